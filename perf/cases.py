@@ -408,3 +408,124 @@ def tolerance(case):
     if k == "prefill":
         return {"rel": 8e-3, "max": 0.15} if c["act_fp8"] else {"rel": 1e-3, "max": 2e-2}
     return {"rel": 5e-3, "max": 5e-2}
+
+
+# ---- the same outputs in 64 bits ---------------------------------------------------------------------------------------------
+def _up(s, b0, b1):
+    return s.double().repeat_interleave(b0, 0).repeat_interleave(b1, 1)
+
+
+def _deq(fmt, w, s=None, zp=None):
+    """A stored matrix as the f64 values its format defines (INT4: W = bf16((u - u_z) s), the checkpoints' own rounding)"""
+    if fmt == "fp8":
+        return w.view(torch.float8_e4m3fn).double() * _up(s, 128, 128)[:w.shape[0]]
+    if fmt == "fp8e":
+        return w.view(torch.float8_e4m3fn).double() * _up(torch.exp2(s.double() - 127.0), 32, 32)
+    if fmt == "int4":
+        sh = torch.arange(8, device=w.device, dtype=torch.int32) * 4
+        u = ((w[..., None] >> sh) & 15).flatten(-2).double()
+        z = ((zp[:, None, :] >> sh[None, :, None]) & 15).flatten(0, 1)
+        return ((u - _up(z, 1, 32)) * _up(s, 1, 32)).to(torch.bfloat16).double()
+    if fmt == "mxfp4":
+        val = torch.tensor([0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0], device=w.device, dtype=torch.float64)
+        code = torch.stack([w & 15, w >> 4], -1).flatten(-2).long()
+        v = val[code & 7] * (1.0 - 2.0 * (code >> 3))
+        return v * _up(torch.exp2(s.double() - 127.0), 1, 32)
+    return w.double()
+
+
+def _experts(c, s):
+    """e -> (gate, up, down) in f64"""
+    H, I = c["H"], c["I"]
+    if c["kind"] in ("dsk", "dsk_prefill"):
+        t = s["keep"]
+        return lambda e: tuple(_deq("mxfp4", t["w" + n][e], t["s" + n][e]) for n in "132")
+    pool, fmt = s["keep"][0], c["fmt"]
+
+    def get(e):
+        at, out = 0, []
+        for N, K in ((I, H), (I, H), (H, I)):
+            o, parts = at, []
+            for shape, dt in {"fp8": [((N, K), torch.uint8), ((N // 128, K // 128), torch.float32)], "bf16": [((N, K), torch.bfloat16)],
+                              "int4": [((N, K // 8), torch.int32), ((N, K // 32), torch.bfloat16), ((N // 8, K // 32), torch.int32)]}[fmt]:
+                n = math.prod(shape) * dt.itemsize
+                parts.append(pool[e, o:o + n].view(dt).view(shape))
+                o += _al256(n)
+            out.append(_deq(fmt, *parts))
+            at += mat_bytes(FMT[fmt], N, K)
+        return out
+    return get
+
+
+def _shared64(c, sh):
+    if c["kind"] in ("dsk", "dsk_prefill"):
+        return tuple(_deq("fp8e", sh["sh_w" + n], sh["sh_s" + n]) for n in "132")
+    if c["fmt"] == "fp8":
+        return tuple(_deq("fp8", q, sc) for q, sc in sh)
+    return sh[0][0::2].double(), sh[0][1::2].double(), sh[1].double()
+
+
+def _route64(logits, topk, scale, softplus):
+    l = logits.double()
+    key = torch.nn.functional.softplus(l).sqrt() if softplus else torch.sigmoid(l)
+    v, idx = key.topk(topk, dim=-1)
+    return idx, v / v.sum(-1, keepdim=True) * scale
+
+
+def _mlp(x, w, limit):
+    g, u = x @ w[0].T, x @ w[1].T
+    if limit:
+        g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+    return (torch.nn.functional.silu(g) * u) @ w[2].T
+
+
+def _moe64(c, x, idx, w, experts, shared, limit=None):
+    """x f64 [T][H] -> the picks' weighted sum, the shared expert's rows"""
+    y = torch.zeros_like(x)
+    for e in idx.unique().tolist():
+        r, k = (idx == e).nonzero(as_tuple=True)
+        y[r] += _mlp(x[r], experts(e), limit) * w[r, k, None]
+    return y, _mlp(x, shared, limit) if shared is not None else None
+
+
+def exact(case, seed):
+    c, s = case, prepare(case, seed)
+    k = c["kind"]
+    mat = lambda segs: _deq(c["fmt"] if segs[0]["fmt"] == FMT[c["fmt"]] else "bf16", segs[0]["w"], segs[0].get("s"), segs[0].get("zp"))
+    if k == "gemv":
+        y = s["x"].double() @ mat(s["segs"]).T
+        return torch.nn.functional.silu(y[:, 0::2]) * y[:, 1::2] if c["out"] == "swiglu" else y
+    if k == "dense":
+        norm = lambda h, w: h * torch.rsqrt((h * h).mean(-1, keepdim=True) + 1e-5) * w.double()
+        o = {"res1": s["res"].double() + s["yr"].double()}
+        o["xn1"] = norm(o["res1"], s["n1"])
+        o["xg"] = o["xn1"] @ mat(s["xproj"]).T
+        o["q"] = o["xg"][:, :c["QL"]] @ mat(s["qb"]).T
+        o["part"] = o["q"] @ mat(s["oproj"]).T
+        o["res2"] = o["res1"] + o["part"]
+        o["xn2"] = norm(o["res2"], s["n2"])
+        o["logits"] = o["xn2"] @ mat(s["router"]).T
+        return {n: o[n] for n in s["out"]}
+    dsk = k in ("dsk", "dsk_prefill")
+    scale = 1.5 if dsk else 1.0 if c["fmt"] == "fp8" else 2.5
+    layers = range(STEP_LAYERS) if k in ("moe", "dsk") else [None]
+    at = lambda v, l: v if l is None else v[l]
+    res = []
+    for l in layers:
+        idx, w = _route64(at(s["logits"], l), c["topk"], scale, dsk)
+        if dsk:
+            x = at(s["xq"], l).view(torch.float8_e4m3fn).double() * _up(torch.exp2(at(s["xs"], l).double() - 127.0), 1, 32)
+        else:
+            x = at(s["x"], l).double()
+        sh = None if not c["shared"] else s["keep"] if dsk else at(s["keep"][2], l)
+        y, ys = _moe64(c, x, idx, w, _experts(c, s), _shared64(c, sh) if c["shared"] else None, 10.0 if dsk else None)
+        res.append((w, y, ys))
+    w, y, ys = [torch.stack(v) if v[0] is not None else None for v in zip(*res)]
+    both = y + ys if ys is not None else y
+    if k == "moe":
+        return [both, ys] if c["shared"] else [both]
+    if k == "dsk":
+        return [both, None, w]
+    if dsk:
+        return [None, w[0], both[0]]
+    return [None, w[0], y[0], ys[0], both[0]] if c["shared"] else [None, w[0], y[0]]
