@@ -59,6 +59,17 @@ struct Shape {
   static constexpr int kLds = kStages * kStageBytes;  // (the epilogues reuse it: UP kPos x 256 B, DOWN 8 x 2 WP KiB)
 };
 
+// The shared expert's side of a launch that holds both its tiles and the routed experts' (k_gemm_mixed): the first `grid`
+// workgroups are its tiles' (grid_of of them, so the others keep their XCDs).
+struct SharedRows {
+  unsigned grid;
+  const uint8_t* aq;
+  const float* as;
+  uint16_t* h;
+  uint8_t* hq;
+  float* hs;
+  float* d;
+};
 struct Args {
   const uint8_t* aq;   // activations, e4m3 [rows][K]
   const float* as;     // their scales [rows][K / 128]
@@ -67,13 +78,14 @@ struct Args {
   const int* tile_m0;
   const int* ntiles;
   const int* off;
-  int nrows;           // shared expert: T
+  int nrows;           // the shared expert's rows: T
   int fast_act;        // UP: SwiGLU by the hardware's exp2 / rcp instead of expf() and the IEEE division
   dsgx_layer_w L;
   uint16_t* h;         // UP: h bf16 [position][I]
   uint8_t* hq;         // UP: h quantised, e4m3 [position][I]
   float* hs;           // UP: its scales [position][I / 128]
   float* d;            // DOWN: f32 [position][H]
+  SharedRows sh;       // k_gemm_mixed: the shared expert's rows in the same launch (grid 0: not in it)
 #ifdef DSGX_PF_TRACE
   unsigned long long* trace;  // (diagnostic build: thread 0's wall-clock stamps, 8 a workgroup)
 #endif
@@ -98,8 +110,8 @@ __host__ __device__ inline unsigned grid_of(int tiles, int NS) {
 // where every tile streams the same weights: 0.241 against 0.250 ms at 8192 rows); else the row groups of one tile (the
 // routed experts' list: 1.63 against 1.75 ms for gate/up).
 template <bool TILE_MINOR>
-__device__ __forceinline__ void task_of(int NS, int& tile, int& ns) {
-  const int x = blockIdx.x % kXcds, j = blockIdx.x / kXcds;
+__device__ __forceinline__ void task_of(int NS, int& tile, int& ns, unsigned wg = blockIdx.x) {
+  const int x = wg % kXcds, j = wg / kXcds;
   const int b = (j / (kMapTiles * kMapNs)) * kXcds + x, i = j % (kMapTiles * kMapNs);
   const int NG = (NS + kMapNs - 1) / kMapNs;
   tile = (b / NG) * kMapTiles + (TILE_MINOR ? i % kMapTiles : i / kMapNs);
@@ -417,7 +429,17 @@ __global__ void __launch_bounds__(kThreads) k_gemm_mixed(Args g) {
   const int NS = UP ? g.L.I / (kWgRows / 2) : g.L.H / kWgRows;
   int tile, ns;
   PF_STAMP(g, 0);
-  task_of<false>(NS, tile, ns);
+  if (blockIdx.x < g.sh.grid) {  // (the same for the whole workgroup)
+    task_of<true>(NS, tile, ns);
+    const int m0 = tile * Shape<2>::kPos, mend = g.nrows;
+    if (ns >= NS || m0 >= mend) return;
+    Args q = g;
+    q.aq = g.sh.aq, q.as = g.sh.as, q.gather = nullptr, q.h = g.sh.h, q.hq = g.sh.hq, q.hs = g.sh.hs, q.d = g.sh.d;
+    if (mend - m0 > Shape<1>::kPos) gemm_tile<UP, 2, DIAG>(q, smem, -1, m0, mend, ns);
+    else gemm_tile<UP, 1, DIAG>(q, smem, -1, m0, mend, ns);
+    return;
+  }
+  task_of<false>(NS, tile, ns, blockIdx.x - g.sh.grid);
   if (ns >= NS || tile >= *g.ntiles) return;
   const int te = g.tile_e[tile], e = te & 0xFFFF;
   const int m0 = g.off[e] + g.tile_m0[tile], mend = g.off[e + 1];

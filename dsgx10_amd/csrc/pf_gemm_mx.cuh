@@ -43,6 +43,14 @@ struct Shape {
   static constexpr int kLds = kStages * kStageBytes;        // (the epilogues reuse it: UP kPos x 256 B, DOWN 8 x 2 WP KiB)
 };
 
+// The shared expert's side of a launch that holds its tiles too (k_gemm_mixed): the first `grid` workgroups are theirs
+struct SharedRows {
+  unsigned grid;
+  const uint8_t *aq, *as, *wa, *sa, *wb, *sb;
+  uint16_t* h;
+  uint8_t *hq, *hs;
+  uint16_t* d;
+};
 struct Args {
   const uint8_t* aq;   // activations, e4m3 [rows][K]
   const uint8_t* as;   // their ue8m0 scales [rows][K / 32]
@@ -61,6 +69,7 @@ struct Args {
   uint8_t* hq;         // UP: h as e4m3 [position][I]
   uint8_t* hs;         // UP: its ue8m0 scales [position][I / 32]
   uint16_t* d;         // DOWN: bf16 [position][H]
+  SharedRows sh;       // (grid 0: the launch holds routed tiles only)
 };
 
 __device__ __forceinline__ int sw4(int r) { return (r >> 2) & 3; }
@@ -359,7 +368,17 @@ __global__ void __launch_bounds__(kThreads) k_gemm_mixed(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int NS = UP ? g.I / (kWgRows / 2) : g.H / kWgRows;
   int tile, ns;
-  pf8::task_of<false>(NS, tile, ns);
+  if (blockIdx.x < g.sh.grid) {  // (the same for the whole workgroup)
+    pf8::task_of<true>(NS, tile, ns);
+    const int m0 = tile * Shape<2, DSGX_FMT_FP8_B32E>::kPos, mend = g.nrows;
+    if (ns >= NS || m0 >= mend) return;
+    Args q = g;
+    q.aq = g.sh.aq, q.as = g.sh.as, q.gather = nullptr, q.posw = nullptr, q.wstride = q.sstride = 0;
+    q.wa = g.sh.wa, q.sa = g.sh.sa, q.wb = g.sh.wb, q.sb = g.sh.sb, q.h = g.sh.h, q.hq = g.sh.hq, q.hs = g.sh.hs, q.d = g.sh.d;
+    gemm_tile<UP, 2, DSGX_FMT_FP8_B32E, DIAG>(q, smem, -1, m0, mend, ns);
+    return;
+  }
+  pf8::task_of<false>(NS, tile, ns, blockIdx.x - g.sh.grid);
   if (ns >= NS || tile >= *g.ntiles) return;
   const int te = g.tile_e[tile], e = te & 0xFFFF;
   const int m0 = g.off[e] + g.tile_m0[tile], mend = g.off[e + 1];

@@ -222,6 +222,21 @@ def test_prefill_tile_order_does_not_change_a_bit():
         _prefill(hl, x, idx, w, T, tile_order=3)
 
 
+@pytest.mark.parametrize("fmt,shared,T", [(abi.FMT_FP8, "fp8", 1), (abi.FMT_FP8, "fp8", 128), (abi.FMT_FP8, "fp8", 129), (abi.FMT_FP8, "fp8", 300)])
+def test_prefill_shared_expert_in_the_routed_launches(fmt, shared, T):
+    """a whole step runs the shared expert's tiles in the routed experts' launches: the bits of its own launches (phase 16)"""
+    H, I, E, topk = 512, 256, 8, 2
+    hl = helpers.make_layer(fmt, H, I, E, topk, 5, seed=33, shared=shared)
+    x, _, idx, w = helpers.rows_and_routing(23, T, H, E, topk, 2.5)
+    yr, ys, _, dl = _prefill(hl, x, idx, w, T)
+    ws, r2, s2 = gpu.empty(lib.prefill_ws_bytes(dl.w, T), 0), gpu.empty(T * H * 4, 0xFF), gpu.empty(T * H * 4, 0xFF)
+    dx, di, dw = gpu.dev(x), gpu.dev(idx), gpu.dev(w)
+    for ph in (1, 2, 4, 8, 16):
+        lib.moe_prefill(dl.w, dx, di, dw, T, ws, r2, s2, phases=ph)
+    assert np.array_equal(gpu.host(r2, np.uint32, (T, H)), yr.view(np.uint32))
+    assert np.array_equal(gpu.host(s2, np.uint32, (T, H)), ys.view(np.uint32))
+
+
 def test_prefill_argument_errors():
     hl = helpers.make_layer(abi.FMT_BF16, 512, 256, 8, 2, 4, seed=1)
     dl = hl.upload()
