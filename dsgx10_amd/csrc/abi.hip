@@ -127,10 +127,13 @@ __global__ void __launch_bounds__(256) k_dequant_int4(const uint32_t* __restrict
   uint32_t* o = reinterpret_cast<uint32_t*>(out + (size_t)n * ld + 32 * g);
   if (hot) {
     const float s = bf16_bits_to_f32(sb), nzs = -((float)uz * s);
+    const I4Group grp = i4_group(s, uz);
+    const bool large = !(fabsf(s) < kI4MaxScale);  // (a lane of its own choice here; the streams decide for a wave)
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       uint32_t p[4];
-      i4x8_to_bf16(w[c], s, nzs, p);
+      if (large) i4x8_to_bf16_any(w[c], s, nzs, p);
+      else i4x8_to_bf16(w[c], grp, p);
 #pragma unroll
       for (int j = 0; j < 4; ++j) o[4 * c + j] = p[j];
     }

@@ -310,17 +310,26 @@ __device__ __forceinline__ void mf_stream(uint8_t* smem, size_t rows_bytes, uint
         }
       }
     } else if constexpr (FMT == DSGX_FMT_INT4_G32) {
+      const float s0 = bf16_bits_to_f32(e.s & 0xFFFFu), s1 = bf16_bits_to_f32(e.s >> 16);
+      auto sums = [&](auto&& decode) {
 #pragma unroll
-      for (int jj = 0; jj < 2; ++jj) {
-        const u32x4_t pc = *reinterpret_cast<const u32x4_t*>(W + rd_off[jj]);
-        const float s = bf16_bits_to_f32(jj ? e.s >> 16 : e.s & 0xFFFFu);
-        const float nzs = -((float)(((jj ? e.z.y : e.z.x) >> zsh) & 15u) * s);
+        for (int jj = 0; jj < 2; ++jj) {
+          const u32x4_t pc = *reinterpret_cast<const u32x4_t*>(W + rd_off[jj]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          uint32_t o[4];
-          i4x8_to_bf16(pc[j], s, nzs, o);
-          acc = mfma(o, 32 * jj + 8 * j, acc);
+          for (int j = 0; j < 4; ++j) {
+            uint32_t o[4];
+            decode(jj, pc[j], o);
+            acc = mfma(o, 32 * jj + 8 * j, acc);
+          }
         }
+      };
+      const uint32_t z0 = (e.z.x >> zsh) & 15u, z1 = (e.z.y >> zsh) & 15u;
+      if (__builtin_expect(i4_any_large(fmaxf(fabsf(s0), fabsf(s1))), 0)) {
+        const float n0 = -((float)z0 * s0), n1 = -((float)z1 * s1);
+        sums([&](int jj, uint32_t w, uint32_t (&o)[4]) { i4x8_to_bf16_any(w, jj ? s1 : s0, jj ? n1 : n0, o); });
+      } else {
+        const I4Group g0 = i4_group(s0, z0), g1 = i4_group(s1, z1);
+        sums([&](int jj, uint32_t w, uint32_t (&o)[4]) { i4x8_to_bf16(w, jj ? g1 : g0, o); });
       }
     } else {
 #pragma unroll

@@ -495,7 +495,7 @@ __global__ void __launch_bounds__(kGemmThreads) k_pf_gemm16(Gemm16Args g) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           uint32_t o[4];
-          i4x8_to_bf16(j == 0 ? w.x : j == 1 ? w.y : j == 2 ? w.z : w.w, sc, nzs, o);
+          i4x8_to_bf16_any(j == 0 ? w.x : j == 1 ? w.y : j == 2 ? w.z : w.w, sc, nzs, o);
           fa[t][j] = u32x4_t{o[0], o[1], o[2], o[3]};
         }
       } else if (F8) {

@@ -154,21 +154,35 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   // landed: with three stages it waits for every load issued so far and issues block kb + 2's; with four, block kb + 2 may
   // still be in flight and it issues block kb + 3's.
   u32x4_t raw[2];
-  float sc[2], nzs[2];
+  I4Group grp[2];
+  uint32_t uz[2];
+  bool large = false;  // (the same in every lane) the opened block holds a scale that i4x8_to_bf16 is not for
   auto open_block = [&](int kb) {  // the lane's raw words, scale and -(zero point * scale) of the wave's two tiles of block kb
     const uint8_t* st = smem + (size_t)(kb % kStages) * kStageBytes;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       raw[t] = *reinterpret_cast<const u32x4_t*>(st + wave * 2048 + t * 1024 + rdw);
-      sc[t] = bf16_bits_to_f32(*reinterpret_cast<const uint16_t*>(st + kStageW + kStageX + wave * 256 + t * 128 + rds));
-      nzs[t] = -((float)((*reinterpret_cast<const uint32_t*>(st + kStageW + kStageX + kStageS + wave * 64 + t * 32 + rdz) >> zsh) & 15u) * sc[t]);
+      uz[t] = (*reinterpret_cast<const uint32_t*>(st + kStageW + kStageX + kStageS + wave * 64 + t * 32 + rdz) >> zsh) & 15u;
+      grp[t] = i4_group(bf16_bits_to_f32(*reinterpret_cast<const uint16_t*>(st + kStageW + kStageX + wave * 256 + t * 128 + rds)), uz[t]);
     }
+    large = i4_any_large(fmaxf(fabsf(grp[0].s), fabsf(grp[1].s)));
   };
   auto piece = [&](u32x4_t (&fa)[2][4], int pc) {  // piece pc = 4 t + j of the opened block
     const int t = pc >> 2, j = pc & 3;
     uint32_t o[4];
-    i4x8_to_bf16(j == 0 ? raw[t].x : j == 1 ? raw[t].y : j == 2 ? raw[t].z : raw[t].w, sc[t], nzs[t], o);
+    i4x8_to_bf16(j == 0 ? raw[t].x : j == 1 ? raw[t].y : j == 2 ? raw[t].z : raw[t].w, grp[t], o);
     fa[t][j] = u32x4_t{o[0], o[1], o[2], o[3]};
+  };
+  // a block with a scale of 2^116 or more (none in a checkpoint): its pieces once more, by the routine for every scale
+  auto redo = [&](u32x4_t (&fa)[2][4]) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        uint32_t o[4];
+        i4x8_to_bf16_any(j == 0 ? raw[t].x : j == 1 ? raw[t].y : j == 2 ? raw[t].z : raw[t].w, grp[t].s, -((float)uz[t] * grp[t].s), o);
+        fa[t][j] = u32x4_t{o[0], o[1], o[2], o[3]};
+      }
   };
   auto run = [&](auto nj_c) {
     constexpr int NJ = decltype(nj_c)::value;
@@ -180,6 +194,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
     open_block(0);
 #pragma unroll
     for (int pc = 0; pc < 8; ++pc) piece(fa, pc);
+    if (__builtin_expect(large, 0)) redo(fa);
     auto turn = [&](int kb, u32x4_t (&fa)[2][4], u32x4_t (&fn)[2][4]) {
       // block kb + 1 has landed (four stages: block kb + 2 may be in flight)
       if (brings_x) wait_loads<(kStages - 3) * kLoads>();
@@ -204,6 +219,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
           for (int t = 0; t < 2; ++t)
             acc[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf_t, fa[t][j]), __builtin_bit_cast(v8bf_t, fb[j]), acc[t][mt], 0, 0, 0);
       }
+      if (__builtin_expect(large, 0)) redo(fn);
     };
     for (int kb = 0; kb < KB; kb += 2) {  // (two turns a pass: the two fragment buffers swap roles without copies)
       turn(kb, fa, fn);

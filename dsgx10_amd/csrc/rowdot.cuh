@@ -168,7 +168,7 @@ __device__ __forceinline__ void step_dot(const Raw (&raw_in)[RB], const uint4* _
       for (int r = 0; r < RB; ++r) {
         const uint32_t w = c == 0 ? raw[r].v.x : c == 1 ? raw[r].v.y : c == 2 ? raw[r].v.z : raw[r].v.w;
         uint32_t o[4];
-        i4x8_to_bf16(w, s[r], nzs[r], o);
+        i4x8_to_bf16_any(w, s[r], nzs[r], o);
 #pragma unroll
         for (int m = 0; m < M; ++m) {
           float t = acc[r][m];
