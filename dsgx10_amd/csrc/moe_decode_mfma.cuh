@@ -191,23 +191,24 @@ __device__ __forceinline__ void mf_stream(uint8_t* smem, size_t rows_bytes, uint
   uint8_t* W = smem + rows_bytes + wave * 2048;  // one step's weights: 16 rows x 128 bytes
   const size_t rs = (size_t)K * 2 + pad;
   // LDS offsets. The row-major writes stay whole 128-byte rows; a row's eight 16-byte pieces are exchanged so that the
-  // MFMA-order reads (16 lanes: 16 rows, one k part) touch every bank once: by (row / 2) % 8 for FP8's reads of 8 bytes,
-  // by row % 8 for the reads of 16 bytes.
+  // MFMA-order reads touch every bank once: by (row / 2) % 8 for FP8's reads of 8 bytes, by row % 8 for BF16's pieces part and
+  // 4 + part, by row % 8 ^ row / 8 for the formats whose lane takes pieces 2 part and 2 part + 1 (a 16-byte read is served
+  // rows 0-3 and 12-15 of one k part with rows 4-11 of the next: row % 8 alone put two of those lanes on a bank).
   constexpr bool F8 = FMT == DSGX_FMT_FP8_B128 || FMT == DSGX_FMT_FP8_B32E;   // 8-byte fragment reads, four MFMAs a 128-k step
   constexpr bool G32 = FMT == DSGX_FMT_INT4_G32 || FMT == DSGX_FMT_MXFP4_G32;  // a lane's 16 bytes = one scale group of 32 values
-  constexpr int RSH = F8 ? 1 : 0;
+  auto row_x = [](int r) { return F8 ? (r >> 1) & 7 : G32 ? (r & 7) ^ (r >> 3) : r & 7; };
   int wr_off[2], rd_off[F8 ? 4 : 2];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) wr_off[h] = (8 * h + r8) * 128 + ((q ^ (((8 * h + r8) >> RSH) & 7)) * 16);
+  for (int h = 0; h < 2; ++h) wr_off[h] = (8 * h + r8) * 128 + ((q ^ row_x(8 * h + r8)) * 16);
   if constexpr (F8) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) rd_off[j] = r16 * 128 + (((2 * j + (part >> 1)) ^ ((r16 >> 1) & 7)) * 16) + 8 * (part & 1);
+    for (int j = 0; j < 4; ++j) rd_off[j] = r16 * 128 + (((2 * j + (part >> 1)) ^ row_x(r16)) * 16) + 8 * (part & 1);
   } else if constexpr (G32) {  // pieces 2 part, 2 part + 1: two scale groups
 #pragma unroll
-    for (int j = 0; j < 2; ++j) rd_off[j] = r16 * 128 + (((2 * part + j) ^ (r16 & 7)) * 16);
+    for (int j = 0; j < 2; ++j) rd_off[j] = r16 * 128 + (((2 * part + j) ^ row_x(r16)) * 16);
   } else {  // pieces part, 4 + part: the lane's 8 k of the step's two MFMAs
 #pragma unroll
-    for (int j = 0; j < 2; ++j) rd_off[j] = r16 * 128 + (((4 * j + part) ^ (r16 & 7)) * 16);
+    for (int j = 0; j < 2; ++j) rd_off[j] = r16 * 128 + (((4 * j + part) ^ row_x(r16)) * 16);
   }
   const bool live = r16 < M;  // positions beyond the step's rows read the zero bytes
   // the lane's activations: row r16 from k0 + (FP8, BF16: 8 part; INT4: 64 part)

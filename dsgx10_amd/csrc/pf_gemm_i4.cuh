@@ -6,12 +6,12 @@
 // channels, gate and up), a wave 32 rows x every position; both operands and the weights' scales and zero points go from
 // memory straight into a stage of LDS (global_load_lds, three stages of one 128-k block, hand-counted waits, one workgroup
 // barrier a block), a turn's loads are issued one at a time between its MFMAs. What is its own:
-//   * a weight row of a block is 64 bytes of packed nibbles (four lanes a row, piece q of row r at slot q ^ (r / 4 % 4));
+//   * a weight row of a block is 64 bytes of packed nibbles (four lanes a row, piece q of row r at slot q ^ sw4(r));
 //     lane (row, part) reads ONE piece = the 32 values of one scale group, its bf16 scale and its zero-point word, decodes
 //     them in registers (the decode kernels' routine: one rounding of the exact product) into the A fragments of four MFMAs;
 //     MFMA j takes the lane's values 8 j .. 8 j + 7, i.e. k = 32 part + 8 j + [0, 8), and the activation fragment of MFMA j
 //     holds the same k (the permutation of k inside a block is invisible to the sums);
-//   * an activation row of a block is 256 bytes of bf16: sixteen 16-byte pieces, piece c of position r at slot c ^ r, four
+//   * an activation row of a block is 256 bytes of bf16: sixteen 16-byte pieces, piece c of position r at slot c ^ sw16(r), four
 //     instructions a 16-position tile; a lane's piece for MFMA j is 4 part + j;
 //   * a block's weights are decoded a turn ahead, between the MFMAs of the block before: vector unit and matrix unit run
 //     beside each other.
@@ -62,7 +62,14 @@ struct Args {
   float* d;            // DOWN: f32 [position][H]
 };
 
-__device__ __forceinline__ int sw4(int r) { return (r >> 2) & 3; }
+// Where piece q of a row lies. A 16-byte LDS read of 64 lanes is served sixteen lanes at a time, and the sixteen are lanes
+// 0-3, 12-15, 20-27 (and 4-11, 16-19, 28-31; the same from 32 on): rows 0-3 and 12-15 of one k part beside rows 4-11 of the
+// next. Slots q ^ (r / 4 % 4) (64-byte rows) and c ^ r (256-byte rows), one-to-one on sixteen neighbouring rows, put two lanes
+// of such a set on every bank (a loop of these reads: 427 us, 222 with the slots below; gate/up's LDS cycles were half
+// conflicts). sw4 takes rows 0-3, 4-7, 8-11, 12-15 to 0, 2, 3, 1 and sw16 exchanges rows 4-7 and 12-15: one-to-one on both
+// kinds of sixteen.
+__device__ __forceinline__ int sw4(int r) { return (((r >> 2) ^ (r >> 3)) & 1) << 1 | ((r >> 3) & 1); }
+__device__ __forceinline__ int sw16(int r) { return r ^ ((r & 4) << 1); }
 
 template <bool UP, int POS>
 __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, int m0, int mend, int ns) {
@@ -103,13 +110,13 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
     const int rowz = tile_row(tz, base);
     pzp = base + zoff + ((size_t)((rowz >> 3) + oz) * G + (lane & 3)) * 4;
   }
-  const uint8_t* px[4];   // activations: the wave brings 16-position tile `wave`; instruction i: position 4 i + lane / 16, piece (lane % 16) ^ position
+  const uint8_t* px[4];   // activations: the wave brings 16-position tile `wave`; instruction i: position 4 i + lane / 16, piece (lane % 16) ^ sw16(position)
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = 4 * i + (lane >> 4);
     int pos = m0 + 16 * wave + r;
     if (pos >= mend) pos = mend - 1;  // a ragged tile re-reads its last row (never stored)
-    px[i] = reinterpret_cast<const uint8_t*>(g.x) + (size_t)(g.gather ? g.gather[pos] : pos) * K * 2 + 16 * ((lane & 15) ^ r);
+    px[i] = reinterpret_cast<const uint8_t*>(g.x) + (size_t)(g.gather ? g.gather[pos] : pos) * K * 2 + 16 * ((lane & 15) ^ sw16(r));
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
   // load number i of block kb (clamped past the end: the last block again, into a stage nobody reads): the small ones first,
@@ -140,7 +147,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   const uint32_t zsh = 4 * (r16 & 7);
   int rdx[4];                                         // the activation piece of MFMA j: 4 part + j of position r16
 #pragma unroll
-  for (int j = 0; j < 4; ++j) rdx[j] = r16 * 256 + (((4 * part + j) ^ r16) & 15) * 16;
+  for (int j = 0; j < 4; ++j) rdx[j] = r16 * 256 + ((4 * part + j) ^ sw16(r16)) * 16;
 
   v4f_t acc[2][8];
 #pragma unroll

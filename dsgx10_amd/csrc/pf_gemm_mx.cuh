@@ -8,7 +8,7 @@
 //
 // The tiling, the LDS staging by global_load_lds (lane-permuted sources so that the fragment reads are conflict-free),
 // the hand-counted waits and the workgroup -> (tile, row group) map are those of pf_gemm_fp8.cuh; what differs:
-//   * a weight row of a 128-k block is 64 bytes (e2m1) - four lanes a row, piece q of row r at slot q ^ (r / 4 % 4);
+//   * a weight row of a 128-k block is 64 bytes (e2m1) - four lanes a row, piece q of row r at slot q ^ sw4(r);
 //   * the scales travel with the block: 4 bytes a weight row and 4 a position, read back a byte a lane (ds_read_u8);
 //   * UP's epilogue is DeepSeek's: gate, up rounded to bf16, up clamped to +-limit and gate from above, silu(gate) * up
 //     times the position's routing weight (none for the shared expert), rounded to bf16, then quantised per 32 channels
@@ -72,7 +72,8 @@ struct Args {
   SharedRows sh;       // (grid 0: the launch holds routed tiles only)
 };
 
-__device__ __forceinline__ int sw4(int r) { return (r >> 2) & 3; }
+// (the slot of a 64-byte row's piece: one-to-one on the rows whose lanes the LDS serves together, see pf_gemm_i4.cuh's sw4)
+__device__ __forceinline__ int sw4(int r) { return (((r >> 2) ^ (r >> 3)) & 1) << 1 | ((r >> 3) & 1); }
 // 128-byte rows (activations, e4m3 weights) lie in LDS in pf_gemm_fp8.cuh's layout, whose fragment reads (a lane's two
 // neighbouring slots 2 part, 2 part + 1, swizzled by row) run without bank conflicts; what differs is WHICH 16 bytes of the
 // row a slot holds: the block-scaled instruction wants bytes 16 part ... and 64 + 16 part ... in a lane, so logical piece
