@@ -48,18 +48,28 @@ __device__ __forceinline__ void stage_rows(uint4* xs, const GemvArgs& a, float* 
                  });
 }
 
-template <int FMT, int M, int RB, int D>
-__global__ void __launch_bounds__(256) k_gemv(GemvArgs a) {
+// NW: wavefronts a workgroup, in groups of four: the first batches of the walk go to every workgroup's first group, so that
+// fewer batches than wavefronts still spread over all CUs. SPLIT: the split-K order of adds (k_gemv_sk's slices, in their
+// order, the same bits) by one wavefront that walks the slices one after the other.
+// Bound by the vector unit (INT4, or from 3 activation rows) or by latency: eight wavefronts a CU in ONE workgroup stage the
+// activations once a CU and keep two wavefronts a SIMD where 64 KB and more of activations left room for one workgroup of
+// four (INT4 6144 x 16384, 4 rows: 36.1 us with four waves, 27.1 with eight, 29.6 with sixteen; FP8 12000 x 8192, 8 rows:
+// 41.6, 33.8, 52.5). Two rows a wavefront: four leave half the waves without a batch or make a longer last round (INT4
+// 16384 x 2048, 1 row: 13.4 against 10.6).
+template <int FMT, int M, int RB, int D, int NW, bool SPLIT>
+__global__ void __launch_bounds__(NW * 64) k_gemv(GemvArgs a) {
   extern __shared__ uint4 xs[];
   __shared__ float red[4];
   const int lane = threadIdx.x & 63;
   // (the wave's number is the same in every lane: said so, which keeps the row cursors and the segment's descriptor on the
   // scalar unit - read from a vector register they came through vector loads of the kernel's arguments, which a wave's
   // weight loads then queued behind, one ring entry after the other)
-  const int gw = uni(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)), GW = gridDim.x * (blockDim.x >> 6);
+  const int wave = uni(threadIdx.x >> 6);
+  const int gw = uni((wave >> 2) * (int)gridDim.x * 4 + (int)blockIdx.x * 4 + (wave & 3)), GW = gridDim.x * NW;
   const int nbatch = a.total_rows / RB;
   const int nmine = gw < nbatch ? (nbatch - gw + GW - 1) / GW : 0;
   const int nsteps = nmine * a.nsegk;
+  const int sk = SPLIT ? a.splitk : 1, slices = SPLIT ? min(sk, a.nsegk) : 1;  // the K slices of a row, and those that hold a segment
 
   auto locate = [&](int row, int& si) {
     si = 0;
@@ -82,7 +92,7 @@ __global__ void __launch_bounds__(256) k_gemv(GemvArgs a) {
     if (a.nsegs > 1) locate(row, si);
     dummy = a.sg[si].m.w + (size_t)(row - a.sg[si].row0) * FmtT<FMT>::row_bytes(a.K);
   }
-  int lt = 0, lj = 0, lseg = 0;  // the load cursor: step, batch number of this wave, segment
+  int lt = 0, lj = 0, lsl = 0, lseg = 0;  // the load cursor: step, batch number of this wave, slice, segment
   // the matrix of the batch under the load cursor and the batch's first row in it: fetched from the kernel's arguments when
   // the cursor enters a batch, not at every step (scalar loads, but each is a wait in front of the step's weight loads)
   // (a call with one segment, the common one, fetches once: every later fetch would be two dependent scalar round trips)
@@ -104,29 +114,34 @@ __global__ void __launch_bounds__(256) k_gemv(GemvArgs a) {
     ++lt;
 #pragma unroll
     for (int i = 0; i < RB; ++i) load_raw<FMT, true>(r[i], lm, lrow + i, lseg, lane, a.K, acc[i][0], ok ? nullptr : dummy);
-    if (ok && ++lseg == a.nsegk) {
-      lseg = 0, ++lj;
-      enter();
+    if (ok && (lseg += sk) >= a.nsegk) {
+      if (++lsl == slices) lsl = 0, ++lj, enter();
+      lseg = lsl;
     }
   };
-  int cj = 0, cseg = 0;
+  int cj = 0, csl = 0, cseg = 0;
+  float mine = 0.f, mine2 = 0.f;  // lane r * M + m: output (row r, activation row m) of the batch, and the pair's other row (SwiGLU)
   auto compute = [&](const Raw (&raw)[RB]) {
     step_dot<FMT, M, RB, true>(raw, xs, a.nq, cseg, lane, acc, a.K);
-    if (++cseg < a.nsegk) return;
-    cseg = 0;
-    // the batch is complete: add the lanes' partials, lane r * M + m keeps output (row r, activation row m)
-    const int row = (gw + cj * GW) * RB;
-    ++cj;
-    float mine = 0.f, mine2 = 0.f;
+    if ((cseg += sk) < a.nsegk) return;
+    // the slice is complete: add the lanes' partials, then the slices' sums in their order
+    float v1 = 0.f, v2 = 0.f;
 #pragma unroll
     for (int i = 0; i < RB; ++i)
 #pragma unroll
       for (int m = 0; m < M; ++m) {
         const float v = wave_sum(acc[i][m]);
         acc[i][m] = 0.f;
-        if (lane == i * M + m) mine = v;
-        if (lane == (i ^ 1) * M + m) mine2 = v;  // the pair's other row (SwiGLU)
+        if (lane == i * M + m) v1 = v;
+        if (lane == (i ^ 1) * M + m) v2 = v;
       }
+    mine = SPLIT && csl ? __fadd_rn(mine, v1) : v1, mine2 = SPLIT && csl ? __fadd_rn(mine2, v2) : v2;
+    cseg = ++csl;
+    if (SPLIT && csl < slices) return;
+    if (SPLIT && slices < sk) mine = __fadd_rn(mine, 0.f), mine2 = __fadd_rn(mine2, 0.f);  // (an empty slice's sum, as k_gemv_sk adds it)
+    csl = cseg = 0;
+    const int row = (gw + cj * GW) * RB;
+    ++cj;
     if (lane >= RB * M) return;
     int si = 0;
     if (a.nsegs > 1) locate(row, si);
@@ -159,7 +174,8 @@ __global__ void __launch_bounds__(256) k_gemv(GemvArgs a) {
 // four waves holds 4 / SK row batches, the SK waves of a batch take the K segments slice, slice + SK, ... of its rows;
 // the waves' sums meet in LDS and the batch's first wave adds them in slice order (a fixed order, as the reference's
 // finish(), gemv.cu:138-151), then the epilogue of k_gemv. One batch a group and launch: this form is for matrices of
-// few rows, where whole-K waves would leave most of the chip idle and walk K in several dependent round trips.
+// few rows, where whole-K waves would leave most of the chip idle and walk K in several dependent round trips; the others
+// take the same slices one after the other in k_gemv.
 template <int FMT, int M, int RB, int SK>
 __global__ void __launch_bounds__(256) k_gemv_sk(GemvArgs a) {
   extern __shared__ uint4 xs[];
@@ -246,44 +262,57 @@ int launch_gemv_sk(const GemvArgs& a, hipStream_t st) {
   return DSGX_OK;
 }
 
-template <int FMT, int M, int RB>
-int launch_gemv(const GemvArgs& a, hipStream_t st) {
-  constexpr int D = 4;
+template <int FMT, int M, int NW, bool SPLIT>
+int launch_gemv_nw(const GemvArgs& a, hipStream_t st) {
+  constexpr int RB = 2, D = 4;
   const size_t lds = (size_t)M * a.nq * 16;
   const int nbatch = a.total_rows / RB;
-  // two workgroups of four wavefronts a CU when the activations leave room in LDS, never more workgroups than batches
-  const int per_cu = lds <= 64 * 1024 ? 2 : 1;
+  // never more workgroups than it takes to give every group of four wavefronts a batch
+  const int per_cu = NW == 4 && lds <= 64 * 1024 ? 2 : 1;
   int grid = num_cus_cached() * per_cu;
   if (grid > (nbatch + 3) / 4) grid = (nbatch + 3) / 4;
   if (grid < 1) grid = 1;
-  auto kern = k_gemv<FMT, M, RB, D>;
+  auto kern = k_gemv<FMT, M, RB, D, NW, SPLIT>;
   if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, st, a);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(NW * 64), lds, st, a);
   DSGX_HIP(hipGetLastError());
   return DSGX_OK;
 }
+template <int FMT, int M, int NW>
+int launch_gemv(const GemvArgs& a, hipStream_t st) {
+  return a.splitk > 1 ? launch_gemv_nw<FMT, M, NW, true>(a, st) : launch_gemv_nw<FMT, M, NW, false>(a, st);
+}
 template <int FMT, int M>
-int launch_gemv_rb(const GemvArgs& a, hipStream_t st) {
-  // split-K as asked for, where the rows are few enough for one batch a wave group and launch
-  if (a.splitk > 1 && a.total_rows / 2 <= 16 * num_cus_cached()) {
+int launch_gemv_rows(const GemvArgs& a, hipStream_t st) {
+  const int nbatch = a.total_rows / 2, cus = num_cus_cached();
+  // Slices on waves of their own (k_gemv_sk) only where the matrix is too small for the chip without: every workgroup of
+  // it stages all activation rows. BF16 256 x 4096 over 4, 3 rows: 4.7 us, 6.5 by one wave a batch; INT4 6144 x 16384 over
+  // 4, 4 rows: 126 and 27; FP8 2048 x 4096 over 4, 1 row: 8.8 and 5.8; BF16 1000 x 7168 over 4, 1 row: 6.3 and 7.8 (many
+  // segments a slice); BF16 2112 x 4096 over 2, 1 row: 6.8 and 7.0, 3 rows: 9.7 and 7.9.
+  const int waves = nbatch * a.splitk;
+  const bool few = waves <= 4 * cus || (nbatch <= 2 * cus && a.nsegk >= 3 * a.splitk && (size_t)M * a.nq * 16 <= 64 * 1024) ||
+                   (M == 1 && waves <= 12 * cus && a.nsegk >= 4 * a.splitk);
+  if (a.splitk > 1 && few) {
     if (a.splitk == 2) return launch_gemv_sk<FMT, M, 2>(a, st);
     return launch_gemv_sk<FMT, M, 4>(a, st);
   }
-  // few rows: two rows a wavefront so that every wavefront of the launch (two workgroups of four a CU) has rows to stream
-  if (a.total_rows / 4 < 2 * 8 * num_cus_cached()) return launch_gemv<FMT, M, 2>(a, st);
-  return launch_gemv<FMT, M, 4>(a, st);
+  // Two workgroups of four a CU where the add + norm prologue is 256 threads' work, and where a wave has one batch at most:
+  // at one row, or with few batches (BF16 1000 x 7168, 2 rows: 8.1 us, 9.0 with eight a workgroup;
+  // INT4 1536 x 6144, 4 rows: 9.2 and 8.3).
+  if (a.norm.part || nbatch < 3 * cus || (M == 1 && nbatch <= 8 * cus)) return launch_gemv<FMT, M, 4>(a, st);
+  return launch_gemv<FMT, M, 8>(a, st);
 }
 template <int FMT>
 int launch_gemv_m(int M, const GemvArgs& a, hipStream_t st) {
   switch (M) {
-    case 1: return launch_gemv_rb<FMT, 1>(a, st);
-    case 2: return launch_gemv_rb<FMT, 2>(a, st);
-    case 3: return launch_gemv_rb<FMT, 3>(a, st);
-    case 4: return launch_gemv_rb<FMT, 4>(a, st);
-    case 5: return launch_gemv_rb<FMT, 5>(a, st);
-    case 6: return launch_gemv_rb<FMT, 6>(a, st);
-    case 7: return launch_gemv_rb<FMT, 7>(a, st);
-    case 8: return launch_gemv_rb<FMT, 8>(a, st);
+    case 1: return launch_gemv_rows<FMT, 1>(a, st);
+    case 2: return launch_gemv_rows<FMT, 2>(a, st);
+    case 3: return launch_gemv_rows<FMT, 3>(a, st);
+    case 4: return launch_gemv_rows<FMT, 4>(a, st);
+    case 5: return launch_gemv_rows<FMT, 5>(a, st);
+    case 6: return launch_gemv_rows<FMT, 6>(a, st);
+    case 7: return launch_gemv_rows<FMT, 7>(a, st);
+    case 8: return launch_gemv_rows<FMT, 8>(a, st);
   }
   return fail(DSGX_EINVAL, "gemv: %d rows a launch", M);
 }

@@ -222,3 +222,20 @@ def test_add_norm(H, mode):
     r2 = gpu.dev(res)
     lib.add_norm(gpu.dev(part), None if part2 is None else gpu.dev(part2), M, H, r2, r2, None, 1e-5, None, round2=mode == "round2")
     assert np.array_equal(gpu.host(r2, np.uint16, (M, H)), o_ro)
+
+
+@pytest.mark.parametrize("splitk", [1, 2, 4])
+@pytest.mark.parametrize("M", [1, 3, 8])
+@pytest.mark.parametrize("N", [1528, 1544, 4104, 6200])
+def test_a_row_does_not_depend_on_the_matrix_it_stands_in(N, M, splitk):
+    """Few rows, a wave a slice; more, one wave for all slices; from 1536 rows eight waves a workgroup, several batches a wave:
+    the same order of adds, so the same bits (K of five segments, the last one partial; SwiGLU pairs as well)"""
+    K = 2048 + 256
+    x = orc.normal_bf16(M, 1, (M, K), 1.0)
+    w = orc.normal_bf16(0, 4, (N, K), 0.02)
+    for out in (abi.OUT_F32, abi.OUT_SWIGLU):
+        y = _run(x, abi.FMT_BF16, (w,), N, K, out, splitk=splitk)
+        for r0 in (0, N // 2 // 8 * 8, N - 64):
+            part = _run(x, abi.FMT_BF16, (w[r0:r0 + 64].copy(),), 64, K, out, splitk=splitk)
+            c0, c1 = (r0, r0 + 64) if out == abi.OUT_F32 else (r0 // 2, r0 // 2 + 32)
+            assert np.array_equal(y[:, c0:c1], part)
