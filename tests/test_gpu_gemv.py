@@ -239,3 +239,22 @@ def test_a_row_does_not_depend_on_the_matrix_it_stands_in(N, M, splitk):
             part = _run(x, abi.FMT_BF16, (w[r0:r0 + 64].copy(),), 64, K, out, splitk=splitk)
             c0, c1 = (r0, r0 + 64) if out == abi.OUT_F32 else (r0 // 2, r0 // 2 + 32)
             assert np.array_equal(y[:, c0:c1], part)
+
+
+@pytest.mark.parametrize("fmt,K", [(abi.FMT_FP8, 4096 + 128), (abi.FMT_INT4, 4096 + 256), (abi.FMT_BF16, 2048 + 256)])
+def test_split_k_is_ignored_above_32_rows_a_cu(fmt, K):
+    """dsgx.h: from 32 rows a CU on every split adds as splitk 1 does; up to there the slices' order, that of a small matrix"""
+    import torch
+    lim = 32 * torch.cuda.get_device_properties(0).multi_processor_count
+    N, M = lim + 8, 3
+    x = orc.normal_bf16(17, 1, (M, K), 1.0)
+    parts = {abi.FMT_FP8: lambda: orc.fp8_random(17, N, K, 1.0 / 256), abi.FMT_INT4: lambda: orc.int4_random(17, N, K),
+             abi.FMT_BF16: lambda: (orc.normal_bf16(17, 4, (N, K), 0.02),)}[fmt]()
+    whole = _run(x, fmt, parts, N, K, abi.OUT_F32)
+    for sk in (2, 4):
+        assert np.array_equal(_run(x, fmt, parts, N, K, abi.OUT_F32, splitk=sk), whole)
+        # (INT4 zero points are packed over 8 rows: an eighth of the rows; the FP8 scales of the first `lim` rows are those of the large matrix)
+        first = lambda n: [p[:(-(-n * p.shape[0] // N) if fmt == abi.FMT_INT4 else n if i == 0 else -(-n // 128))].copy() for i, p in enumerate(parts)]
+        at = _run(x, fmt, first(lim), lim, K, abi.OUT_F32, splitk=sk)
+        assert np.array_equal(at[:, :64], _run(x, fmt, first(64), 64, K, abi.OUT_F32, splitk=sk))
+        assert not np.array_equal(at, whole[:, :lim])
