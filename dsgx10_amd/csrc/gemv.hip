@@ -30,9 +30,10 @@ struct GemvArgs {
 // The activation rows into LDS: from x, or (fused add + norm) computed by this workgroup from the partial sums and the
 // residual - every workgroup makes all M rows for itself (M H values: a few KB from L2), workgroup 0 also writes the new
 // residual and the normed rows to memory for the kernels that follow.
-template <int KL, int M>
+// (add_norm_row is 256 threads' work: a workgroup of another size, NORM false, has no code for it.)
+template <int KL, int M, bool NORM>
 __device__ __forceinline__ void stage_rows(uint4* xs, const GemvArgs& a, float* red) {
-  if (!a.norm.part) {
+  if (!NORM || !a.norm.part) {
     stage_x<KL>(xs, a.x, a.ldx, M, a.K, a.nq * 8);
     return;
   }
@@ -159,7 +160,7 @@ __global__ void __launch_bounds__(NW * 64) k_gemv(GemvArgs a) {
   // first product (these calls are a few microseconds long: latency is most of them)
 #pragma unroll
   for (int d = 0; d < D; ++d) load(w[d]);
-  stage_rows<FmtT<FMT>::KL, M>(xs, a, red);
+  stage_rows<FmtT<FMT>::KL, M, NW == 4>(xs, a, red);
   __syncthreads();
   for (int t = 0; t < nsteps; t += D) {
 #pragma unroll
@@ -213,7 +214,7 @@ __global__ void __launch_bounds__(256) k_gemv_sk(GemvArgs a) {
   };
 #pragma unroll
   for (int d = 0; d < D; ++d) load(w[d]);
-  stage_rows<FmtT<FMT>::KL, M>(xs, a, red);
+  stage_rows<FmtT<FMT>::KL, M, true>(xs, a, red);
   __syncthreads();
   for (int t = 0; t < nmine; t += D) {
 #pragma unroll
@@ -265,6 +266,7 @@ int launch_gemv_sk(const GemvArgs& a, hipStream_t st) {
 template <int FMT, int M, int NW, bool SPLIT>
 int launch_gemv_nw(const GemvArgs& a, hipStream_t st) {
   constexpr int RB = 2, D = 4;
+  if (NW != 4 && a.norm.part) return fail(DSGX_EINVAL, "gemv: the add + norm prologue runs in workgroups of four wavefronts");
   const size_t lds = (size_t)M * a.nq * 16;
   const int nbatch = a.total_rows / RB;
   // never more workgroups than it takes to give every group of four wavefronts a batch

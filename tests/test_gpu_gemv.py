@@ -258,3 +258,22 @@ def test_split_k_is_ignored_above_32_rows_a_cu(fmt, K):
         at = _run(x, fmt, first(lim), lim, K, abi.OUT_F32, splitk=sk)
         assert np.array_equal(at[:, :64], _run(x, fmt, first(64), 64, K, abi.OUT_F32, splitk=sk))
         assert not np.array_equal(at, whole[:, :lim])
+
+
+@pytest.mark.parametrize("splitk", [1, 2, 4])
+@pytest.mark.parametrize("fmt,N,M", [(abi.FMT_BF16, 64, 2), (abi.FMT_BF16, 2312, 3), (abi.FMT_FP8, 2312, 8), (abi.FMT_INT4, 2312, 1), (abi.FMT_INT4, 6152, 8)])
+def test_add_norm_gemv_at_every_size_of_matrix(fmt, N, M, splitk):
+    """The add + norm prologue (256 threads' work) in a GEMV whose plain form runs in workgroups of eight waves too: the bits of
+    dsgx_add_norm followed by dsgx_gemv, the rows it writes included"""
+    K = 2048
+    part, res, w = orc.normal_f32(19, 1, (M, K), 0.7), orc.normal_bf16(19, 3, (M, K), 1.5), orc.normal_bf16(19, 4, (K,), 1.0)
+    parts = {abi.FMT_FP8: lambda: orc.fp8_random(19, N, K, 1.0 / 256), abi.FMT_INT4: lambda: orc.int4_random(19, N, K),
+             abi.FMT_BF16: lambda: (orc.normal_bf16(19, 5, (N, K), 0.02),)}[fmt]()
+    dp, dr, dw, keep = gpu.dev(part), gpu.dev(res), gpu.dev(w), [gpu.dev(p) for p in parts]
+    ro, xn, y = [gpu.empty(M * K * 2, 0xFF) for _ in range(2)], [gpu.empty(M * K * 2, 0xFF) for _ in range(2)], [gpu.empty(M * N * 4, 0xFF) for _ in range(2)]
+    seg = [dict(fmt=fmt, w=keep[0], s=keep[1] if len(keep) > 1 else None, zp=keep[2] if len(keep) > 2 else None, n=N, y=v, ldy=N) for v in y]
+    lib.add_norm_gemv(dp, None, dr, ro[0], dw, 1e-5, xn[0], M, K, [seg[0]], abi.OUT_F32, splitk=splitk)
+    lib.add_norm(dp, None, M, K, dr, ro[1], dw, 1e-5, xn[1])
+    lib.gemv(xn[1], K, M, K, [seg[1]], abi.OUT_F32, splitk=splitk)
+    for a, b in (ro, xn, y):
+        assert np.array_equal(gpu.host(a, np.uint8, (-1,)), gpu.host(b, np.uint8, (-1,)))
