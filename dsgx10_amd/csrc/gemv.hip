@@ -286,22 +286,31 @@ int launch_gemv(const GemvArgs& a, hipStream_t st) {
 }
 template <int FMT, int M>
 int launch_gemv_rows(const GemvArgs& a, hipStream_t st) {
-  const int nbatch = a.total_rows / 2, cus = num_cus_cached();
-  // Slices on waves of their own (k_gemv_sk) only where the matrix is too small for the chip without: every workgroup of
-  // it stages all activation rows. BF16 256 x 4096 over 4, 3 rows: 4.7 us, 6.5 by one wave a batch; INT4 6144 x 16384 over
-  // 4, 4 rows: 126 and 27; FP8 2048 x 4096 over 4, 1 row: 8.8 and 5.8; BF16 1000 x 7168 over 4, 1 row: 6.3 and 7.8 (many
-  // segments a slice); BF16 2112 x 4096 over 2, 1 row: 6.8 and 7.0, 3 rows: 9.7 and 7.9.
-  const int waves = nbatch * a.splitk;
-  const bool few = waves <= 4 * cus || (nbatch <= 2 * cus && a.nsegk >= 3 * a.splitk && (size_t)M * a.nq * 16 <= 64 * 1024) ||
-                   (M == 1 && waves <= 12 * cus && a.nsegk >= 4 * a.splitk);
-  if (a.splitk > 1 && few) {
-    if (a.splitk == 2) return launch_gemv_sk<FMT, M, 2>(a, st);
-    return launch_gemv_sk<FMT, M, 4>(a, st);
+  const int nbatch = a.total_rows / 2, cus = num_cus_cached(), sk = a.splitk;
+  constexpr bool kBf16 = FMT == DSGX_FMT_BF16;
+  const size_t lds = (size_t)M * a.nq * 16;
+  // Slices on waves of their own (k_gemv_sk): a workgroup stages all activation rows for 4 / sk batches, so what counts is how
+  // many of its workgroups a CU holds at once. (us below: own waves / one wave walking the slices in k_gemv)
+  //   one a CU: always (BF16 1000 x 4096 over 2, 8 rows: 8.1 / 9.5; FP8 384 x 2048 over 4, 1 row: 4.4 / 4.6);
+  //   two: BF16, whose steps are short, from two segments a row (1024 x 6144 over 4, 6 rows: 9.4 / 11.8; 2048 x 512 over 2 only
+  //   at many rows: 8 rows 5.3 / 5.7); the others only where slices are long: over 4 from four segments (INT4 1000 x 12288,
+  //   2 rows: 10.1 / 11.2; FP8 768 x 2048, 3 rows: 5.7 / 5.6), three at one or two rows (INT4 768 x 6144, 1 row: 6.5 / 6.9), over
+  //   2 at one row from five (INT4 1152 x 10240: 8.4 / 9.3);
+  //   three, which registers allow at one BF16 row: from six segments (1152 x 8192 over 2: 7.7 / 8.1);
+  //   more, a second round: never (INT4 6144 x 16384 over 4, 4 rows: 125 / 28).
+  const long waves = (long)nbatch * sk;
+  bool own = sk > 1 && waves <= 4 * cus;
+  // (under the add + norm prologue every workgroup makes the rows: one a CU or none. FP8 768 x 4096 over 4, 3 rows: 18.7 / 14.8)
+  if (sk > 1 && !a.norm.part) {
+    const bool two_fit = waves <= 8 * cus && 2 * (lds + 1024) <= 160 * 1024;
+    own = own || (two_fit && (kBf16 ? a.nsegk >= 2 || M >= 4 : sk == 4 ? a.nsegk >= (M <= 2 ? 3 : 4) : M == 1 && a.nsegk >= 5));
+    own = own || (kBf16 && M == 1 && waves <= 12 * cus && a.nsegk >= 6);
   }
-  // Two workgroups of four a CU where the add + norm prologue is 256 threads' work, and where a wave has one batch at most:
-  // at one row, or with few batches (BF16 1000 x 7168, 2 rows: 8.1 us, 9.0 with eight a workgroup;
-  // INT4 1536 x 6144, 4 rows: 9.2 and 8.3).
-  if (a.norm.part || nbatch < 3 * cus || (M == 1 && nbatch <= 8 * cus)) return launch_gemv<FMT, M, 4>(a, st);
+  if (own) return sk == 2 ? launch_gemv_sk<FMT, M, 2>(a, st) : launch_gemv_sk<FMT, M, 4>(a, st);
+  // Two workgroups of four a CU under the add + norm prologue (256 threads' work), and for few and short BF16 rows, which are
+  // over before eight waves' staging returns anything (1024 x 2048, 1 row: 4.8 us, 5.1 with eight a workgroup; 1024 x 8192,
+  // 8 rows, beyond 32 KB of activations: 14.2 and 12.9). FP8 and INT4 take eight at every size (64 x 1024: the same time).
+  if (a.norm.part || (kBf16 && nbatch <= 4 * cus && lds <= 32 * 1024)) return launch_gemv<FMT, M, 4>(a, st);
   return launch_gemv<FMT, M, 8>(a, st);
 }
 template <int FMT>
