@@ -112,8 +112,8 @@ __global__ void __launch_bounds__(256) k_add_norm(NormIn a, int H) {
 }
 
 // INT4 canonical tensors -> the contract's bf16 weight, one thread a group of 32 (the subtract-first form, exact for
-// every finite scale). hot: decode through the streaming kernels' own i4x8_to_bf16 instead (the probe the tests use to
-// pin the hot loop's arithmetic, as the reference's k_deq does: engine/experts/tests/test_experts.cu:217-235).
+// every finite scale). hot 1: decode as the matrix-unit streams do instead, hot 2: as the vector-unit streams do (the probes the
+// tests use to pin the hot loops' arithmetic, as the reference's k_deq does: engine/experts/tests/test_experts.cu:217-235).
 __global__ void __launch_bounds__(256) k_dequant_int4(const uint32_t* __restrict__ packed, const uint16_t* __restrict__ scale,
                                                       const uint32_t* __restrict__ zp, int N, int K, uint16_t* __restrict__ out, size_t ld, int hot) {
   const int G = K / 32;
@@ -128,11 +128,11 @@ __global__ void __launch_bounds__(256) k_dequant_int4(const uint32_t* __restrict
   if (hot) {
     const float s = bf16_bits_to_f32(sb), nzs = -((float)uz * s);
     const I4Group grp = i4_group(s, uz);
-    const bool large = !(fabsf(s) < kI4MaxScale);  // (a lane of its own choice here; the streams decide for a wave)
+    const bool any = hot == 2 || !(fabsf(s) < kI4MaxScale);  // (a lane's own choice here; the matrix-unit streams decide for a wave)
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       uint32_t p[4];
-      if (large) i4x8_to_bf16_any(w[c], s, nzs, p);
+      if (any) i4x8_to_bf16_any(w[c], s, nzs, p);
       else i4x8_to_bf16(w[c], grp, p);
 #pragma unroll
       for (int j = 0; j < 4; ++j) o[4 * c + j] = p[j];
@@ -308,6 +308,9 @@ int dsgx_dequant_int4(const void* packed, const void* scale, const void* zp, int
 }
 int dsgx_probe_dequant_int4(const void* packed, const void* scale, const void* zp, int N, int K, uint16_t* out, size_t ld, void* stream) {
   return dequant_int4_impl(packed, scale, zp, N, K, out, ld, stream, 1);
+}
+int dsgx_probe_dequant_int4_any(const void* packed, const void* scale, const void* zp, int N, int K, uint16_t* out, size_t ld, void* stream) {
+  return dequant_int4_impl(packed, scale, zp, N, K, out, ld, stream, 2);
 }
 int dsgx_widen_fp8(const void* codes, int N, int K, uint16_t* out, size_t ld, void* stream) {
   if (!codes || !out || N < 1 || K < 8 || K % 8 || ld < (size_t)K || ld % 8) return fail(DSGX_EINVAL, "widen_fp8: [%d][%d], ld %zu", N, K, ld);

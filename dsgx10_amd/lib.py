@@ -49,7 +49,7 @@ def lib():
         L.dsgx_add_norm.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_float,
                                     C.c_void_p, C.c_int, C.c_void_p]
         L.dsgx_gemv.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int, C.POINTER(abi.GemvSeg), C.c_int, C.c_int, C.c_int, C.c_void_p]
-        for f in ("dsgx_dequant_int4", "dsgx_probe_dequant_int4"):
+        for f in ("dsgx_dequant_int4", "dsgx_probe_dequant_int4", "dsgx_probe_dequant_int4_any"):
             getattr(L, f).argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_void_p, C.c_size_t, C.c_void_p]
         L.dsgx_widen_fp8.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_void_p, C.c_size_t, C.c_void_p]
         L.dsgx_act_quant.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p]
@@ -237,7 +237,8 @@ def launch_floor(kind, buf=None, sink=None, stream=None):
 
 
 def dequant_int4(packed, scale, zp, N, K, out, ld=None, stream=None, probe=False):
-    f = lib().dsgx_probe_dequant_int4 if probe else lib().dsgx_dequant_int4
+    """probe: the matrix-unit kernels' decode; "any": the vector-unit kernels'"""
+    f = lib().dsgx_probe_dequant_int4_any if probe == "any" else lib().dsgx_probe_dequant_int4 if probe else lib().dsgx_dequant_int4
     _check(f(_ptr(packed), _ptr(scale), _ptr(zp), N, K, _ptr(out), ld or K, _stream(stream)))
 
 

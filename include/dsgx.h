@@ -316,12 +316,16 @@ DSGX_API int dsgx_add_norm_gemv(const dsgx_norm_in* n, int rows, int K, const ds
 /* glm::dequant_int4 (engine/attn/attn.h:154-158): the contract's bf16 weight [N][ld] from the canonical tensors */
 DSGX_API int dsgx_dequant_int4(const void* packed, const void* scale, const void* zp, int N, int K, uint16_t* out,
                                size_t ld, void* stream);
-/* The same through the streaming kernels' own in-register decode: the probe that pins the hot loops' INT4 arithmetic to
-   the contract bit for bit, as the reference's k_deq does (engine/experts/tests/test_experts.cu:217-235). Bit-exact for
+/* The same through the streaming kernels' own in-register decodes: the probes that pin the hot loops' INT4 arithmetic to
+   the contract bit for bit, as the reference's k_deq does (engine/experts/tests/test_experts.cu:217-235): the first the decode of
+   the matrix-unit kernels (prefill, decode variant 1), which takes the other's from 2^116 on; _any the decode of the
+   vector-unit kernels (dsgx_gemv, decode variant 0), at every scale. Bit-exact for
    positive scales below 2^124 (the checkpoint's are 2^-15 .. 2^-4; a negative scale, which the format forbids, gives
    +0 instead of -0 where u = u_z); dsgx_dequant_int4 is exact for every finite scale. */
 DSGX_API int dsgx_probe_dequant_int4(const void* packed, const void* scale, const void* zp, int N, int K, uint16_t* out,
                                      size_t ld, void* stream);
+DSGX_API int dsgx_probe_dequant_int4_any(const void* packed, const void* scale, const void* zp, int N, int K, uint16_t* out,
+                                         size_t ld, void* stream);
 /* FP8 codes -> bf16 bits of the exact e4m3 values [N][ld] (the widening the GEMV and MoE kernels use;
    engine/experts/formats.cuh:121-128, tests/test_experts.cu:124-134) */
 DSGX_API int dsgx_widen_fp8(const void* codes, int N, int K, uint16_t* out, size_t ld, void* stream);

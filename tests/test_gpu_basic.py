@@ -30,7 +30,7 @@ def _dequant(packed, scale, zp, probe):
     return gpu.host(out, np.uint16, (N, K))
 
 
-@pytest.mark.parametrize("probe", [False, True])
+@pytest.mark.parametrize("probe", [False, True, "any"])
 def test_int4_dequant_random_matrices(probe):
     for (N, K, seed) in [(2048, 6144, 40), (6144, 2048, 42), (24, 1024, 6)]:
         packed, scale, zp = orc.int4_random(seed, N, K)
@@ -56,8 +56,9 @@ def test_int4_dequant_whole_domain_operator():
     assert nan.mean() < 1e-3
 
 
-def test_int4_hot_decode_scales():
-    """the streaming kernels' own decode on the reference's 145 test scales (subnormal, extreme) and on every finite scale
+@pytest.mark.parametrize("probe", [True, "any"])
+def test_int4_hot_decode_scales(probe):
+    """the streaming kernels' own decodes (matrix unit; vector unit) on the reference's 145 test scales (subnormal, extreme) and on every finite scale
     below 2^124, all (u, u_z)"""
     sc = _i4_test_scales()
     sb = np.arange(0x10000, dtype=np.uint32)
@@ -71,7 +72,7 @@ def test_int4_hot_decode_scales():
     scale = np.full((N, 16), 0x3F80, np.uint16)
     scale[: sc.size] = sc[:, None]
     zp = np.tile((np.arange(16, dtype=np.uint32) * 0x11111111)[None, :], (N // 8, 1)).astype(np.uint32)
-    got, want = _dequant(packed, scale, zp, True), orc.int4_dequant(packed, scale, zp)
+    got, want = _dequant(packed, scale, zp, probe), orc.int4_dequant(packed, scale, zp)
     pos = (scale[:, 0] & 0x8000) == 0
     assert np.array_equal(got[pos], want[pos])          # the format's scales are positive: bit for bit
     # negative scales (refused by the loader's scale check) differ only in the sign of a zero: u = u_z gives +0, not -0
