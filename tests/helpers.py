@@ -42,6 +42,33 @@ def make_layer(fmt, H, I, E, topk, NS, seed=0, shared=None, random_codes=False):
     return HostLayer(fmt, H, I, E, topk, experts, emap, shared_fp8=sh8, shared_bf16=sh16)
 
 
+def int4_layer_with_large_scales(H, I, E, topk, seed, T):
+    """An INT4 layer of random codes whose matrices hold a few scales in [2^116, 2^124) among ordinary ones, and rows for it: gate
+    in the groups 0 and 5 and up in the groups 10 and last, each in a third of the rows (so one of a wave's two row tiles only,
+    in an even, an odd and the last 128-k block), down in the groups 1, 6 and last. The activations there, and the channels of h, are
+    small enough that every sum stays finite, and not subnormal."""
+    experts = make_layer(abi.FMT_INT4, H, I, E, topk, E, seed=seed, random_codes=True).experts
+    rng = np.random.default_rng(seed)
+    x, logits, idx, w = rows_and_routing(seed, T, H, E, topk, 1.0)
+    x = orc.bf16_to_f32(x)
+    large = lambda n, lo=116: ((127 + rng.integers(lo, 124, n)) << 7 | rng.integers(0, 128, n)).astype(np.uint16)
+    small = np.repeat(np.isin(np.arange(I // 32), [1, 6, I // 32 - 1]), 32)  # the channels that down's large groups read
+    for gate, up, down in experts:
+        for m, groups in ((gate, (0, 5)), (up, (10, H // 32 - 1))):
+            for i, g in enumerate(groups):
+                rows = np.arange(i, I, 3)
+                m[1][rows, g] = large(rows.size)
+                x[:, 32 * g:32 * g + 32] = np.copysign(np.maximum(np.abs(x[:, 32 * g:32 * g + 32]), 0.25), x[:, 32 * g:32 * g + 32])
+        for m in (gate, up):
+            m[1][small] = (127 - 62) << 7
+        for g in (1, 6, I // 32 - 1):
+            rows = np.arange(g % 3, H, 3)
+            down[1][rows, g] = large(rows.size, 118)
+    for g in (0, 5, 10, H // 32 - 1):
+        x[:, 32 * g:32 * g + 32] *= np.float32(2.0 ** -120)
+    return HostLayer(abi.FMT_INT4, H, I, E, topk, experts), orc.f32_to_bf16(x), idx, w
+
+
 def rows_and_routing(seed, M, H, E, topk, scale, bias=None):
     x = orc.normal_bf16(seed, 1, (M, H), 1.0)
     logits = orc.normal_f32(seed, 2, (M, E), 1.0)

@@ -9,7 +9,7 @@ import torch
 
 from dsgx10_amd import abi, lib
 from tests import gpu, orc
-from tests.helpers import check_outputs, check_sums, make_layer, rel_l2, rows_and_routing
+from tests.helpers import check_outputs, check_sums, int4_layer_with_large_scales, make_layer, rel_l2, rows_and_routing
 
 pytestmark = pytest.mark.gpu
 
@@ -249,6 +249,27 @@ def test_decode_mfma_variant_every_bit_against_the_matrix_unit_oracle(fmt, H, I,
             assert np.array_equal(yr.view(np.uint32), dn["yr32"].view(np.uint32)), (M, int((yr != dn["yr32"]).sum()))
             if hl.has_shared:
                 assert np.array_equal(ys.view(np.uint32), dn["ys32"].view(np.uint32)), (M, int((ys != dn["ys32"]).sum()))
+    finally:
+        orc.set_dot_rule(0)
+
+
+@pytest.mark.parametrize("up", [0, 1])
+def test_decode_int4_scales_above_the_fast_decodes_range(up):
+    """a wave of variant 1 that meets a scale of 2^116 or more decodes the step by the routine for every scale, which variant 0 has
+    only: every bit against the oracle in the kernels' order of adds"""
+    H, I, E, topk = 2048, 2048, 8, 4
+    hl, x, idx, w = int4_layer_with_large_scales(H, I, E, topk, 62, 8)
+    dl = hl.upload()
+    orc.set_dot_rule(2 if up else 3)
+    try:
+        for M in (1, 8):
+            yr, _, ws = gpu.decode_layer(dl, x[:M], idx[:M], w[:M], M, up=up)
+            uni = orc.union(idx[:M], E)
+            hg, ho = gpu.h_of(ws, dl, M, len(uni)), orc.moe_up(hl, x[:M], uni)["h32"]
+            assert np.array_equal(hg, ho), (M, int((hg != ho).sum()))
+            dn = orc.moe_down(hl, ho, idx[:M], w[:M], uni)
+            assert np.isfinite(yr).all() and (yr != 0).mean() > 0.9
+            assert np.array_equal(yr.view(np.uint32), dn["yr32"].view(np.uint32)), (M, int((yr != dn["yr32"]).sum()))
     finally:
         orc.set_dot_rule(0)
 

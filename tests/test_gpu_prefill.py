@@ -316,6 +316,25 @@ def test_prefill_int4_lds_staged_kernels_give_the_register_ring_kernels_bits():
         assert np.array_equal(a, b)
 
 
+def test_prefill_int4_scales_above_the_fast_decodes_range():
+    """scales of 2^116 and more make a wave decode the block once more by the routine for every scale: the bits of the
+    register-ring kernel, which has that routine only, in tiles of 128 positions and in ragged ones"""
+    import os
+    H, I, E, topk, T = 512, 256, 4, 2, 300
+    hl, x, idx, w = helpers.int4_layer_with_large_scales(H, I, E, topk, 61, T)
+    outs = []
+    for old in ("0", "1"):
+        os.environ["DSGX_PF_I4_OLD"] = old
+        try:
+            yr, _, ws, dl = _prefill(hl, x, idx, w, T)
+            v = lib.prefill_view(dl.w, ws, T)
+            outs.append((yr, orc.bf16_to_f32(gpu.host(gpu.view(ws, v.h, T * topk * I * 2), np.uint16, (-1,)))))
+        finally:
+            os.environ.pop("DSGX_PF_I4_OLD", None)
+    for a, b in zip(*outs):
+        assert np.isfinite(a).all() and (a != 0).mean() > 0.9 and np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
 @pytest.mark.parametrize("H,I,E,topk,T,shared", [(512, 256, 8, 2, 150, "fp8"), (1024, 128, 16, 4, 37, None)])
 def test_prefill_fp8_bf16_activations_against_oracle(H, I, E, topk, T, shared):
     """FP8 weights under the engine's own prefill contract (prefill.cu:337-352: bf16 activations, per 128-k block the sum
