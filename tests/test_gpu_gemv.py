@@ -277,3 +277,53 @@ def test_add_norm_gemv_at_every_size_of_matrix(fmt, N, M, splitk):
     lib.gemv(xn[1], K, M, K, [seg[1]], abi.OUT_F32, splitk=splitk)
     for a, b in (ro, xn, y):
         assert np.array_equal(gpu.host(a, np.uint8, (-1,)), gpu.host(b, np.uint8, (-1,)))
+
+
+def _cut(fmt, parts, r0, n):
+    """rows r0 ... r0 + n of a matrix (FP8: r0 a multiple of its 128-row scale blocks; INT4: of the 8 rows a zero-point word holds)"""
+    if fmt == abi.FMT_FP8:
+        return parts[0][r0:r0 + n].copy(), parts[1][r0 // 128:(r0 + n + 127) // 128].copy()
+    if fmt == abi.FMT_INT4:
+        return parts[0][r0:r0 + n].copy(), parts[1][r0:r0 + n].copy(), parts[2][r0 // 8:(r0 + n) // 8].copy()
+    return (parts[0][r0:r0 + n].copy(),)
+
+
+_MATRIX = {abi.FMT_FP8: lambda t, n, K: orc.fp8_random(t, n, K, 1.0 / 256), abi.FMT_INT4: lambda t, n, K: orc.int4_random(t, n, K),
+           abi.FMT_BF16: lambda t, n, K: (orc.normal_bf16(0, t, (n, K), 0.02),)}
+
+
+@pytest.mark.parametrize("splitk", [1, 2, 4])
+@pytest.mark.parametrize("M", [1, 8])
+@pytest.mark.parametrize("fmt,N,K", [(abi.FMT_FP8, 1040, 8192 - 128), (abi.FMT_FP8, 4104, 2048 + 128), (abi.FMT_FP8, 6200, 2048 + 128), (abi.FMT_INT4, 776, 6144 - 256),
+                                     (abi.FMT_INT4, 4104, 2048 + 256), (abi.FMT_INT4, 6200, 4096 + 256), (abi.FMT_BF16, 1152, 4096 - 64), (abi.FMT_BF16, 2048, 512)])
+def test_every_route_gives_a_row_the_same_bits(fmt, N, K, M, splitk):
+    """both sides of the launch rule's lines (slices on waves of their own, one wave for all, four and eight waves a workgroup), a
+    second group of waves and several batches a wave, with each format's scales and zero points on later batches: rows at
+    the start, inside and at the end of the matrix against a matrix of these 64 rows"""
+    x = orc.normal_bf16(M, 1, (M, K), 1.0)
+    parts = _MATRIX[fmt](23, N, K)
+    y = _run(x, fmt, parts, N, K, abi.OUT_F32, splitk=splitk)
+    for r0 in (0, N // 2 // 128 * 128, (N - 1) // 128 * 128):
+        n = min(64, N - r0)
+        assert np.array_equal(y[:, r0:r0 + n], _run(x, fmt, _cut(fmt, parts, r0, n), n, K, abi.OUT_F32, splitk=splitk)), r0
+
+
+@pytest.mark.parametrize("splitk", [1, 2, 4])
+@pytest.mark.parametrize("fmt,K,M", [(abi.FMT_FP8, 1024 + 128, 3), (abi.FMT_INT4, 2048 + 256, 8), (abi.FMT_BF16, 1024 + 64, 2)])
+def test_segment_boundaries_inside_a_waves_later_batches(fmt, K, M, splitk):
+    """four segments in one launch, the boundaries after 16, 4120 and 5152 rows: a wave goes on from one matrix to another; each
+    segment's rows are those of a call of its own"""
+    x = orc.normal_bf16(29, 1, (M, K), 1.0)
+    ns = (16, 4104, 1032, 1048)
+    mats = [_MATRIX[fmt](40 + i, n, K) for i, n in enumerate(ns)]
+    keep, segs, ys = [], [], []
+    for n, parts in zip(ns, mats):
+        keep.append([gpu.dev(p) for p in parts])
+        k = keep[-1]
+        ys.append(gpu.empty(M * (n + 24) * 4, 0xFF))
+        segs.append(dict(fmt=fmt, w=k[0], s=k[1] if len(k) > 1 else None, zp=k[2] if len(k) > 2 else None, n=n, y=ys[-1], ldy=n + 24))
+    lib.gemv(gpu.dev(x), K, M, K, segs, abi.OUT_F32, splitk=splitk)
+    for n, parts, y in zip(ns, mats, ys):
+        got = gpu.host(y, np.float32, (M, n + 24))
+        assert np.array_equal(got[:, :n], _run(x, fmt, parts, n, K, abi.OUT_F32, splitk=splitk))
+        assert np.all(got[:, n:].view(np.uint32) == 0xFFFFFFFF)
