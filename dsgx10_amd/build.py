@@ -46,8 +46,8 @@ def _compile(src, force, extra=(), suffix=""):
 
 def build(jobs=None, force=False, extra=(), suffix=""):
     """extra / suffix: a diagnostic variant (e.g. extra=["-DDSGX_TRACE"], suffix="_trace" -> libdsgx_trace.so; DSGX_TRACE:
-    the decode kernels' phase stamps, DSGX_PF_TRACE: the FP8 prefill GEMM's, eight wall-clock stamps a workgroup into the
-    buffer whose address DSGX_PF_TRACE_PTR names; DSGX_LIB=libdsgx_trace.so loads the variant)"""
+    the decode kernels' phase stamps, DSGX_PF_TRACE: the FP8 prefill GEMM's, eight wall-clock stamps a workgroup of the routed
+    experts' grid into the buffer whose address DSGX_PF_TRACE_PTR names; DSGX_LIB=libdsgx_trace.so loads the variant)"""
     srcs = [s for s in SOURCES if os.path.exists(os.path.join(CSRC, s))]
     jobs = jobs or min(len(srcs), os.cpu_count() or 4)
     so = SO.replace(".so", suffix + ".so")

@@ -87,11 +87,11 @@ struct Args {
   float* d;            // DOWN: f32 [position][H]
   SharedRows sh;       // k_gemm_mixed: the shared expert's rows in the same launch (grid 0: not in it)
 #ifdef DSGX_PF_TRACE
-  unsigned long long* trace;  // (diagnostic build: thread 0's wall-clock stamps, 8 a workgroup)
+  unsigned long long* trace;  // (diagnostic build: thread 0's wall-clock stamps, 8 a workgroup of the routed experts' grid)
 #endif
 };
 #ifdef DSGX_PF_TRACE
-#define PF_STAMP(g, k) do { if ((g).trace && threadIdx.x == 0) (g).trace[(size_t)blockIdx.x * 8 + (k)] = wall_clock64(); } while (0)
+#define PF_STAMP(g, k) do { if ((g).trace && threadIdx.x == 0) (g).trace[(size_t)(blockIdx.x - (g).sh.grid) * 8 + (k)] = wall_clock64(); } while (0)
 #else
 #define PF_STAMP(g, k) do { } while (0)
 #endif
@@ -428,24 +428,27 @@ __global__ void __launch_bounds__(kThreads) k_gemm_mixed(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int NS = UP ? g.L.I / (kWgRows / 2) : g.L.H / kWgRows;
   int tile, ns;
-  PF_STAMP(g, 0);
   if (blockIdx.x < g.sh.grid) {  // (the same for the whole workgroup)
     task_of<true>(NS, tile, ns);
     const int m0 = tile * Shape<2>::kPos, mend = g.nrows;
     if (ns >= NS || m0 >= mend) return;
     Args q = g;
+#ifdef DSGX_PF_TRACE
+    q.trace = nullptr;
+#endif
     q.aq = g.sh.aq, q.as = g.sh.as, q.gather = nullptr, q.h = g.sh.h, q.hq = g.sh.hq, q.hs = g.sh.hs, q.d = g.sh.d;
     if (mend - m0 > Shape<1>::kPos) gemm_tile<UP, 2, DIAG>(q, smem, -1, m0, mend, ns);
     else gemm_tile<UP, 1, DIAG>(q, smem, -1, m0, mend, ns);
     return;
   }
+  PF_STAMP(g, 0);
   task_of<false>(NS, tile, ns, blockIdx.x - g.sh.grid);
   if (ns >= NS || tile >= *g.ntiles) return;
   const int te = g.tile_e[tile], e = te & 0xFFFF;
   const int m0 = g.off[e] + g.tile_m0[tile], mend = g.off[e + 1];
   if (m0 >= 0) PF_STAMP(g, 1);
 #ifdef DSGX_PF_TRACE
-  if (g.trace && threadIdx.x == 0) g.trace[(size_t)blockIdx.x * 8 + 7] = ((te >> 30) ? 0x10000 : 0) | min(mend - m0, (te >> 30) ? 256 : 128);
+  if (g.trace && threadIdx.x == 0) g.trace[(size_t)(blockIdx.x - g.sh.grid) * 8 + 7] = ((te >> 30) ? 0x10000 : 0) | min(mend - m0, (te >> 30) ? 256 : 128);
 #endif
   if (te >> 30) gemm_tile<UP, 2, DIAG>(g, smem, e, m0, mend, ns);
   else gemm_tile<UP, 1, DIAG>(g, smem, e, m0, mend, ns);
