@@ -849,16 +849,6 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
   void (*k_dn)(pf8::Args) = pf8::k_gemm_mixed<false>;
   void (*k_up2)(pf8::Args) = pf8::k_gemm<true, 2>;      // the shared expert: 256-position tiles
   void (*k_dn2)(pf8::Args) = pf8::k_gemm<false, 2>;
-#ifdef DSGX_PF_DIAG
-  {  // diagnostic build: DSGX_PF_DIAG=<bits> switches parts of the kernels off (wrong results; for timing only)
-    const char* dv = std::getenv("DSGX_PF_DIAG");
-    switch (dv ? std::atoi(dv) : 0) {
-#define DSGX_DIAG_CASE(n) case n: k_up = pf8::k_gemm_mixed<true, n>, k_dn = pf8::k_gemm_mixed<false, n>, k_up2 = pf8::k_gemm<true, 2, n>, k_dn2 = pf8::k_gemm<false, 2, n>; break;
-      DSGX_DIAG_CASE(1) DSGX_DIAG_CASE(2) DSGX_DIAG_CASE(4) DSGX_DIAG_CASE(8) DSGX_DIAG_CASE(16) DSGX_DIAG_CASE(3) DSGX_DIAG_CASE(9) DSGX_DIAG_CASE(25) DSGX_DIAG_CASE(32) DSGX_DIAG_CASE(64) DSGX_DIAG_CASE(128) DSGX_DIAG_CASE(256) DSGX_DIAG_CASE(384)
-#undef DSGX_DIAG_CASE
-    }
-  }
-#endif
   constexpr int kLdsMix = pf8::Shape<1>::kLds > pf8::Shape<2>::kLds ? pf8::Shape<1>::kLds : pf8::Shape<2>::kLds;
   for (const void* k : {(const void*)k_up, (const void*)k_dn})
     if (int rc = allow_dynamic_lds(k, kLdsMix)) return rc;
@@ -1013,16 +1003,6 @@ int dsgx_dsk_moe_prefill(const dsgx_dsk_weights* Wt, const uint8_t* xq, const ui
   void (*k_dn)(pfmx::Args) = pfmx::k_gemm_mixed<false, F4>;
   void (*k_sup)(pfmx::Args) = pfmx::k_gemm<true, F8>;
   void (*k_sdn)(pfmx::Args) = pfmx::k_gemm<false, F8>;
-#ifdef DSGX_PF_DIAG
-  {  // diagnostic build: DSGX_PF_DIAG=<bits> switches parts of the kernels off (wrong results; for timing only)
-    const char* dv = std::getenv("DSGX_PF_DIAG");
-    switch (dv ? std::atoi(dv) : 0) {
-#define DSGX_DIAG_CASE(n) case n: k_up = pfmx::k_gemm_mixed<true, F4, n>, k_dn = pfmx::k_gemm_mixed<false, F4, n>, k_sup = pfmx::k_gemm<true, F8, n>, k_sdn = pfmx::k_gemm<false, F8, n>; break;
-      DSGX_DIAG_CASE(1) DSGX_DIAG_CASE(4) DSGX_DIAG_CASE(8) DSGX_DIAG_CASE(32) DSGX_DIAG_CASE(64) DSGX_DIAG_CASE(128) DSGX_DIAG_CASE(256) DSGX_DIAG_CASE(384) DSGX_DIAG_CASE(512) DSGX_DIAG_CASE(1024) DSGX_DIAG_CASE(513) DSGX_DIAG_CASE(1025) DSGX_DIAG_CASE(1152) DSGX_DIAG_CASE(1280) DSGX_DIAG_CASE(1408) DSGX_DIAG_CASE(1032) DSGX_DIAG_CASE(1088) DSGX_DIAG_CASE(1056)
-#undef DSGX_DIAG_CASE
-    }
-  }
-#endif
   for (const void* k : {(const void*)k_up, (const void*)k_dn})
     if (int rc = allow_dynamic_lds(k, kLdsRun)) return rc;
   for (const void* k : {(const void*)k_sup, (const void*)k_sdn})

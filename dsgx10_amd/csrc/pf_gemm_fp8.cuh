@@ -132,11 +132,8 @@ __device__ __forceinline__ void wait_loads() {
 }
 __device__ __forceinline__ int swz(int r) { return (r & 7) ^ (r >> 3); }
 
-// DIAG (diagnostic builds only; results are then wrong): 1 no loads after the first stages, 2 the MFMAs accumulate by
-// themselves (no scaled adds on the vector unit), 4 no workgroup barrier in the loop, 8 no MFMAs, 16 no fragment reads
-// after the first turn, 128 the weight loads / 256 the activation loads re-read block 0 (cached) after the first stages
 // one tile: expert e (-1: the shared expert), rows [m0, mend) of the activations' positions, row group ns
-template <bool UP, int WP, int DIAG>
+template <bool UP, int WP>
 __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, int m0, int mend, int ns) {
   using S = Shape<WP>;
   const int K = UP ? g.L.H : g.L.I, KB = K / 128;
@@ -214,12 +211,12 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) dma16(pw[t][hh] + (size_t)(((DIAG & 128) && kb >= S::kStages) ? 0 : kc) * 128, uni(wbase + t * 2048 + hh * 1024));
+      for (int hh = 0; hh < 2; ++hh) dma16(pw[t][hh] + (size_t)kc * 128, uni(wbase + t * 2048 + hh * 1024));
 #pragma unroll
     for (int t = 0; t < WP; ++t) {
       if (t >= nx) break;  // (a ragged tile: nobody reads the 16-position tiles past its end)
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) dma16(px[t][hh] + (size_t)(((DIAG & 256) && kb >= S::kStages) ? 0 : kc) * 128, uni(xbase + t * 2048 + hh * 1024));
+      for (int hh = 0; hh < 2; ++hh) dma16(px[t][hh] + (size_t)kc * 128, uni(xbase + t * 2048 + hh * 1024));
     }
     if (nx > 0 && lane < 16 * WP) dma4(pxs + kc, uni(st + S::kStageW + S::kStageX + (uint32_t)wave * (64 * WP)));
   };
@@ -258,20 +255,20 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
 
   auto run = [&](auto nj_c) {
     constexpr int NJ = decltype(nj_c)::value;
-    for (int kb = 0; kb < ((DIAG & 32) ? 2 : KB); ++kb) {
+    for (int kb = 0; kb < KB; ++kb) {
       // this wave's loads of block kb have landed (later blocks may be in flight); after the barrier everyone's have, and
       // everyone is done reading the stage of block kb - 1, which the loads of block kb + kStages - 1 now overwrite
       if (S::kStages == 2) wait_loads<0>();
       else if (nx == WP) wait_loads<(S::kStages - 2) * S::kLoads>();
       else if (nx == 0) wait_loads<(S::kStages - 2) * 4>();
       else wait_loads<(S::kStages - 2) * (5 + 2 * (WP - 1))>();  // (WP 2 with one live tile; two stages wait for all anyway)
-      if (!(DIAG & 4)) __syncthreads();
+      __syncthreads();
       if (kb == 0) PF_STAMP(g, 4);
-      if (!(DIAG & 1)) issue(kb + S::kStages - 1);
+      issue(kb + S::kStages - 1);
       if (NJ == 0) continue;
       const float wsa = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wsa_l), kb & 63));
       const float wsb = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wsb_l), kb & 63));
-      const uint8_t* st = smem + (size_t)(((DIAG & 16) ? 0 : kb) % S::kStages) * S::kStageBytes;
+      const uint8_t* st = smem + (size_t)(kb % S::kStages) * S::kStageBytes;
       const uint8_t* W = st + S::RA * rg * 2048;
       const uint8_t* X = st + S::kStageW + pg * 2048;
       const float* XS = reinterpret_cast<const float*>(st + S::kStageW + S::kStageX) + 16 * pg;
@@ -285,13 +282,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
         const float s0 = __fmul_rn(xv, wsa), s1 = __fmul_rn(xv, wsb);
 #pragma unroll
         for (int t = 0; t < S::RA; ++t) {
-          if (DIAG & 2) {
-            acc[t][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fa[t], fb, acc[t][j], 0, 0, 0, 0, 0, 0);
-            continue;
-          }
-          v4f_t p;
-          if (DIAG & 8) p = v4f_t{__builtin_bit_cast(float, fa[t][0] ^ fb[0]), __builtin_bit_cast(float, fa[t][1] ^ fb[3]), __builtin_bit_cast(float, fa[t][4] ^ fb[4]), __builtin_bit_cast(float, fa[t][7] ^ fb[7])};
-          else p = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fa[t], fb, v4f_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+          const v4f_t p = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fa[t], fb, v4f_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
           const float sc = (UP && (t & 1)) ? s1 : s0;
 #pragma unroll
           for (int q = 0; q < 4; ++q) acc[t][j][q] = fmaf(sc, p[q], acc[t][j][q]);
@@ -313,15 +304,6 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   wait_loads<0>();   // the trailing loads into unused stages: nothing may still be landing in LDS from here on
   __syncthreads();   // ... in any wave's part of it: the epilogues reuse the stages
   PF_STAMP(g, 5);
-  if (DIAG & 64) {   // (diagnostic: no epilogue; one store keeps the sums alive)
-    float sum = 0.f;
-#pragma unroll
-    for (int t = 0; t < S::RA; ++t)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) sum += acc[t][j][0] + acc[t][j][1] + acc[t][j][2] + acc[t][j][3];
-    if (sum == 12345.678f) reinterpret_cast<float*>(UP ? (void*)g.h : (void*)g.d)[tid] = sum;
-    return;
-  }
 
   // register q of lane l is weight row 4 (l / 16) + q of the 16-row tile, position l % 16 of the 16 positions
   if (UP) {
@@ -404,7 +386,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
 }
 
 // The shared expert (tile_e null: tiles of Shape<WP>::kPos rows over [0, nrows)) or one list of tiles of one shape.
-template <bool UP, int WP, int DIAG = 0>
+template <bool UP, int WP>
 __global__ void __launch_bounds__(kThreads) k_gemm(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int NS = UP ? g.L.I / (kWgRows / 2) : g.L.H / kWgRows;
@@ -420,10 +402,10 @@ __global__ void __launch_bounds__(kThreads) k_gemm(Args g) {
   } else if (m0 >= mend) {
     return;
   }
-  gemm_tile<UP, WP, DIAG>(g, smem, e, m0, mend, ns);
+  gemm_tile<UP, WP>(g, smem, e, m0, mend, ns);
 }
 // The routed experts' list of both shapes (bit 30 of tile_e: a 256-position tile), an expert's tiles next to each other.
-template <bool UP, int DIAG = 0>
+template <bool UP>
 __global__ void __launch_bounds__(kThreads) k_gemm_mixed(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int NS = UP ? g.L.I / (kWgRows / 2) : g.L.H / kWgRows;
@@ -437,8 +419,8 @@ __global__ void __launch_bounds__(kThreads) k_gemm_mixed(Args g) {
     q.trace = nullptr;
 #endif
     q.aq = g.sh.aq, q.as = g.sh.as, q.gather = nullptr, q.h = g.sh.h, q.hq = g.sh.hq, q.hs = g.sh.hs, q.d = g.sh.d;
-    if (mend - m0 > Shape<1>::kPos) gemm_tile<UP, 2, DIAG>(q, smem, -1, m0, mend, ns);
-    else gemm_tile<UP, 1, DIAG>(q, smem, -1, m0, mend, ns);
+    if (mend - m0 > Shape<1>::kPos) gemm_tile<UP, 2>(q, smem, -1, m0, mend, ns);
+    else gemm_tile<UP, 1>(q, smem, -1, m0, mend, ns);
     return;
   }
   PF_STAMP(g, 0);
@@ -450,8 +432,8 @@ __global__ void __launch_bounds__(kThreads) k_gemm_mixed(Args g) {
 #ifdef DSGX_PF_TRACE
   if (g.trace && threadIdx.x == 0) g.trace[(size_t)(blockIdx.x - g.sh.grid) * 8 + 7] = ((te >> 30) ? 0x10000 : 0) | min(mend - m0, (te >> 30) ? 256 : 128);
 #endif
-  if (te >> 30) gemm_tile<UP, 2, DIAG>(g, smem, e, m0, mend, ns);
-  else gemm_tile<UP, 1, DIAG>(g, smem, e, m0, mend, ns);
+  if (te >> 30) gemm_tile<UP, 2>(g, smem, e, m0, mend, ns);
+  else gemm_tile<UP, 1>(g, smem, e, m0, mend, ns);
 }
 
 }  // namespace pf8

@@ -86,16 +86,14 @@ __device__ __forceinline__ v4f_t mfma_mx(v8i_t a, v8i_t b, v4f_t c, int sa, int 
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, CBSZ, 0, 0, sa, 0, sb);
 }
 
-// DIAG (diagnostic builds only; results are then wrong): 1 no loads after the first stages, 4 no workgroup barrier in the
-// loop, 8 no MFMAs, 16 no fragment reads after the first turn, 32 two blocks only, 64 no epilogue
-template <bool UP, int WP, int WF, int DIAG = 0>
+template <bool UP, int WP, int WF>
 __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, int m0, int mend, int ns) {
   using S = Shape<WP, WF>;
   constexpr bool F4 = S::F4;
   constexpr int CBSZ = F4 ? 4 : 0;
   const int K = UP ? g.H : g.I, KB = K / 128, G = K / 32;
   if (mend > m0 + S::kPos) mend = m0 + S::kPos;
-  const size_t eo = (e < 0 || (DIAG & 128)) ? 0 : (size_t)e;  // (diagnostic 128: every tile reads expert 0's weights)
+  const size_t eo = e < 0 ? 0 : (size_t)e;
   const uint8_t *wa = g.wa + eo * g.wstride, *sa = g.sa + eo * g.sstride;
   const uint8_t *wb = UP ? g.wb + eo * g.wstride : wa, *sb = UP ? g.sb + eo * g.sstride : sa;
   const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6), r16 = lane & 15, part = lane >> 4;
@@ -143,7 +141,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
       const int r = 8 * hh + lr;
       int pos = m0 + 16 * (WP * wave + t) + r;
       if (pos >= mend) pos = mend - 1;
-      px[t][hh] = g.aq + (size_t)((DIAG & 256) ? pos & 255 : g.gather ? g.gather[pos] : pos) * K + 16 * pc8(lq ^ swz(r));  // (diagnostic 256: 256 hot rows)
+      px[t][hh] = g.aq + (size_t)(g.gather ? g.gather[pos] : pos) * K + 16 * pc8(lq ^ swz(r));
     }
   const uint8_t* pxs;  // lanes 0 .. 16 WP - 1: the scale word of position 16 WP wave + lane
   {
@@ -208,19 +206,18 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
 
   auto run = [&](auto nj_c) {
     constexpr int NJ = decltype(nj_c)::value;
-    for (int kb = 0; kb < ((DIAG & 32) ? 2 : KB); ++kb) {
+    for (int kb = 0; kb < KB; ++kb) {
       wait_loads<(S::kStages - 2) * S::kLoads>();
-      if (!(DIAG & 4)) __syncthreads();
-      if (!(DIAG & 1) && NJ == 0) issue(kb + S::kStages - 1);
+      __syncthreads();
+      if (NJ == 0) issue(kb + S::kStages - 1);
       if (NJ == 0) continue;
       // loads i with i * NJ / kLoads == j go out after the fragment reads of 16-position tile j
       auto issue_some = [&](int j) {
-        if (DIAG & 1) return;
 #pragma unroll
         for (int i = 0; i < S::kLoads; ++i)
           if (i * (NJ > 0 ? NJ : 1) / S::kLoads == j) issue_one(kb + S::kStages - 1, i);
       };
-      const uint8_t* st = smem + (size_t)(((DIAG & 16) ? 0 : kb) % S::kStages) * S::kStageBytes;
+      const uint8_t* st = smem + (size_t)(kb % S::kStages) * S::kStageBytes;
       const uint8_t* W = st + S::RA * rg * (16 * S::kRowB);
       const uint8_t* X = st + S::kStageW + pg * 2048;
       const uint8_t* WS = st + S::kStageW + S::kStageX + S::RA * rg * 64 + rds;
@@ -239,8 +236,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
         issue_some(j);
 #pragma unroll
         for (int t = 0; t < S::RA; ++t) {
-          if (DIAG & 8) acc[t][j][0] += __builtin_bit_cast(float, fa[t][0] ^ fb[1] ^ fs[t] ^ xsb), acc[t][j][2] += __builtin_bit_cast(float, fa[t][3] ^ fb[6]);
-          else acc[t][j] = mfma_mx<CBSZ>(fa[t], fb, acc[t][j], fs[t], xsb);
+          acc[t][j] = mfma_mx<CBSZ>(fa[t], fb, acc[t][j], fs[t], xsb);
         }
       }
     }
@@ -258,15 +254,6 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   }
   wait_loads<0>();
   __syncthreads();
-  if (DIAG & 64) {
-    float sum = 0.f;
-#pragma unroll
-    for (int t = 0; t < S::RA; ++t)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) sum += acc[t][j][0] + acc[t][j][1] + acc[t][j][2] + acc[t][j][3];
-    if (sum == 12345.678f) reinterpret_cast<float*>(UP ? (void*)g.h : (void*)g.d)[tid] = sum;
-    return;
-  }
 
   // register q of lane l is weight row 4 (l / 16) + q of the 16-row tile, position l % 16 of the 16 positions
   if (UP) {
@@ -352,7 +339,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
 }
 
 // The shared expert (tile_e null: tiles of 256 rows over [0, nrows)).
-template <bool UP, int WF, int DIAG = 0>
+template <bool UP, int WF>
 __global__ void __launch_bounds__(kThreads) k_gemm(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int NS = UP ? g.I / (kWgRows / 2) : g.H / kWgRows;
@@ -361,10 +348,10 @@ __global__ void __launch_bounds__(kThreads) k_gemm(Args g) {
   if (ns >= NS) return;
   const int m0 = tile * Shape<2, WF>::kPos, mend = g.nrows;
   if (m0 >= mend) return;
-  gemm_tile<UP, 2, WF, DIAG>(g, smem, -1, m0, mend, ns);
+  gemm_tile<UP, 2, WF>(g, smem, -1, m0, mend, ns);
 }
 // The routed experts' list of both tile shapes (bit 30 of tile_e: a 256-position tile), an expert's tiles next to each other.
-template <bool UP, int WF, int DIAG = 0>
+template <bool UP, int WF>
 __global__ void __launch_bounds__(kThreads) k_gemm_mixed(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int NS = UP ? g.I / (kWgRows / 2) : g.H / kWgRows;
@@ -376,17 +363,15 @@ __global__ void __launch_bounds__(kThreads) k_gemm_mixed(Args g) {
     Args q = g;
     q.aq = g.sh.aq, q.as = g.sh.as, q.gather = nullptr, q.posw = nullptr, q.wstride = q.sstride = 0;
     q.wa = g.sh.wa, q.sa = g.sh.sa, q.wb = g.sh.wb, q.sb = g.sh.sb, q.h = g.sh.h, q.hq = g.sh.hq, q.hs = g.sh.hs, q.d = g.sh.d;
-    gemm_tile<UP, 2, DSGX_FMT_FP8_B32E, DIAG>(q, smem, -1, m0, mend, ns);
+    gemm_tile<UP, 2, DSGX_FMT_FP8_B32E>(q, smem, -1, m0, mend, ns);
     return;
   }
   pf8::task_of<false>(NS, tile, ns, blockIdx.x - g.sh.grid);
   if (ns >= NS || tile >= *g.ntiles) return;
   const int te = g.tile_e[tile], e = te & 0xFFFF;
   const int m0 = g.off[e] + g.tile_m0[tile], mend = g.off[e + 1];
-  if ((DIAG & 512) && !(te >> 30)) return;  // (diagnostic: the 256-position tiles only / the remainders only)
-  if ((DIAG & 1024) && (te >> 30)) return;
-  if (te >> 30) gemm_tile<UP, 2, WF, DIAG>(g, smem, e, m0, mend, ns);
-  else gemm_tile<UP, 1, WF, DIAG>(g, smem, e, m0, mend, ns);
+  if (te >> 30) gemm_tile<UP, 2, WF>(g, smem, e, m0, mend, ns);
+  else gemm_tile<UP, 1, WF>(g, smem, e, m0, mend, ns);
 }
 
 }  // namespace pfmx
