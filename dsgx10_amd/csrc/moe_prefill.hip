@@ -862,7 +862,7 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
 #endif
   const int NSU = I / (pf8::kWgRows / 2), NSD = H / pf8::kWgRows;
   const bool mixed = order >= 1;
-  g.tile_e = I32(mixed ? o.ord_e : o.mix_e), g.tile_m0 = I32(mixed ? o.ord_m0 : o.mix_m0), g.ntiles = I32(o.nmix), g.off = I32(o.off), g.nrows = P;
+  g.tile_e = I32(mixed ? o.ord_e : o.mix_e), g.tile_m0 = I32(mixed ? o.ord_m0 : o.mix_m0), g.ntiles = I32(o.nmix), g.off = I32(o.off), g.nrows = T;
   // A whole step runs the shared expert's tiles in the routed experts' launches, in front of them: alone they are a launch
   // of T / 256 x 16 workgroups, a sixteenth of the chip at T = 200, and two more tails (whole call, hidden 4096, intermediate
   // 2048, 256 experts: T = 200 1058 -> 978 us, T = 8192 3112 -> 3101; same bits).
@@ -874,10 +874,8 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
   if (cfg.phases & 2) {
     g.aq = W + o.xq, g.as = F32(o.xs), g.gather = I32(o.perm);
     g.h = reinterpret_cast<uint16_t*>(W + o.h), g.hq = W + o.hq, g.hs = F32(o.hs), g.d = nullptr;
-    if (fused_sh) {
-      g.nrows = T;
+    if (fused_sh)
       g.sh = pf8::SharedRows{pf8::grid_of(sh_tiles, NSU), W + o.xq, F32(o.xs), reinterpret_cast<uint16_t*>(W + o.hsh), W + o.hshq, F32(o.hshs), nullptr};
-    }
     hipLaunchKernelGGL(k_up, dim3(g.sh.grid + pf8::grid_of(o.max_big + E, NSU)), dim3(pf8::kThreads), kLdsMix, st, g);
     DSGX_HIP(hipGetLastError());
   }
@@ -894,7 +892,7 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
   }
   if ((cfg.phases & 16) && shared && !fused_sh) {
     const int tiles = sh_tiles;
-    g.tile_e = g.tile_m0 = g.ntiles = g.off = nullptr, g.nrows = T;
+    g.tile_e = g.tile_m0 = g.ntiles = g.off = nullptr;
     g.aq = W + o.xq, g.as = F32(o.xs), g.gather = nullptr;
     g.h = reinterpret_cast<uint16_t*>(W + o.hsh), g.hq = W + o.hshq, g.hs = F32(o.hshs), g.d = nullptr;
     hipLaunchKernelGGL(k_up2, dim3(pf8::grid_of(tiles, NSU)), dim3(pf8::kThreads), pf8::Shape<2>::kLds, st, g);
@@ -1022,14 +1020,14 @@ int dsgx_dsk_moe_prefill(const dsgx_dsk_weights* Wt, const uint8_t* xq, const ui
     DSGX_HIP(hipGetLastError());
   }
   pfmx::Args g{};
-  g.H = H, g.I = I, g.limit = cfg.swiglu_limit;
+  g.H = H, g.I = I, g.nrows = T, g.limit = cfg.swiglu_limit;
   // a whole step runs the shared expert's tiles in the routed experts' launches, in front of them (as the FP8 layers do;
   // hidden 5120, intermediate 2304, T = 3000: 1870 -> 1821 us)
   const int sh_tiles = (T + 255) / 256;
   const bool fused_sh = shared && (cfg.phases & (2 | 4 | 8)) == (2 | 4 | 8);
   if ((cfg.phases & 2) && shared && !fused_sh) {
     const int tiles = sh_tiles;
-    g.tile_e = g.tile_m0 = g.ntiles = g.off = nullptr, g.nrows = T, g.gather = nullptr, g.posw = nullptr, g.wstride = g.sstride = 0;
+    g.tile_e = g.tile_m0 = g.ntiles = g.off = nullptr, g.gather = nullptr, g.posw = nullptr, g.wstride = g.sstride = 0;
     g.aq = xq, g.as = xs, g.wa = Wt->sh_w1, g.sa = Wt->sh_s1, g.wb = Wt->sh_w3, g.sb = Wt->sh_s3;
     g.h = U16(o.hsh), g.hq = W + o.hshq, g.hs = W + o.hshs, g.d = nullptr;
     hipLaunchKernelGGL(k_sup, dim3(pf8::grid_of(tiles, NSU)), dim3(pf8::kThreads), kLdsSh, st, g);
@@ -1038,7 +1036,7 @@ int dsgx_dsk_moe_prefill(const dsgx_dsk_weights* Wt, const uint8_t* xq, const ui
     hipLaunchKernelGGL(k_sdn, dim3(pf8::grid_of(tiles, NSD)), dim3(pf8::kThreads), kLdsSh, st, g);
     DSGX_HIP(hipGetLastError());
   }
-  g.tile_e = I32(o.mix_e), g.tile_m0 = I32(o.mix_m0), g.ntiles = I32(o.nmix), g.off = I32(o.off), g.nrows = T;
+  g.tile_e = I32(o.mix_e), g.tile_m0 = I32(o.mix_m0), g.ntiles = I32(o.nmix), g.off = I32(o.off);
   auto launch = [&](bool up) {
     hipLaunchKernelGGL(up ? k_up : k_dn, dim3(g.sh.grid + pf8::grid_of(o.max_big + E, up ? NSU : NSD)), dim3(pf8::kThreads), kLdsRun, st, g);
   };

@@ -131,6 +131,8 @@ __device__ __forceinline__ void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 __device__ __forceinline__ int swz(int r) { return (r & 7) ^ (r >> 3); }
+// the slot of a 64-byte row's piece q is q ^ sw4(row), in the INT4 and MXFP4 kernels (why: pf_gemm_i4.cuh)
+__device__ __forceinline__ int sw4(int r) { return (((r >> 2) ^ (r >> 3)) & 1) << 1 | ((r >> 3) & 1); }
 
 // one tile: expert e (-1: the shared expert), rows [m0, mend) of the activations' positions, row group ns
 template <bool UP, int WP>

@@ -27,6 +27,7 @@ using pf8::dma16;
 using pf8::dma4;
 using pf8::kThreads;
 using pf8::kWgRows;
+using pf8::sw4;
 using pf8::v4f_t;
 using pf8::wait_loads;
 typedef __bf16 v8bf_t __attribute__((ext_vector_type(8)));
@@ -68,7 +69,6 @@ struct Args {
 // of such a set on every bank (a loop of these reads: 427 us, 222 with the slots below; gate/up's LDS cycles were half
 // conflicts). sw4 takes rows 0-3, 4-7, 8-11, 12-15 to 0, 2, 3, 1 and sw16 exchanges rows 4-7 and 12-15: one-to-one on both
 // kinds of sixteen.
-__device__ __forceinline__ int sw4(int r) { return (((r >> 2) ^ (r >> 3)) & 1) << 1 | ((r >> 3) & 1); }
 __device__ __forceinline__ int sw16(int r) { return r ^ ((r & 4) << 1); }
 
 template <bool UP, int POS>

@@ -23,6 +23,7 @@ using pf8::dma16;
 using pf8::dma4;
 using pf8::kThreads;
 using pf8::kWgRows;
+using pf8::sw4;
 using pf8::swz;
 using pf8::v4f_t;
 using pf8::v8i_t;
@@ -72,8 +73,6 @@ struct Args {
   SharedRows sh;       // (grid 0: the launch holds routed tiles only)
 };
 
-// (the slot of a 64-byte row's piece: one-to-one on the rows whose lanes the LDS serves together, see pf_gemm_i4.cuh's sw4)
-__device__ __forceinline__ int sw4(int r) { return (((r >> 2) ^ (r >> 3)) & 1) << 1 | ((r >> 3) & 1); }
 // 128-byte rows (activations, e4m3 weights) lie in LDS in pf_gemm_fp8.cuh's layout, whose fragment reads (a lane's two
 // neighbouring slots 2 part, 2 part + 1, swizzled by row) run without bank conflicts; what differs is WHICH 16 bytes of the
 // row a slot holds: the block-scaled instruction wants bytes 16 part ... and 64 + 16 part ... in a lane, so logical piece
