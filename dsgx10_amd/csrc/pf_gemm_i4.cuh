@@ -50,6 +50,7 @@ struct Shape {
 };
 constexpr int kLoads = 2 + 4 + 1 + 1;        // a wave's loads a turn: two weight tiles, one activation tile (four pieces of 4 rows), scales, zero points
 constexpr int kLds = Shape<128>::kLds > Shape<64>::kLds ? Shape<128>::kLds : Shape<64>::kLds;
+constexpr int kLdsRun = kLds + kThreads / 64 * 4;  // ... and a word a wave: whether it met a scale above the fast decode's range
 
 struct Args {
   const uint16_t* x;   // activations bf16 [rows][K]
@@ -66,9 +67,8 @@ struct Args {
 // Where piece q of a row lies. A 16-byte LDS read of 64 lanes is served sixteen lanes at a time, and the sixteen are lanes
 // 0-3, 12-15, 20-27 (and 4-11, 16-19, 28-31; the same from 32 on): rows 0-3 and 12-15 of one k part beside rows 4-11 of the
 // next. Slots q ^ (r / 4 % 4) (64-byte rows) and c ^ r (256-byte rows), one-to-one on sixteen neighbouring rows, put two lanes
-// of such a set on every bank (a loop of these reads: 427 us, 222 with the slots below; gate/up's LDS cycles were half
-// conflicts). sw4 takes rows 0-3, 4-7, 8-11, 12-15 to 0, 2, 3, 1 and sw16 exchanges rows 4-7 and 12-15: one-to-one on both
-// kinds of sixteen.
+// of such a set on every bank (gate/up at T = 1111: 7.2e7 conflicts in 1.55e8 LDS cycles; 3e5 in 8.3e7 with the slots below).
+// sw4 takes rows 0-3, 4-7, 8-11, 12-15 to 0, 2, 3, 1 and sw16 exchanges rows 4-7 and 12-15: one-to-one on both kinds of sixteen.
 __device__ __forceinline__ int sw16(int r) { return r ^ ((r & 4) << 1); }
 
 template <bool UP, int POS>
@@ -135,10 +135,13 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
       dma16(pw[i - 6] + (size_t)kc * 64, uni(st + (uint32_t)wave * 2048 + (i - 6) * 1024));
     }
   };
+  auto fill = [&]() {
 #pragma unroll
-  for (int s = 0; s + 1 < kStages; ++s)
+    for (int s = 0; s + 1 < kStages; ++s)
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) issue_one(s, i);
+      for (int i = 0; i < kLoads; ++i) issue_one(s, i);
+  };
+  fill();
 
   // fragment reads
   const int rdw = r16 * 64 + (part ^ sw4(r16)) * 16;  // the lane's 32 nibbles: row r16, group `part` of the block
@@ -163,8 +166,8 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   u32x4_t raw[2];
   I4Group grp[2];
   uint32_t uz[2];
-  bool large = false;  // (the same in every lane) the opened block holds a scale that i4x8_to_bf16 is not for
-  auto open_block = [&](int kb) {  // the lane's raw words, scale and -(zero point * scale) of the wave's two tiles of block kb
+  float smax = 0.f;  // the largest scale that this lane has met (in magnitude; a NaN decodes to NaN by either routine)
+  auto open_block = [&](int kb) {  // the lane's raw words, scale and zero point of the wave's two tiles of block kb
     const uint8_t* st = smem + (size_t)(kb % kStages) * kStageBytes;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -172,26 +175,17 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
       uz[t] = (*reinterpret_cast<const uint32_t*>(st + kStageW + kStageX + kStageS + wave * 64 + t * 32 + rdz) >> zsh) & 15u;
       grp[t] = i4_group(bf16_bits_to_f32(*reinterpret_cast<const uint16_t*>(st + kStageW + kStageX + wave * 256 + t * 128 + rds)), uz[t]);
     }
-    large = i4_any_large(fmaxf(fabsf(grp[0].s), fabsf(grp[1].s)));
+    smax = fmaxf(smax, fmaxf(fabsf(grp[0].s), fabsf(grp[1].s)));
   };
-  auto piece = [&](u32x4_t (&fa)[2][4], int pc) {  // piece pc = 4 t + j of the opened block
+  auto piece = [&](auto any, u32x4_t (&fa)[2][4], int pc) {  // piece pc = 4 t + j of the opened block
     const int t = pc >> 2, j = pc & 3;
+    const uint32_t w = j == 0 ? raw[t].x : j == 1 ? raw[t].y : j == 2 ? raw[t].z : raw[t].w;
     uint32_t o[4];
-    i4x8_to_bf16(j == 0 ? raw[t].x : j == 1 ? raw[t].y : j == 2 ? raw[t].z : raw[t].w, grp[t], o);
+    if constexpr (decltype(any)::value) i4x8_to_bf16_any(w, grp[t].s, -((float)uz[t] * grp[t].s), o);
+    else i4x8_to_bf16(w, grp[t], o);
     fa[t][j] = u32x4_t{o[0], o[1], o[2], o[3]};
   };
-  // a block with a scale of 2^116 or more (none in a checkpoint): its pieces once more, by the routine for every scale
-  auto redo = [&](u32x4_t (&fa)[2][4]) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        uint32_t o[4];
-        i4x8_to_bf16_any(j == 0 ? raw[t].x : j == 1 ? raw[t].y : j == 2 ? raw[t].z : raw[t].w, grp[t].s, -((float)uz[t] * grp[t].s), o);
-        fa[t][j] = u32x4_t{o[0], o[1], o[2], o[3]};
-      }
-  };
-  auto run = [&](auto nj_c) {
+  auto run = [&](auto nj_c, auto any) {  // any: decode by the routine for every scale
     constexpr int NJ = decltype(nj_c)::value;
     u32x4_t fa[2][4], fn[2][4];
     // block 0 has landed (the later ones of the first stages may be in flight)
@@ -200,8 +194,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
     __syncthreads();
     open_block(0);
 #pragma unroll
-    for (int pc = 0; pc < 8; ++pc) piece(fa, pc);
-    if (__builtin_expect(large, 0)) redo(fa);
+    for (int pc = 0; pc < 8; ++pc) piece(any, fa, pc);
     auto turn = [&](int kb, u32x4_t (&fa)[2][4], u32x4_t (&fn)[2][4]) {
       // block kb + 1 has landed (four stages: block kb + 2 may be in flight)
       if (brings_x) wait_loads<(kStages - 3) * kLoads>();
@@ -215,7 +208,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
 #pragma unroll
         for (int i = 0; i < kLoads; ++i)
           if (NJ > 0 ? (mt < NJ && i * NJ / kLoads == mt) : mt == 0) issue_one(kb + kStages - 1, i);
-        piece(fn, mt);
+        piece(any, fn, mt);
         if (mt >= NJ) continue;
         u32x4_t fb[4];
 #pragma unroll
@@ -226,7 +219,6 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
           for (int t = 0; t < 2; ++t)
             acc[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf_t, fa[t][j]), __builtin_bit_cast(v8bf_t, fb[j]), acc[t][mt], 0, 0, 0);
       }
-      if (__builtin_expect(large, 0)) redo(fn);
     };
     for (int kb = 0; kb < KB; kb += 2) {  // (two turns a pass: the two fragment buffers swap roles without copies)
       turn(kb, fa, fn);
@@ -234,26 +226,46 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
     }
   };
   switch (nmt) {
-    case 0: run(std::integral_constant<int, 0>{}); break;
-    case 1: run(std::integral_constant<int, 1>{}); break;
-    case 2: run(std::integral_constant<int, 2>{}); break;
-    case 3: run(std::integral_constant<int, 3>{}); break;
+    case 0: run(std::integral_constant<int, 0>{}, std::false_type{}); break;
+    case 1: run(std::integral_constant<int, 1>{}, std::false_type{}); break;
+    case 2: run(std::integral_constant<int, 2>{}, std::false_type{}); break;
+    case 3: run(std::integral_constant<int, 3>{}, std::false_type{}); break;
     default:
       if constexpr (S::kSub == 4) {
-        run(std::integral_constant<int, 4>{});
+        run(std::integral_constant<int, 4>{}, std::false_type{});
       } else {
         switch (nmt) {
-          case 4: run(std::integral_constant<int, 4>{}); break;
-          case 5: run(std::integral_constant<int, 5>{}); break;
-          case 6: run(std::integral_constant<int, 6>{}); break;
-          case 7: run(std::integral_constant<int, 7>{}); break;
-          default: run(std::integral_constant<int, 8>{}); break;
+          case 4: run(std::integral_constant<int, 4>{}, std::false_type{}); break;
+          case 5: run(std::integral_constant<int, 5>{}, std::false_type{}); break;
+          case 6: run(std::integral_constant<int, 6>{}, std::false_type{}); break;
+          case 7: run(std::integral_constant<int, 7>{}, std::false_type{}); break;
+          default: run(std::integral_constant<int, 8>{}, std::false_type{}); break;
         }
       }
       break;
   }
+  // A tile that met a scale which i4x8_to_bf16 is not for (2^116 or more, none in a checkpoint) is done once more, by the routine
+  // for every scale. The turns only keep the maximum: with a vote and the second decode in every turn (two copies in each of
+  // fourteen bodies, 21,500 instructions of gate/up against 16,600) tiles of few positions, which wait for their loads, were
+  // slower than before the fast decode: gate/up at T = 64, hidden 6144, intermediate 2048: 468 -> 492 us, 472 like this.
+  int* met = reinterpret_cast<int*>(smem + kLds);
+  const bool large = i4_any_large(smax);
+  if (lane == 0) met[wave] = large;
   wait_loads<0>();
   __syncthreads();
+  int any_met = 0;
+#pragma unroll
+  for (int i = 0; i < kThreads / 64; ++i) any_met |= met[i];
+  if (__builtin_expect(uni(any_met), 0)) {  // (the same in every wave)
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[t][j] = v4f_t{0.f, 0.f, 0.f, 0.f};
+    fill();
+    run(std::integral_constant<int, S::kSub>{}, std::true_type{});
+    wait_loads<0>();
+    __syncthreads();
+  }
 
   // register q of lane l is weight row 4 (l / 16) + q of the 16-row tile, position l % 16 of the 16 positions
   if (UP) {
