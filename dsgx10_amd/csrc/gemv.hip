@@ -54,9 +54,9 @@ __device__ __forceinline__ void stage_rows(uint4* xs, const GemvArgs& a, float* 
 // order, the same bits) by one wavefront that walks the slices one after the other.
 // Bound by the vector unit (INT4, or from 3 activation rows) or by latency: eight wavefronts a CU in ONE workgroup stage the
 // activations once a CU and keep two wavefronts a SIMD where 64 KB and more of activations left room for one workgroup of
-// four (INT4 6144 x 16384, 4 rows: 36.1 us with four waves, 27.1 with eight, 29.6 with sixteen; FP8 12000 x 8192, 8 rows:
-// 41.6, 33.8, 52.5). Two rows a wavefront: four leave half the waves without a batch or make a longer last round (INT4
-// 16384 x 2048, 1 row: 13.4 against 10.6).
+// four (INT4 6144 x 16384, 4 rows: 36.1 us with four waves, 27.1 with eight - 25.8 since they hold no code of the add + norm
+// prologue -, 29.6 with sixteen; FP8 12000 x 8192, 8 rows: 41.6, 33.8, 52.5). Two rows a wavefront: four leave half the waves
+// without a batch or make a longer last round (INT4 16384 x 2048, 1 row: 13.4 against 10.6).
 template <int FMT, int M, int RB, int D, int NW, bool SPLIT>
 __global__ void __launch_bounds__(NW * 64) k_gemv(GemvArgs a) {
   extern __shared__ uint4 xs[];

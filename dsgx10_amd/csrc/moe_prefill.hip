@@ -865,7 +865,7 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
   g.tile_e = I32(mixed ? o.ord_e : o.mix_e), g.tile_m0 = I32(mixed ? o.ord_m0 : o.mix_m0), g.ntiles = I32(o.nmix), g.off = I32(o.off), g.nrows = T;
   // A whole step runs the shared expert's tiles in the routed experts' launches, in front of them: alone they are a launch
   // of T / 256 x 16 workgroups, a sixteenth of the chip at T = 200, and two more tails (whole call, hidden 4096, intermediate
-  // 2048, 256 experts: T = 200 1058 -> 978 us, T = 8192 3112 -> 3101; same bits).
+  // 2048, 256 experts: T = 17 387 -> 341 us, T = 200 1061 -> 973, T = 2000 1565 -> 1544, T = 8192 within the noise; same bits).
   const int sh_tiles = (T + 255) / 256;
   const bool fused_sh = shared && (cfg.phases & (2 | 4 | 16)) == (2 | 4 | 16);
   if (cfg.phases & (2 | 16)) {
@@ -1022,7 +1022,7 @@ int dsgx_dsk_moe_prefill(const dsgx_dsk_weights* Wt, const uint8_t* xq, const ui
   pfmx::Args g{};
   g.H = H, g.I = I, g.nrows = T, g.limit = cfg.swiglu_limit;
   // a whole step runs the shared expert's tiles in the routed experts' launches, in front of them (as the FP8 layers do;
-  // hidden 5120, intermediate 2304, T = 3000: 1870 -> 1821 us)
+  // hidden 5120, intermediate 2304, T = 17: 417 -> 362 us, T = 600: 1405 -> 1334, T = 3000: 1870 -> 1821)
   const int sh_tiles = (T + 255) / 256;
   const bool fused_sh = shared && (cfg.phases & (2 | 4 | 8)) == (2 | 4 | 8);
   if ((cfg.phases & 2) && shared && !fused_sh) {

@@ -289,9 +289,10 @@ typedef struct dsgx_gemv_seg {
   int32_t ldy;        /* y's row stride in elements */
 } dsgx_gemv_seg;
 /* y[r][n] = sum_k x[r][k] W[n][k]; x bf16 [rows][ldx], rows 1..16, K a multiple of 128 (INT4: of 256).
-   out: DSGX_OUT_*; SwiGLU: rows interleaved gate/up in pairs. splitk 1, 2 or 4 (engine/attn/attn.h:119): with 2 or 4 the
-   waves of a workgroup share a row pair's K range and their sums are added in a fixed order (for matrices of few rows,
-   e.g. the router's; ignored above 32 rows a CU, where whole-K waves already fill the chip). A given splitk always gives
+   out: DSGX_OUT_*; SwiGLU: rows interleaved gate/up in pairs. splitk 1, 2 or 4 (engine/attn/attn.h:119): with 2 or 4 a row's
+   K segments are dealt to that many slices whose sums are added in slice order - by waves that share a workgroup where the matrix
+   is too small for the chip (e.g. the router's), else by one wave, with the same bits; ignored above 32 rows a CU, where
+   whole-K waves already fill the chip. A given splitk always gives
    the same bits; different values add in different orders. */
 DSGX_API int dsgx_gemv(const uint16_t* x, int ldx, int rows, int K, const dsgx_gemv_seg* segs, int nseg, int out,
                        int splitk, void* stream);
