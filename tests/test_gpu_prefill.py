@@ -317,7 +317,7 @@ def test_prefill_int4_lds_staged_kernels_give_the_register_ring_kernels_bits():
 
 
 def test_prefill_int4_scales_above_the_fast_decodes_range():
-    """scales of 2^116 and more make a wave decode the block once more by the routine for every scale: the bits of the
+    """scales of 2^116 and more make a workgroup do its tile once more by the routine for every scale: the bits of the
     register-ring kernel, which has that routine only, in tiles of 128 positions and in ragged ones"""
     import os
     H, I, E, topk, T = 512, 256, 4, 2, 300
