@@ -326,8 +326,9 @@ __device__ __forceinline__ void mf_stream(uint8_t* smem, size_t rows_bytes, uint
       };
       const uint32_t z0 = (e.z.x >> zsh) & 15u, z1 = (e.z.y >> zsh) & 15u;
       // (one row: the stream waits for its loads, not for the vector unit, and the vote costs more than the shorter decode saves:
-      // layers of 6144 x 2048, 168 experts, four of them 215.3 -> 209.4 us with one decode; 5120 x 2048 198.6 -> 192.0; the other
-      // way round at 4096 x 2048, 202.3 -> 205.0. From two rows the shorter decode gains 1%.)
+      // layers of 6144 x 2048, 168 experts, four of them 215.3 -> 209.4 us with one decode. With 96 experts, 28 shapes: 5120 x 2048
+      // 197.6 -> 189.6, 1024 x 2048 98.6 -> 94.8, the others 0-4%, except 1% the other way round at hidden 4096, 200.7 -> 203.0. At two
+      // rows the two are within 2%, at six the shorter decode gains 1%.)
       if (M == 1 || __builtin_expect(i4_any_large(fmaxf(fabsf(s0), fabsf(s1))), 0)) {
         const float n0 = -((float)z0 * s0), n1 = -((float)z1 * s1);
         sums([&](int jj, uint32_t w, uint32_t (&o)[4]) { i4x8_to_bf16_any(w, jj ? s1 : s0, jj ? n1 : n0, o); });
