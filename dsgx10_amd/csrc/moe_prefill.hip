@@ -14,6 +14,7 @@
 // The FP8-activation GEMMs run on v_mfma_f32_16x16x128_f8f6f4 (one instruction a 128-k scale block), the bf16-activation
 // ones on v_mfma_f32_16x16x32_bf16: weights are the A operand (rows n), activations the B operand, so a lane's four
 // accumulators of a 16 x 16 tile belong to ONE token row and the block's combined scale is one value a lane.
+#include <algorithm>
 #include <cstdlib>
 
 #include "abi_internal.h"
@@ -994,13 +995,13 @@ int dsgx_dsk_moe_prefill(const dsgx_dsk_weights* Wt, const uint8_t* xq, const ui
   auto U16 = [&](size_t off) { return reinterpret_cast<uint16_t*>(W + off); };
   const int H = Wt->H, I = Wt->I, E = Wt->E, topk = Wt->topk, P = o.P;
   constexpr int F4 = DSGX_FMT_MXFP4_G32, F8 = DSGX_FMT_FP8_B32E;
-  constexpr int kLdsMix = pfmx::Shape<1, F4>::kLds > pfmx::Shape<2, F4>::kLds ? pfmx::Shape<1, F4>::kLds : pfmx::Shape<2, F4>::kLds;
-  constexpr int kLdsSh = pfmx::Shape<2, F8>::kLds;
-  constexpr int kLdsRun = kLdsMix > kLdsSh ? kLdsMix : kLdsSh;  // (a routed launch may hold the shared expert's tiles)
-  void (*k_up)(pfmx::Args) = pfmx::k_gemm_mixed<true, F4>;
-  void (*k_dn)(pfmx::Args) = pfmx::k_gemm_mixed<false, F4>;
-  void (*k_sup)(pfmx::Args) = pfmx::k_gemm<true, F8>;
-  void (*k_sdn)(pfmx::Args) = pfmx::k_gemm<false, F8>;
+  constexpr int kLdsSh = std::max({pfmx::Shape<256, F8>::kLds, pfmx::Shape<128, F8>::kLds, pfmx::Shape<64, F8>::kLds});
+  constexpr int kLdsRun = std::max({kLdsSh, pfmx::Shape<256, F4>::kLds, pfmx::Shape<128, F4>::kLds, pfmx::Shape<64, F4>::kLds});  // (a routed launch may hold the shared expert's tiles)
+  static_assert(kLdsRun <= 160 * 1024, "a workgroup's LDS");
+  void (*k_up)(pfmx::Args) = pfmx::k_gemm_mixed<true>;
+  void (*k_dn)(pfmx::Args) = pfmx::k_gemm_mixed<false>;
+  void (*k_sup)(pfmx::Args) = pfmx::k_gemm<true>;
+  void (*k_sdn)(pfmx::Args) = pfmx::k_gemm<false>;
   for (const void* k : {(const void*)k_up, (const void*)k_dn})
     if (int rc = allow_dynamic_lds(k, kLdsRun)) return rc;
   for (const void* k : {(const void*)k_sup, (const void*)k_sdn})

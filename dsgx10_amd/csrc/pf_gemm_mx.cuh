@@ -8,8 +8,8 @@
 //
 // The tiling, the LDS staging by global_load_lds (lane-permuted sources so that the fragment reads are conflict-free),
 // the hand-counted waits and the workgroup -> (tile, row group) map are those of pf_gemm_fp8.cuh; what differs:
-//   * a weight row of a 128-k block is 64 bytes (e2m1) - four lanes a row, piece q of row r at slot q ^ sw4(r);
-//   * the scales travel with the block: 4 bytes a weight row and 4 a position, read back a byte a lane (ds_read_u8);
+//   * a weight row of a 128-k block is 64 bytes (e2m1) - four lanes a row, piece q of row r at slot q ^ sw4(r) -, or 128 of two blocks;
+//   * the scales come in words of four blocks' bytes a weight row and a position, read back a word a lane;
 //   * UP's epilogue is DeepSeek's: gate, up rounded to bf16, up clamped to +-limit and gate from above, silu(gate) * up
 //     times the position's routing weight (none for the shared expert), rounded to bf16, then quantised per 32 channels
 //     (ue8m0) for the down projection; DOWN rounds each position's outputs to bf16 (the reference's per-pick rounding).
@@ -29,19 +29,35 @@ using pf8::v4f_t;
 using pf8::v8i_t;
 using pf8::wait_loads;
 
-template <int WP, int WF>
+// A tile's shape by its positions (64, 128 or 256) and its weights' format. What a turn waits for is the way of its operands into
+// LDS, and there the lines that a load instruction names count as much as its bytes (hidden 5120, intermediate 2304, 256
+// experts of 32 rows each, gate/up 895 us before):
+//   * a scale word of 4 bytes a row and block named 32 lines for 128 bytes; e2m1 experts' scale words therefore come for four
+//     blocks at a time, 16 bytes a row, into two buffers of their own (with no scale loads at all 640 us, with those a
+//     block 729 with coalesced stand-ins); e4m3 rows share a word by 32 and keep theirs with the block;
+//   * half a line a weight row and block (e2m1: 64 bytes) named every line twice: tiles of up to 64 positions, whose weights are
+//     most of their bytes, take two blocks a turn and whole lines (the larger shapes: 2% at 192 rows an expert, and LDS holds
+//     three stages of one block only).
+// Together 895 -> 693 us; the whole call at T = 3000 (Zipf) 1777 -> 1546, at T = 300 1115 -> 878. Four to eight stages instead of
+// three return nothing, two cost 15%.
+template <int POS, int WF>
 struct Shape {
   static constexpr bool F4 = WF == DSGX_FMT_MXFP4_G32;
-  static constexpr int kPos = 128 * WP, kSub = 8 * WP, WR = 8 / WP, RA = 2 * WP;
-  static constexpr int kRowB = F4 ? 64 : 128;       // bytes of a weight row in a 128-k block
+  static constexpr int WP = POS == 256 ? 2 : 1;     // position groups of waves
+  static constexpr int kPos = POS, kSub = POS / 16, WR = 8 / WP, RA = 2 * WP;
+  static constexpr int TB = F4 && POS <= 64 ? 2 : 1;  // 128-k blocks a turn
+  static constexpr int kRowB = F4 ? 64 * TB : 128;  // bytes of a weight row in a turn
   static constexpr int kStageW = kWgRows * kRowB;
-  static constexpr int kStageX = kPos * 128;
-  static constexpr int kStageWS = kWgRows * 4;      // the weight rows' four scale bytes of the block
-  static constexpr int kStageXS = kPos * 4;         // the positions'
-  static constexpr int kStageBytes = kStageW + kStageX + kStageWS + kStageXS;
-  static constexpr int kStages = 3 * kStageBytes <= 160 * 1024 ? 3 : 2;
-  static constexpr int kLoads = (F4 ? 2 : 4) + 2 * WP + 2;  // a wave's loads a turn: weights, activations, the two scale words
-  static constexpr int kLds = kStages * kStageBytes;        // (the epilogues reuse it: UP kPos x 256 B, DOWN 8 x 2 WP KiB)
+  static constexpr int kStageX = kPos * 128;        // one block's activations
+  static constexpr int kStageBytes = kStageW + TB * kStageX;
+  static constexpr int kWords = F4 ? 4 : 1;         // blocks whose scale words come together
+  static constexpr int kGroupW = kWgRows * 4 * kWords, kGroupX = kPos * 4 * kWords;  // their scale words: the weight rows', the positions'
+  static constexpr int kGroup = kGroupW + kGroupX, kGroups = F4 ? 2 : 3;  // (e4m3: a buffer a stage)
+  static constexpr int kStages = 3 * kStageBytes + kGroups * kGroup <= 160 * 1024 ? 3 : 2;
+  static constexpr int kLoadsW = kRowB == 64 ? 2 : 4;       // a wave's loads a turn: its two weight tiles ...
+  static constexpr int kHalfX = kPos / 64;                  // ... and its half tiles of eight positions, a load a block
+  static constexpr int kLoads = kLoadsW + TB * kHalfX + (F4 ? 0 : 2);  // (e4m3: and its two loads of scale words)
+  static constexpr int kLds = kStages * kStageBytes + kGroups * kGroup;  // (the epilogues reuse it: UP kPos x 256 B, DOWN 8 x 2 WP KiB)
 };
 
 // The shared expert's side of a launch that holds its tiles too (k_gemm_mixed): the first `grid` workgroups are theirs
@@ -85,10 +101,11 @@ __device__ __forceinline__ v4f_t mfma_mx(v8i_t a, v8i_t b, v4f_t c, int sa, int 
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, CBSZ, 0, 0, sa, 0, sb);
 }
 
-template <bool UP, int WP, int WF>
+template <bool UP, int POS, int WF>
 __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, int m0, int mend, int ns) {
-  using S = Shape<WP, WF>;
+  using S = Shape<POS, WF>;
   constexpr bool F4 = S::F4;
+  constexpr int WP = S::WP, kPosWave = S::kPos / 8;
   constexpr int CBSZ = F4 ? 4 : 0;
   const int K = UP ? g.H : g.I, KB = K / 128, G = K / 32;
   if (mend > m0 + S::kPos) mend = m0 + S::kPos;
@@ -108,17 +125,17 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   };
   const int nmt = uni(min(S::kSub, (mend - m0 + 15) / 16));
   const int nj = uni(nmt > pg ? (nmt - pg + WP - 1) / WP : 0);
-
   // ---- what this lane fetches ----
-  // weights: the wave brings tiles 2 wave, 2 wave + 1. e2m1: one instruction a tile, lane -> row lane / 4, piece
-  // (lane % 4) ^ sw4(row); e4m3: two instructions a tile (rows 0-7, 8-15), lane -> row lane / 8, piece (lane % 8) ^ swz(row)
+  // weights: the wave brings tiles 2 wave, 2 wave + 1. 64-byte rows: one instruction a tile, lane -> row lane / 4, piece
+  // (lane % 4) ^ sw4(row); 128-byte rows: two instructions a tile (rows 0-7, 8-15), lane -> row lane / 8, piece (lane % 8) ^
+  // swz(row) (e4m3) or (lane % 8) ^ (row % 8) (two blocks of e2m1, whose lanes read pieces part and 4 + part)
   const uint8_t* pw[2][2];
-  const uint8_t* pws;  // lanes 0-31: the scale word of row lane % 16 of tile 2 wave + lane / 16
+  const uint8_t* pws;  // lanes 0-31: the scale words of row lane % 16 of tile 2 wave + lane / 16
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
     const uint8_t *wbase, *sbase;
     const int row = tile_row(2 * wave + t, wbase, sbase);
-    if (F4) {
+    if (S::kRowB == 64) {
       const int r = lane >> 2;
       pw[t][0] = wbase + (size_t)(row + r) * (K / 2) + 16 * ((lane & 3) ^ sw4(r));
       pw[t][1] = pw[t][0];
@@ -126,57 +143,76 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh) {
         const int r = 8 * hh + (lane >> 3);
-        pw[t][hh] = wbase + (size_t)(row + r) * K + 16 * pc8((lane & 7) ^ swz(r));
+        pw[t][hh] = F4 ? wbase + (size_t)(row + r) * (K / 2) + 16 * ((lane & 7) ^ (r & 7)) : wbase + (size_t)(row + r) * K + 16 * pc8((lane & 7) ^ swz(r));
       }
     }
     if (((lane >> 4) & 1) == t) pws = sbase + (size_t)(F4 ? row + r16 : (row + r16) / 32) * G;
   }
-  const int lr = lane >> 3, lq = lane & 7;
-  const uint8_t* px[WP][2];
+  // activations: half tile kHalfX wave + i is positions 8 (kHalfX wave + i) ...; a wave whose half tiles hold no rows brings none
+  const bool brings_x = POS > 64 || m0 + 8 * wave < mend;
+  auto row_of = [&](int p) {  // the activation row of the tile's position p (a ragged tile re-reads its last row: never stored)
+    const int pos = min(m0 + p, mend - 1);
+    return (size_t)(g.gather ? g.gather[pos] : pos);
+  };
+  const uint8_t* px[S::kHalfX];
 #pragma unroll
-  for (int t = 0; t < WP; ++t)
-#pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      const int r = 8 * hh + lr;
-      int pos = m0 + 16 * (WP * wave + t) + r;
-      if (pos >= mend) pos = mend - 1;
-      px[t][hh] = g.aq + (size_t)(g.gather ? g.gather[pos] : pos) * K + 16 * pc8(lq ^ swz(r));
-    }
-  const uint8_t* pxs;  // lanes 0 .. 16 WP - 1: the scale word of position 16 WP wave + lane
-  {
-    int pos = m0 + 16 * WP * wave + (lane & (16 * WP - 1));
-    if (pos >= mend) pos = mend - 1;
-    pxs = g.as + (size_t)(g.gather ? g.gather[pos] : pos) * G;
+  for (int i = 0; i < S::kHalfX; ++i) {
+    const int p = 8 * (S::kHalfX * wave + i) + (lane >> 3);
+    px[i] = g.aq + row_of(p) * K + 16 * pc8((lane & 7) ^ swz(p & 15));
   }
+  const uint8_t* pxs = g.as + row_of(kPosWave * wave + (lane & (kPosWave - 1))) * G;  // lanes 0 .. kPosWave - 1: the scale words of the wave's positions
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
-  // load number i (0 .. kLoads - 1) of block kb: the two scale words, the activations (L2 hits mostly), the weights last: a
-  // wave's loads return in issue order, so a load that waits for HBM holds back every later one of its wave and the
-  // cache's miss slots with them (weights first: 7% slower, measured). A turn issues them one at a time between its MFMAs (issue_some), so that the
+  constexpr int kGroups0 = S::kStages * S::kStageBytes;  // the groups' scale words behind the stages
+  // load number i (0 .. kLoads - 1) of turn t: the activations (L2 hits mostly), the weights last: a wave's loads return in
+  // issue order, so a load that waits for HBM holds back every later one of its wave and the cache's miss slots with them
+  // (weights first: 7% slower, measured). A turn issues them one at a time between its MFMAs (issue_some), so that the
   // texture unit works through a block's 50 KB while the matrix unit runs instead of in front of it: issued together after
   // the barrier they cost every wave the time the unit takes to accept them all (measured: a third of a turn).
-  auto issue_one = [&](int kb, int i) {
-    const int kc = kb < KB ? kb : KB - 1;
-    const uint32_t st = lds0 + (uint32_t)(kb % S::kStages) * S::kStageBytes;
-    const uint32_t wbase = st + (uint32_t)wave * (2 * 16 * S::kRowB), xbase = st + S::kStageW + (uint32_t)wave * (2048 * WP);
-    if (i == 0) {
-      if (lane < 16 * WP) dma4(reinterpret_cast<const float*>(pxs + 4 * kc), uni(st + S::kStageW + S::kStageX + S::kStageWS + (uint32_t)wave * (64 * WP)));
-    } else if (i == 1) {
-      if (lane < 32) dma4(reinterpret_cast<const float*>(pws + 4 * kc), uni(st + S::kStageW + S::kStageX + (uint32_t)wave * 128));
-    } else if (i < 2 + 2 * WP) {
-      const int q = i - 2;
-      dma16(px[q >> 1][q & 1] + (size_t)kc * 128, uni(xbase + (q >> 1) * 2048 + (q & 1) * 1024));
+  const int TN = KB / S::TB;
+  constexpr int kFirst = F4 ? 0 : 2;  // (e4m3: the turn's scale words in front; 32 weight rows share a word, so they name few lines)
+  auto issue_one = [&](int t, int i) {
+    const int tc = t < TN ? t : TN - 1;  // (past the end: the last turn again, into a stage nobody reads)
+    const uint32_t st = lds0 + (uint32_t)(t % S::kStages) * S::kStageBytes;
+    const uint32_t wbase = st + (uint32_t)wave * (2 * 16 * S::kRowB), xbase = st + S::kStageW + (uint32_t)wave * (S::kHalfX * 1024);
+    if (i < kFirst) {
+      const uint32_t at = lds0 + kGroups0 + (uint32_t)(t % S::kStages) * S::kGroup;
+      if (i == 0) {
+        if (brings_x && lane < kPosWave) dma4(reinterpret_cast<const float*>(pxs + 4 * tc), uni(at + S::kGroupW + (uint32_t)wave * (4 * kPosWave)));
+      } else {
+        if (lane < 32) dma4(reinterpret_cast<const float*>(pws + 4 * tc), uni(at + (uint32_t)wave * 128));
+      }
+    } else if (i < kFirst + S::TB * S::kHalfX) {
+      const int b = (i - kFirst) / S::kHalfX, q = (i - kFirst) % S::kHalfX;
+      if (brings_x) dma16(px[q] + (size_t)tc * (128 * S::TB) + 128 * b, uni(xbase + b * S::kStageX + q * 1024));
     } else {
-      const int q = i - 2 - 2 * WP;
-      if (F4) dma16(pw[q][0] + (size_t)kc * 64, uni(wbase + q * 1024));
-      else dma16(pw[q >> 1][q & 1] + (size_t)kc * 128, uni(wbase + (q >> 1) * 2048 + (q & 1) * 1024));
+      const int q = i - kFirst - S::TB * S::kHalfX;
+      if (S::kRowB == 64) dma16(pw[q][0] + (size_t)tc * 64, uni(wbase + q * 1024));
+      else dma16(pw[q >> 1][q & 1] + (size_t)tc * 128, uni(wbase + (q >> 1) * 2048 + (q & 1) * 1024));
     }
   };
-  auto issue = [&](int kb) {
-#pragma unroll
-    for (int i = 0; i < S::kLoads; ++i) issue_one(kb, i);
+  // e2m1: the scale words of the group that turn t opens (blocks 4 q ... 4 q + 3; the last ones of a row from its end): two loads
+  // a wave. Rows of fewer than four blocks have no 16 bytes: their words are put in place by hand.
+  constexpr int kGroupTurns = 4 / S::TB;
+  auto first_block = [&](int q) { return min(4 * q, KB - 4); };
+  auto issue_scales = [&](int t) {
+    const int q = t / kGroupTurns, kb = first_block(q);
+    const uint32_t at = lds0 + kGroups0 + (uint32_t)(q & 1) * S::kGroup;
+    if (lane < 32) dma16(pws + 4 * kb, uni(at + (uint32_t)wave * 512));
+    if (brings_x && lane < kPosWave) dma16(pxs + 4 * kb, uni(at + S::kGroupW + (uint32_t)wave * (16 * kPosWave)));
   };
+  if (F4 && KB >= 4) {
+    issue_scales(0);
+  } else if (F4) {
+    for (int kb = 0; kb < KB; ++kb) {
+      uint32_t* at = reinterpret_cast<uint32_t*>(smem + kGroups0) + kb;
+      if (lane < 32) at[(32 * wave + lane) * 4] = ldg_u32(pws + 4 * kb);
+      if (lane < kPosWave) at[S::kGroupW / 4 + (kPosWave * wave + lane) * 4] = ldg_u32(pxs + 4 * kb);
+    }
+  }
 #pragma unroll
-  for (int s = 0; s + 1 < S::kStages; ++s) issue(s);
+  for (int s = 0; s + 1 < S::kStages; ++s)
+#pragma unroll
+    for (int i = 0; i < S::kLoads; ++i) issue_one(s, i);
 
   // fragment reads. The instruction numbers an 8-bit operand's k as 64 h + 16 part + i (h: the lane's first or second four
   // registers, i: the byte) and a 4-bit operand's as 32 part + i, and takes the scale of k block g = k / 32 from the lanes
@@ -186,15 +222,17 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   const int rd0 = (r16 >> 3) * 1024 + (r16 & 7) * 128 + ((2 * part) ^ swz(r16)) * 16;
   const int rd1 = (r16 >> 3) * 1024 + (r16 & 7) * 128 + ((2 * part + 1) ^ swz(r16)) * 16;
   const int rd4 = r16 * 64 + (part ^ sw4(r16)) * 16;
+  const int rd4b[2] = {(r16 >> 3) * 1024 + (r16 & 7) * 128 + (part ^ (r16 & 7)) * 16, (r16 >> 3) * 1024 + (r16 & 7) * 128 + ((4 + part) ^ (r16 & 7)) * 16};
   auto frag8 = [&](const uint8_t* t) {
     const u32x4_t lo = *reinterpret_cast<const u32x4_t*>(t + rd0), hi = *reinterpret_cast<const u32x4_t*>(t + rd1);
     return v8i_t{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
   };
-  auto frag4 = [&](const uint8_t* t) {
-    const u32x4_t lo = *reinterpret_cast<const u32x4_t*>(t + rd4);
+  auto frag4 = [&](const uint8_t* t, int b) {
+    const u32x4_t lo = *reinterpret_cast<const u32x4_t*>(t + (S::TB == 2 ? rd4b[b] : rd4));
     return v8i_t{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, 0, 0, 0, 0};
   };
-  const int rds = r16 * 4;         // the lane's row's scale word within a 16-row (16-position) tile's 64 bytes; its byte: `part`
+  constexpr int kScaleT = 64 * S::kWords;   // bytes of a 16-row (16-position) tile's scale words
+  const int rds = r16 * (4 * S::kWords);    // the lane's row's among them; its byte: `part`
   const int rsh = 8 * part;
 
   v4f_t acc[S::RA][8];
@@ -205,52 +243,64 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
 
   auto run = [&](auto nj_c) {
     constexpr int NJ = decltype(nj_c)::value;
-    for (int kb = 0; kb < KB; ++kb) {
-      wait_loads<(S::kStages - 2) * S::kLoads>();
+    for (int t = 0; t < TN; ++t) {
+      // turn t's loads have landed; with three stages turn t + 1's may be in flight (the scale words of the group that it opens,
+      // which come first, are waited for: a count of its own for those turns is a branch in every turn and 1% slower)
+      if (S::kStages == 2) wait_loads<0>();
+      else if (brings_x) wait_loads<S::kLoads>();
+      else wait_loads<S::kLoadsW + kFirst / 2>();
       __syncthreads();
-      if (NJ == 0) issue(kb + S::kStages - 1);
-      if (NJ == 0) continue;
-      // loads i with i * NJ / kLoads == j go out after the fragment reads of 16-position tile j
+      const int tn = t + S::kStages - 1;
+      // loads i with i * NJ / kLoads == j go out after the fragment reads of 16-position tile j, a group's scale words after the
+      // first tile's (in front of the turn's first reads they cost the 256-position tiles 2%, at its end every shape 4%)
       auto issue_some = [&](int j) {
+        if (F4 && j == 0 && tn % kGroupTurns == 0 && tn < TN) issue_scales(tn);
 #pragma unroll
         for (int i = 0; i < S::kLoads; ++i)
-          if (i * (NJ > 0 ? NJ : 1) / S::kLoads == j) issue_one(kb + S::kStages - 1, i);
+          if (i * (NJ > 0 ? NJ : 1) / S::kLoads == j) issue_one(tn, i);
       };
-      const uint8_t* st = smem + (size_t)(kb % S::kStages) * S::kStageBytes;
+      if (NJ == 0) issue_some(0);
+      if (NJ == 0) continue;
+      const uint8_t* st = smem + (size_t)(t % S::kStages) * S::kStageBytes;
       const uint8_t* W = st + S::RA * rg * (16 * S::kRowB);
       const uint8_t* X = st + S::kStageW + pg * 2048;
-      const uint8_t* WS = st + S::kStageW + S::kStageX + S::RA * rg * 64 + rds;
-      const uint8_t* XS = st + S::kStageW + S::kStageX + S::kStageWS + pg * 64 + rds;
-      v8i_t fa[S::RA];
-      int fs[S::RA];
+      const int q = t / kGroupTurns, word = S::TB * t - (KB >= 4 ? first_block(q) : 0);  // e2m1: the turn's first word of its group's
+      const uint8_t* GS = smem + kGroups0 + (F4 ? (size_t)(q & 1) * S::kGroup + 4 * word : (size_t)(t % S::kStages) * S::kGroup);
+      const uint8_t* WS = GS + S::RA * rg * kScaleT + rds;
+      const uint8_t* XS = GS + S::kGroupW + pg * kScaleT + rds;
+      v8i_t fa[S::TB][S::RA];
+      int fs[S::TB][S::RA];
 #pragma unroll
-      for (int t = 0; t < S::RA; ++t) {
-        fa[t] = F4 ? frag4(W + t * 1024) : frag8(W + t * 2048);
-        fs[t] = (*reinterpret_cast<const uint32_t*>(WS + t * 64) >> rsh) & 0xFFu;
-      }
+      for (int b = 0; b < S::TB; ++b)
+#pragma unroll
+        for (int i = 0; i < S::RA; ++i) {
+          fa[b][i] = F4 ? frag4(W + i * (16 * S::kRowB), b) : frag8(W + i * 2048);
+          fs[b][i] = (*reinterpret_cast<const uint32_t*>(WS + i * kScaleT + 4 * b) >> rsh) & 0xFFu;
+        }
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
-        const v8i_t fb = frag8(X + j * (2048 * WP));
-        const int xsb = (*reinterpret_cast<const uint32_t*>(XS + j * (64 * WP)) >> rsh) & 0xFFu;
+        v8i_t fb[S::TB];
+        int xsb[S::TB];
+#pragma unroll
+        for (int b = 0; b < S::TB; ++b) {
+          fb[b] = frag8(X + b * S::kStageX + j * (2048 * WP));
+          xsb[b] = (*reinterpret_cast<const uint32_t*>(XS + j * (kScaleT * WP) + 4 * b) >> rsh) & 0xFFu;
+        }
         issue_some(j);
 #pragma unroll
-        for (int t = 0; t < S::RA; ++t) {
-          acc[t][j] = mfma_mx<CBSZ>(fa[t], fb, acc[t][j], fs[t], xsb);
-        }
+        for (int b = 0; b < S::TB; ++b)
+#pragma unroll
+          for (int i = 0; i < S::RA; ++i) acc[i][j] = mfma_mx<CBSZ>(fa[b][i], fb[b], acc[i][j], fs[b][i], xsb[b]);
       }
     }
   };
-  switch (nj) {
-    case 0: run(std::integral_constant<int, 0>{}); break;
-    case 1: run(std::integral_constant<int, 1>{}); break;
-    case 2: run(std::integral_constant<int, 2>{}); break;
-    case 3: run(std::integral_constant<int, 3>{}); break;
-    case 4: run(std::integral_constant<int, 4>{}); break;
-    case 5: run(std::integral_constant<int, 5>{}); break;
-    case 6: run(std::integral_constant<int, 6>{}); break;
-    case 7: run(std::integral_constant<int, 7>{}); break;
-    default: run(std::integral_constant<int, 8>{}); break;
-  }
+  constexpr int kMaxNJ = S::kSub / WP, kMinNJ = WP == 2 ? 0 : 1;
+  auto run_nj = [&](auto self, auto n) {
+    constexpr int N = decltype(n)::value;
+    if (N == kMaxNJ || nj == N) run(n);
+    else if constexpr (N < kMaxNJ) self(self, std::integral_constant<int, N + 1>{});
+  };
+  run_nj(run_nj, std::integral_constant<int, kMinNJ>{});
   wait_loads<0>();
   __syncthreads();
 
@@ -337,40 +387,49 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   }
 }
 
+// The tile of the shared expert's rows from m0 on (e4m3 weights), in the smallest shape that holds them
+template <bool UP>
+__device__ __forceinline__ void shared_tile(const Args& g, uint8_t* smem, int m0, int mend, int ns) {
+  constexpr int F8 = DSGX_FMT_FP8_B32E;
+  if (mend - m0 > 128) gemm_tile<UP, 256, F8>(g, smem, -1, m0, mend, ns);
+  else if (mend - m0 > 64) gemm_tile<UP, 128, F8>(g, smem, -1, m0, mend, ns);
+  else gemm_tile<UP, 64, F8>(g, smem, -1, m0, mend, ns);
+}
 // The shared expert (tile_e null: tiles of 256 rows over [0, nrows)).
-template <bool UP, int WF>
+template <bool UP>
 __global__ void __launch_bounds__(kThreads) k_gemm(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int NS = UP ? g.I / (kWgRows / 2) : g.H / kWgRows;
   int tile, ns;
   pf8::task_of<true>(NS, tile, ns);
-  if (ns >= NS) return;
-  const int m0 = tile * Shape<2, WF>::kPos, mend = g.nrows;
-  if (m0 >= mend) return;
-  gemm_tile<UP, 2, WF>(g, smem, -1, m0, mend, ns);
+  if (ns >= NS || tile * 256 >= g.nrows) return;
+  shared_tile<UP>(g, smem, tile * 256, g.nrows, ns);
 }
 // The routed experts' list of both tile shapes (bit 30 of tile_e: a 256-position tile), an expert's tiles next to each other.
-template <bool UP, int WF>
+// A remainder of up to 64 rows runs two blocks a turn where K is pairs of blocks.
+template <bool UP>
 __global__ void __launch_bounds__(kThreads) k_gemm_mixed(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  constexpr int F4 = DSGX_FMT_MXFP4_G32;
   const int NS = UP ? g.I / (kWgRows / 2) : g.H / kWgRows;
   int tile, ns;
   if (blockIdx.x < g.sh.grid) {  // (the same for the whole workgroup)
     pf8::task_of<true>(NS, tile, ns);
-    const int m0 = tile * Shape<2, DSGX_FMT_FP8_B32E>::kPos, mend = g.nrows;
-    if (ns >= NS || m0 >= mend) return;
+    if (ns >= NS || tile * 256 >= g.nrows) return;
     Args q = g;
     q.aq = g.sh.aq, q.as = g.sh.as, q.gather = nullptr, q.posw = nullptr, q.wstride = q.sstride = 0;
     q.wa = g.sh.wa, q.sa = g.sh.sa, q.wb = g.sh.wb, q.sb = g.sh.sb, q.h = g.sh.h, q.hq = g.sh.hq, q.hs = g.sh.hs, q.d = g.sh.d;
-    gemm_tile<UP, 2, DSGX_FMT_FP8_B32E>(q, smem, -1, m0, mend, ns);
+    shared_tile<UP>(q, smem, tile * 256, g.nrows, ns);
     return;
   }
   pf8::task_of<false>(NS, tile, ns, blockIdx.x - g.sh.grid);
   if (ns >= NS || tile >= *g.ntiles) return;
   const int te = g.tile_e[tile], e = te & 0xFFFF;
   const int m0 = g.off[e] + g.tile_m0[tile], mend = g.off[e + 1];
-  if (te >> 30) gemm_tile<UP, 2, WF>(g, smem, e, m0, mend, ns);
-  else gemm_tile<UP, 1, WF>(g, smem, e, m0, mend, ns);
+  const bool pairs = (UP ? g.H : g.I) % 256 == 0;
+  if (te >> 30) gemm_tile<UP, 256, F4>(g, smem, e, m0, mend, ns);
+  else if (mend - m0 <= 64 && pairs) gemm_tile<UP, 64, F4>(g, smem, e, m0, mend, ns);
+  else gemm_tile<UP, 128, F4>(g, smem, e, m0, mend, ns);
 }
 
 }  // namespace pfmx

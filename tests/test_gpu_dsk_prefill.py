@@ -208,6 +208,20 @@ def test_dsk_prefill_against_oracle(H, I, E, T, shared):
         assert np.array_equal(gpu.host(y2, np.uint32, (T, H)), got["y"].view(np.uint32))
 
 
+@pytest.mark.parametrize("H,I,T", [(256, 128, 17), (256, 384, 10), (512, 640, 64), (768, 1152, 90), (1024, 1280, 33)])
+def test_dsk_prefill_scale_groups_and_block_pairs(H, I, T):
+    """The scale words come for four 128-k blocks at a time and small tiles take blocks by pairs: rows of K with fewer than four
+    blocks (1, 2, 3), with a last group that is not whole (5, 6, 9, 10), odd numbers of blocks; 8 to 64 positions and over"""
+    E, topk = 8, 6
+    L = Stacked(43, H, I, E, topk, 5, True)
+    x = orc.normal_bf16(43, 1, (T, H), 1.5)
+    idx, w = orc.route(orc.normal_f32(43, 2, (T, E), 1.0), orc.normal_f32(43, 3, (E,), 0.2), topk, 1.5, score_fn=1)
+    xq, xs = orc.act_quant_ue8m0(x)
+    # (end to end: a bf16 step of one of h's few values is a larger part of a short row; the stages are checked bit for bit)
+    check_chunk(L, x, idx, w, sorted({0, T // 2, T - 1}), run_prefill(L, xq, xs, idx, w), e2e=1e-2)
+
+
+
 def test_dsk_prefill_refuses_what_it_cannot_run():
     L = Stacked(42, 1024, 512, 16, 6, 2, False)
     xq = gpu.empty(4 * 1024, 0)
