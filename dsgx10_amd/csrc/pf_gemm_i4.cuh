@@ -4,9 +4,9 @@
 //
 // The structure is pf_gemm_fp8.cuh's: a workgroup (8 waves) computes up to 128 positions against 256 weight rows (UP: 128
 // channels, gate and up), a wave 32 rows x every position; both operands and the weights' scales and zero points go from
-// memory straight into a stage of LDS (global_load_lds, three stages of one 128-k block, hand-counted waits, one workgroup
-// barrier a block), a turn's loads are issued one at a time between its MFMAs. What is its own:
-//   * a weight row of a block is 64 bytes of packed nibbles (four lanes a row, piece q of row r at slot q ^ sw4(r));
+// memory straight into rings in LDS (global_load_lds, hand-counted waits, one workgroup barrier a 128-k block), a turn's loads
+// are issued one at a time between its MFMAs. What is its own:
+//   * a weight row of a block is 64 bytes of packed nibbles (four lanes a row, piece q of row r at slot q ^ sw4(r)), or 128 of two;
 //     lane (row, part) reads ONE piece = the 32 values of one scale group, its bf16 scale and its zero-point word, decodes
 //     them in registers (the decode kernels' routine: one rounding of the exact product) into the A fragments of four MFMAs;
 //     MFMA j takes the lane's values 8 j .. 8 j + 7, i.e. k = 32 part + 8 j + [0, 8), and the activation fragment of MFMA j
@@ -32,24 +32,28 @@ using pf8::v4f_t;
 using pf8::wait_loads;
 typedef __bf16 v8bf_t __attribute__((ext_vector_type(8)));
 
-constexpr int kStageW = kWgRows * 64;        // 16 KiB of nibbles
-constexpr int kStageS = kWgRows * 8;         // four bf16 scales a row
-constexpr int kStageZ = (kWgRows / 8) * 16;  // four zero-point words a group of eight rows
-// A tile's shape by its positions: 128 (three stages), or 64 for the tiles that hold no more rows (four stages). What a
-// turn waits for is the trip to HBM of a block's 18.5 KB of weights, scales and zero points, not their rate (9 GB/s a CU):
-// with three stages a block has one turn to land (it is decoded a turn ahead), with four it has two. Most tiles of a
-// chunk of 2048 rows are such tiles (the median bucket holds 34 rows).
+// A tile's shape by its positions: 64 or 128. LDS holds three rings of three slots each: activations (a slot a 128-k block),
+// nibbles (64: a slot two blocks, whole lines of a weight row; 128: a block) and the scales and zero points of two blocks. A
+// wave's weights, scales and zero points are its own, so their slot is free as soon as the wave has opened the block, a turn
+// before its MFMAs: a load has two turns to land in either shape.
+// What the launch waits for besides is the lines that its loads name (pf_gemm_mx.cuh): 8 bytes of scales a row and block were 32
+// lines an instruction, 64 bytes of weights a row and block named every line twice. Hidden 6144, intermediate 2048, 168
+// experts, gate/up with 16 / 32 / 64 / 128 rows an expert: 686 / 741 / 855 / 1301 us with a stage of every operand a block and its
+// scales in it, 606 / 690 / 840 / 1180 like this (with the weights in the caches 540 / 600 / 742 / 1032).
 template <int POS>
 struct Shape {
   static constexpr int kPos = POS;
-  static constexpr int kSub = POS / 16;                  // its 16-position tiles: waves 0 .. kSub - 1 bring one each
-  static constexpr int kStageX = POS * 256;              // bf16 rows of the block
-  static constexpr int kStageBytes = kStageW + kStageX + kStageS + kStageZ;  // 51,712 | 35,328
-  static constexpr int kStages = POS == 128 ? 3 : 4;
-  static constexpr int kLds = kStages * kStageBytes;     // (the epilogues reuse it: UP POS x 256 B, DOWN 8 x 2 KiB)
+  static constexpr int kSub = POS / 16;
+  static constexpr bool kPair = POS == 64;               // two blocks a weight slot
+  static constexpr int kX = POS * 256;                   // bf16 rows of a block
+  static constexpr int kW = kWgRows * (kPair ? 128 : 64);
+  static constexpr int kS = kWgRows * 16, kZ = (kWgRows / 8) * 32;  // two blocks: eight bf16 scales a row, eight zero-point words a group of eight rows
+  static constexpr int kOffW = 3 * kX, kOffS = kOffW + 3 * kW, kOffZ = kOffS + 3 * kS;
+  static constexpr int kLds = kOffZ + 3 * kZ;            // 162,816 (the epilogues reuse it: UP POS x 256 B, DOWN 8 x 2 KiB)
+  static constexpr int kLoadsX = POS / 32, kLoads = 1 + 2 + kLoadsX;  // a wave's loads a turn: scales or zero points, weights, activations
 };
-constexpr int kLoads = 2 + 4 + 1 + 1;        // a wave's loads a turn: two weight tiles, one activation tile (four pieces of 4 rows), scales, zero points
-constexpr int kLds = Shape<128>::kLds > Shape<64>::kLds ? Shape<128>::kLds : Shape<64>::kLds;
+constexpr int kLds = Shape<128>::kLds;
+static_assert(kLds == Shape<64>::kLds, "one launch, either shape");
 constexpr int kLdsRun = kLds + kThreads / 64 * 4;  // ... and a word a wave: whether it met a scale above the fast decode's range
 
 struct Args {
@@ -74,7 +78,7 @@ __device__ __forceinline__ int sw16(int r) { return r ^ ((r & 4) << 1); }
 template <bool UP, int POS>
 __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, int m0, int mend, int ns) {
   using S = Shape<POS>;
-  constexpr int kPos = S::kPos, kStageX = S::kStageX, kStageBytes = S::kStageBytes, kStages = S::kStages;
+  constexpr int kPos = S::kPos;
   const int K = UP ? g.L.H : g.L.I, N = UP ? g.L.I : g.L.H, KB = K / 128, G = K / 32;
   if (mend > m0 + kPos) mend = m0 + kPos;
   const dsgx_mat_desc* dsc = g.L.desc + (size_t)e * 3;
@@ -90,65 +94,93 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
     return UP ? c0 + 16 * wave : r0 + 32 * wave + 16 * t;
   };
   const int nmt = uni(min(S::kSub, (mend - m0 + 15) / 16));
-  const bool brings_x = wave < S::kSub;  // (a wave's loads a turn: kLoads, or kLoads - 4)
 
   // ---- what this lane fetches ----
-  const uint8_t* pw[2];   // weights: row lane / 4 of tile t, piece (lane % 4) ^ sw4(row)
-  const uint8_t* psc;     // scales: lane -> (tile lane / 32, row lane / 2 % 16, half lane % 2): 4 bytes = two groups' bf16
-  const uint8_t* pzp;     // lanes 0-15: zero points: (tile lane / 8, octet lane / 4 % 2, group lane % 4): one word
+  // weights: 64-byte rows: one instruction a tile, lane -> row lane / 4, piece (lane % 4) ^ sw4(row); 128-byte rows: two
+  // instructions a tile (rows 0-7, 8-15), lane -> row lane / 8, piece (lane % 8) ^ (row % 8)
+  const uint8_t* pw[2];
+  const uint8_t* psc;  // scales, lanes 0-31: the 16 bytes of tile lane / 16, row lane % 16
+  const uint8_t* pzp;  // zero points, lanes 0-7: 16 of the 32 bytes of tile lane / 4, octet lane / 2 % 2
   {
     const uint8_t* base;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      const int row = tile_row(t, base), r = lane >> 2;
-      pw[t] = base + (size_t)(row + r) * (K / 2) + 16 * ((lane & 3) ^ sw4(r));
+      const int row = tile_row(t, base), rl = lane >> (S::kPair ? 3 : 2);
+      pw[t] = base + (size_t)(row + rl) * (K / 2) + 16 * (S::kPair ? (lane & 7) ^ rl : (lane & 3) ^ sw4(rl));
     }
-    const int ts = lane >> 5, rs = (lane >> 1) & 15;
-    const int rows = tile_row(ts, base);
-    psc = base + soff + ((size_t)(rows + rs) * G) * 2 + 4 * (lane & 1);
-    const int tz = (lane >> 3) & 1, oz = (lane >> 2) & 1;
-    const int rowz = tile_row(tz, base);
-    pzp = base + zoff + ((size_t)((rowz >> 3) + oz) * G + (lane & 3)) * 4;
+    const int rows = tile_row((lane >> 4) & 1, base);
+    psc = base + soff + (size_t)(rows + r16) * G * 2;
+    const int rowz = tile_row((lane >> 2) & 1, base);
+    pzp = base + zoff + (size_t)((rowz >> 3) + ((lane >> 1) & 1)) * G * 4 + (KB > 1 ? 16 * (lane & 1) : 0);
   }
-  const uint8_t* px[4];   // activations: the wave brings 16-position tile `wave`; instruction i: position 4 i + lane / 16, piece (lane % 16) ^ sw16(position)
+  // activations: the wave brings positions kPos / 8 wave ... (none if they lie past a small tile's end); instruction i: position
+  // 4 i + lane / 16 of them, piece (lane % 16) ^ sw16(position)
+  const bool brings_x = !S::kPair || m0 + 8 * wave < mend;
+  const uint8_t* px[S::kLoadsX];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = 4 * i + (lane >> 4);
-    int pos = m0 + 16 * wave + r;
-    if (pos >= mend) pos = mend - 1;  // a ragged tile re-reads its last row (never stored)
-    px[i] = reinterpret_cast<const uint8_t*>(g.x) + (size_t)(g.gather ? g.gather[pos] : pos) * K * 2 + 16 * ((lane & 15) ^ sw16(r));
+  for (int i = 0; i < S::kLoadsX; ++i) {
+    const int p = kPos / 8 * wave + 4 * i + (lane >> 4);
+    const int pos = min(m0 + p, mend - 1);  // (a ragged tile re-reads its last row: never stored)
+    px[i] = reinterpret_cast<const uint8_t*>(g.x) + (size_t)(g.gather ? g.gather[pos] : pos) * K * 2 + 16 * ((lane & 15) ^ sw16(p & 15));
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
-  // load number i of block kb (clamped past the end: the last block again, into a stage nobody reads): the small ones first,
-  // then the activations (L2 hits mostly), the weights last (a wave's loads return in issue order: the ones that wait for HBM
-  // hold back every later one)
+  // The loads, each clamped past K's end (the last block again, into a slot nobody reads). Scales and zero points: pair q of
+  // blocks; the last pair of an odd number of blocks starts a block early.
+  auto first_block = [&](int q) { return max(0, min(2 * q, KB - 2)); };
+  auto load_s = [&](int q) {
+    if (lane < 32) dma16(psc + 8 * first_block(q), uni(lds0 + S::kOffS + (uint32_t)(q % 3) * S::kS + (uint32_t)wave * 512));
+  };
+  auto load_z = [&](int q) {
+    if (lane < 8) dma16(pzp + 16 * first_block(q), uni(lds0 + S::kOffZ + (uint32_t)(q % 3) * S::kZ + (uint32_t)wave * 128));
+  };
+  auto load_x = [&](int kb, int i) {
+    if (brings_x) dma16(px[i] + (size_t)min(kb, KB - 1) * 256, uni(lds0 + (uint32_t)(kb % 3) * S::kX + (uint32_t)wave * (kPos * 32) + i * 1024));
+  };
+  auto load_w = [&](int q, int t, int hh) {  // slot q: block q, or pair q (its rows 8 hh ...)
+    const int last = S::kPair ? KB / 2 - 1 : KB - 1;
+    dma16(pw[t] + (S::kPair ? (size_t)hh * 4 * K : 0) + (size_t)min(q, last) * (S::kPair ? 128 : 64),  // (rows 8-15: the same pieces)
+          uni(lds0 + S::kOffW + (uint32_t)(q % 3) * S::kW + (uint32_t)wave * (S::kPair ? 4096 : 2048) + t * (S::kPair ? 2048 : 1024) + hh * 1024));
+  };
+  // load i of turn kb: activations of block kb + 2, weights of block kb + 3, or half the rows of pair kb / 2 + 2, scales (even
+  // turns) or zero points (odd turns) of pair kb / 2 + 2; the small ones first, then the activations (L2 hits mostly), the weights
+  // last (a wave's loads return in issue order: the ones that wait for HBM hold back every later one)
   auto issue_one = [&](int kb, int i) {
-    const int kc = kb < KB ? kb : KB - 1;
-    const uint32_t st = lds0 + (uint32_t)(kb % kStages) * kStageBytes;
+    const int q = (kb >> 1) + 2;
     if (i == 0) {
-      dma4(reinterpret_cast<const float*>(psc + (size_t)kc * 8), uni(st + kStageW + kStageX + (uint32_t)wave * 256));
-    } else if (i == 1) {
-      if (lane < 16) dma4(reinterpret_cast<const float*>(pzp + (size_t)kc * 16), uni(st + kStageW + kStageX + kStageS + (uint32_t)wave * 64));
-    } else if (i < 6) {
-      if (brings_x) dma16(px[i - 2] + (size_t)kc * 256, uni(st + kStageW + (uint32_t)wave * 4096 + (i - 2) * 1024));
+      if (kb & 1) load_z(q);
+      else load_s(q);
+    } else if (i <= S::kLoadsX) {
+      load_x(kb + 2, i - 1);
     } else {
-      dma16(pw[i - 6] + (size_t)kc * 64, uni(st + (uint32_t)wave * 2048 + (i - 6) * 1024));
+      const int t = i - 1 - S::kLoadsX;
+      if (S::kPair) load_w(q, t, kb & 1);
+      else load_w(kb + 3, t, 0);
     }
   };
+  // what the first turns need: blocks 0 (and 1, opened in turn 0), then block 1's activations and the next weights
   auto fill = [&]() {
 #pragma unroll
-    for (int s = 0; s + 1 < kStages; ++s)
+    for (int n = 0; n < 2; ++n) {
+      load_s(n), load_z(n);
 #pragma unroll
-      for (int i = 0; i < kLoads; ++i) issue_one(s, i);
+      for (int i = 0; i < S::kLoadsX; ++i) load_x(n, i);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        if (S::kPair) load_w(n, t, 0), load_w(n, t, 1);
+        else if (n == 0) load_w(0, t, 0), load_w(1, t, 0);
+        else load_w(2, t, 0);
+      }
+    }
   };
+  constexpr int kSecond = 2 + S::kLoadsX + (S::kPair ? 4 : 2);  // a wave's loads of fill's second pass
   fill();
 
-  // fragment reads
-  const int rdw = r16 * 64 + (part ^ sw4(r16)) * 16;  // the lane's 32 nibbles: row r16, group `part` of the block
-  const int rds = r16 * 8 + part * 2;                 // its bf16 scale
-  const int rdz = (r16 >> 3) * 16 + part * 4;         // its zero-point word (the row's nibble: r16 % 8)
+  // fragment reads: the lane's 32 nibbles (row r16, group `part` of the block), its bf16 scale, its zero-point word (the row's
+  // nibble: r16 % 8), the activation piece of MFMA j: 4 part + j of position r16
+  const int rdw = S::kPair ? (r16 >> 3) * 1024 + (r16 & 7) * 128 + (part ^ (r16 & 7)) * 16 : r16 * 64 + (part ^ sw4(r16)) * 16;  // (a pair's second block: ^ 64)
+  const int rds = r16 * 16 + part * 2, rdz = (r16 >> 3) * 32 + part * 4;
   const uint32_t zsh = 4 * (r16 & 7);
-  int rdx[4];                                         // the activation piece of MFMA j: 4 part + j of position r16
+  int rdx[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) rdx[j] = r16 * 256 + ((4 * part + j) ^ sw16(r16)) * 16;
 
@@ -160,20 +192,21 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
 
   // A block's weights are decoded a turn ahead, a piece (one MFMA's fragment) at a time between the MFMAs of the turn before:
   // the decode is vector-unit work and the MFMAs run beside it. (Decoded in front of its own MFMAs it stood in their way: both
-  // waves of a SIMD reach it together behind the barrier: 1.39 -> 1.1 ms for gate/up.) Turn kb therefore needs block kb + 1
-  // landed: with three stages it waits for every load issued so far and issues block kb + 2's; with four, block kb + 2 may
-  // still be in flight and it issues block kb + 3's.
+  // waves of a SIMD reach it together behind the barrier: 1.39 -> 1.1 ms for gate/up.)
   u32x4_t raw[2];
   I4Group grp[2];
   uint32_t uz[2];
   float smax = 0.f;  // the largest scale that this lane has met (in magnitude; a NaN decodes to NaN by either routine)
   auto open_block = [&](int kb) {  // the lane's raw words, scale and zero point of the wave's two tiles of block kb
-    const uint8_t* st = smem + (size_t)(kb % kStages) * kStageBytes;
+    const int q = kb >> 1, o = kb - first_block(q);  // the pair whose scales and zero points the block's are among, which of the two
+    const uint8_t* W = smem + S::kOffW + (size_t)((S::kPair ? q : kb) % 3) * S::kW + wave * (S::kPair ? 4096 : 2048) + (S::kPair ? rdw ^ ((kb & 1) * 64) : rdw);
+    const uint8_t* SC = smem + S::kOffS + (size_t)(q % 3) * S::kS + wave * 512 + 8 * o + rds;
+    const uint8_t* Z = smem + S::kOffZ + (size_t)(q % 3) * S::kZ + wave * 128 + 16 * o + rdz;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      raw[t] = *reinterpret_cast<const u32x4_t*>(st + wave * 2048 + t * 1024 + rdw);
-      uz[t] = (*reinterpret_cast<const uint32_t*>(st + kStageW + kStageX + kStageS + wave * 64 + t * 32 + rdz) >> zsh) & 15u;
-      grp[t] = i4_group(bf16_bits_to_f32(*reinterpret_cast<const uint16_t*>(st + kStageW + kStageX + wave * 256 + t * 128 + rds)), uz[t]);
+      raw[t] = *reinterpret_cast<const u32x4_t*>(W + t * (S::kPair ? 2048 : 1024));
+      uz[t] = (*reinterpret_cast<const uint32_t*>(Z + t * 64) >> zsh) & 15u;
+      grp[t] = i4_group(bf16_bits_to_f32(*reinterpret_cast<const uint16_t*>(SC + t * 256)), uz[t]);
     }
     smax = fmaxf(smax, fmaxf(fabsf(grp[0].s), fabsf(grp[1].s)));
   };
@@ -188,26 +221,29 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   auto run = [&](auto nj_c, auto any) {  // any: decode by the routine for every scale
     constexpr int NJ = decltype(nj_c)::value;
     u32x4_t fa[2][4], fn[2][4];
-    // block 0 has landed (the later ones of the first stages may be in flight)
-    if (brings_x) wait_loads<(kStages - 2) * kLoads>();
-    else wait_loads<(kStages - 2) * (kLoads - 4)>();
+    // fill's first pass has landed (the second may be in flight)
+    if (brings_x) wait_loads<kSecond>();
+    else wait_loads<kSecond - S::kLoadsX>();
     __syncthreads();
     open_block(0);
 #pragma unroll
     for (int pc = 0; pc < 8; ++pc) piece(any, fa, pc);
     auto turn = [&](int kb, u32x4_t (&fa)[2][4], u32x4_t (&fn)[2][4]) {
-      // block kb + 1 has landed (four stages: block kb + 2 may be in flight)
-      if (brings_x) wait_loads<(kStages - 3) * kLoads>();
-      else wait_loads<(kStages - 3) * (kLoads - 4)>();
+      // what turn kb - 2 asked for has landed: the activations of block kb, the weights of block kb + 1 (turn kb - 1's loads may be
+      // in flight; turn 0: fill's first pass)
+      if (kb > 0) {
+        if (brings_x) wait_loads<S::kLoads>();
+        else wait_loads<S::kLoads - S::kLoadsX>();
+      }
       __syncthreads();
-      open_block(kb + 1);
-      const uint8_t* X = smem + (size_t)(kb % kStages) * kStageBytes + kStageW;
+      open_block(min(kb + 1, KB - 1));
+      const uint8_t* X = smem + (size_t)(kb % 3) * S::kX;
 #pragma unroll
       for (int mt = 0; mt < 8; ++mt) {
         // (the turn's loads between its MFMAs; a ragged tile issues what is left behind its last 16-position tile)
 #pragma unroll
-        for (int i = 0; i < kLoads; ++i)
-          if (NJ > 0 ? (mt < NJ && i * NJ / kLoads == mt) : mt == 0) issue_one(kb + kStages - 1, i);
+        for (int i = 0; i < S::kLoads; ++i)
+          if (mt < NJ && i * NJ / S::kLoads == mt) issue_one(kb, i);
         piece(any, fn, mt);
         if (mt >= NJ) continue;
         u32x4_t fb[4];
@@ -226,7 +262,6 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
     }
   };
   switch (nmt) {
-    case 0: run(std::integral_constant<int, 0>{}, std::false_type{}); break;
     case 1: run(std::integral_constant<int, 1>{}, std::false_type{}); break;
     case 2: run(std::integral_constant<int, 2>{}, std::false_type{}); break;
     case 3: run(std::integral_constant<int, 3>{}, std::false_type{}); break;
@@ -325,7 +360,7 @@ __global__ void __launch_bounds__(kThreads) k_gemm(Args g) {
   if (ns >= NS || tile >= *g.ntiles) return;
   const int e = g.tile_e[tile];
   const int m0 = g.off[e] + g.tile_m0[tile], mend = g.off[e + 1];
-  if (mend - m0 <= 64) gemm_tile<UP, 64>(g, smem, e, m0, mend, ns);
+  if (mend - m0 <= 64 && (UP ? g.L.H : g.L.I) % 256 == 0) gemm_tile<UP, 64>(g, smem, e, m0, mend, ns);
   else gemm_tile<UP, 128>(g, smem, e, m0, mend, ns);
 }
 

@@ -316,6 +316,27 @@ def test_prefill_int4_lds_staged_kernels_give_the_register_ring_kernels_bits():
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("H,I,T", [(256, 128, 9), (256, 384, 20), (512, 640, 64), (768, 1152, 70), (1280, 256, 130)])
+def test_prefill_int4_rings_at_the_edges_of_k_and_of_the_tiles(H, I, T):
+    """pf_gemm_i4.cuh's rings (two blocks of scales and zero points a load, two of weights for up to 64 rows): one 128-k block, odd
+    numbers of them, the shortest pairs; tiles of a few rows, of 64 and over - the register-ring kernel's bits"""
+    import os
+    E, topk = 4, 4
+    hl = helpers.make_layer(abi.FMT_INT4, H, I, E, topk, 4, seed=23, shared=None)
+    x, _, idx, w = helpers.rows_and_routing(29, T, H, E, topk, 2.5)
+    outs = []
+    for old in ("0", "1"):
+        os.environ["DSGX_PF_I4_OLD"] = old
+        try:
+            yr, _, ws, dl = _prefill(hl, x, idx, w, T)
+            v = lib.prefill_view(dl.w, ws, T)
+            outs.append((yr.view(np.uint32), gpu.host(gpu.view(ws, v.h, T * topk * I * 2), np.uint16, (-1,))))
+        finally:
+            os.environ.pop("DSGX_PF_I4_OLD", None)
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b)
+
+
 def test_prefill_int4_scales_above_the_fast_decodes_range():
     """scales of 2^116 and more make a workgroup do its tile once more by the routine for every scale: the bits of the
     register-ring kernel, which has that routine only, in tiles of 128 positions and in ragged ones"""
