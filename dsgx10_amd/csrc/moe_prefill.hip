@@ -300,14 +300,14 @@ __device__ __forceinline__ void pf_task(int NS, int& tile, int& ns) {
   ns = (b % NG) * kMapNs + i % kMapNs;
 }
 
-// ---- the grouped GEMM with bf16 activations (INT4 layers, and their BF16 shared expert) -----------------------------
+// ---- the grouped GEMM with bf16 activations and a register ring of weights (FP8 layers; INT4 layers: DSGX_PF_I4_OLD) ---
 // The same streaming structure for the altar-1 contract (engine/experts/prefill.cu:337-352, 772-831): activations stay
-// bf16, a weight is the bf16 value W = bf16((u - u_z) s) (INT4; decoded in registers by the decode kernels' routine) or
-// the stored bf16 (the shared expert), products are summed in f32 by v_mfma_f32_16x16x32_bf16, whose accumulators the
-// MFMA itself carries across K (no per-block scale here: the scales are inside W).
+// bf16, a weight is the bf16 value W = bf16((u - u_z) s) (INT4; decoded in registers by the decode kernels' routine), products
+// are summed in f32 by v_mfma_f32_16x16x32_bf16, whose accumulators the MFMA itself carries across K (INT4: no per-block
+// scale, the scales are inside W).
 // A 128-k block is four MFMAs (j = 0..3) a 16-row tile. INT4: a lane's 16 bytes are the 32 values of ONE scale group:
 // lane (row, part) holds k = 32 part + 8 j + [0, 8) for MFMA j (four lanes a row: 64 contiguous bytes an instruction),
-// one scale and one zero-point word a lane and block. BF16: k = 32 j + 8 part + [0, 8), one 16-byte load an MFMA.
+// one scale and one zero-point word a lane and block.
 // The activation panel in LDS is in fragment order for the same k map: piece (tile mt, j, lane) at 16 ((4 mt + j) 64 + lane).
 typedef __bf16 v8bf_t __attribute__((ext_vector_type(8)));
 constexpr int kPanel16 = kTile * 256;  // bytes of one bf16 activation panel (128 positions x 128 k)
@@ -326,7 +326,7 @@ struct Gemm16Args {
   float* d;            // DOWN: f32 [position][H]
 };
 
-// WF: the weights' format (DSGX_FMT_INT4_G32: the routed experts; DSGX_FMT_BF16: the shared expert, gate/up interleaved;
+// WF: the weights' format (DSGX_FMT_INT4_G32: the routed experts;
 // DSGX_FMT_FP8_B128: e4m3 experts or shared expert with bf16 activations, the reference engine's own prefill contract
 // for FP8 weights, prefill.cu:337-352: per 128-k block the bf16 x bf16 products summed from zero, acc = fma(S, sum, acc))
 template <bool UP, int WF>
@@ -360,7 +360,7 @@ __global__ void __launch_bounds__(kGemmThreads) k_pf_gemm16(Gemm16Args g) {
   const uint8_t* pz[2] = {nullptr, nullptr};
   uint32_t zsh[2] = {0, 0};
   float s2a = 1.f, s2b = 1.f;
-  if (I4) {
+  if constexpr (I4) {
     const dsgx_mat_desc* d = g.L.desc + (size_t)e * 3;
     const int G = K / 32;
     const size_t soff = ((size_t)N * K / 2 + 255) / 256 * 256, zoff = soff + ((size_t)N * G * 2 + 255) / 256 * 256;
@@ -375,7 +375,7 @@ __global__ void __launch_bounds__(kGemmThreads) k_pf_gemm16(Gemm16Args g) {
       zsh[t] = 4 * (n & 7);
     }
     if (UP) s2a = d[0].s2, s2b = d[1].s2;
-  } else if (F8) {
+  } else {
     const uint8_t *wa, *wb;
     const float *sa, *sb;
     if (e < 0) {
@@ -393,13 +393,6 @@ __global__ void __launch_bounds__(kGemmThreads) k_pf_gemm16(Gemm16Args g) {
     pw[1] = (UP ? wb + (size_t)(n0 + lrow) * K : wa + (size_t)(n0 + 16 + lrow) * K) + lq * 16;
     ps[0] = reinterpret_cast<const uint8_t*>(sa + (size_t)(n0 / 128) * KB);  // the tiles' scale rows (32 rows: one 128-row block)
     ps[1] = UP ? reinterpret_cast<const uint8_t*>(sb + (size_t)(n0 / 128) * KB) : ps[0];
-  } else {
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      // shared expert: gate row c is row 2 c of bgu, up row c is row 2 c + 1; down rows plain
-      const size_t row = UP ? 2 * (size_t)(n0 + lrow) + t : (size_t)(n0 + 16 * t + lrow);
-      pw[t] = reinterpret_cast<const uint8_t*>(UP ? g.L.sh.bgu : g.L.sh.bd) + row * K * 2 + lq * 16;
-    }
   }
   // activation staging: wave w brings the 16 positions 16 w ..., the lane the four 16-byte pieces of its fragments
   const uint8_t* px;
@@ -409,11 +402,11 @@ __global__ void __launch_bounds__(kGemmThreads) k_pf_gemm16(Gemm16Args g) {
     px = reinterpret_cast<const uint8_t*>(g.x) + (size_t)(g.gather ? g.gather[pos] : pos) * K * 2 + lq * 16;
   }
   // Activation load i of a lane is the 16-byte piece c = 4 i + lq of its row's block (k = 8 c ...): the piece of MFMA j,
-  // part p with c = 4 p + j (INT4 map: k = 32 p + 8 j) or c = 4 j + p (BF16 map: k = 32 j + 8 p).
+  // part p with c = 4 p + j (INT4 map: k = 32 p + 8 j).
   // FP8 map: a lane's 32 codes are the 16 at 16 p and the 16 at 64 + 16 p of the block: k = 64 (j / 2) + 16 p + 8 (j % 2), c = k / 8.
   auto slot_of = [&](int i) {
     const int c = 4 * i + lq;
-    const int j = I4 ? c & 3 : F8 ? 2 * (c >> 3) + (c & 1) : c >> 2, p = I4 ? c >> 2 : F8 ? (c >> 1) & 3 : c & 3;
+    const int j = I4 ? c & 3 : 2 * (c >> 3) + (c & 1), p = I4 ? c >> 2 : (c >> 1) & 3;
     return ((4 * wave + j) * 64 + p * 16 + lrow) * 16;
   };
 
@@ -423,9 +416,9 @@ __global__ void __launch_bounds__(kGemmThreads) k_pf_gemm16(Gemm16Args g) {
 #pragma unroll
     for (int mt = 0; mt < 8; ++mt) acc[t][mt] = v4f_t{};
 
-  constexpr int kRing16 = I4 || F8 ? 3 : 2;
+  constexpr int kRing16 = 3;
   struct WRegs {
-    u32x4_t v[I4 ? 1 : F8 ? 2 : 4];
+    u32x4_t v[I4 ? 1 : 2];
     uint32_t s, z;
   };
   // FP8: the wave's weight scales, lane l holding those of block kb0 + l for the 64 blocks from kb0 (a load inside the
@@ -448,14 +441,10 @@ __global__ void __launch_bounds__(kGemmThreads) k_pf_gemm16(Gemm16Args g) {
         ra[slot][t].v[0] = ldg_stream(p);
         ra[slot][t].s = ldg_u16(ps[t] + (size_t)kc * 8);
         ra[slot][t].z = ldg_u32(pz[t] + (size_t)kc * 16);
-      } else if (F8) {
+      } else {
         const uint8_t* p = pin_after(pw[t] + (size_t)kc * 128, acc[t][0][0]);
         ra[slot][t].v[0] = *reinterpret_cast<const DSGX_GLOBAL u32x4_t*>((uintptr_t)p);
         ra[slot][t].v[F8 ? 1 : 0] = *reinterpret_cast<const DSGX_GLOBAL u32x4_t*>((uintptr_t)(p + 64));
-      } else {
-        const uint8_t* p = pin_after(pw[t] + (size_t)kc * 256, acc[t][0][0]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) ra[slot][t].v[I4 || F8 ? 0 : j] = ldg_stream(p + 64 * j);
       }
     }
   };
@@ -499,7 +488,7 @@ __global__ void __launch_bounds__(kGemmThreads) k_pf_gemm16(Gemm16Args g) {
           i4x8_to_bf16_any(j == 0 ? w.x : j == 1 ? w.y : j == 2 ? w.z : w.w, sc, nzs, o);
           fa[t][j] = u32x4_t{o[0], o[1], o[2], o[3]};
         }
-      } else if (F8) {
+      } else {
         auto mv = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_ds_bpermute(perm_addr, (int)v); };
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -510,13 +499,6 @@ __global__ void __launch_bounds__(kGemmThreads) k_pf_gemm16(Gemm16Args g) {
           fa[t][2 * h] = u32x4_t{o[0], o[1], o[2], o[3]};
           fp8x8_to_bf16(w.z, w.w, o);
           fa[t][2 * h + 1] = u32x4_t{o[0], o[1], o[2], o[3]};
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          auto mv = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_ds_bpermute(perm_addr, (int)v); };
-          const u32x4_t wl = keep_whole(ra[slot][t].v[I4 || F8 ? 0 : j]);
-          fa[t][j] = u32x4_t{mv(wl.x), mv(wl.y), mv(wl.z), mv(wl.w)};
         }
       }
     }
@@ -800,9 +782,7 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
     const size_t lds16 = (size_t)kStages16 * kPanel16;
     auto k_up = i4 ? k_pf_gemm16<true, DSGX_FMT_INT4_G32> : k_pf_gemm16<true, DSGX_FMT_FP8_B128>;
     auto k_dn = i4 ? k_pf_gemm16<false, DSGX_FMT_INT4_G32> : k_pf_gemm16<false, DSGX_FMT_FP8_B128>;
-    auto k_sup = i4 ? k_pf_gemm16<true, DSGX_FMT_BF16> : k_pf_gemm16<true, DSGX_FMT_FP8_B128>;
-    auto k_sdn = i4 ? k_pf_gemm16<false, DSGX_FMT_BF16> : k_pf_gemm16<false, DSGX_FMT_FP8_B128>;
-    for (const void* k : {(const void*)k_up, (const void*)k_dn, (const void*)k_sup, (const void*)k_sdn})
+    for (const void* k : {(const void*)k_up, (const void*)k_dn})
       if (int rc = allow_dynamic_lds(k, lds16)) return rc;
     Gemm16Args q{};
     q.L = *L;
@@ -816,28 +796,44 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
         if (int rc = allow_dynamic_lds(k, pfi4::kLdsRun)) return rc;
       q4.L = *L, q4.tile_e = I32(o.tile_e), q4.tile_m0 = I32(o.tile_m0), q4.ntiles = I32(o.ntiles), q4.off = I32(o.off);
     }
+    // the BF16 shared expert: a whole step runs its tiles in the routed experts' launches (pf_gemm_b16.cuh), phases apart have
+    // launches of their own: the same bits
+    const int sh_tiles = (T + pfb16::kPos - 1) / pfb16::kPos;
+    uint16_t* hsh = reinterpret_cast<uint16_t*>(W + o.hsh);
+    const pfb16::Args sh_up{x, L->sh.bgu, T, H, I, hsh, nullptr}, sh_dn{hsh, L->sh.bd, T, H, I, nullptr, ys};
+    const unsigned sh_gu = pf8::grid_of(sh_tiles, I / (kWgRows / 2)), sh_gd = pf8::grid_of(sh_tiles, H / kWgRows);
+    const bool fused_sh = new4 && shared && (cfg.phases & (2 | 4 | 16)) == (2 | 4 | 16);
     if (cfg.phases & 2) {
       q.x = x, q.gather = I32(o.perm), q.h = reinterpret_cast<uint16_t*>(W + o.h), q.d = nullptr;
+      if (fused_sh) q4.sh_grid = sh_gu, q4.sh = sh_up;
       q4.x = q.x, q4.gather = q.gather, q4.h = q.h, q4.d = nullptr;
-      if (new4) hipLaunchKernelGGL(pfi4::k_gemm<true>, dim3(pf8::grid_of(o.max_tiles, I / (kWgRows / 2))), dim3(pf8::kThreads), pfi4::kLdsRun, st, q4);
+      if (new4) hipLaunchKernelGGL(pfi4::k_gemm<true>, dim3(q4.sh_grid + pf8::grid_of(o.max_tiles, I / (kWgRows / 2))), dim3(pf8::kThreads), pfi4::kLdsRun, st, q4);
       else hipLaunchKernelGGL(k_up, dim3(pf_grid(o.max_tiles, I / (kWgRows / 2))), dim3(kGemmThreads), lds16, st, q);
     }
     if (cfg.phases & 4) {
       q.x = reinterpret_cast<const uint16_t*>(W + o.h), q.gather = nullptr, q.h = nullptr, q.d = F32(o.d);
       q4.x = q.x, q4.gather = nullptr, q4.h = nullptr, q4.d = q.d;
-      if (new4) hipLaunchKernelGGL(pfi4::k_gemm<false>, dim3(pf8::grid_of(o.max_tiles, H / kWgRows)), dim3(pf8::kThreads), pfi4::kLdsRun, st, q4);
+      if (fused_sh) q4.sh_grid = sh_gd, q4.sh = sh_dn;
+      if (new4) hipLaunchKernelGGL(pfi4::k_gemm<false>, dim3(q4.sh_grid + pf8::grid_of(o.max_tiles, H / kWgRows)), dim3(pf8::kThreads), pfi4::kLdsRun, st, q4);
       else hipLaunchKernelGGL(k_dn, dim3(pf_grid(o.max_tiles, H / kWgRows)), dim3(kGemmThreads), lds16, st, q);
     }
     if (cfg.phases & 8) {
       launch_pf_combine(F32(o.d), I32(o.rpos), F32(o.rk), T, H, topk, yr, st);
     }
-    if ((cfg.phases & 16) && shared) {
-      const int tiles = (T + kTile - 1) / kTile;
-      q.tile_e = q.tile_m0 = q.ntiles = q.off = nullptr, q.nrows = T;
-      q.x = x, q.gather = nullptr, q.h = reinterpret_cast<uint16_t*>(W + o.hsh), q.d = nullptr;
-      hipLaunchKernelGGL(k_sup, dim3(pf_grid(tiles, I / (kWgRows / 2))), dim3(kGemmThreads), lds16, st, q);
-      q.x = reinterpret_cast<const uint16_t*>(W + o.hsh), q.h = nullptr, q.d = ys;
-      hipLaunchKernelGGL(k_sdn, dim3(pf_grid(tiles, H / kWgRows)), dim3(kGemmThreads), lds16, st, q);
+    if ((cfg.phases & 16) && shared && !fused_sh) {
+      if (i4) {
+        for (const void* k : {(const void*)pfb16::k_gemm<true>, (const void*)pfb16::k_gemm<false>})
+          if (int rc = allow_dynamic_lds(k, pfb16::kLds)) return rc;
+        hipLaunchKernelGGL(pfb16::k_gemm<true>, dim3(sh_gu), dim3(pf8::kThreads), pfb16::kLds, st, sh_up);
+        hipLaunchKernelGGL(pfb16::k_gemm<false>, dim3(sh_gd), dim3(pf8::kThreads), pfb16::kLds, st, sh_dn);
+      } else {
+        const int tiles = (T + kTile - 1) / kTile;
+        q.tile_e = q.tile_m0 = q.ntiles = q.off = nullptr, q.nrows = T;
+        q.x = x, q.gather = nullptr, q.h = hsh, q.d = nullptr;
+        hipLaunchKernelGGL(k_up, dim3(pf_grid(tiles, I / (kWgRows / 2))), dim3(kGemmThreads), lds16, st, q);
+        q.x = hsh, q.h = nullptr, q.d = ys;
+        hipLaunchKernelGGL(k_dn, dim3(pf_grid(tiles, H / kWgRows)), dim3(kGemmThreads), lds16, st, q);
+      }
     }
     DSGX_HIP(hipGetLastError());
     return DSGX_OK;

@@ -18,7 +18,7 @@
 // The k order of the sums - block after block, inside a block the four MFMAs j = 0 .. 3 - is k_pf_gemm16's, so the bits
 // are the ones that kernel gave.
 #pragma once
-#include "pf_gemm_fp8.cuh"
+#include "pf_gemm_b16.cuh"
 
 namespace dsgx {
 namespace pfi4 {
@@ -54,6 +54,7 @@ struct Shape {
 };
 constexpr int kLds = Shape<128>::kLds;
 static_assert(kLds == Shape<64>::kLds, "one launch, either shape");
+static_assert(pfb16::kLds <= kLds, "a launch may hold the shared expert's tiles");
 constexpr int kLdsRun = kLds + kThreads / 64 * 4;  // ... and a word a wave: whether it met a scale above the fast decode's range
 
 struct Args {
@@ -66,6 +67,8 @@ struct Args {
   dsgx_layer_w L;
   uint16_t* h;         // UP: h bf16 [position][I]
   float* d;            // DOWN: f32 [position][H]
+  unsigned sh_grid;    // the shared expert's workgroups in this launch (pf8::grid_of of them, so the others keep their XCDs; 0: none)
+  pfb16::Args sh;
 };
 
 // Where piece q of a row lies. A 16-byte LDS read of 64 lanes is served sixteen lanes at a time, and the sixteen are lanes
@@ -302,61 +305,21 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
     __syncthreads();
   }
 
-  // register q of lane l is weight row 4 (l / 16) + q of the 16-row tile, position l % 16 of the 16 positions
-  if (UP) {
-    // h = bf16(bf16(silu(bf16 g)) * bf16 u) of the workgroup's 128 channels into an LDS tile [position][256 bytes] (16-byte
-    // pieces exchanged by position: writes and reads spread over the banks), then whole lines to memory, 16 lanes a position
-    const int I = g.L.I;
-#pragma unroll
-    for (int mt = 0; mt < 8; ++mt) {
-      if (mt >= nmt) break;
-      const int p = 16 * mt + r16;
-      uint32_t hb[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        hb[q] = swiglu_bits(bf16_round(__fmul_rn(acc[0][mt][q], s2a)), bf16_round(__fmul_rn(acc[1][mt][q], s2b)));
-      const int ch = 16 * wave + 4 * part;
-      const int piece = (ch >> 3) ^ (p & 15);
-      *reinterpret_cast<uint2*>(smem + p * 256 + piece * 16 + (ch & 4) * 2) = make_uint2(hb[0] | (hb[1] << 16), hb[2] | (hb[3] << 16));
-    }
-    __syncthreads();
-    const int l16 = tid & 15;
-    for (int p = tid >> 4; p < 16 * nmt; p += kThreads / 16) {
-      const int pos = m0 + p;
-      const u32x4_t hv = *reinterpret_cast<const u32x4_t*>(smem + p * 256 + (l16 ^ (p & 15)) * 16);
-      if (pos < mend) *reinterpret_cast<u32x4_t*>(g.h + (size_t)pos * I + c0 + 8 * l16) = hv;
-    }
-  } else {
-    // a 16-position tile at a time through the wave's own 2 KiB: written as held (four rows of a position: 16 bytes), read back
-    // as whole rows (32 rows = 128 bytes a position, 8 lanes a position)
-    const int H = g.L.H;
-    uint8_t* my = smem + wave * 2048;
-    const int row0 = r0 + 32 * wave;
-#pragma unroll
-    for (int mt = 0; mt < 8; ++mt) {
-      if (mt >= nmt) break;
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const int c = 4 * t + part;
-        *reinterpret_cast<v4f_t*>(my + r16 * 128 + ((c ^ r16) & 7) * 16) = acc[t][mt];
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int idx = i * 64 + lane, p = idx >> 3, c = idx & 7;
-        const v4f_t v = *reinterpret_cast<const v4f_t*>(my + p * 128 + ((c ^ p) & 7) * 16);
-        const int pos = m0 + 16 * mt + p;
-        if (pos < mend) *reinterpret_cast<v4f_t*>(g.d + (size_t)pos * H + row0 + 4 * c) = v;
-      }
-    }
-  }
+  if (UP) pfb16::store_h(smem, acc, nmt, s2a, s2b, m0, mend, c0, g.L.I, g.h);
+  else pfb16::store_d(smem, acc, nmt, m0, mend, r0, g.L.H, g.d);
 }
 
+// The routed experts' tiles, and in front of them (workgroups 0 .. sh_grid - 1) the BF16 shared expert's, if the launch holds those
 template <bool UP>
 __global__ void __launch_bounds__(kThreads) k_gemm(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  if (blockIdx.x < g.sh_grid) {  // (the same for the whole workgroup)
+    pfb16::tiles<UP>(g.sh, smem, blockIdx.x);
+    return;
+  }
   const int NS = UP ? g.L.I / (kWgRows / 2) : g.L.H / kWgRows;
   int tile, ns;
-  pf8::task_of<false>(NS, tile, ns);
+  pf8::task_of<false>(NS, tile, ns, blockIdx.x - g.sh_grid);
   if (ns >= NS || tile >= *g.ntiles) return;
   const int e = g.tile_e[tile];
   const int m0 = g.off[e] + g.tile_m0[tile], mend = g.off[e + 1];

@@ -389,3 +389,20 @@ def test_prefill_bf16_activations_every_bit_against_the_matrix_unit_oracle(fmt, 
         assert np.array_equal(yr[t].view(np.uint32), o["yr"].view(np.uint32)), (t, int((yr[t] != o["yr"]).sum()))
         if shared:
             assert np.array_equal(ys[t].view(np.uint32), o["ys"].view(np.uint32)), (t, int((ys[t] != o["ys"]).sum()))
+
+
+@pytest.mark.parametrize("H,I,T", [(256, 128, 1), (512, 384, 128), (1024, 256, 129), (256, 640, 300)])
+def test_prefill_int4_bf16_shared_expert_tiles(H, I, T):
+    """the BF16 shared expert's tiles (pf_gemm_b16.cuh: two 64-k turns of K and more; one row, one tile, one row over, a ragged third)
+    bit for bit against the oracle that adds as the matrix unit does, and in launches of their own the bits that they have in
+    the routed experts' launches"""
+    E, topk = 8, 2
+    test_prefill_bf16_activations_every_bit_against_the_matrix_unit_oracle(abi.FMT_INT4, H, I, E, topk, T, "bf16", {})
+    hl = helpers.make_layer(abi.FMT_INT4, H, I, E, topk, 4, seed=27, shared="bf16")
+    x, _, idx, w = helpers.rows_and_routing(31, T, H, E, topk, 2.5)
+    yr, ys, _, dl = _prefill(hl, x, idx, w, T)
+    ws, r2, s2 = gpu.empty(lib.prefill_ws_bytes(dl.w, T), 0x5A), gpu.empty(T * H * 4, 0xFF), gpu.empty(T * H * 4, 0xFF)
+    for ph in (1, 2, 4, 8, 16):
+        lib.moe_prefill(dl.w, gpu.dev(x), gpu.dev(idx), gpu.dev(w), T, ws, r2, s2, phases=ph)
+    assert np.array_equal(gpu.host(r2, np.uint32, (T, H)), yr.view(np.uint32))
+    assert np.array_equal(gpu.host(s2, np.uint32, (T, H)), ys.view(np.uint32))
