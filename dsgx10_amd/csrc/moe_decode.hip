@@ -207,11 +207,13 @@ static int moe_decode_at(const dsgx_layer_w* L, const uint16_t* x, const int* id
   if ((fp8sh || b16sh || c.ysum) && (c.parts & 2) && !ys) return fail(DSGX_EINVAL, "moe_decode: ys (the shared expert's output) is needed");
   if (((uintptr_t)x | (uintptr_t)ws | (uintptr_t)L->pool) & 15) return fail(DSGX_EINVAL, "moe_decode: x, ws and pool must be 16-byte aligned");
 
-  if (M > 8) {
-    // 9-16 rows (the reference's limit, experts.h:104): two passes of the kernels built for up to eight rows, rows 0-7
-    // then the rest; every row's result is what it is alone or in any batch, so the split is invisible in the output.
-    // The second pass reads the weights of its experts again; the workspace is reused in stream order.
-    const int M1 = 8, topk = L->topk, E = L->E;
+  // 9-16 rows (the reference's limit, experts.h:104): the MFMA kernels take as many in one pass as their LDS holds, the vector-unit
+  // kernels eight
+  const int M1 = M <= 8 ? M : c.up != 1 ? 8 : L->fmt == DSGX_FMT_FP8_B128 ? max_rows_fp8_mfma(H, I, M) : L->fmt == DSGX_FMT_INT4_G32 ? max_rows_int4_mfma(H, I, M) : max_rows_mxfp4_mfma(H, I, M);
+  if (M1 < M) {
+    // two passes, the first as large as it can be; every row's result is what it is alone or in any batch, so the split is
+    // invisible in the output. The second pass reads the weights of its experts again; the workspace is reused in stream order.
+    const int topk = L->topk, E = L->E;
     dsgx_decode_cfg c1 = c, c2 = c;
     c1.parts = c2.parts = c.parts & 3;
     if (c.logits) c2.logits = c.logits + (size_t)M1 * E;

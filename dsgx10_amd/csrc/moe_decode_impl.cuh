@@ -91,6 +91,7 @@ struct DecodeArgs {
   size_t stk_wb[3], stk_sb[3];
   int* idx_out;     // fused routing: the selection is also written here (idx_out / wts_out of dsk::moe_routed, dsk.h:239-241)
   float* wts_out;
+  int down_slots;   // 9 to 16 rows: the slots whose h the down phase stages together, 2 or (where LDS holds no more) 1
 };
 
 int launch_decode_mxfp4_mfma(const DecodeArgs& a, int parts, bool shared_fp8e, hipStream_t st);  // MXFP4 experts (+ FP8_B32E shared)
@@ -99,6 +100,10 @@ int launch_decode_fp8_mfma(const DecodeArgs& a, int parts, bool shared, hipStrea
 int launch_decode_int4(const DecodeArgs& a, int parts, bool shared_bf16, hipStream_t st);
 int launch_decode_int4_mfma(const DecodeArgs& a, int parts, int shared_fmt, hipStream_t st);  // variant 1 (shared: 0, BF16 or FP8_B128)
 int launch_decode_bf16(const DecodeArgs& a, int parts, hipStream_t st);
+// how many of M (9 .. 16) rows the MFMA kernels of a format take in one pass, 8 at least (moe_decode_mfma.cuh)
+int max_rows_fp8_mfma(int H, int I, int M);
+int max_rows_int4_mfma(int H, int I, int M);
+int max_rows_mxfp4_mfma(int H, int I, int M);
 
 // ---- what a workgroup knows about the step -------------------------------------------------------------------------
 struct MatRef {
@@ -111,19 +116,31 @@ struct Slot {
   MatRef g, u, d;
   int hslot, shared;
 };
-template <int M>
+struct DescHead {  // a descriptor's off and s2
+  uint32_t x, y, z;
+};
+// M: the step's rows, or 16 for 9 to 16 of them (step_rows). PICKS: the MFMA kernels, which keep a row's weights by its picks
+template <int M, bool PICKS = false>
 struct Step {
   alignas(16) uint32_t mask[DSGX_MAX_EXPERTS / 32];  // the picked experts (read 16 bytes at a time)
   int n;                               // distinct picked experts
   int ri[M * DSGX_MAX_TOPK];
   float rw[M * DSGX_MAX_TOPK];
-  float wslot[M * DSGX_MAX_TOPK][M];   // per slot the rows' routing weights (0: the row did not pick it)
+  float wslot[PICKS ? 1 : M * DSGX_MAX_TOPK][M];  // per slot the rows' routing weights (0: the row did not pick it)
   Slot slots[M * DSGX_MAX_TOPK + 1];
   int gen;                             // the grid barrier's generation at kernel start
   int next_up;                         // the gate/up phase's batch counter (up_body)
   int rdone, ready;                    // rows routed so far; the slots are complete (resolve)
-  uint4 dtab[DSGX_MAX_EXPERTS * 3];    // the descriptors' first 16 bytes (off, s2, fmt), fetched before the routing is known
+  std::conditional_t<(M > 8), DescHead, uint4> dtab[DSGX_MAX_EXPERTS * 3];  // the descriptors' first 16 bytes (off, s2, fmt) or 12, fetched before the routing is known
+  // PICKS: per slot and row the number m topk + r of the row's pick, r picks of the row lying in lower slots (255: not picked),
+  // and per pick the weight and s2 w
+  uint8_t pick[PICKS ? M * DSGX_MAX_TOPK : 1][M <= 4 ? 4 : M <= 8 ? 8 : 16];
+  float pw[PICKS ? M * DSGX_MAX_TOPK : 1], pfac[PICKS ? M * DSGX_MAX_TOPK : 1];
 };
+// the number of row m's pick of the routed slot (255: it did not pick it); one row picked every slot, its picks are numbered as they are
+template <int M>
+__device__ __forceinline__ int pick_of(const Step<M, true>& S, int slot, int m) { return M == 1 ? slot : S.pick[slot][m]; }
+template <int M> __device__ __forceinline__ int step_rows(const DecodeArgs& a) { return M <= 8 ? M : a.M; }
 
 // The step's set-up comes in two parts, so that the weights that do not depend on the routing (the fused shared
 // expert's, slot 0) stream while the routing's dependent memory round trips are under way:
@@ -137,23 +154,31 @@ struct Step {
 //              S.ready when they need a routed slot (wait_slots()).
 // Every workgroup does both for itself.
 template <int M> __device__ __forceinline__ constexpr int resolver_waves() { return M < 4 ? M : 4; }
-template <int FMT, int SHFMT, int M>
-__device__ __forceinline__ void prep(Step<M>& S, const DecodeArgs& a) {
+template <int FMT, int SHFMT, int M, bool PICKS>
+__device__ __forceinline__ void prep(Step<M, PICKS>& S, const DecodeArgs& a) {
   const int tid = threadIdx.x;
   // every expert's descriptors into S.dtab (their first 16 of 64 bytes), three loads in flight a thread
   // (loads past the end re-read the last descriptor: unconditional loads into named registers stay in flight together)
   const DSGX_GLOBAL u32x4_t* d = (const DSGX_GLOBAL u32x4_t*)(uintptr_t)a.L.desc;
-  u32x4_t* tab = reinterpret_cast<u32x4_t*>(S.dtab);
+  auto put = [&](int i, u32x4_t v) {
+    if constexpr (M > 8) S.dtab[i] = DescHead{v.x, v.y, v.z};
+    else *reinterpret_cast<u32x4_t*>(&S.dtab[i]) = v;
+  };
   const int nd = a.stk_w[0] ? 0 : a.L.E * 3, bd = blockDim.x;  // (stacked experts are addressed by their id alone)
   for (int i0 = tid; i0 < nd; i0 += 3 * bd) {
     const int i1 = i0 + bd, i2 = i1 + bd;
     const u32x4_t v0 = d[(size_t)i0 * 4], v1 = d[(size_t)min(i1, nd - 1) * 4], v2 = d[(size_t)min(i2, nd - 1) * 4];
-    tab[i0] = v0;
-    if (i1 < nd) tab[i1] = v1;
-    if (i2 < nd) tab[i2] = v2;
+    put(i0, v0);
+    if (i1 < nd) put(i1, v1);
+    if (i2 < nd) put(i2, v2);
   }
   if (tid < DSGX_MAX_EXPERTS / 32) S.mask[tid] = 0;
-  for (int i = tid; i < M * DSGX_MAX_TOPK * M; i += blockDim.x) (&S.wslot[0][0])[i] = 0.f;
+  if constexpr (PICKS) {
+    for (int i = tid; M > 1 && i < (int)sizeof(S.pick) / 4; i += blockDim.x) reinterpret_cast<uint32_t*>(S.pick)[i] = 0xFFFFFFFFu;
+    if (tid < M * DSGX_MAX_TOPK) S.pfac[tid] = 0.f;
+  } else {
+    for (int i = tid; i < M * DSGX_MAX_TOPK * M; i += blockDim.x) (&S.wslot[0][0])[i] = 0.f;
+  }
   if (tid == 0) {
     S.next_up = 0, S.ready = 0, S.rdone = 0;
     if (SHFMT != 0) {
@@ -196,17 +221,18 @@ __device__ __forceinline__ MatDev mat_dev(const MatRef& r, int N, int K) {
 struct ResolveRegs {
   float lg[kRouteRJ], bs[kRouteRJ];
 };
-template <int M>
-__device__ __forceinline__ void resolve_fetch(Step<M>& S, const DecodeArgs& a, int rw, int nr, ResolveRegs& R) {
+template <int M, bool PICKS>
+__device__ __forceinline__ void resolve_fetch(Step<M, PICKS>& S, const DecodeArgs& a, int rw, int nr, ResolveRegs& R) {
   const int lane = threadIdx.x & 63, E = a.L.E;
   if (a.logits) {
-    route_fetch(rw < M ? a.logits + (size_t)rw * E : nullptr, E, lane, R.lg);
+    route_fetch(rw < step_rows<M>(a) ? a.logits + (size_t)rw * E : nullptr, E, lane, R.lg);
     route_fetch(a.bias, E, lane, R.bs);
   }
 }
-template <int FMT, int SHFMT, int M>
-__device__ __forceinline__ void resolve(Step<M>& S, const DecodeArgs& a, int rw, int nr, ResolveRegs& R) {
-  const int lane = threadIdx.x & 63, E = a.L.E, topk = a.L.topk, ne = M * topk;
+template <int FMT, int SHFMT, int M, bool PICKS>
+__device__ __forceinline__ void resolve(Step<M, PICKS>& S, const DecodeArgs& a, int rw, int nr, ResolveRegs& R) {
+  const int rows = step_rows<M>(a);
+  const int lane = threadIdx.x & 63, E = a.L.E, topk = a.L.topk, ne = rows * topk;
   const int H = a.L.H, I = a.L.I, nsh = SHFMT != 0 ? 1 : 0;
   __builtin_amdgcn_s_setprio(3);
   // the routed slot of expert e, its place r among the step's experts
@@ -214,12 +240,13 @@ __device__ __forceinline__ void resolve(Step<M>& S, const DecodeArgs& a, int rw,
     Slot t;
     auto ref = [&](int which, int N, int K) {
       if (a.stk_w[0]) return MatRef{a.stk_w[which] + (size_t)e * a.stk_wb[which], a.stk_s[which] + (size_t)e * a.stk_sb[which], 1.f, 0};
-      const uint4 d = S.dtab[e * 3 + which];
+      const auto d = S.dtab[e * 3 + which];
       return mat_ref<FMT>(a.L.pool + (((uint64_t)d.y << 32) | d.x), N, K, __uint_as_float(d.z));
     };
     t.g = ref(0, I, H), t.u = ref(1, I, H), t.d = ref(2, H, I);
     t.hslot = r, t.shared = 0;
     S.slots[nsh + r] = t;
+    return t.d.s2;
   };
   if constexpr (M == 1) {
     // One row: its picks are the step's experts, and a pick's slot is the number of picks with a lower id - counted in
@@ -240,8 +267,9 @@ __device__ __forceinline__ void resolve(Step<M>& S, const DecodeArgs& a, int rw,
       DSGX_MARKW(9);
       if (lane < topk) {
         if (a.idx_out && blockIdx.x == 0) a.idx_out[lane] = id, a.wts_out[lane] = w;
-        S.wslot[r][0] = w;
-        make_slot(id, r);
+        const float s2 = make_slot(id, r);
+        if constexpr (PICKS) S.pw[r] = w, S.pfac[r] = __fmul_rn(s2, w);
+        else S.wslot[r][0] = w;
       }
       if (lane == 0) S.n = topk;
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -252,7 +280,7 @@ __device__ __forceinline__ void resolve(Step<M>& S, const DecodeArgs& a, int rw,
     }
   }
   int mine = 0;
-  for (int row = rw; row < M; row += nr, ++mine) {
+  for (int row = rw; row < rows; row += nr, ++mine) {
     int id = 0;
     float w = 0.f;
     if (a.logits) {
@@ -271,7 +299,7 @@ __device__ __forceinline__ void resolve(Step<M>& S, const DecodeArgs& a, int rw,
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   int before = 0;
   if (lane == 0) before = __hip_atomic_fetch_add(&S.rdone, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-  if (uni(before) + mine < M) {  // another resolver finishes later: it does the rest
+  if (uni(before) + mine < rows) {  // another resolver finishes later: it does the rest
     __builtin_amdgcn_s_setprio(0);
     return;
   }
@@ -293,8 +321,16 @@ __device__ __forceinline__ void resolve(Step<M>& S, const DecodeArgs& a, int rw,
       const uint32_t below = j < (e >> 5) ? 0xFFFFFFFFu : j == (e >> 5) ? (1u << (e & 31)) - 1 : 0u;
       r += __popc(mk[j] & below);
     }
-    S.wslot[r][i / topk] = S.rw[i];
-    make_slot(e, r);  // (rows that picked the same expert write the same values)
+    const int m = i / topk;
+    const float s2 = make_slot(e, r);  // (rows that picked the same expert write the same values)
+    if constexpr (PICKS) {
+      int p = M == 1 ? r : m * topk;  // the row's pick: its picks below e before it (one row: pick_of)
+      for (int j = 0; M > 1 && j < topk; ++j) p += S.ri[m * topk + j] < e ? 1 : 0;
+      if (M > 1) S.pick[r][m] = p;
+      S.pw[p] = S.rw[i], S.pfac[p] = __fmul_rn(s2, S.rw[i]);
+    } else {
+      S.wslot[r][m] = S.rw[i];
+    }
   }
   if (lane == 0) {
     int n = 0;
@@ -479,12 +515,12 @@ __device__ __forceinline__ void up_phase(const DecodeArgs& a, uint4* xs, Step<M>
   const bool resolver = wave >= nw - NR;
   ResolveRegs rr;
   if (resolver) resolve_fetch(S, a, wave - (nw - NR), NR, rr);
-  prep<FMT, SHFMT, M>(S, a);
+  prep<FMT, SHFMT>(S, a);
   if (shared_wg) stage_x<FmtT<DSGX_FMT_BF16>::KL>(xs, a.x, H, M, H, num_segs<DSGX_FMT_BF16>(H) * 512);
   else stage_x<FmtT<FMT>::KL>(xs, a.x, H, M, H, num_segs<FMT>(H) * FmtT<FMT>::SEGK);
   __syncthreads();
   DSGX_MARK(1);
-  if (resolver) resolve<FMT, SHFMT, M>(S, a, wave - (nw - NR), NR, rr);
+  if (resolver) resolve<FMT, SHFMT>(S, a, wave - (nw - NR), NR, rr);
   if (shared_wg) {
     up_body<kMixed ? DSGX_FMT_BF16 : FMT, M, kMixed, kUpCH, kUpD>(a, xs, S.slots, 1, &S.next_up, blockIdx.x, shared_wgs, [&] {
       wait_slots(S);
@@ -760,9 +796,9 @@ __global__ void __launch_bounds__(DSGX_DECODE_THREADS) k_down_part(DecodeArgs a,
     const int wave = uni((int)(threadIdx.x >> 6)), nw = blockDim.x >> 6;
     ResolveRegs rr;
     if (wave >= nw - NR) resolve_fetch(S, a, wave - (nw - NR), NR, rr);
-    prep<FMT, SHFMT, M>(S, a);
+    prep<FMT, SHFMT>(S, a);
     __syncthreads();
-    if (wave >= nw - NR) resolve<FMT, SHFMT, M>(S, a, wave - (nw - NR), NR, rr);
+    if (wave >= nw - NR) resolve<FMT, SHFMT>(S, a, wave - (nw - NR), NR, rr);
     __syncthreads();
   }
   const int nrouted = uni(S.n);
@@ -818,6 +854,32 @@ __global__ void __launch_bounds__(256) k_down_combine(DecodeArgs a) {
   if (SH) a.ys[i] = sv = a.dsk ? bf16_round(a.dpart[i]) : a.dpart[i];
   else if (a.ysum) sv = a.ys[i];
   if (a.ysum || (a.dsk && SH)) acc = __fadd_rn(acc, sv);  // (DeepSeek: the shared expert last, always)
+  a.yr[i] = acc;
+}
+
+// The same sums after the MFMA kernels' down phase, whose dots are kept by pick: dpart [row m][pick r of topk, by slot][H], then
+// the shared expert's rows [m][H]; fac[8 + m topk + r] = s2 w (0: no such pick, or a weight of 0: nothing is added). A dot that
+// no row's routing asks for is neither stored nor read: by slot and row, as for k_down_combine, eight rows with 58 slots moved 15 MB a
+// layer of hidden 4096, now 2.4 (FP8, four layers of eight rows 1010 -> 972 us; INT4, six rows, 886 -> 862).
+template <bool SH>
+__global__ void __launch_bounds__(256) k_pick_combine(DecodeArgs a) {
+  const int H = a.L.H, topk = a.L.topk, M = a.M;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= M * H) return;
+  const int m = i / H, n = i - m * H;
+  const float* d = a.dpart + (size_t)m * topk * H + n;
+  float v[DSGX_MAX_TOPK], f[DSGX_MAX_TOPK];
+#pragma unroll
+  for (int r = 0; r < DSGX_MAX_TOPK; ++r) v[r] = d[(size_t)min(r, topk - 1) * H], f[r] = r < topk ? a.fac[8 + m * topk + r] : 0.f;
+  const float sh = SH ? a.dpart[(size_t)(M * topk + m) * H + n] : 0.f;
+  float acc = 0.f;
+#pragma unroll
+  for (int r = 0; r < DSGX_MAX_TOPK; ++r)
+    if (f[r] != 0.f) acc = a.dsk ? __fadd_rn(acc, bf16_round(v[r])) : fmaf(f[r], v[r], acc);  // (dsk: see k_down_combine)
+  float sv = 0.f;
+  if (SH) a.ys[i] = sv = a.dsk ? bf16_round(sh) : sh;
+  else if (a.ysum) sv = a.ys[i];
+  if (a.ysum || (a.dsk && SH)) acc = __fadd_rn(acc, sv);
   a.yr[i] = acc;
 }
 
@@ -918,9 +980,9 @@ __global__ void __launch_bounds__(256) k_down(DecodeArgs a, int spc) {
     const int wave = uni((int)(threadIdx.x >> 6)), nw = blockDim.x >> 6;
     ResolveRegs rr;
     if (wave >= nw - NR) resolve_fetch(S, a, wave - (nw - NR), NR, rr);
-    prep<FMT, SHFMT, M>(S, a);
+    prep<FMT, SHFMT>(S, a);
     __syncthreads();
-    if (wave >= nw - NR) resolve<FMT, SHFMT, M>(S, a, wave - (nw - NR), NR, rr);
+    if (wave >= nw - NR) resolve<FMT, SHFMT>(S, a, wave - (nw - NR), NR, rr);
     __syncthreads();
   }
   const int H = a.L.H, gw = uni((int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)));

@@ -15,7 +15,7 @@
 //   * the slices' sums are added in slice order through LDS (one workgroup barrier a round of units), then the epilogue.
 // gate/up: unit = 8 channels, rows interleaved (g0, u0, g1, u1, ...), so that g and u of a channel meet in one lane.
 // down: units are (slot, 16 output rows), cut into equal contiguous ranges a workgroup; the complete dots go to memory
-// as f32 [slot][M][H] and k_down_combine chains them in slot order (as after k_down_part).
+// by row and pick and k_pick_combine chains them in slot order.
 // Every output depends on its own activation row only: a row's bits do not depend on the rows beside it.
 #pragma once
 #include "moe_decode_impl.cuh"
@@ -58,7 +58,8 @@ __host__ __device__ inline int mf_slices(int K, int stepk, int minsteps) {
 }
 __host__ __device__ inline size_t mf_rows_bytes(int M, int K, int pad) { return (size_t)M * ((size_t)K * 2 + pad) + 256; }
 // + one step's weights a wave + the waves' slice sums of two rounds (the lanes of positions < M only: 4 M x 16 bytes a wave)
-__host__ __device__ inline size_t mf_lds_bytes(int M, int K, int pad) { return mf_rows_bytes(M, K, pad) + kMfWaves * 2048 + 2 * kMfWaves * 64 * M; }
+// (rows: the staged ones, the step's M or two slots' 2 M)
+__host__ __device__ inline size_t mf_lds_bytes(int rows, int M, int K, int pad) { return mf_rows_bytes(rows, K, pad) + kMfWaves * 2048 + 2 * kMfWaves * 64 * M; }
 
 // M rows of K bf16 (row m at src + m * ld) to LDS with the padded stride.
 // COHERENT: rows written by other workgroups of the same kernel (h after the grid barrier)
@@ -161,8 +162,8 @@ struct MfUnit {
 // the LDS (units of different slots in one stream); zoff: 256 zero bytes. pre() is called once by every wave, after
 // its first kMfD steps' loads are issued and before anything is read from LDS: the caller waits for and stages the
 // activations there (a workgroup barrier at its end), with the first weights already on their way.
-template <int FMT, int M, class Open, class XOff, class Done, class Pre>
-__device__ __forceinline__ void mf_stream(uint8_t* smem, size_t rows_bytes, uint32_t zoff, int pad, int K, int k0, int ns, int nu, int steps, Open&& open,
+template <int FMT, class Open, class XOff, class Done, class Pre>
+__device__ __forceinline__ void mf_stream(const int M, uint8_t* smem, size_t rows_bytes, uint32_t zoff, int pad, int K, int k0, int ns, int nu, int steps, Open&& open,
                                           XOff&& xoff_of, Done&& done, Pre&& pre) {
   constexpr int STEPK = MfFmt<FMT>::STEPK;
   const uint32_t lane = threadIdx.x & 63;
@@ -376,7 +377,7 @@ __device__ __forceinline__ void mf_stream(uint8_t* smem, size_t rows_bytes, uint
 // expert in another format (INT4 or MXFP4 experts) its first tiles - tile g by workgroup g - stream while the routing is
 // being resolved (mf_shared_early), when nothing else could.
 template <int FMT, int SHFMT, int M, bool UP>
-__device__ __forceinline__ void mf_setup(Step<M>& S, const DecodeArgs& a, uint8_t* mf_smem);
+__device__ __forceinline__ void mf_setup(Step<M, true>& S, const DecodeArgs& a, uint8_t* mf_smem);
 // A unit of a gate/up matrix pair in format F: tile t = channels 8 t .. 8 t + 7, unit rows 2 c and 2 c + 1 gate and up of
 // channel 8 t + c. (BF16: the shared expert's interleaved matrix, whose rows already come in this order.)
 template <int F>
@@ -453,15 +454,17 @@ __device__ __forceinline__ MfUnit mf_open_down(const Slot& T, int t, int H, int 
 // The gate/up epilogue of a unit's complete sums (v4f of lane l: gate, up of channel 8 t + 2 (l / 16) and of the next,
 // activation row l % 16): SwiGLU and the store of h
 template <int SHFMT, int M>
-__device__ __forceinline__ void mf_up_store(Step<M>& S, const DecodeArgs& a, int sl, int t, v4f_t sum, uint32_t lane) {
+__device__ __forceinline__ void mf_up_store(Step<M, true>& S, const DecodeArgs& a, int sl, int t, v4f_t sum, uint32_t lane) {
   constexpr int nsh = SHFMT != 0 ? 1 : 0;
+  const int rows = step_rows<M>(a);
   const int I = a.L.I;
   const int pos = lane & 15, part = lane >> 4;
-  if (pos >= M) return;
+  if (pos >= rows) return;
   const Slot& T = S.slots[sl];
   const float sg = T.g.s2, su = T.u.s2;
   uint32_t h0, h1;
   if (a.dsk) {
+    const int pk = T.shared ? 255 : pick_of<M>(S, sl - nsh, pos);
     // ds41f engine/kernels/moe.cu:519-528: gate and up rounded to bf16, up clamped to +-limit and gate from above,
     // silu(gate) * up, times the row's routing weight (routed slots), rounded to bf16; quantised per 32 when the down
     // phase stages it
@@ -470,7 +473,7 @@ __device__ __forceinline__ void mf_up_store(Step<M>& S, const DecodeArgs& a, int
       up = fminf(fmaxf(up, -a.dsk_limit), a.dsk_limit);
       gt = fminf(gt, a.dsk_limit);
       float h = __fmul_rn(__fdiv_rn(gt, __fadd_rn(1.f, expf(-gt))), up);
-      if (!T.shared) h = __fmul_rn(S.wslot[sl - nsh][pos], h);
+      if (!T.shared) h = __fmul_rn(pk == 255 ? 0.f : S.pw[pk], h);
       return f32_to_bf16_bits(h);
     };
     h0 = hd(sum[0], sum[1]), h1 = hd(sum[2], sum[3]);
@@ -478,7 +481,7 @@ __device__ __forceinline__ void mf_up_store(Step<M>& S, const DecodeArgs& a, int
     h0 = swiglu_bits(bf16_round(__fmul_rn(sum[0], sg)), bf16_round(__fmul_rn(sum[1], su)));
     h1 = swiglu_bits(bf16_round(__fmul_rn(sum[2], sg)), bf16_round(__fmul_rn(sum[3], su)));
   }
-  uint16_t* dst = a.h + ((size_t)T.hslot * M + pos) * I + 8 * t + 2 * part;
+  uint16_t* dst = a.h + ((size_t)T.hslot * rows + pos) * I + 8 * t + 2 * part;
   __hip_atomic_store((DSGX_GLOBAL uint32_t*)(uintptr_t)dst, h0 | (h1 << 16), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -491,15 +494,16 @@ __device__ __forceinline__ void mf_up_store(Step<M>& S, const DecodeArgs& a, int
 #endif
 __host__ __device__ inline int mf_early_tiles(int I, int G) { return DSGX_MF_EARLY ? (I / 8 < G ? I / 8 : G) : 0; }
 template <int FMT, int SHFMT, int M>
-__device__ __forceinline__ void mf_shared_early(Step<M>& S, const DecodeArgs& a, uint8_t* mf_smem) {
+__device__ __forceinline__ void mf_shared_early(Step<M, true>& S, const DecodeArgs& a, uint8_t* mf_smem) {
   constexpr int F = SHFMT, pad = mf_pad(FMT);
+  const int rows = step_rows<M>(a);
   const int H = a.L.H, I = a.L.I, t = blockIdx.x;
   if (t >= mf_early_tiles(I, gridDim.x)) return;
   const uint32_t lane = threadIdx.x & 63;
   const int wave = uni((int)(threadIdx.x >> 6));
   const int ns = mf_slices(H, MfFmt<F>::STEPK, MfFmt<F>::MINSTEPS), KS = H / ns, act = ns < 4 ? ns : 4;
   if (wave >= act) return;
-  const size_t rows_bytes = mf_rows_bytes(M, H, pad);
+  const size_t rows_bytes = mf_rows_bytes(rows, H, pad);
   float* red = reinterpret_cast<float*>(mf_smem + rows_bytes + kMfWaves * 2048);
   // mf_stream's unit u of this wave (u = wave, wave + 8, ...) is K slice wave + act (u / 8)
   auto slice_of = [&](int u) { return (u & 7) + act * (u >> 3); };
@@ -507,27 +511,28 @@ __device__ __forceinline__ void mf_shared_early(Step<M>& S, const DecodeArgs& a,
   auto xoff = [&](int u) { return (uint32_t)(slice_of(u) * KS * 2); };
   auto fin = [&](int u, v4f_t sum) {
     const int pos = lane & 15, part = lane >> 4;
-    if (pos < M) *reinterpret_cast<v4f_t*>(red + ((size_t)slice_of(u) * 4 * M + part * M + pos) * 4) = sum;
+    if (pos < rows) *reinterpret_cast<v4f_t*>(red + ((size_t)slice_of(u) * 4 * rows + part * rows + pos) * 4) = sum;
   };
-  mf_stream<F, M>(mf_smem, rows_bytes, (uint32_t)(M * ((size_t)H * 2 + pad)), pad, H, 0, 1, kMfWaves * (ns / act), KS / MfFmt<F>::STEPK, open, xoff, fin,
+  mf_stream<F>(rows, mf_smem, rows_bytes, (uint32_t)(rows * ((size_t)H * 2 + pad)), pad, H, 0, 1, kMfWaves * (ns / act), KS / MfFmt<F>::STEPK, open, xoff, fin,
                   [] {});
 }
 template <int FMT, int SHFMT, int M>
-__device__ __forceinline__ void mf_shared_early_finish(Step<M>& S, const DecodeArgs& a, uint8_t* mf_smem) {
+__device__ __forceinline__ void mf_shared_early_finish(Step<M, true>& S, const DecodeArgs& a, uint8_t* mf_smem) {
   constexpr int F = SHFMT, pad = mf_pad(FMT);
+  const int rows = step_rows<M>(a);
   const int H = a.L.H, I = a.L.I, t = blockIdx.x;
   if (t >= mf_early_tiles(I, gridDim.x) || threadIdx.x >= 64) return;
   const uint32_t lane = threadIdx.x;
   const int ns = mf_slices(H, MfFmt<F>::STEPK, MfFmt<F>::MINSTEPS);
-  const float* red = reinterpret_cast<const float*>(mf_smem + mf_rows_bytes(M, H, pad) + kMfWaves * 2048);
+  const float* red = reinterpret_cast<const float*>(mf_smem + mf_rows_bytes(rows, H, pad) + kMfWaves * 2048);
   const int pos = lane & 15, part = lane >> 4;
   v4f_t sum = {0.f, 0.f, 0.f, 0.f};
-  if (pos < M)
-    for (int w = 0; w < ns; ++w) sum += *reinterpret_cast<const v4f_t*>(red + ((size_t)w * 4 * M + part * M + pos) * 4);
+  if (pos < rows)
+    for (int w = 0; w < ns; ++w) sum += *reinterpret_cast<const v4f_t*>(red + ((size_t)w * 4 * rows + part * rows + pos) * 4);
   mf_up_store<SHFMT, M>(S, a, 0, t, sum, lane);
 }
 template <int FMT, int SHFMT, int M, bool UP>
-__device__ __forceinline__ void mf_setup(Step<M>& S, const DecodeArgs& a, uint8_t* mf_smem) {
+__device__ __forceinline__ void mf_setup(Step<M, true>& S, const DecodeArgs& a, uint8_t* mf_smem) {
   constexpr int NR = resolver_waves<M>();
 #ifndef DSGX_MF_EARLY_SAME
 #define DSGX_MF_EARLY_SAME 1
@@ -536,16 +541,16 @@ __device__ __forceinline__ void mf_setup(Step<M>& S, const DecodeArgs& a, uint8_
   const int wave = uni((int)(threadIdx.x >> 6)), nw = blockDim.x >> 6;
   ResolveRegs rr;
   if (wave >= nw - NR) resolve_fetch(S, a, wave - (nw - NR), NR, rr);
-  prep<FMT, SHFMT, M>(S, a);
+  prep<FMT, SHFMT>(S, a);
   if constexpr (UP) {
     constexpr int pad = mf_pad(FMT);
-    const int H = a.L.H;
-    if (a.dsk_xq) mf_stage_rows_q(mf_smem, a.dsk_xq, a.dsk_xs, M, H, pad);
-    else mf_stage_rows<false>(mf_smem, a.x, H, M, H, pad);
-    mf_zero_bytes(mf_smem + (size_t)M * ((size_t)H * 2 + pad));
+    const int H = a.L.H, rows = step_rows<M>(a);
+    if (a.dsk_xq) mf_stage_rows_q(mf_smem, a.dsk_xq, a.dsk_xs, rows, H, pad);
+    else mf_stage_rows<false>(mf_smem, a.x, H, rows, H, pad);
+    mf_zero_bytes(mf_smem + (size_t)rows * ((size_t)H * 2 + pad));
   }
   __syncthreads();
-  if (wave >= nw - NR) resolve<FMT, SHFMT, M>(S, a, wave - (nw - NR), NR, rr);
+  if (wave >= nw - NR) resolve<FMT, SHFMT>(S, a, wave - (nw - NR), NR, rr);
   else if constexpr (EARLY) mf_shared_early<FMT, SHFMT, M>(S, a, mf_smem);
   __syncthreads();
   if constexpr (EARLY) {
@@ -557,9 +562,9 @@ __device__ __forceinline__ void mf_setup(Step<M>& S, const DecodeArgs& a, uint8_
 // SHFMT: 0 (no fused shared expert), FMT (slot 0 streams with the routed slots) or another format (slot 0 first, in a
 // stream of its own)
 template <int FMT, int SHFMT, int M>
-__device__ __forceinline__ void mf_up_phase(Step<M>& S, const DecodeArgs& a, uint8_t* mf_smem) {
+__device__ __forceinline__ void mf_up_phase(Step<M, true>& S, const DecodeArgs& a, uint8_t* mf_smem) {
   constexpr int nsh = SHFMT != 0 ? 1 : 0;
-  const int H = a.L.H, I = a.L.I;
+  const int H = a.L.H, I = a.L.I, rows = step_rows<M>(a);
   const uint32_t lane = threadIdx.x & 63;
   const int wave = uni((int)(threadIdx.x >> 6));
   constexpr int pad = mf_pad(FMT);
@@ -584,7 +589,7 @@ __device__ __forceinline__ void mf_up_phase(Step<M>& S, const DecodeArgs& a, uin
       const int q = t0 + g + u * G, sl = uni(q / tiles);
       done(s0 + sl, q - sl * tiles, sum);
     };
-    mf_stream<F, M>(mf_smem, mf_rows_bytes(M, H, pad), (uint32_t)(M * ((size_t)H * 2 + pad)), pad, H, k0, ns, mine, KS / MfFmt<F>::STEPK, open,
+    mf_stream<F>(rows, mf_smem, mf_rows_bytes(rows, H, pad), (uint32_t)(rows * ((size_t)H * 2 + pad)), pad, H, k0, ns, mine, KS / MfFmt<F>::STEPK, open,
                     [](int) { return 0u; }, fin, [] {});
   };
   const int nrouted = uni(S.n);
@@ -615,23 +620,19 @@ __device__ __forceinline__ void mf_up_phase(Step<M>& S, const DecodeArgs& a, uin
 // The units (slot, tile of 16 output rows) are cut into equal contiguous ranges a workgroup; a shared slot in another
 // format counts WSH units a tile (BF16 beside INT4: 3.5 times the bytes, but streamed at the memory's rate where an INT4
 // tile waits for the vector unit: twice the time, measured). A workgroup's range is walked in segments of
-// up to two slots, a stream each (with no more slots than workgroups, the whole range is one segment): the h rows of
+// up to two slots (one, for many rows), a stream each (with no more slots than workgroups, the whole range is one segment): the h rows of
 // the segment's slots are staged together and the ring runs on across the slot boundary. FUSED: h was written by this
 // launch; the first segment's weights are requested before the grid barrier is waited for.
 template <int FMT, int SHFMT, int M, bool FUSED>
-__device__ __forceinline__ void mf_down_phase(Step<M>& S, const DecodeArgs& a, uint8_t* mf_smem) {
+__device__ __forceinline__ void mf_down_phase(Step<M, true>& S, const DecodeArgs& a, uint8_t* mf_smem) {
   constexpr int nsh = SHFMT != 0 ? 1 : 0;
   constexpr bool SH2 = SHFMT != 0 && SHFMT != FMT;
   constexpr int WSH = 2;
-  const int H = a.L.H, I = a.L.I;
+  const int H = a.L.H, I = a.L.I, rows = step_rows<M>(a), topk = a.L.topk;
   const uint32_t lane = threadIdx.x & 63;
   const int wave = uni((int)(threadIdx.x >> 6));
   const int nrouted = uni(S.n);
-  if (blockIdx.x == 0) {  // the slot table for k_down_combine
-    if (threadIdx.x == 0) reinterpret_cast<int*>(a.fac)[0] = nrouted;
-    for (int i = threadIdx.x; i < nrouted * M; i += blockDim.x)
-      a.fac[8 + (i / M) * 8 + i % M] = __fmul_rn(S.slots[nsh + i / M].d.s2, S.wslot[i / M][i % M]);
-  }
+  if (blockIdx.x == 0 && (int)threadIdx.x < rows * topk) a.fac[8 + threadIdx.x] = S.pfac[threadIdx.x];  // (for k_pick_combine)
   const int tps = H / 16;  // tiles a slot
   const int s0 = SH2 ? 1 : 0, nsl = nsh + nrouted - s0;  // the slots in format FMT
   const long csh = SH2 ? (long)WSH * tps : 0;
@@ -639,7 +640,8 @@ __device__ __forceinline__ void mf_down_phase(Step<M>& S, const DecodeArgs& a, u
   const long c_lo = total * blockIdx.x / gridDim.x, c_hi = total * (blockIdx.x + 1) / gridDim.x;
   constexpr int pad = mf_pad(FMT);
   const size_t rs = (size_t)I * 2 + pad;
-  const size_t rows_bytes = mf_rows_bytes(2 * M, I, pad);
+  const int seg = M <= 8 ? 2 : a.down_slots;  // slots a segment
+  const size_t rows_bytes = mf_rows_bytes(seg * rows, I, pad);
   bool waited = !FUSED;  // the grid barrier is behind this workgroup
   // units [ua, ub) of the slots from sl0 on (unit = slot * tps + tile, slots counted from sl0), all in format F
   auto run = [&](auto fmt_tag, int sl0, int ua, int ub) {
@@ -650,11 +652,11 @@ __device__ __forceinline__ void mf_down_phase(Step<M>& S, const DecodeArgs& a, u
       else __syncthreads();
       waited = true;
       for (int j = 0; j < nss; ++j)
-        mf_stage_rows<FUSED>(mf_smem + (size_t)j * M * rs, a.h + (size_t)S.slots[sl0 + j].hslot * M * I, I, M, I, pad);
-      mf_zero_bytes(mf_smem + (size_t)2 * M * rs);
+        mf_stage_rows<FUSED>(mf_smem + (size_t)j * rows * rs, a.h + (size_t)S.slots[sl0 + j].hslot * rows * I, I, rows, I, pad);
+      mf_zero_bytes(mf_smem + (size_t)seg * rows * rs);
       __syncthreads();
       if (a.dsk) {  // w2's input is act_quant(h): e4m3 with a ue8m0 scale per 32 values (moe.cu:529-534), again bf16 values
-        mf_quant_rows(mf_smem, nss * M, I, rs);
+        mf_quant_rows(mf_smem, nss * rows, I, rs);
         __syncthreads();
       }
     };
@@ -663,12 +665,15 @@ __device__ __forceinline__ void mf_down_phase(Step<M>& S, const DecodeArgs& a, u
       const int j = uni((ua + u) / tps);
       return mf_open_down<F>(S.slots[sl0 + j], ua + u - j * tps, H, I, k0, lane);
     };
-    auto xoff = [&](int u) { return (uint32_t)(uni((ua + u) / tps) * M * rs); };
+    auto xoff = [&](int u) { return (uint32_t)(uni((ua + u) / tps) * rows * rs); };
     auto fin = [&](int u, v4f_t sum) {
       const int j = uni((ua + u) / tps), t = ua + u - j * tps, pos = lane & 15, part = lane >> 4;
-      if (pos < M) *reinterpret_cast<v4f_t*>(a.dpart + ((size_t)(sl0 + j) * M + pos) * H + 16 * t + 4 * part) = sum;
+      const int sl = sl0 + j;
+      int at = 255;  // the dot's place among the picks' (none: the row did not pick the slot's expert)
+      if (pos < rows) at = nsh && sl == 0 ? rows * topk + pos : pick_of<M>(S, sl - nsh, pos);
+      if (at != 255) *reinterpret_cast<v4f_t*>(a.dpart + (size_t)at * H + 16 * t + 4 * part) = sum;
     };
-    mf_stream<F, M>(mf_smem, rows_bytes, (uint32_t)(2 * M * rs), pad, I, k0, ns, ub - ua, KS / MfFmt<F>::STEPK, open, xoff, fin, pre);
+    mf_stream<F>(rows, mf_smem, rows_bytes, (uint32_t)(seg * rows * rs), pad, I, k0, ns, ub - ua, KS / MfFmt<F>::STEPK, open, xoff, fin, pre);
   };
   if constexpr (SH2) {  // the shared slot's tiles whose first cost unit lies in this workgroup's range
     const long lo = c_lo < csh ? c_lo : csh, hi = c_hi < csh ? c_hi : csh;
@@ -676,8 +681,8 @@ __device__ __forceinline__ void mf_down_phase(Step<M>& S, const DecodeArgs& a, u
     if (tb > ta) run(std::integral_constant<int, SHFMT>{}, 0, ta, tb);
   }
   const int u_lo = (int)((c_lo > csh ? c_lo : csh) - csh), u_hi = (int)((c_hi > csh ? c_hi : csh) - csh);
-  for (int sl = u_lo / tps; sl * tps < u_hi; sl += 2) {  // (the same for every wave of the workgroup)
-    const int ua = max(u_lo, sl * tps) - sl * tps, ub = min(u_hi, (sl + 2) * tps) - sl * tps;
+  for (int sl = u_lo / tps; sl * tps < u_hi; sl += seg) {  // (the same for every wave of the workgroup)
+    const int ua = max(u_lo, sl * tps) - sl * tps, ub = min(u_hi, (sl + seg) * tps) - sl * tps;
     run(std::integral_constant<int, FMT>{}, s0 + sl, ua, ub);
   }
   if (!waited) grid_barrier(a.bar, S.gen, a.spin_limit);  // (a workgroup without a unit)
@@ -686,14 +691,14 @@ __device__ __forceinline__ void mf_down_phase(Step<M>& S, const DecodeArgs& a, u
 template <int FMT, int SHFMT, int M>
 __global__ void __launch_bounds__(kMfThreads) k_up_mfma(DecodeArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t mf_smem[];  // (read and written 16 bytes at a time)
-  __shared__ Step<M> S;
+  __shared__ Step<M, true> S;
   mf_setup<FMT, SHFMT, M, true>(S, a, mf_smem);
   mf_up_phase<FMT, SHFMT, M>(S, a, mf_smem);
 }
 template <int FMT, int SHFMT, int M>
 __global__ void __launch_bounds__(kMfThreads) k_down_mfma(DecodeArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t mf_smem[];  // (read and written 16 bytes at a time)
-  __shared__ Step<M> S;
+  __shared__ Step<M, true> S;
   mf_setup<FMT, SHFMT, M, false>(S, a, mf_smem);
   mf_down_phase<FMT, SHFMT, M, false>(S, a, mf_smem);
 }
@@ -701,44 +706,65 @@ __global__ void __launch_bounds__(kMfThreads) k_down_mfma(DecodeArgs a) {
 template <int FMT, int SHFMT, int M>
 __global__ void __launch_bounds__(kMfThreads) k_decode_mfma(DecodeArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t mf_smem[];  // (read and written 16 bytes at a time)
-  __shared__ Step<M> S;
+  __shared__ Step<M, true> S;
   if (threadIdx.x == 0) S.gen = grid_barrier_gen(a.bar);
   mf_setup<FMT, SHFMT, M, true>(S, a, mf_smem);
   mf_up_phase<FMT, SHFMT, M>(S, a, mf_smem);
   mf_down_phase<FMT, SHFMT, M, true>(S, a, mf_smem);
 }
 
+// The LDS of a step's phases (slots: the slots whose h the down phase stages together), and the rows that the kernels take at
+// once: a step of 9 to 16 rows is one pass where the staged rows and the tables beside them fit a CU's LDS, else as many rows as
+// do and the rest (moe_decode_at). One pass reads the weights of the experts that both would have read once: FP8, 13 rows of top-8
+// of 256, hidden 4096, intermediate 2048: 95 expert reads a layer in passes of 8 and 5, 87 in one, four layers 1697 -> 1600 us;
+// hidden 2048: 9 rows 730 -> 623, 12 rows 910 -> 768.
+template <int FMT>
+size_t mf_step_lds(int rows, int H, int I, int parts, int slots) {
+  const size_t up = mf_lds_bytes(rows, rows, H, mf_pad(FMT)), down = mf_lds_bytes(slots * rows, rows, I, mf_pad(FMT));
+  return parts == 1 ? up : parts == 2 ? down : std::max(up, down);
+}
+template <int FMT>
+bool mf_fits(int rows, int H, int I, int slots) { return mf_step_lds<FMT>(rows, H, I, 3, slots) + sizeof(Step<16, true>) + 64 <= 160 * 1024; }
+template <int FMT>
+int mf_max_rows(int H, int I, int M) {
+  while (M > 8 && !mf_fits<FMT>(M, H, I, 1)) --M;
+  return M;
+}
+
 template <int FMT, int SHFMT, int M>
-int launch_decode_mfma(const DecodeArgs& a, int parts, hipStream_t st) {
-  const int H = a.L.H, I = a.L.I, cus = num_cus_cached();
+int launch_decode_mfma(const DecodeArgs& args, int parts, hipStream_t st) {
+  const int H = args.L.H, I = args.L.I, cus = num_cus_cached();
+  DecodeArgs a = args;
+  a.down_slots = M <= 8 || mf_fits<FMT>(a.M, H, I, 2) ? 2 : 1;
   if (H % 256 || I % 256)
     return fail(DSGX_EINVAL, "moe_decode (variant 1): hidden %d, intermediate %d (whole steps of 256 k)", H, I);
+  auto combine = [&] { hipLaunchKernelGGL((k_pick_combine<SHFMT != 0>), dim3((a.M * H + 255) / 256), dim3(256), 0, st, a); };
   if (parts == 3) {
     auto kern = k_decode_mfma<FMT, SHFMT, M>;
-    const size_t lds = std::max(mf_lds_bytes(M, H, mf_pad(FMT)), mf_lds_bytes(2 * M, I, mf_pad(FMT)));
+    const size_t lds = mf_step_lds<FMT>(a.M, H, I, 3, a.down_slots);
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
     int per_cu = 0;  // the grid barrier needs every workgroup resident
     DSGX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kMfThreads, lds));
     if (per_cu >= 1) {
       hipLaunchKernelGGL(kern, dim3(cus), dim3(kMfThreads), lds, st, a);
-      hipLaunchKernelGGL((k_down_combine<M, SHFMT != 0>), dim3((M * H + 255) / 256), dim3(256), 0, st, a);
+      combine();
       DSGX_HIP(hipGetLastError());
       return DSGX_OK;
     }
   }
   if (parts & 1) {
     auto kern = k_up_mfma<FMT, SHFMT, M>;
-    const size_t lds = mf_lds_bytes(M, H, mf_pad(FMT));
+    const size_t lds = mf_step_lds<FMT>(a.M, H, I, 1, a.down_slots);
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
     hipLaunchKernelGGL(kern, dim3(cus), dim3(kMfThreads), lds, st, a);
     DSGX_HIP(hipGetLastError());
   }
   if (parts & 2) {
     auto kern = k_down_mfma<FMT, SHFMT, M>;
-    const size_t lds = mf_lds_bytes(2 * M, I, mf_pad(FMT));
+    const size_t lds = mf_step_lds<FMT>(a.M, H, I, 2, a.down_slots);
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
     hipLaunchKernelGGL(kern, dim3(cus), dim3(kMfThreads), lds, st, a);
-    hipLaunchKernelGGL((k_down_combine<M, SHFMT != 0>), dim3((M * H + 255) / 256), dim3(256), 0, st, a);
+    combine();
     DSGX_HIP(hipGetLastError());
   }
   return DSGX_OK;
@@ -756,6 +782,7 @@ int launch_decode_mfma_m(const DecodeArgs& a, int parts, hipStream_t st) {
     case 7: return launch_decode_mfma<FMT, SHFMT, 7>(a, parts, st);
     case 8: return launch_decode_mfma<FMT, SHFMT, 8>(a, parts, st);
   }
+  if (a.M >= 9 && a.M <= DSGX_MAX_ROWS) return launch_decode_mfma<FMT, SHFMT, 16>(a, parts, st);
   return fail(DSGX_EUNSUPPORTED, "moe_decode (variant 1): %d rows", a.M);
 }
 

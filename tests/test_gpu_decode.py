@@ -400,3 +400,23 @@ def test_decode_status_reports_a_timeout_and_repairs_the_workspace():
             got = gpu.decode_layer(dl, x, idx, w, 2, ws=ws)
             assert np.array_equal(got[0].view(np.uint32), want[0].view(np.uint32)) and np.array_equal(got[1].view(np.uint32), want[1].view(np.uint32))
         lib.decode_status(dl.w, ws)
+
+
+@pytest.mark.parametrize("fmt,H,I,E,topk,shared,rows", [(abi.FMT_FP8, 2048, 2048, 48, 8, "fp8", (9, 13, 14, 16)), (abi.FMT_FP8, 4096, 512, 32, 8, None, (13, 16)),
+                                                       (abi.FMT_INT4, 2048, 2048, 24, 8, "bf16", (11, 16)), (abi.FMT_INT4, 6144, 512, 16, 4, None, (9, 10))],
+                         ids=["fp8", "fp8-two-passes", "int4", "int4-H6144"])
+def test_decode_nine_to_sixteen_rows_in_one_pass(fmt, H, I, E, topk, shared, rows):
+    """9 to 16 rows in one pass of the MFMA kernels, with the h of two slots staged together and of one, and as many rows as LDS
+    holds and the rest: every row's bits are those of the row alone; fused routing the bits of given picks"""
+    hl, dl = _layer(fmt, H, I, E, topk, 3, shared, seed=11)
+    x, logits, idx, w = rows_and_routing(37, max(rows), H, E, topk, 2.5)
+    alone = [gpu.decode_layer(dl, x[m:m + 1], idx[m:m + 1], w[m:m + 1], 1, up=1)[:2] for m in range(max(rows))]
+    for M in rows:
+        ws = gpu.empty(lib.decode_ws_bytes(dl.w), 0)
+        runs = [gpu.decode_layer(dl, x[:M], idx[:M], w[:M], M, ws=ws, up=1)[:2],
+                gpu.decode_layer(dl, x[:M], None, None, M, ws=ws, logits=gpu.dev(logits[:M]), route_scale=2.5, up=1)[:2]]
+        for yr, ys in runs:
+            for m in range(M):
+                assert np.array_equal(yr[m].view(np.uint32), alone[m][0][0].view(np.uint32)), (M, m)
+                if hl.has_shared:
+                    assert np.array_equal(ys[m].view(np.uint32), alone[m][1][0].view(np.uint32)), (M, m)
