@@ -17,12 +17,10 @@ constexpr int kWave = 64;
 __device__ __forceinline__ float bf16_bits_to_f32(uint32_t b) { return __uint_as_float(b << 16); }
 // Round to nearest even, the contract's integer form (engine/experts/formats.cuh:33-37 of the reference): used where
 // a single value is rounded (epilogues); the packed hardware conversion below is used in the streaming loops.
-__device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
-  uint32_t u = __float_as_uint(f);
-  u += 0x7FFFu + ((u >> 16) & 1u);
-  return u >> 16;
-}
-__device__ __forceinline__ float bf16_round(float f) { return __uint_as_float(f32_to_bf16_bits(f) << 16); }
+// f32 -> bf16, round to nearest even: v_cvt_pk_bf16_f32, one instruction (two for the rounded f32) where adding half a step by hand
+// is four; the same bits for every number (all 2^32 compared), and a NaN stays one
+__device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
+__device__ __forceinline__ float bf16_round(float f) { return (float)(__bf16)f; }
 // two f32 -> packed bf16 (lo = a, hi = b), round to nearest even: v_cvt_pk_bf16_f32
 __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
   bf16x2_t v = {(__bf16)a, (__bf16)b};
@@ -494,21 +492,55 @@ __device__ __forceinline__ void route_row(const float (&logit)[kRouteRJ], const 
   else route_row_nj<kRouteRJ>(logit, bias, E, topk, scale, score_fn, lane, id_out, w_out);
 }
 
+__device__ __forceinline__ float bf16_lo(uint32_t p) { return __uint_as_float(p << 16); }  // the values of a packed pair
+__device__ __forceinline__ float bf16_hi(uint32_t p) { return __uint_as_float(p & 0xFFFF0000u); }
+// silu(g) = g / (1 + e^-g) of four bf16 values, the division IEEE's: by the divisor's reciprocal and one correction step where |g| < 60
+// (the divisor is then in [1, 2^87]: no scaling; equal to the division for every bf16 g, all compared, but the sign of a zero, which
+// is g's), by the division itself if a value of the wave lies outside. The prefill GEMMs' epilogues are bound by the vector unit, and
+// beside them the tiles' loads wait: with the conversions above, ~20 instructions a value less, FP8 chunk of 256 rows an expert 2679
+// -> 2644 us, Zipf T = 8192 3063 -> 3000; INT4 T = 1111 1590 -> 1509.
+__device__ __forceinline__ void silu4(const float (&g)[4], float (&s)[4]) {
+  float d[4];
+  bool far = false;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    d[i] = __fadd_rn(1.f, expf(-g[i]));
+    const float r = __builtin_amdgcn_rcpf(d[i]), q = __fmul_rn(g[i], r);
+    s[i] = __builtin_copysignf(fmaf(fmaf(-q, d[i], g[i]), r, q), g[i]);
+    far |= !(fabsf(g[i]) < 60.f);
+  }
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(far) != 0, 0)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[i] = __fdiv_rn(g[i], d[i]);
+  }
+}
+// Four of swiglu_bits' values, packed. fast: with the hardware's exponential and reciprocal (each within 1 ulp) in place of expf() and
+// the IEEE division: silu before its rounding to bf16 is within a few f32 ulp of the exact value (the reference's own expf() is
+// specified to 2 ulp), so the bf16 it rounds to differs from swiglu_bits' once in ~10^4 values, by one bf16 step.
+__device__ __forceinline__ uint2 swiglu4(const float (&g)[4], const float (&u)[4], bool fast) {
+  float s[4];
+  if (fast) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[i] = __fmul_rn(g[i], __builtin_amdgcn_rcpf(__fadd_rn(1.f, __builtin_amdgcn_exp2f(__fmul_rn(g[i], -1.44269504088896341f)))));
+  } else {
+    silu4(g, s);
+  }
+  const uint32_t a = pack_bf16(s[0], s[1]), b = pack_bf16(s[2], s[3]);
+  return make_uint2(pack_bf16(__fmul_rn(bf16_lo(a), u[0]), __fmul_rn(bf16_hi(a), u[1])), pack_bf16(__fmul_rn(bf16_lo(b), u[2]), __fmul_rn(bf16_hi(b), u[3])));
+}
+// the accumulators' four values times a matrix's scale, rounded to bf16
+template <class V>
+__device__ __forceinline__ void bf16_round4(const V& acc, float s2, float (&o)[4]) {
+  const uint32_t a = pack_bf16(__fmul_rn(acc[0], s2), __fmul_rn(acc[1], s2)), b = pack_bf16(__fmul_rn(acc[2], s2), __fmul_rn(acc[3], s2));
+  o[0] = bf16_lo(a), o[1] = bf16_hi(a), o[2] = bf16_lo(b), o[3] = bf16_hi(b);
+}
+
 // h = bf16(bf16(silu(g)) * u), g and u already bf16 values (engine/experts/decode.cu:110-113 of the reference)
 __device__ __forceinline__ uint32_t swiglu_bits(float g, float u) {
   const float sl = bf16_round(__fdiv_rn(g, __fadd_rn(1.f, expf(-g))));
   return f32_to_bf16_bits(__fmul_rn(sl, u));
 }
 
-// The same with the hardware's exponential and reciprocal (each within 1 ulp) in place of expf() and the IEEE division:
-// silu before its rounding to bf16 is within a few f32 ulp of the exact value (the reference's own expf() is specified to
-// 2 ulp), so the bf16 it rounds to differs from swiglu_bits' once in ~10^4 values, by one bf16 step. For the prefill
-// GEMMs' epilogues, where the exact form's ~20 extra instructions a value are a tenth of the kernel.
-__device__ __forceinline__ uint32_t swiglu_fast_bits(float g, float u) {
-  const float e = __builtin_amdgcn_exp2f(__fmul_rn(g, -1.44269504088896341f));
-  const float sl = bf16_round(__fmul_rn(g, __builtin_amdgcn_rcpf(__fadd_rn(1.f, e))));
-  return f32_to_bf16_bits(__fmul_rn(sl, u));
-}
 // v / d by d's reciprocal (r = rcp(d), within 1 ulp) and one correction step: the quotient rounded to nearest for every v
 // and d met here (normal numbers far from the format's ends; the IEEE sequence spends twice the instructions on scaling
 // for the ends). Checked against the division bit for bit in tests.

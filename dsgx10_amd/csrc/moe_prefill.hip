@@ -565,11 +565,9 @@ __global__ void __launch_bounds__(kGemmThreads) k_pf_gemm16(Gemm16Args g) {
     for (int mt = 0; mt < 8; ++mt) {
       const int pos = m0 + 16 * mt + r16;
       if (pos >= mend) continue;
-      uint32_t hb[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        hb[q] = swiglu_bits(bf16_round(__fmul_rn(acc[0][mt][q], s2a)), bf16_round(__fmul_rn(acc[1][mt][q], s2b)));
-      *reinterpret_cast<uint2*>(g.h + (size_t)pos * I + n0 + 4 * part) = make_uint2(hb[0] | (hb[1] << 16), hb[2] | (hb[3] << 16));
+      float gv[4], uv[4];
+      bf16_round4(acc[0][mt], s2a, gv), bf16_round4(acc[1][mt], s2b, uv);
+      *reinterpret_cast<uint2*>(g.h + (size_t)pos * I + n0 + 4 * part) = swiglu4(gv, uv, false);
     }
   } else {
     const int H = g.L.H;

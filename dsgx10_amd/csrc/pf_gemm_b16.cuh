@@ -47,13 +47,11 @@ __device__ __forceinline__ void store_h(uint8_t* smem, const v4f_t (&acc)[2][8],
   for (int mt = 0; mt < 8; ++mt) {
     if (mt >= nmt) break;
     const int p = 16 * mt + r16;
-    uint32_t hb[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      hb[q] = swiglu_bits(bf16_round(__fmul_rn(acc[0][mt][q], s2a)), bf16_round(__fmul_rn(acc[1][mt][q], s2b)));
+    float gv[4], uv[4];
+    bf16_round4(acc[0][mt], s2a, gv), bf16_round4(acc[1][mt], s2b, uv);
     const int ch = 16 * wave + 4 * part;
     const int piece = (ch >> 3) ^ (p & 15);
-    *reinterpret_cast<uint2*>(smem + p * 256 + piece * 16 + (ch & 4) * 2) = make_uint2(hb[0] | (hb[1] << 16), hb[2] | (hb[3] << 16));
+    *reinterpret_cast<uint2*>(smem + p * 256 + piece * 16 + (ch & 4) * 2) = swiglu4(gv, uv, false);
   }
   __syncthreads();
   const int l16 = tid & 15;

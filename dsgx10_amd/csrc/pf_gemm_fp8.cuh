@@ -321,15 +321,11 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
       const int p = 16 * (pg + WP * j) + r16;  // position within the tile
 #pragma unroll
       for (int b = 0; b < S::RA / 2; ++b) {
-        uint32_t hb[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float gv = bf16_round(__fmul_rn(acc[2 * b][j][q], s2a)), uv = bf16_round(__fmul_rn(acc[2 * b + 1][j][q], s2b));
-          hb[q] = fast ? swiglu_fast_bits(gv, uv) : swiglu_bits(gv, uv);
-        }
+        float gv[4], uv[4];
+        bf16_round4(acc[2 * b][j], s2a, gv), bf16_round4(acc[2 * b + 1][j], s2b, uv);
         const int ch = 16 * (S::RA / 2 * rg + b) + 4 * part;  // first of the lane's four channels (of the workgroup's 128)
         const int piece = (ch >> 3) ^ (p & 15);
-        *reinterpret_cast<uint2*>(smem + p * 256 + piece * 16 + (ch & 4) * 2) = make_uint2(hb[0] | (hb[1] << 16), hb[2] | (hb[3] << 16));
+        *reinterpret_cast<uint2*>(smem + p * 256 + piece * 16 + (ch & 4) * 2) = swiglu4(gv, uv, fast);
       }
     }
     __syncthreads();

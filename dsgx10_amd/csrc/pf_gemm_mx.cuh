@@ -315,19 +315,19 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
       const float wv = (g.posw && m0 + p < mend) ? g.posw[m0 + p] : 1.f;
 #pragma unroll
       for (int b = 0; b < S::RA / 2; ++b) {
-        uint32_t hb[4];
+        float gt[4], up[4], hv[4];
+        bf16_round4(acc[2 * b][j], 1.f, gt), bf16_round4(acc[2 * b + 1][j], 1.f, up);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) up[q] = fminf(fmaxf(up[q], -lim), lim), gt[q] = fminf(gt[q], lim);
+        silu4(gt, hv);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          float gt = bf16_round(acc[2 * b][j][q]), up = bf16_round(acc[2 * b + 1][j][q]);
-          up = fminf(fmaxf(up, -lim), lim);
-          gt = fminf(gt, lim);
-          float hv = __fmul_rn(__fdiv_rn(gt, __fadd_rn(1.f, expf(-gt))), up);
-          if (g.posw) hv = __fmul_rn(wv, hv);
-          hb[q] = f32_to_bf16_bits(hv);
+          hv[q] = __fmul_rn(hv[q], up[q]);
+          if (g.posw) hv[q] = __fmul_rn(wv, hv[q]);
         }
         const int ch = 16 * (S::RA / 2 * rg + b) + 4 * part;
         const int piece = (ch >> 3) ^ (p & 15);
-        *reinterpret_cast<uint2*>(smem + p * 256 + piece * 16 + (ch & 4) * 2) = make_uint2(hb[0] | (hb[1] << 16), hb[2] | (hb[3] << 16));
+        *reinterpret_cast<uint2*>(smem + p * 256 + piece * 16 + (ch & 4) * 2) = make_uint2(pack_bf16(hv[0], hv[1]), pack_bf16(hv[2], hv[3]));
       }
     }
     __syncthreads();
@@ -371,8 +371,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
       if (j >= nj) break;
 #pragma unroll
       for (int t = 0; t < S::RA; ++t) {
-        const uint32_t lo = f32_to_bf16_bits(acc[t][j][0]) | (f32_to_bf16_bits(acc[t][j][1]) << 16);
-        const uint32_t hi = f32_to_bf16_bits(acc[t][j][2]) | (f32_to_bf16_bits(acc[t][j][3]) << 16);
+        const uint32_t lo = pack_bf16(acc[t][j][0], acc[t][j][1]), hi = pack_bf16(acc[t][j][2], acc[t][j][3]);
         const int c = 2 * t + (part >> 1);  // the 16-byte piece: rows 16 t + 4 part ... are bytes 32 t + 8 part ...
         *reinterpret_cast<uint2*>(my + r16 * RB + ((c ^ r16) & (PC - 1)) * 16 + (part & 1) * 8) = make_uint2(lo, hi);
       }

@@ -406,3 +406,32 @@ def test_prefill_int4_bf16_shared_expert_tiles(H, I, T):
         lib.moe_prefill(dl.w, gpu.dev(x), gpu.dev(idx), gpu.dev(w), T, ws, r2, s2, phases=ph)
     assert np.array_equal(gpu.host(r2, np.uint32, (T, H)), yr.view(np.uint32))
     assert np.array_equal(gpu.host(s2, np.uint32, (T, H)), ys.view(np.uint32))
+
+
+def test_prefill_silu_at_the_ends_of_its_fast_division():
+    """the prefill epilogues divide by the reciprocal where |gate| < 60 and by IEEE's division beyond (common.cuh: silu4); the decode
+    kernels by IEEE's everywhere: h of a BF16 shared expert whose gates are given values, on both sides of +-60, denormal results,
+    zeros and infinities, from both"""
+    H, I, E, topk = 256, 256, 8, 2
+    hl = helpers.make_layer(abi.FMT_INT4, H, I, E, topk, 4, seed=27, shared="bf16")
+    dl = hl.upload()
+    v = np.concatenate([np.float32([0, -0.0, 1e-40, -1e-40, 59.75, -59.75, 60, -60, 60.25, -60.25, 87, -87, 88.5, -88.5, 103, -103, 1e30, -1e30, 1e38, -1e38]),
+                        np.linspace(-70, 70, I - 20, dtype=np.float32)])
+    bgu = np.zeros((2 * I, H), np.uint16)
+    bgu[0::2, 0] = orc.f32_to_bf16(v)           # gate of channel c: v[c] x[0]
+    bgu[1::2, 1] = orc.f32_to_bf16(np.float32([1.0]))[0]  # up: x[1]
+    keep = gpu.dev(bgu)
+    dl.w.sh.bgu = keep.data_ptr()
+    x, _, idx, w = helpers.rows_and_routing(31, 1, H, E, topk, 2.5)
+    x[:] = 0
+    x[0, :2] = orc.f32_to_bf16(np.float32([1.0, 3.0]))
+    ws, yr, ys = gpu.empty(lib.prefill_ws_bytes(dl.w, 1), 0), gpu.empty(H * 4), gpu.empty(H * 4)
+    lib.moe_prefill(dl.w, gpu.dev(x), gpu.dev(idx), gpu.dev(w), 1, ws, yr, ys, act_fp8=False)
+    pv = lib.prefill_view(dl.w, ws, 1)
+    h = gpu.host(gpu.view(ws, pv.hsh, I * 2), np.uint16, (I,))
+    _, _, wd = gpu.decode_layer(dl, x, idx, w, 1, up=1)
+    assert np.array_equal(h, gpu.h_of(wd, dl, 1, topk)[-1][0])
+    g = orc.bf16_to_f32(orc.f32_to_bf16(v)).astype(np.float64)
+    with np.errstate(over="ignore"):
+        ref = 3.0 * (g / (1.0 + np.exp(-g)))
+    assert np.allclose(orc.bf16_to_f32(h), ref, rtol=2.0 ** -6, atol=1e-37)
