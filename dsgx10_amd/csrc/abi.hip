@@ -104,11 +104,9 @@ __global__ void __launch_bounds__(256) k_finalize(const float* __restrict__ R, c
 
 // The residual add and the next layer's RMSNorm after an MoE (or MLP) step, one workgroup a row (addnorm.cuh)
 __global__ void __launch_bounds__(256) k_add_norm(NormIn a, int H) {
+  extern __shared__ uint4 xs[];  // the row: H bf16 values
   __shared__ float red[4];
-  const int row = blockIdx.x;
-  add_norm_row(a, row, H, red, a.xn != nullptr,
-               [&](int q, u32x4_t v) { if (a.res_out) *reinterpret_cast<u32x4_t*>(a.res_out + (size_t)row * H + 8 * q) = v; },
-               [&](int q, u32x4_t v) { *reinterpret_cast<u32x4_t*>(a.xn + (size_t)row * H + 8 * q) = v; });
+  add_norm_rows<1>(a, blockIdx.x, H, xs, red, a.xn != nullptr, true, [](int, int q) { return q; });
 }
 
 // INT4 canonical tensors -> the contract's bf16 weight, one thread a group of 32 (the subtract-first form, exact for
@@ -289,7 +287,7 @@ int dsgx_add_norm(const float* part, const float* part2, int M, int H, const uin
   if (H < 2048 || H % 2048 || H > 16384) return fail(DSGX_EINVAL, "add_norm: hidden %d (a multiple of 2048 up to 16384)", H);
   if (xn && !w) return fail(DSGX_EINVAL, "add_norm: the norm needs its weight");
   if (!xn && !res_out) return fail(DSGX_EINVAL, "add_norm: no output");
-  hipLaunchKernelGGL(k_add_norm, dim3(M), dim3(256), 0, static_cast<hipStream_t>(stream), NormIn{part, part2, res, res_out, w, xn, eps, round2}, H);
+  hipLaunchKernelGGL(k_add_norm, dim3(M), dim3(256), (size_t)H * 2, static_cast<hipStream_t>(stream), NormIn{part, part2, res, res_out, w, xn, eps, round2}, H);
   DSGX_HIP(hipGetLastError());
   return DSGX_OK;
 }

@@ -30,23 +30,14 @@ struct GemvArgs {
 // The activation rows into LDS: from x, or (fused add + norm) computed by this workgroup from the partial sums and the
 // residual - every workgroup makes all M rows for itself (M H values: a few KB from L2), workgroup 0 also writes the new
 // residual and the normed rows to memory for the kernels that follow.
-// (add_norm_row is 256 threads' work: a workgroup of another size, NORM false, has no code for it.)
+// (add_norm_rows is 256 threads' work: a workgroup of another size, NORM false, has no code for it.)
 template <int KL, int M, bool NORM>
 __device__ __forceinline__ void stage_rows(uint4* xs, const GemvArgs& a, float* red) {
   if (!NORM || !a.norm.part) {
     stage_x<KL>(xs, a.x, a.ldx, M, a.K, a.nq * 8);
     return;
   }
-  const bool writer = blockIdx.x == 0;
-  const int H = a.K;
-#pragma unroll 1
-  for (int m = 0; m < M; ++m)
-    add_norm_row(a.norm, m, H, red, true,
-                 [&](int q, u32x4_t v) { if (writer && a.norm.res_out) *reinterpret_cast<u32x4_t*>(a.norm.res_out + (size_t)m * H + 8 * q) = v; },
-                 [&](int q, u32x4_t v) {
-                   xs[(size_t)m * a.nq + xchunk_index<KL>(q)] = make_uint4(v.x, v.y, v.z, v.w);
-                   if (writer && a.norm.xn) *reinterpret_cast<u32x4_t*>(a.norm.xn + (size_t)m * H + 8 * q) = v;
-                 });
+  add_norm_rows<M>(a.norm, 0, a.K, xs, red, true, blockIdx.x == 0, [&](int m, int q) { return (size_t)m * a.nq + xchunk_index<KL>(q); });
 }
 
 // NW: wavefronts a workgroup, in groups of four: the first batches of the walk go to every workgroup's first group, so that
@@ -60,7 +51,7 @@ __device__ __forceinline__ void stage_rows(uint4* xs, const GemvArgs& a, float* 
 template <int FMT, int M, int RB, int D, int NW, bool SPLIT>
 __global__ void __launch_bounds__(NW * 64) k_gemv(GemvArgs a) {
   extern __shared__ uint4 xs[];
-  __shared__ float red[4];
+  __shared__ float red[4 * M];
   const int lane = threadIdx.x & 63;
   // (the wave's number is the same in every lane: said so, which keeps the row cursors and the segment's descriptor on the
   // scalar unit - read from a vector register they came through vector loads of the kernel's arguments, which a wave's
@@ -181,7 +172,7 @@ template <int FMT, int M, int RB, int SK>
 __global__ void __launch_bounds__(256) k_gemv_sk(GemvArgs a) {
   extern __shared__ uint4 xs[];
   __shared__ float part[4][RB * M];
-  __shared__ float red[4];
+  __shared__ float red[4 * M];
   const int lane = threadIdx.x & 63, wave = uni(threadIdx.x >> 6);  // (uniform: the segment's descriptor stays on the scalar unit)
   constexpr int GPW = 4 / SK;  // batches a workgroup
   const int grp = wave / SK, slice = wave % SK;
