@@ -54,9 +54,10 @@ struct Shape {
   static constexpr int kStages = WP == 1 ? 3 : 2;
   static constexpr int kStageW = kWgRows * 128;    // sixteen 16-row tiles of 2 KiB
   static constexpr int kStageX = kPos * 128;
-  static constexpr int kStageBytes = kStageW + kStageX + kPos * 4;  // + the positions' scales of the block
-  static constexpr int kLoads = 5 + 2 * WP;        // a wave's loads a turn: 4 weight, 2 WP activation, 1 scale
-  static constexpr int kLds = kStages * kStageBytes;  // (the epilogues reuse it: UP kPos x 256 B, DOWN 8 x 2 WP KiB)
+  static constexpr int kStageBytes = kStageW + kStageX;
+  static constexpr int kGroup = kPos * 16;         // the positions' scales of four blocks; two such buffers behind the stages
+  static constexpr int kLoads = 4 + 2 * WP;        // a wave's loads a turn: 4 weight, 2 WP activation (and, every fourth turn, one of scales)
+  static constexpr int kLds = kStages * kStageBytes + 2 * kGroup;  // (the epilogues reuse it: UP kPos x 256 B, DOWN 8 x 2 WP KiB)
 };
 
 // The shared expert's side of a launch that holds both its tiles and the routed experts' (k_gemm_mixed): the first `grid`
@@ -203,8 +204,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
   // the 16-position tiles this wave brings that hold rows: a ragged tile's other slots are neither fetched nor read (a
   // remainder of a few rows otherwise spends a third of its loads on them; gate/up 1.6% and down 0.8% faster at the
-  // benchmark's chunk; the same change in the INT4 and MXFP4 kernels, whose loads sit between their MFMAs, gained nothing
-  // and is not in them). A wave's loads a turn are then 4, or 4 + 2 nx + 1, which its waits count.
+  // benchmark's chunk). A wave's loads a turn are then 4 + 2 nx, which its waits count.
   const int nx = uni(min(WP, max(0, nmt - WP * wave)));
   auto issue = [&](int kb) {  // block kb (clamped: past the end the last block again, into a stage nobody reads) -> its stage
     const int kc = kb < KB ? kb : KB - 1;
@@ -220,8 +220,22 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh) dma16(px[t][hh] + (size_t)kc * 128, uni(xbase + t * 2048 + hh * 1024));
     }
-    if (nx > 0 && lane < 16 * WP) dma4(pxs + kc, uni(st + S::kStageW + S::kStageX + (uint32_t)wave * (64 * WP)));
   };
+  // The positions' scales come for four blocks at a time, 16 bytes a position, into two buffers (blocks 4 q ... 4 q + 3, the last
+  // ones of a row from its end): a scale of 4 bytes a position and block named as many cache lines an instruction as all of the
+  // block's activations do (pf_gemm_mx.cuh): gate/up of 128 / 256 rows an expert 1021 / 1425 us before, 964 / 1366 like this. Rows of fewer than four blocks have no 16 bytes: put in place by hand.
+  constexpr int kGroups0 = S::kStages * S::kStageBytes;
+  auto first_block = [&](int q) { return min(4 * q, KB - 4); };
+  auto issue_scales = [&](int q) {
+    if (nx > 0 && lane < 16 * WP)
+      dma16(reinterpret_cast<const uint8_t*>(pxs + first_block(q)), uni(lds0 + kGroups0 + (uint32_t)(q & 1) * S::kGroup + (uint32_t)wave * (256 * WP)));
+  };
+  if (KB >= 4) {
+    issue_scales(0);
+  } else if (lane < 16 * WP) {
+    for (int kb = 0; kb < KB; ++kb)
+      *reinterpret_cast<float*>(smem + kGroups0 + (16 * WP * wave + lane) * 16 + 4 * kb) = *(const DSGX_GLOBAL float*)(uintptr_t)(pxs + kb);
+  }
   // The wave's weight scales: lane l holds those of block l; one value
   // a 16-row tile pair (UP: gate and up; DOWN: all of a wave's rows lie in one 128-row block). They are loaded with
   // ordinary loads and WAITED FOR before any of the loads above is issued (the compiler's own wait for them would
@@ -262,10 +276,10 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
       // everyone is done reading the stage of block kb - 1, which the loads of block kb + kStages - 1 now overwrite
       if (S::kStages == 2) wait_loads<0>();
       else if (nx == WP) wait_loads<(S::kStages - 2) * S::kLoads>();
-      else if (nx == 0) wait_loads<(S::kStages - 2) * 4>();
-      else wait_loads<(S::kStages - 2) * (5 + 2 * (WP - 1))>();  // (WP 2 with one live tile; two stages wait for all anyway)
+      else wait_loads<(S::kStages - 2) * 4>();  // (no live tile; WP 2 with one: two stages wait for all anyway)
       __syncthreads();
       if (kb == 0) PF_STAMP(g, 4);
+      if ((kb + S::kStages - 1) % 4 == 0 && kb + S::kStages - 1 < KB) issue_scales((kb + S::kStages - 1) / 4);
       issue(kb + S::kStages - 1);
       if (NJ == 0) continue;
       const float wsa = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wsa_l), kb & 63));
@@ -273,14 +287,14 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
       const uint8_t* st = smem + (size_t)(kb % S::kStages) * S::kStageBytes;
       const uint8_t* W = st + S::RA * rg * 2048;
       const uint8_t* X = st + S::kStageW + pg * 2048;
-      const float* XS = reinterpret_cast<const float*>(st + S::kStageW + S::kStageX) + 16 * pg;
+      const uint8_t* XS = smem + kGroups0 + (size_t)((kb >> 2) & 1) * S::kGroup + (16 * pg + r16) * 16 + 4 * (kb - (KB >= 4 ? first_block(kb >> 2) : 0));
       v8i_t fa[S::RA];
 #pragma unroll
       for (int t = 0; t < S::RA; ++t) fa[t] = frag(W + t * 2048);
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
         const v8i_t fb = frag(X + j * (2048 * WP));
-        const float xv = XS[16 * WP * j + r16];
+        const float xv = *reinterpret_cast<const float*>(XS + j * (256 * WP));
         const float s0 = __fmul_rn(xv, wsa), s1 = __fmul_rn(xv, wsb);
 #pragma unroll
         for (int t = 0; t < S::RA; ++t) {

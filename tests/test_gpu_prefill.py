@@ -180,6 +180,13 @@ def test_prefill_fp8_against_oracle(H, I, E, topk, T, shared, unit_rule):
         assert helpers.rel_l2(ys[:24], seq_s[:24]) <= 6e-3
 
 
+@pytest.mark.parametrize("H,I,T", [(512, 640, 20), (1280, 1152, 300)])
+def test_prefill_fp8_scale_groups(H, I, T, unit_rule):
+    """the rows' scales come for four 128-k blocks at a time: last groups that are not whole (5, 9 and 10 blocks; 4 are one group,
+    1, 2 and 3 are among the shapes above), tiles of a few rows and of 256"""
+    test_prefill_fp8_against_oracle(H, I, 4, 2, T, "fp8", unit_rule)
+
+
 def test_prefill_rows_do_not_depend_on_the_chunk():
     """a row's result is the same bits whatever else is in the chunk (bucket positions differ)"""
     H, I, E, topk = 256, 256, 8, 2
