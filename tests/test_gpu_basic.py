@@ -198,3 +198,24 @@ def test_bf16_mfma_probe_is_the_f32_product_sum():
         assert np.all(np.abs(got - want) <= 1e-6 * mag), float((np.abs(got - want) / mag).max())
         mine = gpu.host(out, np.float32, (16, 16))
         assert np.array_equal(mine.view(np.uint32), orc.mfma_bf16_k32(a, b, c).view(np.uint32))
+
+
+def test_calls_go_to_the_current_stream():
+    """the handle that a call without a stream hands over: the default stream's, a side stream's, a capture's"""
+    import torch
+    same = lambda: lib._stream() == torch.cuda.current_stream().cuda_stream
+    assert same()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert same() and lib._stream() == side.cuda_stream
+    assert same() and lib._stream() != side.cuda_stream and lib._stream(side) == side.cuda_stream
+    a, out = torch.ones(256, device="cuda"), torch.zeros(256, dtype=torch.bfloat16, device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        assert same()
+        lib.finalize(a, a, 256, out)
+    for v in (1.0, 3.0, 5.0):
+        a.fill_(v)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert bool((out.float() == 2 * v).all())
