@@ -40,6 +40,10 @@ __device__ __forceinline__ void stage_rows(uint4* xs, const GemvArgs& a, float* 
   add_norm_rows<M>(a.norm, 0, a.K, xs, red, true, blockIdx.x == 0, [&](int m, int q) { return (size_t)m * a.nq + xchunk_index<KL>(q); });
 }
 
+// the lanes of a row's last segment that lie inside K
+template <int FMT>
+__device__ __forceinline__ int last_seg_lanes(int K, int nsegk) { return (K - (nsegk - 1) * FmtT<FMT>::SEGK + FmtT<FMT>::KL - 1) / FmtT<FMT>::KL; }
+
 // NW: wavefronts a workgroup, in groups of four: the first batches of the walk go to every workgroup's first group, so that
 // fewer batches than wavefronts still spread over all CUs. SPLIT: the split-K order of adds (k_gemv_sk's slices, in their
 // order, the same bits) by one wavefront that walks the slices one after the other.
@@ -75,39 +79,46 @@ __global__ void __launch_bounds__(NW * 64) k_gemv(GemvArgs a) {
   for (int r = 0; r < RB; ++r)
 #pragma unroll
     for (int m = 0; m < M; ++m) acc[r][m] = 0.f;
-  // where the loads past the last step go: the first 16 bytes of this wave's first row (cached; a line of its own, not one
-  // that every wave of the launch reads)
-  const uint8_t* dummy;
-  {
-    const int row = min(gw * RB, a.total_rows - 1);
-    int si = 0;
-    if (a.nsegs > 1) locate(row, si);
-    dummy = a.sg[si].m.w + (size_t)(row - a.sg[si].row0) * FmtT<FMT>::row_bytes(a.K);
-  }
   int lt = 0, lj = 0, lsl = 0, lseg = 0;  // the load cursor: step, batch number of this wave, slice, segment
-  // the matrix of the batch under the load cursor and the batch's first row in it: fetched from the kernel's arguments when
-  // the cursor enters a batch, not at every step (scalar loads, but each is a wait in front of the step's weight loads)
-  // (a call with one segment, the common one, fetches once: every later fetch would be two dependent scalar round trips)
+  // the rows of the batch under the load cursor: their addresses are set up on the scalar unit when the cursor enters a batch, and a
+  // step's loads are a scalar base and a lane offset each. (With 64-bit addresses made on the lanes for every load there were 85
+  // instructions between one load and the next, which is what the waves' first loads waited for: INT4 6144 x 16384 at one / four rows
+  // 20.4 / 27.6 us a call -> 19.4 / 26.2, 1536 x 6144 at one row 6.8 -> 6.4, FP8 16384 x 1536 8.7 -> 8.45, 1000 x 1152 4.25 -> 4.03.)
+  // (a call with one segment, the common one, fetches its descriptor once: every later fetch would be two dependent scalar round trips)
   MatDev lm = a.sg[0].m;
-  int lrow = 0;
+  RowSrc src[RB];
   auto enter = [&]() {
-    const int row = lt < nsteps ? (gw + lj * GW) * RB : 0;
+    const int row = uni(min((gw + lj * GW) * RB, a.total_rows - RB));  // (a wave without a batch: rows of its own as far as there are)
     int row0 = 0;
     if (a.nsegs > 1) {
       int si;
       locate(row, si);
       lm = a.sg[si].m, row0 = a.sg[si].row0;
     }
-    lrow = row - row0;
+#pragma unroll
+    for (int i = 0; i < RB; ++i) src[i] = row_src<FMT>(lm, row - row0 + i, a.K);
   };
   enter();
+  // past the last step the ring's loads go, scales and zero points too, to the first bytes of the wave's last rows: one cached line of
+  // the wave's own (with a line for each kind of load, 2048 x 4096 over 2 took 5.9 us, 5.5 like this)
+  auto park = [&]() {
+#pragma unroll
+    for (int i = 0; i < RB; ++i) src[i].w = src[i].a = src[i].z = src[0].w;
+  };
+  if (nsteps == 0) park();
+  const int last_lanes = last_seg_lanes<FMT>(a.K, a.nsegk);
   auto load = [&](Raw (&r)[RB]) {
     const bool ok = lt < nsteps;
     ++lt;
+    const uint32_t le = lane < uni(ok ? (lseg == a.nsegk - 1 ? last_lanes : kWave) : 0) ? lane : 0;
 #pragma unroll
-    for (int i = 0; i < RB; ++i) load_raw<FMT, true>(r[i], lm, lrow + i, lseg, lane, a.K, acc[i][0], ok ? nullptr : dummy);
+    for (int i = 0; i < RB; ++i) load_row<FMT>(r[i], src[i], uni(ok ? lseg : 0), le, lm.lks, acc[i][0]);
     if (ok && (lseg += sk) >= a.nsegk) {
-      if (++lsl == slices) lsl = 0, ++lj, enter();
+      if (++lsl == slices) {
+        lsl = 0, ++lj;
+        if (lt < nsteps) enter();
+        else park();
+      }
       lseg = lsl;
     }
   };
@@ -179,7 +190,7 @@ __global__ void __launch_bounds__(256) k_gemv_sk(GemvArgs a) {
   const int nbatch = a.total_rows / RB;
   const int batch = blockIdx.x * GPW + grp;
   const bool live = batch < nbatch;
-  const int row = live ? batch * RB : 0;
+  const int row = uni(live ? batch * RB : 0);
   int si = 0;
 #pragma unroll
   for (int i = 1; i < kMaxSegs; ++i)
@@ -193,15 +204,21 @@ __global__ void __launch_bounds__(256) k_gemv_sk(GemvArgs a) {
   for (int r = 0; r < RB; ++r)
 #pragma unroll
     for (int m = 0; m < M; ++m) acc[r][m] = 0.f;
-  // (loads past the last step: the first 16 bytes of this wave's row)
-  const uint8_t* dummy = reinterpret_cast<const uint8_t*>(sg.m.w) + (size_t)(row - sg.row0) * FmtT<FMT>::row_bytes(a.K);
+  RowSrc src[RB];
+#pragma unroll
+  for (int i = 0; i < RB; ++i) src[i] = row_src<FMT>(sg.m, row - sg.row0 + i, a.K);
+  const int last_lanes = last_seg_lanes<FMT>(a.K, a.nsegk);
   int lt = 0;
   auto load = [&](Raw (&r)[RB]) {
     const bool ok = lt < nmine;
-    const int seg = slice + (ok ? lt : 0) * SK;
-    ++lt;
+    if (lt == nmine)  // past the last step: the first bytes of this wave's rows (k_gemv's park)
 #pragma unroll
-    for (int i = 0; i < RB; ++i) load_raw<FMT, true>(r[i], sg.m, row - sg.row0 + i, seg, lane, a.K, acc[i][0], ok ? nullptr : dummy);
+      for (int i = 0; i < RB; ++i) src[i].w = src[i].a = src[i].z = src[0].w;
+    const int seg = uni(ok ? slice + lt * SK : 0);
+    ++lt;
+    const uint32_t le = lane < uni(ok ? (seg == a.nsegk - 1 ? last_lanes : kWave) : 0) ? lane : 0;
+#pragma unroll
+    for (int i = 0; i < RB; ++i) load_row<FMT>(r[i], src[i], seg, le, sg.m.lks, acc[i][0]);
   };
 #pragma unroll
   for (int d = 0; d < D; ++d) load(w[d]);

@@ -40,34 +40,7 @@ template <> struct FmtT<DSGX_FMT_BF16> {
   __device__ static __forceinline__ size_t row_bytes(int K) { return (size_t)K * 2; }
 };
 
-// The lane's 16 bytes of (row n, segment seg) and what it needs to decode them. The loads are unconditional: a lane
-// past the end of K (TAIL: the dense GEMV's partial last segment) reads the row's first bytes instead and step_dot
-// drops them; with `dummy` set (the pipeline's loads past the wave's last step) every lane reads there instead.
-// `pin`: a value of the preceding compute, see pin_after().
-template <int FMT, bool TAIL>
-__device__ __forceinline__ void load_raw(Raw& r, const MatDev& m, int n, int seg, int lane, int K, float pin, const uint8_t* dummy) {
-  using F = FmtT<FMT>;
-  int k0 = seg * F::SEGK + lane * F::KL;
-  if (TAIL && k0 >= K) k0 = 0;
-  const uint8_t* wp = m.w + (size_t)n * F::row_bytes(K) + F::row_bytes(k0);
-  const uint8_t* ap = nullptr;
-  if constexpr (FMT == DSGX_FMT_FP8_B128) ap = m.s + ((size_t)(n >> m.lrs) * m.srow + (k0 >> m.lks)) * 4;
-  if (dummy) wp = ap = dummy;  // (every lane the same 16 bytes: one cache line a load)
-  r.v = ldg_stream(pin_after(wp, pin));
-  if constexpr (FMT == DSGX_FMT_FP8_B128) {
-    r.aux = ldg_u32(ap);
-  } else if constexpr (FMT == DSGX_FMT_INT4_G32) {
-    const int g = k0 >> 5, G = K >> 5;
-    const uint8_t* sp = m.s + ((size_t)n * G + g) * 2;
-    const uint8_t* zp = m.zp + ((size_t)(n >> 3) * G + g) * 4;
-    if (dummy) sp = zp = dummy;
-    r.aux = ldg_u16(sp) | (((ldg_u32(zp) >> (4 * (n & 7))) & 15u) << 16);
-  } else {
-    r.aux = 0;
-  }
-}
-
-// The same loads with the wave-uniform part of the addresses kept apart: a RowSrc is one weight row's bases, set up
+// Where one weight row's loads go, with the wave-uniform part of the addresses kept apart: a RowSrc is the row's bases, set up
 // once a row on the scalar unit; load_row() then issues the step's loads as scalar base + lane offset.
 struct RowSrc {
   const uint8_t* w;  // the row's first byte
@@ -92,7 +65,9 @@ __device__ __forceinline__ RowSrc row_src(const MatDev& m, int n, int K) {
   }
   return r;
 }
-// seg wave-uniform; lks: log2 of the FP8 scale block along k (wave-uniform). No tail handling: K is whole segments.
+// The lane's 16 bytes of segment seg of the row and what it needs to decode them. seg wave-uniform; lks: log2 of the FP8 scale
+// block along k (wave-uniform). The loads are unconditional: a lane past the end of K (the dense GEMV's partial last segment) hands
+// in lane 0's place, and step_dot drops what it gets; `pin`: a value of the preceding compute, see pin_after().
 template <int FMT>
 __device__ __forceinline__ void load_row(Raw& r, const RowSrc& s, int seg, uint32_t lane, int lks, float pin) {
   r.v = ldg_stream(s.w + seg * 1024, pin_after(lane * 16u, pin));
