@@ -494,11 +494,9 @@ __device__ __forceinline__ void route_row(const float (&logit)[kRouteRJ], const 
 
 __device__ __forceinline__ float bf16_lo(uint32_t p) { return __uint_as_float(p << 16); }  // the values of a packed pair
 __device__ __forceinline__ float bf16_hi(uint32_t p) { return __uint_as_float(p & 0xFFFF0000u); }
-// silu(g) = g / (1 + e^-g) of four bf16 values, the division IEEE's: by the divisor's reciprocal and one correction step where |g| < 60
-// (the divisor is then in [1, 2^87]: no scaling; equal to the division for every bf16 g, all compared, but the sign of a zero, which
-// is g's), by the division itself if a value of the wave lies outside. The prefill GEMMs' epilogues are bound by the vector unit, and
-// beside them the tiles' loads wait: with the conversions above, ~20 instructions a value less, FP8 chunk of 256 rows an expert 2679
-// -> 2644 us, Zipf T = 8192 3063 -> 3000; INT4 T = 1111 1590 -> 1509.
+// silu(g) = g / (1 + e^-g) of four values in f32, the division IEEE's: by the divisor's reciprocal and one correction step where
+// |g| < 60 (the divisor is then in [1, 2^87]: no scaling; equal to the division for every bf16 g, all compared, but the sign of a
+// zero, which is g's), by the division itself if a value of the wave lies outside.
 __device__ __forceinline__ void silu4(const float (&g)[4], float (&s)[4]) {
   float d[4];
   bool far = false;
@@ -514,16 +512,27 @@ __device__ __forceinline__ void silu4(const float (&g)[4], float (&s)[4]) {
     for (int i = 0; i < 4; ++i) s[i] = __fdiv_rn(g[i], d[i]);
   }
 }
-// Four of swiglu_bits' values, packed. fast: with the hardware's exponential and reciprocal (each within 1 ulp) in place of expf() and
-// the IEEE division: silu before its rounding to bf16 is within a few f32 ulp of the exact value (the reference's own expf() is
-// specified to 2 ulp), so the bf16 it rounds to differs from swiglu_bits' once in ~10^4 values, by one bf16 step.
+// bf16(g / (1 + e^-g)) of a bf16 value g: where only the rounded value is used, the hardware's exponential and reciprocal do, without
+// expf()'s range reduction, the correction step and the cases apart (9 vector instructions less a value). Both sides of the quotient
+// are a quarter of theirs, which keeps the reciprocal normal up to the largest finite divisor, and the quarter of the divisor's 1 is one
+// step above 1/4: of the 65536 bf16 values, NaN, infinities and zeros included, every one rounds to the bits that the exact sequence
+// (expf, IEEE division) rounds to (all compared; with 1/4 itself 5.9375 alone does not). The prefill GEMMs' epilogues are bound by the
+// vector unit (the FP8 256-position gate/up tile spends an eighth of
+// its time there): FP8 gate/up at 256 rows an expert 1366 -> 1326 us, Zipf T = 8192 2919 -> 2876; INT4 at 64 rows an expert 1490 -> 1461.
+__device__ __forceinline__ float silu_for_bf16(float g) {
+  const float e = __builtin_amdgcn_exp2f(fmaf(g, -1.44269504088896341f, -2.f));
+  return __fmul_rn(__fmul_rn(g, 0.25f), __builtin_amdgcn_rcpf(__fadd_rn(0x1.000002p-2f, e)));
+}
+// Four of swiglu_bits' values, packed (g, u: bf16 values). fast: the same function by the plain formula, the caller's choice: one bf16
+// value of g rounds to the other side.
 __device__ __forceinline__ uint2 swiglu4(const float (&g)[4], const float (&u)[4], bool fast) {
   float s[4];
   if (fast) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) s[i] = __fmul_rn(g[i], __builtin_amdgcn_rcpf(__fadd_rn(1.f, __builtin_amdgcn_exp2f(__fmul_rn(g[i], -1.44269504088896341f)))));
   } else {
-    silu4(g, s);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[i] = silu_for_bf16(g[i]);
   }
   const uint32_t a = pack_bf16(s[0], s[1]), b = pack_bf16(s[2], s[3]);
   return make_uint2(pack_bf16(__fmul_rn(bf16_lo(a), u[0]), __fmul_rn(bf16_hi(a), u[1])), pack_bf16(__fmul_rn(bf16_lo(b), u[2]), __fmul_rn(bf16_hi(b), u[3])));

@@ -416,8 +416,7 @@ def test_prefill_int4_bf16_shared_expert_tiles(H, I, T):
 
 
 def test_prefill_silu_at_the_ends_of_its_fast_division():
-    """the prefill epilogues divide by the reciprocal where |gate| < 60 and by IEEE's division beyond (common.cuh: silu4); the decode
-    kernels by IEEE's everywhere: h of a BF16 shared expert whose gates are given values, on both sides of +-60, denormal results,
+    """silu of the prefill epilogues (common.cuh) against the decode kernels', which divide by IEEE's division everywhere: h of a BF16 shared expert whose gates are given values, on both sides of +-60, denormal results,
     zeros and infinities, from both"""
     H, I, E, topk = 256, 256, 8, 2
     hl = helpers.make_layer(abi.FMT_INT4, H, I, E, topk, 4, seed=27, shared="bf16")
@@ -442,3 +441,29 @@ def test_prefill_silu_at_the_ends_of_its_fast_division():
     with np.errstate(over="ignore"):
         ref = 3.0 * (g / (1.0 + np.exp(-g)))
     assert np.allclose(orc.bf16_to_f32(h), ref, rtol=2.0 ** -6, atol=1e-37)
+
+
+def test_prefill_silu_of_every_finite_bf16_gate():
+    """the prefill epilogues' silu (common.cuh: silu_for_bf16) rounds every bf16 gate to the bits of the decode kernels' (expf and IEEE's
+    division): row t of a one-hot x picks column t of a BF16 shared expert's gate matrix, 256 rows x 256 channels; the up values are 1"""
+    H, I, E, topk, T = 256, 256, 8, 2, 256
+    hl = helpers.make_layer(abi.FMT_INT4, H, I, E, topk, 4, seed=27, shared="bf16")
+    dl = hl.upload()
+    v = np.arange(65536, dtype=np.uint16)
+    v[(v & 0x7F80) == 0x7F80] = 0x3F80  # (one infinite or NaN weight would reach every row of its channel)
+    bgu = np.zeros((2 * I, H), np.uint16)
+    bgu[0::2] = v.reshape(I, H)
+    bgu[1::2] = 0x3F80
+    keep = gpu.dev(bgu)
+    dl.w.sh.bgu = keep.data_ptr()
+    _, _, idx, w = helpers.rows_and_routing(31, T, H, E, topk, 2.5)
+    x = np.zeros((T, H), np.uint16)
+    x[np.arange(T), np.arange(T)] = 0x3F80
+    ws, yr, ys = gpu.empty(lib.prefill_ws_bytes(dl.w, T), 0), gpu.empty(T * H * 4), gpu.empty(T * H * 4)
+    lib.moe_prefill(dl.w, gpu.dev(x), gpu.dev(idx), gpu.dev(w), T, ws, yr, ys, act_fp8=False)
+    h = gpu.host(gpu.view(ws, lib.prefill_view(dl.w, ws, T).hsh, T * I * 2), np.uint16, (T, I))
+    for t0 in range(0, T, 8):
+        _, _, wd = gpu.decode_layer(dl, x[t0:t0 + 8], idx[t0:t0 + 8], w[t0:t0 + 8], 8, up=1)
+        o = gpu.h_of(wd, dl, 8, topk)[-1]
+        for m in range(8):
+            assert np.array_equal(h[t0 + m], o[m]), t0 + m
