@@ -206,20 +206,26 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   // remainder of a few rows otherwise spends a third of its loads on them; gate/up 1.6% and down 0.8% faster at the
   // benchmark's chunk). A wave's loads a turn are then 4 + 2 nx, which its waits count.
   const int nx = uni(min(WP, max(0, nmt - WP * wave)));
-  auto issue = [&](int kb) {  // block kb (clamped: past the end the last block again, into a stage nobody reads) -> its stage
+  // block kb (clamped: past the end the last block again, into a stage nobody reads) -> its stage: the wave's four weight loads, and
+  // its activations
+  auto issue_w = [&](int kb, int i) {
     const int kc = kb < KB ? kb : KB - 1;
-    const uint32_t st = lds0 + (uint32_t)(kb % S::kStages) * S::kStageBytes;
-    const uint32_t wbase = st + (uint32_t)wave * 4096, xbase = st + S::kStageW + (uint32_t)wave * (2048 * WP);
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int hh = 0; hh < 2; ++hh) dma16(pw[t][hh] + (size_t)kc * 128, uni(wbase + t * 2048 + hh * 1024));
+    dma16(pw[i >> 1][i & 1] + (size_t)kc * 128, uni(lds0 + (uint32_t)(kb % S::kStages) * S::kStageBytes + (uint32_t)wave * 4096 + i * 1024));
+  };
+  auto issue_x = [&](int kb) {
+    const int kc = kb < KB ? kb : KB - 1;
+    const uint32_t xbase = lds0 + (uint32_t)(kb % S::kStages) * S::kStageBytes + S::kStageW + (uint32_t)wave * (2048 * WP);
 #pragma unroll
     for (int t = 0; t < WP; ++t) {
       if (t >= nx) break;  // (a ragged tile: nobody reads the 16-position tiles past its end)
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh) dma16(px[t][hh] + (size_t)kc * 128, uni(xbase + t * 2048 + hh * 1024));
     }
+  };
+  auto issue = [&](int kb) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) issue_w(kb, i);
+    issue_x(kb);
   };
   // The positions' scales come for four blocks at a time, 16 bytes a position, into two buffers (blocks 4 q ... 4 q + 3, the last
   // ones of a row from its end): a scale of 4 bytes a position and block named as many cache lines an instruction as all of the
@@ -280,7 +286,13 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
       __syncthreads();
       if (kb == 0) PF_STAMP(g, 4);
       if ((kb + S::kStages - 1) % 4 == 0 && kb + S::kStages - 1 < KB) issue_scales((kb + S::kStages - 1) / 4);
-      issue(kb + S::kStages - 1);
+      const int nb = kb + S::kStages - 1;
+      // WP 1: the weights' loads one by one between the MFMAs of the first 16-position tiles. All of a turn's loads in front of its
+      // MFMAs hold the waves up where the memory takes them slowly: whole call at 96 / 128 rows an expert 1572 / 1753 us -> 1556 / 1733.
+      // (WP 2's two stages leave a load one turn to land: there every load goes first; between the MFMAs gate/up and down lost 1%.)
+      constexpr bool kSpread = WP == 1 && NJ >= 4;
+      if (kSpread) issue_x(nb);
+      else issue(nb);
       if (NJ == 0) continue;
       const float wsa = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wsa_l), kb & 63));
       const float wsb = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wsb_l), kb & 63));
@@ -291,10 +303,14 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
       v8i_t fa[S::RA];
 #pragma unroll
       for (int t = 0; t < S::RA; ++t) fa[t] = frag(W + t * 2048);
+      v8i_t fn = frag(X);
+      float xn = *reinterpret_cast<const float*>(XS);
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
-        const v8i_t fb = frag(X + j * (2048 * WP));
-        const float xv = *reinterpret_cast<const float*>(XS + j * (256 * WP));
+        const v8i_t fb = fn;
+        const float xv = xn;
+        if (j + 1 < NJ) fn = frag(X + (j + 1) * (2048 * WP)), xn = *reinterpret_cast<const float*>(XS + (j + 1) * (256 * WP));
+        if (kSpread && j < 4) issue_w(nb, j);
         const float s0 = __fmul_rn(xv, wsa), s1 = __fmul_rn(xv, wsb);
 #pragma unroll
         for (int t = 0; t < S::RA; ++t) {
