@@ -236,12 +236,6 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
     if (nx > 0 && lane < 16 * WP)
       dma16(reinterpret_cast<const uint8_t*>(pxs + first_block(q)), uni(lds0 + kGroups0 + (uint32_t)(q & 1) * S::kGroup + (uint32_t)wave * (256 * WP)));
   };
-  if (KB >= 4) {
-    issue_scales(0);
-  } else if (lane < 16 * WP) {
-    for (int kb = 0; kb < KB; ++kb)
-      *reinterpret_cast<float*>(smem + kGroups0 + (16 * WP * wave + lane) * 16 + 4 * kb) = *(const DSGX_GLOBAL float*)(uintptr_t)(pxs + kb);
-  }
   // The wave's weight scales: lane l holds those of block l; one value
   // a 16-row tile pair (UP: gate and up; DOWN: all of a wave's rows lie in one 128-row block). They are loaded with
   // ordinary loads and WAITED FOR before any of the loads above is issued (the compiler's own wait for them would
@@ -258,8 +252,14 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   PF_STAMP(g, 2);
   load_ws(0);
   PF_STAMP(g, 3);
+  if (KB < 4 && lane < 16 * WP) {
+    for (int kb = 0; kb < KB; ++kb)
+      *reinterpret_cast<float*>(smem + kGroups0 + (16 * WP * wave + lane) * 16 + 4 * kb) = *(const DSGX_GLOBAL float*)(uintptr_t)(pxs + kb);
+  }
+  issue(0);
+  if (KB >= 4) issue_scales(0);  // (behind the first block's loads, which every turn's wait for that block covers)
 #pragma unroll
-  for (int s = 0; s + 1 < S::kStages; ++s) issue(s);
+  for (int s = 1; s + 1 < S::kStages; ++s) issue(s);
 
   // fragment reads: lane (row r16, part) takes pieces 2 part and 2 part + 1 of its row (32 consecutive k)
   const int rd0 = (r16 >> 3) * 1024 + (r16 & 7) * 128 + ((2 * part) ^ swz(r16)) * 16;
