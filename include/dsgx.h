@@ -177,7 +177,7 @@ DSGX_API int dsgx_finalize(const float* R, const float* S, int n, uint16_t* out,
    the block-scaled products), up clamped to +-limit and gate from above, h = bf16(w_row * (silu(gate) * up)) (no weight for
    the shared expert), h quantised like x, the expert's w2 output rounded to bf16; y = the f32 sum of the picked experts'
    outputs in expert-id order, then the shared expert's. y f32 [M][H] the sum, ys f32 [M][H] the shared expert's bf16
-   output alone. ws: dsgx_decode_ws_bytes(L), zeroed once. M <= 16 (9-16: two passes). */
+   output alone. ws: dsgx_decode_ws_bytes(L), zeroed once. M <= 16 (9-16 in one pass as far as the rows fit LDS, else in two). */
 typedef struct dsgx_dsk_cfg {
   float swiglu_limit;   /* 10 */
   const float* logits;  /* fused routing (moe_routed): f32 [M][E]; idx, w are then not read */
