@@ -209,7 +209,7 @@ static int moe_decode_at(const dsgx_layer_w* L, const uint16_t* x, const int* id
 
   // 9-16 rows (the reference's limit, experts.h:104): the MFMA kernels take as many in one pass as their LDS holds, the vector-unit
   // kernels eight
-  const int M1 = M <= 8 ? M : c.up != 1 ? 8 : L->fmt == DSGX_FMT_FP8_B128 ? max_rows_fp8_mfma(H, I, M) : L->fmt == DSGX_FMT_INT4_G32 ? max_rows_int4_mfma(H, I, M) : max_rows_mxfp4_mfma(H, I, M);
+  const int M1 = M <= 8 ? M : c.up != 1 ? 8 : L->fmt == DSGX_FMT_FP8_B128 ? max_rows_fp8_mfma(H, I, L->E, M) : L->fmt == DSGX_FMT_INT4_G32 ? max_rows_int4_mfma(H, I, L->E, M) : max_rows_mxfp4_mfma(H, I, L->E, M);
   if (M1 < M) {
     // two passes, the first as large as it can be; every row's result is what it is alone or in any batch, so the split is
     // invisible in the output. The second pass reads the weights of its experts again; the workspace is reused in stream order.

@@ -101,9 +101,9 @@ int launch_decode_int4(const DecodeArgs& a, int parts, bool shared_bf16, hipStre
 int launch_decode_int4_mfma(const DecodeArgs& a, int parts, int shared_fmt, hipStream_t st);  // variant 1 (shared: 0, BF16 or FP8_B128)
 int launch_decode_bf16(const DecodeArgs& a, int parts, hipStream_t st);
 // how many of M (9 .. 16) rows the MFMA kernels of a format take in one pass, 8 at least (moe_decode_mfma.cuh)
-int max_rows_fp8_mfma(int H, int I, int M);
-int max_rows_int4_mfma(int H, int I, int M);
-int max_rows_mxfp4_mfma(int H, int I, int M);
+int max_rows_fp8_mfma(int H, int I, int E, int M);
+int max_rows_int4_mfma(int H, int I, int E, int M);
+int max_rows_mxfp4_mfma(int H, int I, int E, int M);
 
 // ---- what a workgroup knows about the step -------------------------------------------------------------------------
 struct MatRef {
@@ -119,6 +119,13 @@ struct Slot {
 struct DescHead {  // a descriptor's off and s2
   uint32_t x, y, z;
 };
+// M > 8: the DescHeads lie in front of the kernel's dynamic LDS, as many as the layer has experts (the table for every layer, 18 KiB,
+// took the LDS of two rows)
+__host__ __device__ constexpr int dyn_dtab_bytes(int M, int E) { return M > 8 ? (E * 3 * (int)sizeof(DescHead) + 255) / 256 * 256 : 0; }
+__device__ __forceinline__ DescHead* dyn_dtab() {
+  extern __shared__ __attribute__((aligned(16))) uint8_t mf_lds[];
+  return reinterpret_cast<DescHead*>(mf_lds);
+}
 // M: the step's rows, or 16 for 9 to 16 of them (step_rows). PICKS: the MFMA kernels, which keep a row's weights by its picks
 template <int M, bool PICKS = false>
 struct Step {
@@ -131,7 +138,7 @@ struct Step {
   int gen;                             // the grid barrier's generation at kernel start
   int next_up;                         // the gate/up phase's batch counter (up_body)
   int rdone, ready;                    // rows routed so far; the slots are complete (resolve)
-  std::conditional_t<(M > 8), DescHead, uint4> dtab[DSGX_MAX_EXPERTS * 3];  // the descriptors' first 16 bytes (off, s2, fmt) or 12, fetched before the routing is known
+  uint4 dtab[M > 8 ? 1 : DSGX_MAX_EXPERTS * 3];  // the descriptors' first 16 bytes (off, s2, fmt), fetched before the routing is known (M > 8: dyn_dtab)
   // PICKS: per slot and row the number m topk + r of the row's pick, r picks of the row lying in lower slots (255: not picked),
   // and per pick the weight and s2 w
   uint8_t pick[PICKS ? M * DSGX_MAX_TOPK : 1][M <= 4 ? 4 : M <= 8 ? 8 : 16];
@@ -161,7 +168,7 @@ __device__ __forceinline__ void prep(Step<M, PICKS>& S, const DecodeArgs& a) {
   // (loads past the end re-read the last descriptor: unconditional loads into named registers stay in flight together)
   const DSGX_GLOBAL u32x4_t* d = (const DSGX_GLOBAL u32x4_t*)(uintptr_t)a.L.desc;
   auto put = [&](int i, u32x4_t v) {
-    if constexpr (M > 8) S.dtab[i] = DescHead{v.x, v.y, v.z};
+    if constexpr (M > 8) dyn_dtab()[i] = DescHead{v.x, v.y, v.z};
     else *reinterpret_cast<u32x4_t*>(&S.dtab[i]) = v;
   };
   const int nd = a.stk_w[0] ? 0 : a.L.E * 3, bd = blockDim.x;  // (stacked experts are addressed by their id alone)
@@ -240,7 +247,10 @@ __device__ __forceinline__ void resolve(Step<M, PICKS>& S, const DecodeArgs& a, 
     Slot t;
     auto ref = [&](int which, int N, int K) {
       if (a.stk_w[0]) return MatRef{a.stk_w[which] + (size_t)e * a.stk_wb[which], a.stk_s[which] + (size_t)e * a.stk_sb[which], 1.f, 0};
-      const auto d = S.dtab[e * 3 + which];
+      const auto d = [&] {
+        if constexpr (M > 8) return dyn_dtab()[e * 3 + which];
+        else return S.dtab[e * 3 + which];
+      }();
       return mat_ref<FMT>(a.L.pool + (((uint64_t)d.y << 32) | d.x), N, K, __uint_as_float(d.z));
     };
     t.g = ref(0, I, H), t.u = ref(1, I, H), t.d = ref(2, H, I);

@@ -8,5 +8,5 @@ int launch_decode_int4_mfma(const DecodeArgs& a, int parts, int shared, hipStrea
   if (shared == DSGX_FMT_FP8_B128) return launch_decode_mfma_m<DSGX_FMT_INT4_G32, DSGX_FMT_FP8_B128>(a, parts, st);
   return launch_decode_mfma_m<DSGX_FMT_INT4_G32, 0>(a, parts, st);
 }
-int max_rows_int4_mfma(int H, int I, int M) { return mf_max_rows<DSGX_FMT_INT4_G32>(H, I, M); }
+int max_rows_int4_mfma(int H, int I, int E, int M) { return mf_max_rows<DSGX_FMT_INT4_G32>(H, I, E, M); }
 }  // namespace dsgx

@@ -690,14 +690,16 @@ __device__ __forceinline__ void mf_down_phase(Step<M, true>& S, const DecodeArgs
 
 template <int FMT, int SHFMT, int M>
 __global__ void __launch_bounds__(kMfThreads) k_up_mfma(DecodeArgs a) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t mf_smem[];  // (read and written 16 bytes at a time)
+  extern __shared__ __attribute__((aligned(16))) uint8_t mf_lds[];  // (read and written 16 bytes at a time)
+  uint8_t* mf_smem = mf_lds + dyn_dtab_bytes(M, a.L.E);
   __shared__ Step<M, true> S;
   mf_setup<FMT, SHFMT, M, true>(S, a, mf_smem);
   mf_up_phase<FMT, SHFMT, M>(S, a, mf_smem);
 }
 template <int FMT, int SHFMT, int M>
 __global__ void __launch_bounds__(kMfThreads) k_down_mfma(DecodeArgs a) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t mf_smem[];  // (read and written 16 bytes at a time)
+  extern __shared__ __attribute__((aligned(16))) uint8_t mf_lds[];  // (read and written 16 bytes at a time)
+  uint8_t* mf_smem = mf_lds + dyn_dtab_bytes(M, a.L.E);
   __shared__ Step<M, true> S;
   mf_setup<FMT, SHFMT, M, false>(S, a, mf_smem);
   mf_down_phase<FMT, SHFMT, M, false>(S, a, mf_smem);
@@ -705,7 +707,8 @@ __global__ void __launch_bounds__(kMfThreads) k_down_mfma(DecodeArgs a) {
 // Both phases in one launch, a grid barrier between them (every workgroup resident: one a CU); the step's set-up runs once
 template <int FMT, int SHFMT, int M>
 __global__ void __launch_bounds__(kMfThreads) k_decode_mfma(DecodeArgs a) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t mf_smem[];  // (read and written 16 bytes at a time)
+  extern __shared__ __attribute__((aligned(16))) uint8_t mf_lds[];  // (read and written 16 bytes at a time)
+  uint8_t* mf_smem = mf_lds + dyn_dtab_bytes(M, a.L.E);
   __shared__ Step<M, true> S;
   if (threadIdx.x == 0) S.gen = grid_barrier_gen(a.bar);
   mf_setup<FMT, SHFMT, M, true>(S, a, mf_smem);
@@ -716,18 +719,21 @@ __global__ void __launch_bounds__(kMfThreads) k_decode_mfma(DecodeArgs a) {
 // The LDS of a step's phases (slots: the slots whose h the down phase stages together), and the rows that the kernels take at
 // once: a step of 9 to 16 rows is one pass where the staged rows and the tables beside them fit a CU's LDS, else as many rows as
 // do and the rest (moe_decode_at). One pass reads the weights of the experts that both would have read once: FP8, 13 rows of top-8
-// of 256, hidden 4096, intermediate 2048: 95 expert reads a layer in passes of 8 and 5, 87 in one, four layers 1697 -> 1600 us;
-// hidden 2048: 9 rows 730 -> 623, 12 rows 910 -> 768.
+// of 256, hidden 4096, intermediate 2048, four layers: in passes of 8 and 5 1690 us, of 12 and 1 (as far as rows fit beside a table of
+// DSGX_MAX_EXPERTS descriptors) 1592, in one 1498; INT4, hidden 6144, 168 experts, 9 rows: of 8 and 1 1324, in one 1193; FP8, hidden
+// 2048: 9 rows 730 -> 623, 12 rows 910 -> 768.
 template <int FMT>
 size_t mf_step_lds(int rows, int H, int I, int parts, int slots) {
   const size_t up = mf_lds_bytes(rows, rows, H, mf_pad(FMT)), down = mf_lds_bytes(slots * rows, rows, I, mf_pad(FMT));
   return parts == 1 ? up : parts == 2 ? down : std::max(up, down);
 }
 template <int FMT>
-bool mf_fits(int rows, int H, int I, int slots) { return mf_step_lds<FMT>(rows, H, I, 3, slots) + sizeof(Step<16, true>) + 64 <= 160 * 1024; }
+bool mf_fits(int rows, int H, int I, int E, int slots) {
+  return mf_step_lds<FMT>(rows, H, I, 3, slots) + dyn_dtab_bytes(16, E) + sizeof(Step<16, true>) + 64 <= 160 * 1024;
+}
 template <int FMT>
-int mf_max_rows(int H, int I, int M) {
-  while (M > 8 && !mf_fits<FMT>(M, H, I, 1)) --M;
+int mf_max_rows(int H, int I, int E, int M) {
+  while (M > 8 && !mf_fits<FMT>(M, H, I, E, 1)) --M;
   return M;
 }
 
@@ -735,13 +741,13 @@ template <int FMT, int SHFMT, int M>
 int launch_decode_mfma(const DecodeArgs& args, int parts, hipStream_t st) {
   const int H = args.L.H, I = args.L.I, cus = num_cus_cached();
   DecodeArgs a = args;
-  a.down_slots = M <= 8 || mf_fits<FMT>(a.M, H, I, 2) ? 2 : 1;
+  a.down_slots = M <= 8 || mf_fits<FMT>(a.M, H, I, a.L.E, 2) ? 2 : 1;
   if (H % 256 || I % 256)
     return fail(DSGX_EINVAL, "moe_decode (variant 1): hidden %d, intermediate %d (whole steps of 256 k)", H, I);
   auto combine = [&] { hipLaunchKernelGGL((k_pick_combine<SHFMT != 0>), dim3((a.M * H + 255) / 256), dim3(256), 0, st, a); };
   if (parts == 3) {
     auto kern = k_decode_mfma<FMT, SHFMT, M>;
-    const size_t lds = mf_step_lds<FMT>(a.M, H, I, 3, a.down_slots);
+    const size_t lds = dyn_dtab_bytes(M, a.L.E) + mf_step_lds<FMT>(a.M, H, I, 3, a.down_slots);
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
     int per_cu = 0;  // the grid barrier needs every workgroup resident
     DSGX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kMfThreads, lds));
@@ -754,14 +760,14 @@ int launch_decode_mfma(const DecodeArgs& args, int parts, hipStream_t st) {
   }
   if (parts & 1) {
     auto kern = k_up_mfma<FMT, SHFMT, M>;
-    const size_t lds = mf_step_lds<FMT>(a.M, H, I, 1, a.down_slots);
+    const size_t lds = dyn_dtab_bytes(M, a.L.E) + mf_step_lds<FMT>(a.M, H, I, 1, a.down_slots);
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
     hipLaunchKernelGGL(kern, dim3(cus), dim3(kMfThreads), lds, st, a);
     DSGX_HIP(hipGetLastError());
   }
   if (parts & 2) {
     auto kern = k_down_mfma<FMT, SHFMT, M>;
-    const size_t lds = mf_step_lds<FMT>(a.M, H, I, 2, a.down_slots);
+    const size_t lds = dyn_dtab_bytes(M, a.L.E) + mf_step_lds<FMT>(a.M, H, I, 2, a.down_slots);
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
     hipLaunchKernelGGL(kern, dim3(cus), dim3(kMfThreads), lds, st, a);
     combine();

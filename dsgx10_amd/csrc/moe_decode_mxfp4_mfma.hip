@@ -8,5 +8,5 @@ int launch_decode_mxfp4_mfma(const DecodeArgs& a, int parts, bool shared_fp8e, h
   if (shared_fp8e) return launch_decode_mfma_m<DSGX_FMT_MXFP4_G32, DSGX_FMT_FP8_B32E>(a, parts, st);
   return launch_decode_mfma_m<DSGX_FMT_MXFP4_G32, 0>(a, parts, st);
 }
-int max_rows_mxfp4_mfma(int H, int I, int M) { return mf_max_rows<DSGX_FMT_MXFP4_G32>(H, I, M); }
+int max_rows_mxfp4_mfma(int H, int I, int E, int M) { return mf_max_rows<DSGX_FMT_MXFP4_G32>(H, I, E, M); }
 }  // namespace dsgx
