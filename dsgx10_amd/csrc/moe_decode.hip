@@ -100,7 +100,7 @@ struct DskIn {
   float* wts_out = nullptr;
 };
 static int moe_decode_at(const dsgx_layer_w* L, const uint16_t* x, const int* idx, const float* w, int M, void* ws, const WsLayout& lay,
-                         float* yr, float* ys, void* stream, const dsgx_decode_cfg* cfg, DskIn dsk = DskIn{});
+                         float* yr, float* ys, void* stream, const dsgx_decode_cfg* cfg, DskIn dsk = DskIn{}, int rows_before = 0);
 
 extern "C" {
 size_t dsgx_decode_ws_bytes(const dsgx_layer_w* L) {
@@ -165,7 +165,7 @@ static int decode_by_prefill(const dsgx_layer_w* L, const uint16_t* x, const int
 }
 
 static int moe_decode_at(const dsgx_layer_w* L, const uint16_t* x, const int* idx, const float* w, int M, void* ws, const WsLayout& lay,
-                         float* yr, float* ys, void* stream, const dsgx_decode_cfg* cfg, DskIn dsk) {
+                         float* yr, float* ys, void* stream, const dsgx_decode_cfg* cfg, DskIn dsk, int rows_before) {
   dsgx_decode_cfg c;
   if (cfg) c = *cfg;
   else dsgx_decode_cfg_default(&c);
@@ -212,7 +212,8 @@ static int moe_decode_at(const dsgx_layer_w* L, const uint16_t* x, const int* id
   const int M1 = M <= 8 ? M : c.up != 1 ? 8 : L->fmt == DSGX_FMT_FP8_B128 ? max_rows_fp8_mfma(H, I, L->E, M) : L->fmt == DSGX_FMT_INT4_G32 ? max_rows_int4_mfma(H, I, L->E, M) : max_rows_mxfp4_mfma(H, I, L->E, M);
   if (M1 < M) {
     // two passes, the first as large as it can be; every row's result is what it is alone or in any batch, so the split is
-    // invisible in the output. The second pass reads the weights of its experts again; the workspace is reused in stream order.
+    // invisible in the output. The second pass reads the weights of its experts again. Its h lies behind the first one's (the
+    // workspace holds the slots of DSGX_MAX_ROWS rows): a call of the up phase leaves both passes' h for a call of the down phase.
     const int topk = L->topk, E = L->E;
     dsgx_decode_cfg c1 = c, c2 = c;
     c1.parts = c2.parts = c.parts & 3;
@@ -222,11 +223,11 @@ static int moe_decode_at(const dsgx_layer_w* L, const uint16_t* x, const int* id
     if (dsk.xq) dsk2.xq = dsk.xq + (size_t)M1 * H, dsk2.xs = dsk.xs + (size_t)M1 * (H / 32);
     if (dsk.idx_out) dsk2.idx_out = dsk.idx_out + (size_t)M1 * topk, dsk2.wts_out = dsk.wts_out + (size_t)M1 * topk;
     return moe_decode_at(L, x + (size_t)M1 * H, idx ? idx + (size_t)M1 * topk : nullptr, w ? w + (size_t)M1 * topk : nullptr, M - M1, ws, lay,
-                         yr ? yr + (size_t)M1 * H : nullptr, ys ? ys + (size_t)M1 * H : nullptr, stream, &c2, dsk2);
+                         yr ? yr + (size_t)M1 * H : nullptr, ys ? ys + (size_t)M1 * H : nullptr, stream, &c2, dsk2, M1);
   }
   DecodeArgs a{};
   a.x = x, a.M = M, a.idx = idx, a.w = w, a.logits = c.logits, a.bias = c.bias, a.route_scale = c.route_scale, a.score_fn = c.score_fn;
-  a.L = *L, a.h = static_cast<uint16_t*>(ws), a.yr = yr, a.ys = ys, a.ysum = c.ysum;
+  a.L = *L, a.h = static_cast<uint16_t*>(ws) + (size_t)(DSGX_MAX_UNION + 1) * rows_before * I, a.yr = yr, a.ys = ys, a.ysum = c.ysum;
   uint8_t* wsb = static_cast<uint8_t*>(ws);
   a.bar = reinterpret_cast<int*>(wsb + lay.bar_off());
   a.fac = reinterpret_cast<float*>(wsb + lay.fac_off());

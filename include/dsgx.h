@@ -151,7 +151,9 @@ DSGX_API size_t dsgx_decode_ws_flag_offset(const dsgx_layer_w* L);
 DSGX_API int dsgx_decode_status(const dsgx_layer_w* L, void* ws, void* stream);
 /* x bf16 [M][H]; idx, w from dsgx_route; yr, ys f32 [M][H]. ys is written when the layer has a fused shared expert,
    otherwise it is an input (only read with ysum). h of the step stays in ws: slot s (the s-th picked expert in
-   expert-id order) at ((s * M + m) * I + c), the shared expert's at slot DSGX_SH_SLOT. */
+   expert-id order) at ((s * M + m) * I + c), the shared expert's at slot DSGX_SH_SLOT. A step of more rows than one pass of
+   the kernels takes (up 0: 8; up 1: what LDS holds, 8 at least) runs as two, of M1 rows and the rest, each with slots of its own: the
+   second one's begin at (DSGX_MAX_UNION + 1) * M1 * I. */
 DSGX_API int dsgx_moe_decode(const dsgx_layer_w* L, const uint16_t* x, const int* idx, const float* w, int M, void* ws,
                              float* yr, float* ys, void* stream, const dsgx_decode_cfg* cfg);
 /* dsgx_moe_decode on a workspace inside the library, for callers that cannot allocate device memory (code under HIP graph

@@ -421,3 +421,21 @@ def test_decode_nine_to_sixteen_rows_in_one_pass(fmt, H, I, E, topk, shared, row
                 assert np.array_equal(yr[m].view(np.uint32), alone[m][0][0].view(np.uint32)), (M, m)
                 if hl.has_shared:
                     assert np.array_equal(ys[m].view(np.uint32), alone[m][1][0].view(np.uint32)), (M, m)
+
+
+@pytest.mark.parametrize("fmt,H,I,E,topk,shared,up,rows", [(abi.FMT_FP8, 2048, 1024, 32, 8, "fp8", 0, (12,)), (abi.FMT_BF16, 1024, 512, 16, 4, None, 0, (13,)),
+                                                          (abi.FMT_FP8, 4096, 512, 32, 8, None, 1, (13, 16)), (abi.FMT_INT4, 6144, 512, 16, 4, "bf16", 1, (9, 16))],
+                         ids=["fp8-vector", "bf16-vector", "fp8", "int4"])
+def test_decode_phases_apart_over_eight_rows(fmt, H, I, E, topk, shared, up, rows):
+    """the up phase in one call and the down phase in the next give the whole step's bits, whether the rows are one pass of the
+    kernels (13 of the FP8 layer, 9 of the INT4 layer) or two, whose h then lie one behind the other"""
+    hl, dl = _layer(fmt, H, I, E, topk, 3, shared, seed=11)
+    x, _, idx, w = rows_and_routing(43, max(rows), H, E, topk, 2.5)
+    for M in rows:
+        yr, ys, ws = gpu.decode_layer(dl, x[:M], idx[:M], w[:M], M, up=up)
+        r2, s2 = gpu.empty(M * H * 4, 0xFF), gpu.empty(M * H * 4, 0xFF)
+        ws.fill_(0)
+        for parts in (1, 2):
+            lib.moe_decode(dl.w, gpu.dev(x[:M]), gpu.dev(idx[:M]), gpu.dev(w[:M]), M, ws, r2, s2, parts=parts, up=up)
+        assert np.array_equal(gpu.host(r2, np.uint32, (M, H)), yr.view(np.uint32)), M
+        assert np.array_equal(gpu.host(s2, np.uint32, (M, H)), ys.view(np.uint32)), M
