@@ -14,8 +14,8 @@ extern "C" unsigned long long* dsgx_trace_buf() { return g_trace_buf; }
 #endif
 
 // The workspace of dsgx_moe_decode_noalloc: a device array of the library itself, sized for the largest layer that entry
-// point takes (h of 129 slots x 16 rows x DSGX_NOALLOC_MAX_I, the barrier's words, the slot-partitioned down phase's
-// table and its f32 [129][8][DSGX_NOALLOC_MAX_H] results: 34.0 MB on every GPU the library runs on, zero when the
+// point takes (h of 129 slots x 16 rows x DSGX_NOALLOC_MAX_I, the barrier's words, the down phase's factors and its
+// [129 x 8][DSGX_NOALLOC_MAX_H] f32 dots (DecodeArgs): 34.0 MB on every GPU the library runs on, zero when the
 // module loads, which is the barrier's initial state). In host code the array's name is not a device address: the
 // address is asked for once a device (static_ws) and only that pointer is used.
 static constexpr size_t kStaticWsBytes = (size_t)(DSGX_MAX_UNION + 1) * DSGX_MAX_ROWS * DSGX_NOALLOC_MAX_I * 2 + dsgx::kBarBytes +
@@ -69,19 +69,22 @@ static int decode_variant(uint32_t fmt, int M, int H, int I) {
 
 }  // extern "C"
 
-// The workspace: h [DSGX_MAX_UNION + 1 slots][DSGX_MAX_ROWS][I] | the barrier's words (kBarBytes) | the slot-partitioned down
-// phase's slot table (kFacBytes) and its f32 results [slot][8 rows][H] | a reserved row buffer [16][H] bf16. I and H here are the LAYOUT's: the layer's own for a
-// caller's workspace; the built-in workspace is laid out for its largest shapes whatever the layer, so that every layer run
+// The workspace: h [DSGX_MAX_UNION + 1 slots][DSGX_MAX_ROWS][I] | the barrier's words (kBarBytes) | the down phase's factors
+// (kFacBytes) and kDots rows of f32 [H] dots (DecodeArgs: by slot, 129 of eight rows, or by pick, sixteen rows' top-k and shared
+// expert) | a reserved row buffer [16][H] bf16. I and H here are the LAYOUT's: the layer's own for a caller's workspace; the built-in workspace is laid out for its largest shapes whatever the layer, so that every layer run
 // on it finds the barrier's words in one place (at an offset that moved with the layer, one layer's h or partial sums would
 // lie where another's counters are expected to be zero).
 struct WsLayout {
   int I, H;
   static constexpr size_t kFacBytes = (size_t)(8 + (DSGX_MAX_UNION + 1) * 8) * 4 + 192;  // (a multiple of 256)
+  static constexpr size_t kDots = (size_t)(DSGX_MAX_UNION + 1) * 8;
+  static_assert((8 + DSGX_MAX_ROWS * DSGX_MAX_TOPK) * 4 <= kFacBytes && (DSGX_MAX_TOPK + 1) * DSGX_MAX_ROWS <= kDots, "the factors and dots by pick");
+  static_assert(DSGX_MAX_ROWS * DSGX_MAX_TOPK < 255, "a pick's number is a byte, 255 no pick");
   constexpr size_t h_bytes() const { return (size_t)(DSGX_MAX_UNION + 1) * DSGX_MAX_ROWS * I * 2; }
   constexpr size_t bar_off() const { return h_bytes(); }
   constexpr size_t fac_off() const { return bar_off() + kBarBytes; }
   constexpr size_t dpart_off() const { return fac_off() + kFacBytes; }
-  constexpr size_t xdeq_off() const { return dpart_off() + (size_t)(DSGX_MAX_UNION + 1) * 8 * H * 4; }  // (reserved)
+  constexpr size_t xdeq_off() const { return dpart_off() + kDots * H * 4; }  // (reserved)
   constexpr size_t bytes() const { return xdeq_off() + (size_t)DSGX_MAX_ROWS * H * 2; }
   // dsgx_dsk_moe_stacked's workspace: the same, then the shared expert's output rows f32 [DSGX_MAX_ROWS][H]
   constexpr size_t dsk_ys_off() const { return (bytes() + 255) / 256 * 256; }

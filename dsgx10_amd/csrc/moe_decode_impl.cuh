@@ -71,8 +71,12 @@ struct DecodeArgs {
   float* ys;
   int ysum;
   int* bar;     // the grid barrier's words in the workspace (grid_barrier)
-  float* dpart; // the slot-partitioned down phase's results, f32 [slot][M][H] (k_down_part -> k_down_combine)
-  float* fac;   // its slot table: fac[0] = slots (as int bits), fac[8 + slot * 8 + m] = s2_down * w of row m
+  // The down phase's dots and their factors, between its kernel and the one that chains them. The vector-unit kernels (k_down_part ->
+  // k_down_combine, up to eight rows a pass) keep them by slot: dpart f32 [slot][M][H], fac[0] = slots (as int bits), fac[8 + slot * 8 +
+  // m] = s2_down * w of row m. The MFMA kernels (-> k_pick_combine, up to 16 rows) keep them by pick: dpart f32 [m topk + r][H], then
+  // the shared expert's rows [M topk + m][H]; fac[8 + m topk + r] = s2_down * w.
+  float* dpart;
+  float* fac;
 #ifdef DSGX_TRACE
   unsigned long long* trace;
 #endif
