@@ -74,7 +74,7 @@ struct DecodeArgs {
   // The down phase's dots and their factors, between its kernel and the one that chains them. The vector-unit kernels (k_down_part ->
   // k_down_combine, up to eight rows a pass) keep them by slot: dpart f32 [slot][M][H], fac[0] = slots (as int bits), fac[8 + slot * 8 +
   // m] = s2_down * w of row m. The MFMA kernels (-> k_pick_combine, up to 16 rows) keep them by pick: dpart f32 [m topk + r][H], then
-  // the shared expert's rows [M topk + m][H]; fac[8 + m topk + r] = s2_down * w.
+  // the shared expert's rows [M topk + m][H]; fac[8 + m topk + r] = s2_down * w, or kNoPick.
   float* dpart;
   float* fac;
 #ifdef DSGX_TRACE
@@ -148,6 +148,13 @@ struct Step {
   uint8_t pick[PICKS ? M * DSGX_MAX_TOPK : 1][M <= 4 ? 4 : M <= 8 ? 8 : 16];
   float pw[PICKS ? M * DSGX_MAX_TOPK : 1], pfac[PICKS ? M * DSGX_MAX_TOPK : 1];
 };
+// A pick's factor, s2 w; kNoPick (a NaN that no product is taken as) where the row has no such pick, its picks naming an expert twice,
+// and in DeepSeek's fold, which adds the outputs as they are, where the weight is 0
+constexpr uint32_t kNoPick = 0x7FFFFFFFu;
+__device__ __forceinline__ float pick_factor(float s2, float w, int dsk) {
+  const float f = __fmul_rn(s2, w);
+  return f != f ? __uint_as_float(0x7FC00000u) : dsk && f == 0.f ? __uint_as_float(kNoPick) : f;
+}
 // the number of row m's pick of the routed slot (255: it did not pick it); one row picked every slot, its picks are numbered as they are
 template <int M>
 __device__ __forceinline__ int pick_of(const Step<M, true>& S, int slot, int m) { return M == 1 ? slot : S.pick[slot][m]; }
@@ -186,7 +193,7 @@ __device__ __forceinline__ void prep(Step<M, PICKS>& S, const DecodeArgs& a) {
   if (tid < DSGX_MAX_EXPERTS / 32) S.mask[tid] = 0;
   if constexpr (PICKS) {
     for (int i = tid; M > 1 && i < (int)sizeof(S.pick) / 4; i += blockDim.x) reinterpret_cast<uint32_t*>(S.pick)[i] = 0xFFFFFFFFu;
-    if (tid < M * DSGX_MAX_TOPK) S.pfac[tid] = 0.f;
+    if (tid < M * DSGX_MAX_TOPK) S.pfac[tid] = __uint_as_float(kNoPick);
   } else {
     for (int i = tid; i < M * DSGX_MAX_TOPK * M; i += blockDim.x) (&S.wslot[0][0])[i] = 0.f;
   }
@@ -282,7 +289,7 @@ __device__ __forceinline__ void resolve(Step<M, PICKS>& S, const DecodeArgs& a, 
       if (lane < topk) {
         if (a.idx_out && blockIdx.x == 0) a.idx_out[lane] = id, a.wts_out[lane] = w;
         const float s2 = make_slot(id, r);
-        if constexpr (PICKS) S.pw[r] = w, S.pfac[r] = __fmul_rn(s2, w);
+        if constexpr (PICKS) S.pw[r] = w, S.pfac[r] = pick_factor(s2, w, a.dsk);
         else S.wslot[r][0] = w;
       }
       if (lane == 0) S.n = topk;
@@ -341,7 +348,7 @@ __device__ __forceinline__ void resolve(Step<M, PICKS>& S, const DecodeArgs& a, 
       int p = M == 1 ? r : m * topk;  // the row's pick: its picks below e before it (one row: pick_of)
       for (int j = 0; M > 1 && j < topk; ++j) p += S.ri[m * topk + j] < e ? 1 : 0;
       if (M > 1) S.pick[r][m] = p;
-      S.pw[p] = S.rw[i], S.pfac[p] = __fmul_rn(s2, S.rw[i]);
+      S.pw[p] = S.rw[i], S.pfac[p] = pick_factor(s2, S.rw[i], a.dsk);
     } else {
       S.wslot[r][m] = S.rw[i];
     }
@@ -857,23 +864,18 @@ __global__ void __launch_bounds__(256) k_down_combine(DecodeArgs a) {
     }
 #pragma unroll
     for (int j = 0; j < B; ++j)
-      if (s0 + j < nrouted) {
-        // DeepSeek's fold: the outputs of the experts the row picked (their routing weight, never zero, went in before
-        // w2), each rounded to bf16, added in expert-id order (ds41f engine/kernels/moe.cu:974-981)
-        if (a.dsk) acc = f[j] != 0.f ? __fadd_rn(acc, bf16_round(v[j])) : acc;
-        else acc = fmaf(f[j], v[j], acc);
-      }
+      if (s0 + j < nrouted) acc = fmaf(f[j], v[j], acc);
   }
   float sv = 0.f;
-  if (SH) a.ys[i] = sv = a.dsk ? bf16_round(a.dpart[i]) : a.dpart[i];
+  if (SH) a.ys[i] = sv = a.dpart[i];
   else if (a.ysum) sv = a.ys[i];
-  if (a.ysum || (a.dsk && SH)) acc = __fadd_rn(acc, sv);  // (DeepSeek: the shared expert last, always)
+  if (a.ysum) acc = __fadd_rn(acc, sv);
   a.yr[i] = acc;
 }
 
 // The same sums after the MFMA kernels' down phase, whose dots are kept by pick: dpart [row m][pick r of topk, by slot][H], then
-// the shared expert's rows [m][H]; fac[8 + m topk + r] = s2 w (0: no such pick, or a weight of 0: nothing is added). A dot that
-// no row's routing asks for is neither stored nor read: by slot and row, as for k_down_combine, eight rows with 58 slots moved 15 MB a
+// the shared expert's rows [m][H]; fac[8 + m topk + r] = s2 w, or kNoPick (a weight of 0 is added: what it multiplies may be
+// infinite). A dot that no row's routing asks for is neither stored nor read: by slot and row, as for k_down_combine, eight rows with 58 slots moved 15 MB a
 // layer of hidden 4096, now 2.4 (FP8, four layers of eight rows 1010 -> 972 us; INT4, six rows, 886 -> 862).
 template <bool SH>
 __global__ void __launch_bounds__(256) k_pick_combine(DecodeArgs a) {
@@ -884,12 +886,16 @@ __global__ void __launch_bounds__(256) k_pick_combine(DecodeArgs a) {
   const float* d = a.dpart + (size_t)m * topk * H + n;
   float v[DSGX_MAX_TOPK], f[DSGX_MAX_TOPK];
 #pragma unroll
-  for (int r = 0; r < DSGX_MAX_TOPK; ++r) v[r] = d[(size_t)min(r, topk - 1) * H], f[r] = r < topk ? a.fac[8 + m * topk + r] : 0.f;
+  for (int r = 0; r < DSGX_MAX_TOPK; ++r) v[r] = d[(size_t)min(r, topk - 1) * H], f[r] = a.fac[8 + m * topk + min(r, topk - 1)];
   const float sh = SH ? a.dpart[(size_t)(M * topk + m) * H + n] : 0.f;
+  // (DeepSeek's fold: the picked experts' outputs, their routing weight in them before w2, each rounded to bf16, added in expert-id
+  // order, the shared expert's last: ds41f engine/kernels/moe.cu:974-981)
   float acc = 0.f;
 #pragma unroll
-  for (int r = 0; r < DSGX_MAX_TOPK; ++r)
-    if (f[r] != 0.f) acc = a.dsk ? __fadd_rn(acc, bf16_round(v[r])) : fmaf(f[r], v[r], acc);  // (dsk: see k_down_combine)
+  for (int r = 0; r < DSGX_MAX_TOPK; ++r) {
+    const float s = a.dsk ? __fadd_rn(acc, bf16_round(v[r])) : fmaf(f[r], v[r], acc);
+    acc = r < topk && __float_as_uint(f[r]) != kNoPick ? s : acc;
+  }
   float sv = 0.f;
   if (SH) a.ys[i] = sv = a.dsk ? bf16_round(sh) : sh;
   else if (a.ysum) sv = a.ys[i];

@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from dsgx10_amd import abi, lib
+from dsgx10_amd.layer import HostLayer
 from tests import gpu, orc
 from tests.helpers import check_outputs, check_sums, int4_layer_with_large_scales, make_layer, rel_l2, rows_and_routing
 
@@ -439,3 +440,25 @@ def test_decode_phases_apart_over_eight_rows(fmt, H, I, E, topk, shared, up, row
             lib.moe_decode(dl.w, gpu.dev(x[:M]), gpu.dev(idx[:M]), gpu.dev(w[:M]), M, ws, r2, s2, parts=parts, up=up)
         assert np.array_equal(gpu.host(r2, np.uint32, (M, H)), yr.view(np.uint32)), M
         assert np.array_equal(gpu.host(s2, np.uint32, (M, H)), ys.view(np.uint32)), M
+
+
+@pytest.mark.parametrize("M", [1, 3, 12])
+def test_decode_weight_of_zero_on_an_infinite_output(M):
+    """the last row picks, with a weight of 0, an expert whose outputs overflow: the row is NaN, as the sum of products says and as
+    the vector-unit kernels give it; a row that did not pick that expert keeps the bits that it has alone"""
+    H, I, E, topk = 1024, 1024, 16, 4
+    hl = make_layer(abi.FMT_FP8, H, I, E, topk, 4, seed=13)
+    bad = int(hl.emap[0])
+    hl.experts[bad][2][1][:] = 3.3e38
+    dl = HostLayer(abi.FMT_FP8, H, I, E, topk, hl.experts, hl.emap).upload()
+    x, _, _, _ = rows_and_routing(44, M, H, E, topk, 1.0)
+    good = [e for e in range(E) if hl.emap[e] != bad]
+    idx = np.array([[good[(m + j) % len(good)] for j in range(topk)] for m in range(M)], np.int32)
+    w = np.full((M, topk), 0.25, np.float32)
+    idx[-1, 2], w[-1, 2] = 0, 0.0
+    yr, _, _ = gpu.decode_layer(dl, x, idx, w, M, up=1)
+    y0, _, _ = gpu.decode_layer(dl, x[-1:], idx[-1:], w[-1:], 1, up=0)
+    assert np.isnan(y0).all() and np.isnan(yr[-1]).all()
+    for m in range(M - 1):
+        y1, _, _ = gpu.decode_layer(dl, x[m:m + 1], idx[m:m + 1], w[m:m + 1], 1, up=1)
+        assert np.isfinite(y1).all() and np.array_equal(yr[m].view(np.uint32), y1[0].view(np.uint32)), m
