@@ -229,7 +229,9 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   };
   // The positions' scales come for four blocks at a time, 16 bytes a position, into two buffers (blocks 4 q ... 4 q + 3, the last
   // ones of a row from its end): a scale of 4 bytes a position and block named as many cache lines an instruction as all of the
-  // block's activations do (pf_gemm_mx.cuh): gate/up of 128 / 256 rows an expert 1021 / 1425 us before, 964 / 1366 like this. Rows of fewer than four blocks have no 16 bytes: put in place by hand.
+  // block's activations do (pf_gemm_mx.cuh): gate/up of 128 / 256 rows an expert 1021 / 1425 us before, 964 / 1366 like this. Rows of fewer
+  // than four blocks have no 16 bytes: put in place by hand, their loads in flight together (one after the other they cost a call of hidden 2048,
+  // intermediate 384 and 17 rows 1.4 us of 61).
   constexpr int kGroups0 = S::kStages * S::kStageBytes;
   auto first_block = [&](int q) { return min(4 * q, KB - 4); };
   auto issue_scales = [&](int q) {
@@ -250,11 +252,16 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
     asm volatile("" : "+v"(wsa_l), "+v"(wsb_l));  // (uses that make the compiler place its wait here)
   };
   PF_STAMP(g, 2);
+  float xw[3];  // (KB < 4: the positions' scales, on their way with the weights')
+  if (KB < 4) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) xw[i] = *(const DSGX_GLOBAL float*)(uintptr_t)(pxs + min(i, KB - 1));
+  }
   load_ws(0);
   PF_STAMP(g, 3);
   if (KB < 4 && lane < 16 * WP) {
-    for (int kb = 0; kb < KB; ++kb)
-      *reinterpret_cast<float*>(smem + kGroups0 + (16 * WP * wave + lane) * 16 + 4 * kb) = *(const DSGX_GLOBAL float*)(uintptr_t)(pxs + kb);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) reinterpret_cast<float*>(smem + kGroups0)[(16 * WP * wave + lane) * 4 + i] = xw[i];
   }
   issue(0);
   if (KB >= 4) issue_scales(0);  // (behind the first block's loads, which every turn's wait for that block covers)
