@@ -405,8 +405,9 @@ def test_decode_status_reports_a_timeout_and_repairs_the_workspace():
 
 @pytest.mark.parametrize("fmt,H,I,E,topk,shared,rows", [(abi.FMT_FP8, 2048, 2048, 48, 8, "fp8", (9, 13, 14, 16)), (abi.FMT_FP8, 4096, 512, 32, 8, None, (13, 16)),
                                                        (abi.FMT_INT4, 2048, 2048, 24, 8, "bf16", (11, 16)), (abi.FMT_INT4, 6144, 512, 16, 4, None, (9, 10)),
-                                                       (abi.FMT_FP8, 256, 256, 512, 8, "fp8", (9, 16)), (abi.FMT_INT4, 512, 256, 37, 4, None, (9, 16))],
-                         ids=["fp8", "fp8-two-passes", "int4", "int4-H6144", "fp8-E512", "int4-E37"])
+                                                       (abi.FMT_FP8, 256, 256, 512, 8, "fp8", (9, 16)), (abi.FMT_INT4, 512, 256, 37, 4, None, (9, 16)),
+                                                       (abi.FMT_INT4, 2048, 1024, 24, 8, "fp8", (9, 16))],
+                         ids=["fp8", "fp8-two-passes", "int4", "int4-H6144", "fp8-E512", "int4-E37", "int4-fp8-shared"])
 def test_decode_nine_to_sixteen_rows_in_one_pass(fmt, H, I, E, topk, shared, rows):
     """9 to 16 rows in one pass of the MFMA kernels, with the h of two slots staged together and of one, and as many rows as LDS
     holds and the rest: every row's bits are those of the row alone; fused routing the bits of given picks"""

@@ -145,8 +145,8 @@ def test_dsk_moe_every_bit_against_the_matrix_unit_oracle(H, I, E, M, shared):
 
 @pytest.mark.parametrize("M", [12, 16])
 def test_dsk_moe_nine_to_sixteen_rows(M):
-    """9-16 rows run as two passes of the kernels built for eight (dsk.h:211-223's up16 / down16 range): every row's bits are
-    what the row gives in a call of its own, whose parity with the oracle the test above holds; routing fused and apart"""
+    """9-16 rows (dsk.h:211-223's up16 / down16 range; one pass of the kernels at this size): every row's bits are what the row gives in
+    a call of its own, whose parity with the oracle the test above holds; routing fused and apart"""
     H, I, E, topk = 2048, 768, 32, 6
     hl = _layer(22, H, I, E, topk, 5, True)
     dl = hl.upload()
@@ -173,3 +173,35 @@ def test_dsk_moe_nine_to_sixteen_rows(M):
         y1, ys1 = run([m], False)
         assert np.array_equal(y[m], y1[0]) and np.array_equal(ys[m], ys1[0]), m
     assert np.isfinite(y.view(np.float32)).all()
+
+
+@pytest.mark.parametrize("H,I,rows", [(1024, 2304, (13, 16)), (6144, 512, (9, 10, 16))], ids=["one-slot", "two-passes"])
+def test_dsk_moe_stacked_over_eight_rows(H, I, rows):
+    """stacked experts at more than eight rows: h of one slot at a time staged and quantised in the down phase (13 rows and more of
+    intermediate 2304), and nine rows and the rest (hidden 6144); routing fused, its selection written for the caller, and the phases in
+    two calls: every row's bits are those of the row alone"""
+    from tests.test_gpu_dsk_prefill import Stacked
+    E, topk, N = 16, 6, max(rows)
+    L = Stacked(45, H, I, E, topk, 5, True)
+    xq, xs = orc.act_quant_ue8m0(orc.normal_bf16(45, 1, (N, H), 1.5))
+    logits, bias = orc.normal_f32(45, 2, (N, E), 1.0), orc.normal_f32(45, 3, (E,), 0.2)
+    idx, w = orc.route(logits, bias, topk, 1.5, score_fn=1)
+
+    def run(a, b, parts=(3,), fused=False):
+        n = b - a
+        ws, y = gpu.empty(lib.dsk_ws_bytes(H, I), 0), gpu.empty(n * H * 4, 0xFF)
+        io, wo = gpu.empty(n * topk * 4, 0xFF), gpu.empty(n * topk * 4, 0xFF)
+        for p in parts:
+            if fused:
+                lib.dsk_moe_stacked(L.w, gpu.dev(xq[a:b]), gpu.dev(xs[a:b]), None, None, n, ws, y, logits=gpu.dev(logits[a:b]), bias=gpu.dev(bias), route_scale=1.5,
+                                    parts=p, idx_out=io, wts_out=wo)
+            else:
+                lib.dsk_moe_stacked(L.w, gpu.dev(xq[a:b]), gpu.dev(xs[a:b]), gpu.dev(idx[a:b]), gpu.dev(w[a:b]), n, ws, y, parts=p)
+        return gpu.host(y, np.uint32, (n, H)), gpu.host(io, np.int32, (n, topk)), gpu.host(wo, np.float32, (n, topk))
+    alone = np.concatenate([run(m, m + 1)[0] for m in range(N)])
+    for M in rows:
+        y, io, wo = run(0, M, fused=True)
+        assert np.array_equal(y, alone[:M]), M
+        assert np.array_equal(io, idx[:M]) and np.array_equal(wo.view(np.uint32), w[:M].view(np.uint32)), M
+        assert np.array_equal(run(0, M)[0], y) and np.array_equal(run(0, M, parts=(1, 2))[0], y), M
+    assert np.isfinite(alone.view(np.float32)).all()
