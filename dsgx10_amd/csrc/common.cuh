@@ -15,10 +15,9 @@ constexpr int kWave = 64;
 
 // ---- scalar codecs ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ float bf16_bits_to_f32(uint32_t b) { return __uint_as_float(b << 16); }
-// Round to nearest even, the contract's integer form (engine/experts/formats.cuh:33-37 of the reference): used where
-// a single value is rounded (epilogues); the packed hardware conversion below is used in the streaming loops.
-// f32 -> bf16, round to nearest even: v_cvt_pk_bf16_f32, one instruction (two for the rounded f32) where adding half a step by hand
-// is four; the same bits for every number (all 2^32 compared), and a NaN stays one
+// f32 -> bf16, round to nearest even (engine/experts/formats.cuh:33-37 of the reference): v_cvt_pk_bf16_f32, one instruction (two for
+// the rounded f32) where adding half a step by hand is four; the same bits for every number, and a NaN stays a NaN (by hand the carry
+// takes some to infinity or -0). A test compares all 2^32.
 __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 __device__ __forceinline__ float bf16_round(float f) { return (float)(__bf16)f; }
 // two f32 -> packed bf16 (lo = a, hi = b), round to nearest even: v_cvt_pk_bf16_f32
@@ -495,8 +494,8 @@ __device__ __forceinline__ void route_row(const float (&logit)[kRouteRJ], const 
 __device__ __forceinline__ float bf16_lo(uint32_t p) { return __uint_as_float(p << 16); }  // the values of a packed pair
 __device__ __forceinline__ float bf16_hi(uint32_t p) { return __uint_as_float(p & 0xFFFF0000u); }
 // silu(g) = g / (1 + e^-g) of four values in f32, the division IEEE's: by the divisor's reciprocal and one correction step where
-// |g| < 60 (the divisor is then in [1, 2^87]: no scaling; equal to the division for every bf16 g, all compared, but the sign of a
-// zero, which is g's), by the division itself if a value of the wave lies outside.
+// |g| < 60 (the divisor is then in [1, 2^87]: no scaling; equal to the division for every f32 g there, all compared, so a gate clamped
+// to a limit that is no bf16 value is in; a zero takes g's sign), by the division itself if a value of the wave lies outside.
 __device__ __forceinline__ void silu4(const float (&g)[4], float (&s)[4]) {
   float d[4];
   bool far = false;
@@ -523,8 +522,8 @@ __device__ __forceinline__ float silu_for_bf16(float g) {
   const float e = __builtin_amdgcn_exp2f(fmaf(g, -1.44269504088896341f, -2.f));
   return __fmul_rn(__fmul_rn(g, 0.25f), __builtin_amdgcn_rcpf(__fadd_rn(0x1.000002p-2f, e)));
 }
-// Four of swiglu_bits' values, packed (g, u: bf16 values). fast: the same function by the plain formula, the caller's choice: one bf16
-// value of g rounds to the other side.
+// Four of swiglu_bits' values, packed (g, u: bf16 values). fast: the same function by the plain formula, the caller's choice: silu of four
+// bf16 gates is another, one step at 5.9375 and -0 at -87.5, -88 and -88.5, whose divisor's reciprocal is not normal.
 __device__ __forceinline__ uint2 swiglu4(const float (&g)[4], const float (&u)[4], bool fast) {
   float s[4];
   if (fast) {

@@ -100,7 +100,7 @@ __global__ void __launch_bounds__(NW * 64) k_gemv(GemvArgs a) {
   };
   enter();
   // past the last step the ring's loads go, scales and zero points too, to the first bytes of the wave's last rows: one cached line of
-  // the wave's own (with a line for each kind of load, 2048 x 4096 over 2 took 5.9 us, 5.5 like this)
+  // the wave's own (with a line for each kind of load, 2048 x 4096 over 2 took 5.9 us, 5.4 like this)
   auto park = [&]() {
 #pragma unroll
     for (int i = 0; i < RB; ++i) src[i].w = src[i].a = src[i].z = src[0].w;

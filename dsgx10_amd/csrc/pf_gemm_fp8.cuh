@@ -80,7 +80,7 @@ struct Args {
   const int* ntiles;
   const int* off;
   int nrows;           // the shared expert's rows: T
-  int fast_act;        // UP: SwiGLU by the hardware's exp2 / rcp instead of expf() and the IEEE division
+  int fast_act;        // UP: SwiGLU by the plain formula (swiglu4)
   dsgx_layer_w L;
   uint16_t* h;         // UP: h bf16 [position][I]
   uint8_t* hq;         // UP: h quantised, e4m3 [position][I]

@@ -24,7 +24,6 @@ namespace dsgx {
 namespace pfi4 {
 
 using pf8::dma16;
-using pf8::dma4;
 using pf8::kThreads;
 using pf8::kWgRows;
 using pf8::sw4;

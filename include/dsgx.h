@@ -252,10 +252,10 @@ typedef struct dsgx_prefill_cfg {
   int32_t act_fp8;  /* FP8 layers: 1 = quantise activations per row and 128 k to e4m3 and run the fp8 MFMA
                        (ds41f-4xgx10-switchless/ref/torchref/kernel.py:56-77, ref/inference/kernel.py:207-274);
                        0 = bf16 activations, weights widened to bf16 (the altar-1 contract) */
-  int32_t fast_act; /* FP8 activations only. 0 (the default): SwiGLU with expf() and the IEEE division, as the decode kernels
-                       and the reference compute it (engine/experts/decode.cu:110-113); 1: the hardware's exponential and
-                       reciprocal (each within 1 ulp; h then differs from the exact form's in about one value in 10^4, by one
-                       bf16 step), for callers that trade that for the epilogue's time */
+  int32_t fast_act; /* FP8 activations only. 0 (the default): SwiGLU with the bits of the decode kernels and the reference
+                       (engine/experts/decode.cu:110-113: expf() and the IEEE division, then the rounding to bf16) for every bf16
+                       gate; 1: the plain formula on the hardware's exponential and reciprocal, whose silu differs at four bf16
+                       gates (one step at 5.9375; -0 instead of -9e-37 ... -3e-37 at -87.5, -88 and -88.5) */
   int32_t tile_order; /* FP8 activations only: the order in which the grouped GEMMs walk the tiles (the reference's
                        prefill_tuning tord, ds41f-4xgx10-switchless/engine/kernels/dsk.h:252, prefill.cu:658-668). 0: by
                        expert id, an expert's tiles next to each other; 1: the experts by falling count, their

@@ -3,6 +3,7 @@ streaming kernels' own in-register routine), the router's ids and weight bits, f
 Mirrors the reference's test_deq / test_route (altar1-4xgx10-switchless/engine/experts/tests/test_experts.cu:217-319)."""
 import numpy as np
 import pytest
+import torch
 
 from dsgx10_amd import abi, lib
 from tests import gpu, orc
@@ -219,3 +220,19 @@ def test_calls_go_to_the_current_stream():
         graph.replay()
         torch.cuda.synchronize()
         assert bool((out.float() == 2 * v).all())
+
+
+def test_bf16_rounding_of_every_f32():
+    """the kernels' rounding to bf16 (through finalize: bf16(R) + bf16(-0) is bf16(R)) is to nearest, ties to even, for all 2^32 patterns;
+    a NaN stays a NaN"""
+    n = 1 << 28
+    S = torch.full((n,), -0.0, device="cuda")
+    out = torch.empty(n, dtype=torch.int16, device="cuda")
+    for k in range(16):
+        u = torch.arange(n, dtype=torch.int32, device="cuda") + ((k << 28) - (1 << 32) * (k >= 8))
+        lib.finalize(u.view(torch.float32), S, n, out)
+        want = (u + 0x7FFF + ((u >> 16) & 1)) >> 16
+        nan = (u & 0x7FFFFFFF) > 0x7F800000
+        got = out.int()
+        assert bool(((got == want) | nan).all()), k
+        assert bool((((got & 0x7FFF) > 0x7F80) == nan).all()), k

@@ -260,3 +260,41 @@ def test_dsk_prefill_at_the_layer_shape():
     sub = rows[:3]
     got1 = run_prefill(L, xq[sub], xs[sub], idx[sub], w[sub])
     assert np.array_equal(got1["y"].view(np.uint32), got["y"][sub].view(np.uint32))
+
+
+@pytest.mark.parametrize("limit", [3e38, 57.3, 1.7, 1.0 / 3.0])
+def test_dsk_prefill_silu_of_given_gates(limit):
+    """silu of the MXFP4 prefill's epilogue (common.cuh: silu4) against the decode kernels', which take expf and IEEE's division: h of a
+    shared expert whose gates are, row by row of powers of two, all bf16 significands of both signs - tiny ones, both sides of +-60 in one
+    tile, and those whose divisor overflows -, unclamped and with limits that are no bf16 values"""
+    H, I, E, topk = 256, 256, 8, 6
+    L = Stacked(46, H, I, E, topk, 2, True)
+    exps = np.arange(-110, 121)
+    T = len(exps)
+    code = lambda v: orc.f32_to_e4m3(np.asarray(v, np.float32))
+    sig, sign = 128 + np.arange(I) % 128, np.where(np.arange(I) < 128, 1.0, -1.0)
+    gate, up = np.zeros((I, H), np.uint8), np.zeros((I, H), np.uint8)
+    gate[:, 0], gate[:, 32] = code(sign * (sig >> 4)), code(sign * (sig & 15))  # g = +-(hi 2^-3 + lo 2^-7) 2^e
+    up[:, 64] = code(1.0)
+    gs, us = np.full((I // 32, H // 32), 127, np.uint8), np.full((I // 32, H // 32), 127, np.uint8)
+    gs[:, 0], gs[:, 1] = 127 - 3, 127 - 7
+    keep = [gpu.dev(a) for a in (gate, gs, up, us)]
+    L.w.sh_w1, L.w.sh_s1, L.w.sh_w3, L.w.sh_s3 = [k.data_ptr() for k in keep]
+    xq, xs = np.zeros((T, H), np.uint8), np.full((T, H // 32), 127, np.uint8)
+    xq[:, [0, 32, 64]] = code(1.0)
+    xs[:, 0] = xs[:, 1] = 127 + exps
+    idx = np.tile(np.arange(topk, dtype=np.int32), (T, 1))
+    w = np.full((T, topk), 0.25, np.float32)
+    ws, y = gpu.empty(lib.dsk_prefill_ws_bytes(H, I, E, topk, T), 0xEE), gpu.empty(T * H * 4)
+    lib.dsk_moe_prefill(L.w, gpu.dev(xq), gpu.dev(xs), gpu.dev(idx), gpu.dev(w), T, ws, y, limit=limit)
+    h = gpu.host(gpu.view(ws, lib.dsk_prefill_view(L.w, ws, T).hsh, T * I * 2), np.uint16, (T, I))
+    g = np.minimum(sign * sig * 2.0 ** -7 * 2.0 ** exps[:, None].astype(np.float64), np.float32(limit))
+    with np.errstate(over="ignore"):
+        ref = g / (1.0 + np.exp(-g)) * min(1.0, np.float32(limit))
+    assert np.allclose(orc.bf16_to_f32(h), ref, rtol=2.0 ** -7, atol=1e-36)  # (the divisor overflows from g = -88.75 on: -0 for up to 3e-37)
+    for t0 in range(0, T, 8):
+        n = min(8, T - t0)
+        wd, yd = gpu.empty(lib.dsk_ws_bytes(H, I), 0), gpu.empty(n * H * 4)
+        lib.dsk_moe_stacked(L.w, gpu.dev(xq[t0:t0 + n]), gpu.dev(xs[t0:t0 + n]), gpu.dev(idx[t0:t0 + n]), gpu.dev(w[t0:t0 + n]), n, wd, yd, limit=limit)
+        hd = gpu.host(wd[abi.SH_SLOT * n * I * 2:(abi.SH_SLOT + 1) * n * I * 2], np.uint16, (n, I))
+        assert np.array_equal(h[t0:t0 + n], hd), (t0, np.argwhere(h[t0:t0 + n] != hd)[:4].tolist())

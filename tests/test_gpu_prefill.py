@@ -416,8 +416,9 @@ def test_prefill_int4_bf16_shared_expert_tiles(H, I, T):
 
 
 def test_prefill_silu_at_the_ends_of_its_fast_division():
-    """silu of the prefill epilogues (common.cuh) against the decode kernels', which divide by IEEE's division everywhere: h of a BF16 shared expert whose gates are given values, on both sides of +-60, denormal results,
-    zeros and infinities, from both"""
+    """silu of the INT4 prefill's epilogue (common.cuh: silu_for_bf16) against the decode kernels', which divide by IEEE's division
+    everywhere: h of a BF16 shared expert whose gates are given values, denormal results, zeros and overflowing divisors among them, from
+    both (silu4, whose division has ends at +-60: test_dsk_prefill_silu_of_given_gates)"""
     H, I, E, topk = 256, 256, 8, 2
     hl = helpers.make_layer(abi.FMT_INT4, H, I, E, topk, 4, seed=27, shared="bf16")
     dl = hl.upload()
@@ -467,3 +468,46 @@ def test_prefill_silu_of_every_finite_bf16_gate():
         o = gpu.h_of(wd, dl, 8, topk)[-1]
         for m in range(8):
             assert np.array_equal(h[t0 + m], o[m]), t0 + m
+
+
+def test_prefill_fp8_silu_of_given_gates_exact_and_by_the_plain_formula():
+    """the FP8 prefill's silu rounds every bf16 gate met here - all significands of both signs, row by row of powers of two up to those that
+    overflow - to the bits of the decode kernels'; with fast_act four gates are others, as dsgx.h lists them"""
+    H, I, E, topk = 256, 512, 8, 2
+    hl = helpers.make_layer(abi.FMT_FP8, H, I, E, topk, 4, seed=27, shared="fp8")
+    dl = hl.upload()
+    exps = np.arange(-22, 116)  # (beyond, the decode kernels' sums overflow before their scale of 2^-90)
+    T = len(exps)
+    code = lambda v: orc.f32_to_e4m3(np.asarray(v, np.float32))
+    sig, sign = 128 + np.arange(I) % 128, np.where(np.arange(I) // 128 % 2 == 0, 1.0, -1.0)
+    gate, up = np.zeros((I, H), np.uint8), np.zeros((I, H), np.uint8)
+    gate[:, 0], gate[:, 1] = code(sign * (sig >> 4)), code(sign * (sig & 15))  # g = +-(256 hi + 16 lo) 2^e s
+    up[:, 129] = code(1.0)
+    gs, us = np.ones((I // 128, H // 128), np.float32), np.full((I // 128, H // 128), 2.0 ** -8, np.float32)
+    gs[:2], gs[2:] = 2.0 ** 4, 2.0 ** -90
+    keep = [gpu.dev(a) for a in (gate, gs, up, us)]
+    dl.w.sh.g, dl.w.sh.gs, dl.w.sh.u, dl.w.sh.us = [k.data_ptr() for k in keep]
+    x = np.zeros((T, H), np.float32)
+    x[:, 0], x[:, 1], x[:, 2] = 256 * 2.0 ** exps, 16 * 2.0 ** exps, 448 * 2.0 ** exps  # (the largest makes the block's scale 2^e)
+    x[:, 128], x[:, 129] = 448, 256
+    x = orc.f32_to_bf16(x)
+    _, _, idx, w = helpers.rows_and_routing(31, T, H, E, topk, 2.5)
+
+    def prefill(fast):
+        ws, yr, ys = gpu.empty(lib.prefill_ws_bytes(dl.w, T), 0), gpu.empty(T * H * 4), gpu.empty(T * H * 4)
+        lib.moe_prefill(dl.w, gpu.dev(x), gpu.dev(idx), gpu.dev(w), T, ws, yr, ys, fast_act=fast)
+        return gpu.host(gpu.view(ws, lib.prefill_view(dl.w, ws, T).hsh, T * I * 2), np.uint16, (T, I))
+    h, hf = prefill(False), prefill(True)
+    nan = lambda b: (b & 0x7FFF) > 0x7F80
+    for t0 in range(0, T, 8):
+        n = min(8, T - t0)
+        _, _, wd = gpu.decode_layer(dl, x[t0:t0 + n], idx[t0:t0 + n], w[t0:t0 + n], n, up=1)
+        hd = gpu.h_of(wd, dl, n, topk)[-1]
+        assert np.array_equal(np.where(nan(hd), 0x7FC0, hd), np.where(nan(h[t0:t0 + n]), 0x7FC0, h[t0:t0 + n])), t0
+    with np.errstate(over="ignore"):
+        g = (sign * sig * 16.0 * np.repeat(gs[:, 0], 128)[None, :]) * 2.0 ** exps[:, None]
+        g32 = g.astype(np.float32)
+    assert nan(h[g32 == -np.inf]).all() and (h[g32 == np.inf] == 0x7F80).all() and np.isinf(g32).any()
+    other = (h != hf) & ~(nan(h) & nan(hf))
+    assert sorted(set(g[other].tolist())) == [-88.5, -88.0, -87.5, 5.9375]
+    assert (hf[other & (g < 0)] == 0x8000).all()
