@@ -71,9 +71,10 @@ static int decode_variant(uint32_t fmt, int M, int H, int I) {
 
 // The workspace: h [DSGX_MAX_UNION + 1 slots][DSGX_MAX_ROWS][I] | the barrier's words (kBarBytes) | the down phase's factors
 // (kFacBytes) and kDots rows of f32 [H] dots (DecodeArgs: by slot, 129 of eight rows, or by pick, sixteen rows' top-k and shared
-// expert) | a reserved row buffer [16][H] bf16. I and H here are the LAYOUT's: the layer's own for a caller's workspace; the built-in workspace is laid out for its largest shapes whatever the layer, so that every layer run
-// on it finds the barrier's words in one place (at an offset that moved with the layer, one layer's h or partial sums would
-// lie where another's counters are expected to be zero).
+// expert) | a reserved row buffer [16][H] bf16. I and H here are the LAYOUT's: the layer's own for a caller's workspace; the
+// built-in workspace is laid out for its largest shapes whatever the layer, so that every layer run on it finds the barrier's
+// words in one place (at an offset that moved with the layer, one layer's h or partial sums would lie where another's
+// counters are expected to be zero).
 struct WsLayout {
   int I, H;
   static constexpr size_t kFacBytes = (size_t)(8 + (DSGX_MAX_UNION + 1) * 8) * 4 + 192;  // (a multiple of 256)

@@ -876,7 +876,7 @@ __global__ void __launch_bounds__(256) k_down_combine(DecodeArgs a) {
 // The same sums after the MFMA kernels' down phase, whose dots are kept by pick: dpart [row m][pick r of topk, by slot][H], then
 // the shared expert's rows [m][H]; fac[8 + m topk + r] = s2 w, or kNoPick (a weight of 0 is added: what it multiplies may be
 // infinite). A dot that no row's routing asks for is neither stored nor read: by slot and row, as for k_down_combine, eight rows with 58 slots moved 15 MB a
-// layer of hidden 4096, now 2.4 (FP8, four layers of eight rows 1010 -> 972 us; INT4, six rows, 886 -> 862).
+// layer of hidden 4096, now 2.4 (FP8, four layers of eight rows 1010 -> 972 us; INT4, six rows, 886 -> 868).
 template <bool SH>
 __global__ void __launch_bounds__(256) k_pick_combine(DecodeArgs a) {
   const int H = a.L.H, topk = a.L.topk, M = a.M;
