@@ -788,9 +788,10 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
     // INT4 experts: the LDS-staged kernels of pf_gemm_i4.cuh (DSGX_PF_I4_OLD=1: the register-ring kernel they replaced, same bits)
     const char* old4 = std::getenv("DSGX_PF_I4_OLD");
     const bool new4 = i4 && !(old4 && old4[0] == '1');
+    const auto k_dn4 = I % 256 ? pfi4::k_gemm<false, false> : pfi4::k_gemm<false, true>;
     pfi4::Args q4{};
     if (new4) {
-      for (const void* k : {(const void*)pfi4::k_gemm<true>, (const void*)pfi4::k_gemm<false>})
+      for (const void* k : {(const void*)pfi4::k_gemm<true, true>, (const void*)k_dn4})
         if (int rc = allow_dynamic_lds(k, pfi4::kLdsRun)) return rc;
       q4.L = *L, q4.tile_e = I32(o.tile_e), q4.tile_m0 = I32(o.tile_m0), q4.ntiles = I32(o.ntiles), q4.off = I32(o.off);
     }
@@ -805,14 +806,14 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
       q.x = x, q.gather = I32(o.perm), q.h = reinterpret_cast<uint16_t*>(W + o.h), q.d = nullptr;
       if (fused_sh) q4.sh_grid = sh_gu, q4.sh = sh_up;
       q4.x = q.x, q4.gather = q.gather, q4.h = q.h, q4.d = nullptr;
-      if (new4) hipLaunchKernelGGL(pfi4::k_gemm<true>, dim3(q4.sh_grid + pf8::grid_of(o.max_tiles, I / (kWgRows / 2))), dim3(pf8::kThreads), pfi4::kLdsRun, st, q4);
+      if (new4) hipLaunchKernelGGL((pfi4::k_gemm<true, true>), dim3(q4.sh_grid + pf8::grid_of(o.max_tiles, I / (kWgRows / 2))), dim3(pf8::kThreads), pfi4::kLdsRun, st, q4);
       else hipLaunchKernelGGL(k_up, dim3(pf_grid(o.max_tiles, I / (kWgRows / 2))), dim3(kGemmThreads), lds16, st, q);
     }
     if (cfg.phases & 4) {
       q.x = reinterpret_cast<const uint16_t*>(W + o.h), q.gather = nullptr, q.h = nullptr, q.d = F32(o.d);
       q4.x = q.x, q4.gather = nullptr, q4.h = nullptr, q4.d = q.d;
       if (fused_sh) q4.sh_grid = sh_gd, q4.sh = sh_dn;
-      if (new4) hipLaunchKernelGGL(pfi4::k_gemm<false>, dim3(q4.sh_grid + pf8::grid_of(o.max_tiles, H / kWgRows)), dim3(pf8::kThreads), pfi4::kLdsRun, st, q4);
+      if (new4) hipLaunchKernelGGL(k_dn4, dim3(q4.sh_grid + pf8::grid_of(o.max_tiles, H / kWgRows)), dim3(pf8::kThreads), pfi4::kLdsRun, st, q4);
       else hipLaunchKernelGGL(k_dn, dim3(pf_grid(o.max_tiles, H / kWgRows)), dim3(kGemmThreads), lds16, st, q);
     }
     if (cfg.phases & 8) {

@@ -309,8 +309,13 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   else pfb16::store_d(smem, acc, nmt, m0, mend, r0, g.L.H, g.d);
 }
 
-// The routed experts' tiles, and in front of them (workgroups 0 .. sh_grid - 1) the BF16 shared expert's, if the launch holds those
-template <bool UP>
+// The routed experts' tiles, and in front of them (workgroups 0 .. sh_grid - 1) the BF16 shared expert's, if the launch holds those.
+// PAIR: K is an even number of 128-k blocks; only down has an odd number (up to 64 rows of one: in the 128-position shape every wave
+// fetches activations that nobody reads; whole call of hidden 2048, intermediate 384, 64 experts, T = 17 / 60: 69.5 / 75.7 us there, 68.1 /
+// 74.8 like this). A kernel of its own: as a third shape of one kernel it cost the others up to 1.3% (hidden 6144, intermediate 2048, 168
+// experts, T = 17 / 40 / 60: 396.5 / 551 / 685 us, 391.5 / 544 / 677.5 like this). The check of K under PAIR is always true; it is
+// there for the code that the compiler makes of it: without it 394 / 547.5 / 681.
+template <bool UP, bool PAIR>
 __global__ void __launch_bounds__(kThreads) k_gemm(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   if (blockIdx.x < g.sh_grid) {  // (the same for the whole workgroup)
@@ -323,11 +328,8 @@ __global__ void __launch_bounds__(kThreads) k_gemm(Args g) {
   if (ns >= NS || tile >= *g.ntiles) return;
   const int e = g.tile_e[tile];
   const int m0 = g.off[e] + g.tile_m0[tile], mend = g.off[e + 1];
-  // (up to 64 rows of an odd number of 128-k blocks, which only down has: in the 128-position shape every wave fetches activations
-  // that nobody reads; down of hidden 2048, intermediate 384, 64 experts, T = 60 / 200: 15.3 / 23.5 us there, 14.8 / 22.8 like this)
-  if (mend - m0 > 64) gemm_tile<UP, 128, false>(g, smem, e, m0, mend, ns);
-  else if (UP || g.L.I % 256 == 0) gemm_tile<UP, 64, true>(g, smem, e, m0, mend, ns);
-  else gemm_tile<UP, 64, false>(g, smem, e, m0, mend, ns);
+  if (mend - m0 <= 64 && (!PAIR || (UP ? g.L.H : g.L.I) % 256 == 0)) gemm_tile<UP, 64, PAIR>(g, smem, e, m0, mend, ns);
+  else gemm_tile<UP, 128, false>(g, smem, e, m0, mend, ns);
 }
 
 }  // namespace pfi4
