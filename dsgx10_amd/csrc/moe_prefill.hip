@@ -76,10 +76,9 @@ constexpr int kTile = 128;  // rows of a tile (token positions) and weight rows 
 constexpr int kRowBlock = 128;  // token rows a workgroup of the bucketing kernels
 struct PfLayout {
   size_t cnt, off, ntiles, tile_e, tile_m0, perm, pickpos, posw, rpos, re, rk, xq, xs, h, hq, hs, hsh, hshq, hshs, d, bcnt, boff, bmask, total;
-  size_t nbig, big_e, big_m0, nsmall, small_e, small_m0;  // the FP8 kernels' lists: 256-position tiles, and the experts' remainders
-  size_t nmix, mix_e, mix_m0;                             // ... and the two merged, in expert order
-  size_t ord_e, ord_m0;                                   // ... and merged with the experts by falling count, remainders spread evenly
-  int P, max_tiles, max_big;
+  size_t nwide, wide_e, wide_m0;  // the FP8-activation kernels' list: tiles of pf8::kMaxPos positions
+  size_t ord_e, ord_m0;           // ... in dsgx_prefill_cfg::tile_order's order
+  int P, max_tiles, max_wide;
 };
 PfLayout pf_layout(const dsgx_layer_w* L, int T) {
   PfLayout o{};
@@ -90,11 +89,9 @@ PfLayout pf_layout(const dsgx_layer_w* L, int T) {
   auto take = [&](size_t bytes) { const size_t a = at; at += align256(bytes); return a; };
   o.cnt = take(E * 4), o.off = take((E + 1) * 4), o.ntiles = take(4);
   o.tile_e = take((size_t)o.max_tiles * 4), o.tile_m0 = take((size_t)o.max_tiles * 4);
-  o.max_big = (int)(P / 256 + E);
-  o.nbig = take(4), o.big_e = take((size_t)o.max_big * 4), o.big_m0 = take((size_t)o.max_big * 4);
-  o.nsmall = take(4), o.small_e = take(E * 4), o.small_m0 = take(E * 4);
-  o.nmix = take(4), o.mix_e = take((size_t)(o.max_big + E) * 4), o.mix_m0 = take((size_t)(o.max_big + E) * 4);
-  o.ord_e = take((size_t)(o.max_big + E) * 4), o.ord_m0 = take((size_t)(o.max_big + E) * 4);
+  o.max_wide = (int)(P / pf8::kMaxPos + E);
+  o.nwide = take(4), o.wide_e = take((size_t)o.max_wide * 4), o.wide_m0 = take((size_t)o.max_wide * 4);
+  o.ord_e = take((size_t)o.max_wide * 4), o.ord_m0 = take((size_t)o.max_wide * 4);
   o.perm = take(P * 4), o.pickpos = take(P * 4), o.posw = take(P * 4), o.rpos = take(P * 4), o.re = take(P * 4), o.rk = take(P * 4);
   o.xq = take((size_t)T * H), o.xs = take((size_t)T * (H / 128) * 4);
   o.h = take(P * I * 2), o.hq = take(P * I), o.hs = take(P * (I / 128) * 4);
@@ -133,18 +130,16 @@ __global__ void __launch_bounds__(256) k_pf_mask(const int* __restrict__ idx, in
     *reinterpret_cast<uint4*>(&bmask[((size_t)b * E + e) * 4]) = m;
   }
 }
-// The FP8 kernels' two lists: an expert of c rows gives c / 256 tiles of 256 positions, one more if over 128 rows are left,
-// else (if any are left) one tile of up to 128 positions.
+// The lists of tiles, an expert's next to each other: neighbours run at about the same time on one XCD (pf8::task_of), so part of what
+// an expert's tiles stream, each in full, comes out of that XCD's L2.
 struct TileLists {
-  int *ntiles, *tile_e, *tile_m0;     // all rows in 128-position tiles
-  int *nbig, *big_e, *big_m0;         // 256-position tiles
-  int *nsmall, *small_e, *small_m0;   // the remainders of up to 128 positions
-  int *nmix, *mix_e, *mix_m0;         // both, in expert order (expert | 1 << 30 for a 256-position tile)
-  int *ord_e, *ord_m0;                // both (nmix of them), the experts by falling count (see k_pf_scan)
+  int *ntiles, *tile_e, *tile_m0;  // tiles of kTile positions: the bf16-activation kernels'
+  int *nwide, *wide_e, *wide_m0;   // tiles of pf8::kMaxPos positions: the FP8-activation kernels'
+  int *ord_e, *ord_m0;             // the latter (nwide of them) in the order asked for (below)
 };
 __global__ void __launch_bounds__(DSGX_MAX_EXPERTS) k_pf_scan(const int* __restrict__ bcnt, int NB, int E, int* __restrict__ boff,
                                                               int* __restrict__ cnt, int* __restrict__ off, TileLists tl, int order) {
-  __shared__ int sa[DSGX_MAX_EXPERTS], sb[DSGX_MAX_EXPERTS], sc[DSGX_MAX_EXPERTS], sd[DSGX_MAX_EXPERTS];
+  __shared__ int sa[DSGX_MAX_EXPERTS], sb[DSGX_MAX_EXPERTS], sc[DSGX_MAX_EXPERTS];
   const int e = threadIdx.x;
   int c = 0;
   if (e < E) {
@@ -162,86 +157,70 @@ __global__ void __launch_bounds__(DSGX_MAX_EXPERTS) k_pf_scan(const int* __restr
       c += v;
     }
   }
-  const int nt = (c + kTile - 1) / kTile;
-  const int rem = c % 256, nbig = c / 256 + (rem > 128 ? 1 : 0), nsmall = rem > 0 && rem <= 128 ? 1 : 0;
-  sa[e] = e < E ? c : 0, sb[e] = e < E ? nt : 0, sc[e] = e < E ? nbig : 0, sd[e] = e < E ? nsmall : 0;
+  constexpr int kWide = pf8::kMaxPos;
+  const int nt = (c + kTile - 1) / kTile, nw = (c + kWide - 1) / kWide;
+  sa[e] = e < E ? c : 0, sb[e] = e < E ? nt : 0, sc[e] = e < E ? nw : 0;
   __syncthreads();
   for (int d = 1; d < DSGX_MAX_EXPERTS; d <<= 1) {  // inclusive scans of the counts and of the tile counts
-    const int va = e >= d ? sa[e - d] : 0, vb = e >= d ? sb[e - d] : 0, vc = e >= d ? sc[e - d] : 0, vd = e >= d ? sd[e - d] : 0;
+    const int va = e >= d ? sa[e - d] : 0, vb = e >= d ? sb[e - d] : 0, vc = e >= d ? sc[e - d] : 0;
     __syncthreads();
-    sa[e] += va, sb[e] += vb, sc[e] += vc, sd[e] += vd;
+    sa[e] += va, sb[e] += vb, sc[e] += vc;
     __syncthreads();
   }
   if (e < E) {
     cnt[e] = c;
     off[e] = sa[e] - c;
-    if (e == E - 1) off[E] = sa[e], *tl.ntiles = sb[e], *tl.nbig = sc[e], *tl.nsmall = sd[e];
-    const int t0 = sb[e] - nt;
+    if (e == E - 1) off[E] = sa[e], *tl.ntiles = sb[e], *tl.nwide = sc[e];
+    const int t0 = sb[e] - nt, w0 = sc[e] - nw;
     for (int i = 0; i < nt; ++i) tl.tile_e[t0 + i] = e, tl.tile_m0[t0 + i] = i * kTile;
-    const int b0 = sc[e] - nbig;
-    for (int i = 0; i < nbig; ++i) tl.big_e[b0 + i] = e, tl.big_m0[b0 + i] = i * 256;
-    if (nsmall) tl.small_e[sd[e] - 1] = e, tl.small_m0[sd[e] - 1] = (c / 256) * 256;
+    for (int i = 0; i < nw; ++i) tl.wide_e[w0 + i] = e, tl.wide_m0[w0 + i] = i * kWide;
+    if (!order)  // (the last list is always a valid one: a later call may name it whatever this call was told)
+      for (int i = 0; i < nw; ++i) tl.ord_e[w0 + i] = e, tl.ord_m0[w0 + i] = i * kWide;
   }
-  __syncthreads();
-  const int nb = sc[DSGX_MAX_EXPERTS - 1], nsm = sd[DSGX_MAX_EXPERTS - 1];
-  // The merged list, in expert order: an expert's 256-position tiles, then its remainder. Neighbours in the list run at
-  // about the same time on one XCD (pf8::task_of), so part of what an expert's tiles stream, each in full, comes out of
-  // that XCD's L2: 12% fewer bytes from HBM for gate/up, 19% for down, than with the remainders spread evenly among the
-  // big tiles (measured; the time differs by 1% only: the stream is not what bounds these launches).
-  if (e < E) {
-    const int p0 = (sc[e] - nbig) + (sd[e] - nsmall);
-    for (int i = 0; i < nbig; ++i) tl.mix_e[p0 + i] = e | (1 << 30), tl.mix_m0[p0 + i] = i * 256;
-    if (nsmall) tl.mix_e[p0 + nbig] = e, tl.mix_m0[p0 + nbig] = (c / 256) * 256;
-    if (!order) {  // (the second list is always a valid one: a later call may name it whatever this call was told)
-      for (int i = 0; i < nbig; ++i) tl.ord_e[p0 + i] = e | (1 << 30), tl.ord_m0[p0 + i] = i * 256;
-      if (nsmall) tl.ord_e[p0 + nbig] = e, tl.ord_m0[p0 + nbig] = (c / 256) * 256;
-    }
-  }
-  if (e == 0) *tl.nmix = nb + nsm;
-  // The same tiles in the order of the reference's prefill_tuning tord (ds41f-4xgx10-switchless/engine/kernels/prefill.cu:
+  // The wide tiles in the order of the reference's prefill_tuning tord (ds41f-4xgx10-switchless/engine/kernels/prefill.cu:
   // 658-668: the most-picked experts' tiles with those of the least-picked between them): the experts by falling count
-  // (ties by id), their 256-position tiles as one list B and their remainders as one list S, merged so that both lists
+  // (ties by id), their full tiles as one list B and their remainders as one list S, merged so that both lists
   // run out together (B's tile k at key (k + 1/2) / |B|, S's tile j at (j + 1/2) / |S|, by rising key, B first on a tie).
-  // A 256-position tile is bound by the matrix unit and a remainder by the weight stream, so at any time the chip runs
-  // a mix of the two. The order of the sums does not depend on the list's order.
+  // The order of the sums does not depend on the list's order.
   if (!order) return;  // (the same for every thread)
+  const int full = c / kWide, part = c % kWide;
   __syncthreads();
   sa[e] = e < E ? c : -1;
   __syncthreads();
   int rank = 0, rank2 = 0;  // by falling count; by falling remainder (order 2's list of remainders)
   {
-    const int ce = e < E ? c : -1, re = (e < E && nsmall) ? rem : -1;
+    const int ce = e < E ? c : -1, re = (e < E && part) ? part : -1;
     for (int j = 0; j < DSGX_MAX_EXPERTS; ++j) {
       const int cj = sa[j];
-      const int rj = (cj >= 0 && cj % 256 > 0 && cj % 256 <= 128) ? cj % 256 : -1;
+      const int rj = (cj >= 0 && cj % kWide > 0) ? cj % kWide : -1;
       rank += (cj > ce) || (cj == ce && j < e);
       rank2 += (rj > re) || (rj == re && j < e);
     }
   }
   __syncthreads();
-  sb[rank] = e < E ? nbig : 0, sd[order == 2 ? rank2 : rank] = e < E ? nsmall : 0;
+  sb[rank] = e < E ? full : 0, sc[order == 2 ? rank2 : rank] = e < E && part ? 1 : 0;
   __syncthreads();
   for (int d = 1; d < DSGX_MAX_EXPERTS; d <<= 1) {  // inclusive scans in rank order
-    const int vb = e >= d ? sb[e - d] : 0, vd = e >= d ? sd[e - d] : 0;
+    const int vb = e >= d ? sb[e - d] : 0, vc = e >= d ? sc[e - d] : 0;
     __syncthreads();
-    sb[e] += vb, sd[e] += vd;
+    sb[e] += vb, sc[e] += vc;
     __syncthreads();
   }
   if (e < E) {
-    const long long NB_ = nb, NS_ = nsm;
-    const int k0 = sb[rank] - nbig, j0 = sd[order == 2 ? rank2 : rank] - nsmall;
-    for (int i = 0; i < nbig; ++i) {
+    const long long NB_ = sb[DSGX_MAX_EXPERTS - 1], NS_ = sc[DSGX_MAX_EXPERTS - 1];
+    const int k0 = sb[rank] - full, j0 = sc[order == 2 ? rank2 : rank] - (part ? 1 : 0);
+    for (int i = 0; i < full; ++i) {
       const long long k = k0 + i;
       long long before = NS_ ? ((2 * k + 1) * NS_ + NB_ - 1) / (2 * NB_) : 0;  // S tiles of a key below this one's
       if (before > NS_) before = NS_;
-      if (order == 2) before = 0;  // every 256-position tile before every remainder
-      tl.ord_e[k + before] = e | (1 << 30), tl.ord_m0[k + before] = i * 256;
+      if (order == 2) before = 0;  // every full tile before every remainder
+      tl.ord_e[k + before] = e, tl.ord_m0[k + before] = i * kWide;
     }
-    if (nsmall) {
+    if (part) {
       const long long j = j0;
       long long before = NB_ ? ((2 * j + 1) * NB_ + NS_) / (2 * NS_) : 0;      // B tiles of a key up to this one's
       if (before > NB_ || order == 2) before = NB_;
-      tl.ord_e[j + before] = e, tl.ord_m0[j + before] = (c / 256) * 256;
+      tl.ord_e[j + before] = e, tl.ord_m0[j + before] = full * kWide;
     }
   }
 }
@@ -767,8 +746,7 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
     const int NB = (T + kRowBlock - 1) / kRowBlock;
     uint32_t* bmask = reinterpret_cast<uint32_t*>(W + o.bmask);
     hipLaunchKernelGGL(k_pf_mask, dim3(NB), dim3(256), 0, st, idx, T, topk, E, I32(o.bcnt), bmask);
-    const TileLists tl{I32(o.ntiles), I32(o.tile_e), I32(o.tile_m0), I32(o.nbig), I32(o.big_e), I32(o.big_m0), I32(o.nsmall), I32(o.small_e), I32(o.small_m0),
-                       I32(o.nmix), I32(o.mix_e), I32(o.mix_m0), I32(o.ord_e), I32(o.ord_m0)};
+    const TileLists tl{I32(o.ntiles), I32(o.tile_e), I32(o.tile_m0), I32(o.nwide), I32(o.wide_e), I32(o.wide_m0), I32(o.ord_e), I32(o.ord_m0)};
     hipLaunchKernelGGL(k_pf_scan, dim3(1), dim3(DSGX_MAX_EXPERTS), 0, st, I32(o.bcnt), NB, E, I32(o.boff), I32(o.cnt), I32(o.off), tl, order);
     hipLaunchKernelGGL(k_pf_place, dim3(NB), dim3(256), 0, st, idx, w, T, topk, E, I32(o.off), I32(o.boff), bmask, L->desc, I32(o.perm),
                        I32(o.pickpos), I32(o.rpos), I32(o.re), F32(o.rk), (float*)nullptr);
@@ -838,48 +816,51 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
     return DSGX_OK;
   }
   // FP8 activations: x quantised -> gate/up + SwiGLU (h bf16 for the view, and quantised for the down projection in the
-  // same kernel) -> down (f32 a pick) -> ordered combine. Every GEMM runs twice: the 256-position tiles, then the
-  // experts' remainders of up to 128 positions.
+  // same kernel) -> down (f32 a pick) -> ordered combine.
   if (H > 8192 || I > 8192) return fail(DSGX_EUNSUPPORTED, "moe_prefill: FP8 activations: hidden %d, intermediate %d (up to 8192)", H, I);
-  void (*k_up)(pf8::Args) = pf8::k_gemm_mixed<true>;    // the routed experts: the merged list of both tile shapes
+  void (*k_up)(pf8::Args) = pf8::k_gemm_mixed<true>;  // the routed experts (and the shared one's tiles)
   void (*k_dn)(pf8::Args) = pf8::k_gemm_mixed<false>;
-  void (*k_up2)(pf8::Args) = pf8::k_gemm<true, 2>;      // the shared expert: 256-position tiles
-  void (*k_dn2)(pf8::Args) = pf8::k_gemm<false, 2>;
-  constexpr int kLdsMix = pf8::Shape<1>::kLds > pf8::Shape<2>::kLds ? pf8::Shape<1>::kLds : pf8::Shape<2>::kLds;
+  void (*k_up2)(pf8::Args) = pf8::k_gemm<true>;        // the shared expert alone
+  void (*k_dn2)(pf8::Args) = pf8::k_gemm<false>;
   for (const void* k : {(const void*)k_up, (const void*)k_dn})
-    if (int rc = allow_dynamic_lds(k, kLdsMix)) return rc;
+    if (int rc = allow_dynamic_lds(k, pf8::kLds)) return rc;
   for (const void* k : {(const void*)k_up2, (const void*)k_dn2})
-    if (int rc = allow_dynamic_lds(k, pf8::Shape<2>::kLds)) return rc;
+    if (int rc = allow_dynamic_lds(k, pf8::kLds)) return rc;
   pf8::Args g{};
   g.L = *L;
+  // Which workgroups share an XCD. Few rows an expert: eight row groups of one tile, an expert is a tile and the chip is even in small
+  // blocks; many rows: eight tiles x four row groups, so that an expert's tiles find its weights in L2. 4096 x 2048, 256 experts, top-8,
+  // 1 x 8 / 8 x 4: T = 20 340 / 358 us, T = 200 991 / 1019, T = 700 1271 / 1313, T = 1500 1432 / 1440, T = 3000 1715 / 1716, T = 5000
+  // 2115 / 2106, T = 8192 2844 / 2814 (other shapes of 1 to 8 tiles x 1 to 32 groups lie between or above).
+  auto map_for = [&](int NS) { return (long long)P >= 94LL * E ? pf8::map_of(3, 2, NS) : pf8::map_of(0, 3, NS); };
   g.fast_act = cfg.fast_act;
 #ifdef DSGX_PF_TRACE
   if (const char* tp = std::getenv("DSGX_PF_TRACE_PTR")) g.trace = reinterpret_cast<unsigned long long*>(std::strtoull(tp, nullptr, 0));
 #endif
   const int NSU = I / (pf8::kWgRows / 2), NSD = H / pf8::kWgRows;
   const bool mixed = order >= 1;
-  g.tile_e = I32(mixed ? o.ord_e : o.mix_e), g.tile_m0 = I32(mixed ? o.ord_m0 : o.mix_m0), g.ntiles = I32(o.nmix), g.off = I32(o.off), g.nrows = T;
+  g.tile_e = I32(mixed ? o.ord_e : o.wide_e), g.tile_m0 = I32(mixed ? o.ord_m0 : o.wide_m0), g.ntiles = I32(o.nwide), g.off = I32(o.off), g.nrows = T;
   // A whole step runs the shared expert's tiles in the routed experts' launches, in front of them: alone they are a launch
-  // of T / 256 x 16 workgroups, a sixteenth of the chip at T = 200, and two more tails (whole call, hidden 4096, intermediate
+  // of few workgroups at small T, and two more tails (as kernels of eight waves, whole call, hidden 4096, intermediate
   // 2048, 256 experts: T = 17 387 -> 341 us, T = 200 1061 -> 973, T = 2000 1565 -> 1544, T = 8192 within the noise; same bits).
-  const int sh_tiles = (T + 255) / 256;
+  const int sh_tiles = (T + pf8::kMaxPos - 1) / pf8::kMaxPos;
   const bool fused_sh = shared && (cfg.phases & (2 | 4 | 16)) == (2 | 4 | 16);
   if (cfg.phases & (2 | 16)) {
     if (int rc = dsgx_act_quant(x, T, H, W + o.xq, F32(o.xs), stream)) return rc;
   }
   if (cfg.phases & 2) {
-    g.aq = W + o.xq, g.as = F32(o.xs), g.gather = I32(o.perm);
+    g.aq = W + o.xq, g.as = F32(o.xs), g.gather = I32(o.perm), g.map = map_for(NSU);
     g.h = reinterpret_cast<uint16_t*>(W + o.h), g.hq = W + o.hq, g.hs = F32(o.hs), g.d = nullptr;
     if (fused_sh)
-      g.sh = pf8::SharedRows{pf8::grid_of(sh_tiles, NSU), W + o.xq, F32(o.xs), reinterpret_cast<uint16_t*>(W + o.hsh), W + o.hshq, F32(o.hshs), nullptr};
-    hipLaunchKernelGGL(k_up, dim3(g.sh.grid + pf8::grid_of(o.max_big + E, NSU)), dim3(pf8::kThreads), kLdsMix, st, g);
+      g.sh = pf8::SharedRows{pf8::grid_of(sh_tiles, NSU, g.map), W + o.xq, F32(o.xs), reinterpret_cast<uint16_t*>(W + o.hsh), W + o.hshq, F32(o.hshs), nullptr};
+    hipLaunchKernelGGL(k_up, dim3(g.sh.grid + pf8::grid_of(o.max_wide, NSU, g.map)), dim3(pf8::kThreads4), pf8::kLds, st, g);
     DSGX_HIP(hipGetLastError());
   }
   if (cfg.phases & 4) {
-    g.aq = W + o.hq, g.as = F32(o.hs), g.gather = nullptr;
+    g.aq = W + o.hq, g.as = F32(o.hs), g.gather = nullptr, g.map = map_for(NSD);
     g.h = nullptr, g.hq = nullptr, g.hs = nullptr, g.d = F32(o.d);
-    if (fused_sh) g.sh = pf8::SharedRows{pf8::grid_of(sh_tiles, NSD), W + o.hshq, F32(o.hshs), nullptr, nullptr, nullptr, ys};
-    hipLaunchKernelGGL(k_dn, dim3(g.sh.grid + pf8::grid_of(o.max_big + E, NSD)), dim3(pf8::kThreads), kLdsMix, st, g);
+    if (fused_sh) g.sh = pf8::SharedRows{pf8::grid_of(sh_tiles, NSD, g.map), W + o.hshq, F32(o.hshs), nullptr, nullptr, nullptr, ys};
+    hipLaunchKernelGGL(k_dn, dim3(g.sh.grid + pf8::grid_of(o.max_wide, NSD, g.map)), dim3(pf8::kThreads4), pf8::kLds, st, g);
     DSGX_HIP(hipGetLastError());
   }
   if (cfg.phases & 8) {
@@ -891,9 +872,9 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
     g.tile_e = g.tile_m0 = g.ntiles = g.off = nullptr;
     g.aq = W + o.xq, g.as = F32(o.xs), g.gather = nullptr;
     g.h = reinterpret_cast<uint16_t*>(W + o.hsh), g.hq = W + o.hshq, g.hs = F32(o.hshs), g.d = nullptr;
-    hipLaunchKernelGGL(k_up2, dim3(pf8::grid_of(tiles, NSU)), dim3(pf8::kThreads), pf8::Shape<2>::kLds, st, g);
+    hipLaunchKernelGGL(k_up2, dim3(pf8::grid_of(tiles, NSU)), dim3(pf8::kThreads4), pf8::kLds, st, g);
     g.aq = W + o.hshq, g.as = F32(o.hshs), g.h = nullptr, g.hq = nullptr, g.hs = nullptr, g.d = ys;
-    hipLaunchKernelGGL(k_dn2, dim3(pf8::grid_of(tiles, NSD)), dim3(pf8::kThreads), pf8::Shape<2>::kLds, st, g);
+    hipLaunchKernelGGL(k_dn2, dim3(pf8::grid_of(tiles, NSD)), dim3(pf8::kThreads4), pf8::kLds, st, g);
     DSGX_HIP(hipGetLastError());
   }
   return DSGX_OK;
@@ -989,18 +970,14 @@ int dsgx_dsk_moe_prefill(const dsgx_dsk_weights* Wt, const uint8_t* xq, const ui
   auto F32 = [&](size_t off) { return reinterpret_cast<float*>(W + off); };
   auto U16 = [&](size_t off) { return reinterpret_cast<uint16_t*>(W + off); };
   const int H = Wt->H, I = Wt->I, E = Wt->E, topk = Wt->topk, P = o.P;
-  constexpr int F4 = DSGX_FMT_MXFP4_G32, F8 = DSGX_FMT_FP8_B32E;
-  constexpr int kLdsSh = std::max({pfmx::Shape<256, F8>::kLds, pfmx::Shape<128, F8>::kLds, pfmx::Shape<64, F8>::kLds});
-  constexpr int kLdsRun = std::max({kLdsSh, pfmx::Shape<256, F4>::kLds, pfmx::Shape<128, F4>::kLds, pfmx::Shape<64, F4>::kLds});  // (a routed launch may hold the shared expert's tiles)
-  static_assert(kLdsRun <= 160 * 1024, "a workgroup's LDS");
   void (*k_up)(pfmx::Args) = pfmx::k_gemm_mixed<true>;
   void (*k_dn)(pfmx::Args) = pfmx::k_gemm_mixed<false>;
   void (*k_sup)(pfmx::Args) = pfmx::k_gemm<true>;
   void (*k_sdn)(pfmx::Args) = pfmx::k_gemm<false>;
   for (const void* k : {(const void*)k_up, (const void*)k_dn})
-    if (int rc = allow_dynamic_lds(k, kLdsRun)) return rc;
+    if (int rc = allow_dynamic_lds(k, pfmx::kLds)) return rc;
   for (const void* k : {(const void*)k_sup, (const void*)k_sdn})
-    if (int rc = allow_dynamic_lds(k, kLdsSh)) return rc;
+    if (int rc = allow_dynamic_lds(k, pfmx::kLds)) return rc;
   const int NSU = I / (pf8::kWgRows / 2), NSD = H / pf8::kWgRows;
   uint16_t* dsh = U16(o.d + align256((size_t)P * H * 2));  // the shared expert's outputs behind the picks', both bf16
   // phases (dsk::MoePCfg, dsk.h:278-282): 1 bucketing, 2 shared expert, 4 routed up, 8 routed down, 16 combine
@@ -1008,8 +985,7 @@ int dsgx_dsk_moe_prefill(const dsgx_dsk_weights* Wt, const uint8_t* xq, const ui
     const int NB = (T + kRowBlock - 1) / kRowBlock;
     uint32_t* bmask = reinterpret_cast<uint32_t*>(W + o.bmask);
     hipLaunchKernelGGL(k_pf_mask, dim3(NB), dim3(256), 0, st, idx, T, topk, E, I32(o.bcnt), bmask);
-    const TileLists tl{I32(o.ntiles), I32(o.tile_e), I32(o.tile_m0), I32(o.nbig), I32(o.big_e), I32(o.big_m0), I32(o.nsmall), I32(o.small_e), I32(o.small_m0),
-                       I32(o.nmix), I32(o.mix_e), I32(o.mix_m0), I32(o.ord_e), I32(o.ord_m0)};
+    const TileLists tl{I32(o.ntiles), I32(o.tile_e), I32(o.tile_m0), I32(o.nwide), I32(o.wide_e), I32(o.wide_m0), I32(o.ord_e), I32(o.ord_m0)};
     hipLaunchKernelGGL(k_pf_scan, dim3(1), dim3(DSGX_MAX_EXPERTS), 0, st, I32(o.bcnt), NB, E, I32(o.boff), I32(o.cnt), I32(o.off), tl, 0);
     hipLaunchKernelGGL(k_pf_place, dim3(NB), dim3(256), 0, st, idx, w, T, topk, E, I32(o.off), I32(o.boff), bmask, (const dsgx_mat_desc*)nullptr, I32(o.perm),
                        I32(o.pickpos), I32(o.rpos), I32(o.re), F32(o.rk), F32(o.posw));
@@ -1017,40 +993,43 @@ int dsgx_dsk_moe_prefill(const dsgx_dsk_weights* Wt, const uint8_t* xq, const ui
   }
   pfmx::Args g{};
   g.H = H, g.I = I, g.nrows = T, g.limit = cfg.swiglu_limit;
+  // (as for the FP8 layers; 1 tile x 2 / 4 x 2, T = 20
+  // 237 / 246 us, T = 60 411 / 419, T = 300 803 / 812, T = 1000 1076 / 1078, T = 2000 1267 / 1245, T = 6000 2103 / 2015)
+  auto map_for = [&](int NS) { return (long long)P >= 24LL * E ? pf8::map_of(2, 1, NS) : pf8::map_of(0, 1, NS); };
   // a whole step runs the shared expert's tiles in the routed experts' launches, in front of them (as the FP8 layers do;
   // hidden 5120, intermediate 2304, T = 17: 417 -> 362 us, T = 600: 1405 -> 1334, T = 3000: 1870 -> 1821)
-  const int sh_tiles = (T + 255) / 256;
+  const int sh_tiles = (T + 127) / 128;
   const bool fused_sh = shared && (cfg.phases & (2 | 4 | 8)) == (2 | 4 | 8);
   if ((cfg.phases & 2) && shared && !fused_sh) {
     const int tiles = sh_tiles;
     g.tile_e = g.tile_m0 = g.ntiles = g.off = nullptr, g.gather = nullptr, g.posw = nullptr, g.wstride = g.sstride = 0;
     g.aq = xq, g.as = xs, g.wa = Wt->sh_w1, g.sa = Wt->sh_s1, g.wb = Wt->sh_w3, g.sb = Wt->sh_s3;
     g.h = U16(o.hsh), g.hq = W + o.hshq, g.hs = W + o.hshs, g.d = nullptr;
-    hipLaunchKernelGGL(k_sup, dim3(pf8::grid_of(tiles, NSU)), dim3(pf8::kThreads), kLdsSh, st, g);
+    hipLaunchKernelGGL(k_sup, dim3(pf8::grid_of(tiles, NSU)), dim3(pf8::kThreads4), pfmx::kLds, st, g);
     g.aq = W + o.hshq, g.as = W + o.hshs, g.wa = Wt->sh_w2, g.sa = Wt->sh_s2, g.wb = g.sb = nullptr;
     g.h = nullptr, g.hq = g.hs = nullptr, g.d = dsh;
-    hipLaunchKernelGGL(k_sdn, dim3(pf8::grid_of(tiles, NSD)), dim3(pf8::kThreads), kLdsSh, st, g);
+    hipLaunchKernelGGL(k_sdn, dim3(pf8::grid_of(tiles, NSD)), dim3(pf8::kThreads4), pfmx::kLds, st, g);
     DSGX_HIP(hipGetLastError());
   }
-  g.tile_e = I32(o.mix_e), g.tile_m0 = I32(o.mix_m0), g.ntiles = I32(o.nmix), g.off = I32(o.off);
+  g.tile_e = I32(o.wide_e), g.tile_m0 = I32(o.wide_m0), g.ntiles = I32(o.nwide), g.off = I32(o.off);
   auto launch = [&](bool up) {
-    hipLaunchKernelGGL(up ? k_up : k_dn, dim3(g.sh.grid + pf8::grid_of(o.max_big + E, up ? NSU : NSD)), dim3(pf8::kThreads), kLdsRun, st, g);
+    hipLaunchKernelGGL(up ? k_up : k_dn, dim3(g.sh.grid + pf8::grid_of(o.max_wide, up ? NSU : NSD, g.map)), dim3(pf8::kThreads4), pfmx::kLds, st, g);
   };
   if (cfg.phases & 4) {
-    g.aq = xq, g.as = xs, g.gather = I32(o.perm), g.posw = F32(o.posw);
+    g.aq = xq, g.as = xs, g.gather = I32(o.perm), g.posw = F32(o.posw), g.map = map_for(NSU);
     g.wa = Wt->w1, g.sa = Wt->s1, g.wb = Wt->w3, g.sb = Wt->s3, g.wstride = (size_t)I * H / 2, g.sstride = (size_t)I * H / 32;
     g.h = U16(o.h), g.hq = W + o.hq, g.hs = W + o.hs, g.d = nullptr;
     if (fused_sh)
-      g.sh = pfmx::SharedRows{pf8::grid_of(sh_tiles, NSU), xq, xs, Wt->sh_w1, Wt->sh_s1, Wt->sh_w3, Wt->sh_s3, U16(o.hsh), W + o.hshq, W + o.hshs, nullptr};
+      g.sh = pfmx::SharedRows{pf8::grid_of(sh_tiles, NSU, g.map), xq, xs, Wt->sh_w1, Wt->sh_s1, Wt->sh_w3, Wt->sh_s3, U16(o.hsh), W + o.hshq, W + o.hshs, nullptr};
     launch(true);
     DSGX_HIP(hipGetLastError());
   }
   if (cfg.phases & 8) {
-    g.aq = W + o.hq, g.as = W + o.hs, g.gather = nullptr, g.posw = nullptr;
+    g.aq = W + o.hq, g.as = W + o.hs, g.gather = nullptr, g.posw = nullptr, g.map = map_for(NSD);
     g.wa = Wt->w2, g.sa = Wt->s2, g.wb = g.sb = nullptr, g.wstride = (size_t)I * H / 2, g.sstride = (size_t)I * H / 32;
     g.h = nullptr, g.hq = g.hs = nullptr, g.d = U16(o.d);
     if (fused_sh)
-      g.sh = pfmx::SharedRows{pf8::grid_of(sh_tiles, NSD), W + o.hshq, W + o.hshs, Wt->sh_w2, Wt->sh_s2, nullptr, nullptr, nullptr, nullptr, nullptr, dsh};
+      g.sh = pfmx::SharedRows{pf8::grid_of(sh_tiles, NSD, g.map), W + o.hshq, W + o.hshs, Wt->sh_w2, Wt->sh_s2, nullptr, nullptr, nullptr, nullptr, nullptr, dsh};
     launch(false);
     DSGX_HIP(hipGetLastError());
   }

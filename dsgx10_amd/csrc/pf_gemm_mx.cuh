@@ -20,44 +20,41 @@ namespace dsgx {
 namespace pfmx {
 
 using pf8::dma16;
-using pf8::dma4;
-using pf8::kThreads;
+using pf8::kMaxPos;
+using pf8::kThreads4;
+using pf8::kWaves;
 using pf8::kWgRows;
+using pf8::sc_half;
+using pf8::static_for;
 using pf8::sw4;
 using pf8::swz;
 using pf8::v4f_t;
 using pf8::v8i_t;
 using pf8::wait_loads;
 
-// A tile's shape by its positions (64, 128 or 256) and its weights' format. What a turn waits for is the way of its operands into
-// LDS, and there the lines that a load instruction names count as much as its bytes (hidden 5120, intermediate 2304, 256
-// experts of 32 rows each, gate/up 895 us before):
-//   * a scale word of 4 bytes a row and block named 32 lines for 128 bytes; e2m1 experts' scale words therefore come for four
-//     blocks at a time, 16 bytes a row, into two buffers of their own (with no scale loads at all 640 us, with those a
-//     block 729 with coalesced stand-ins); e4m3 rows share a word by 32 and keep theirs with the block;
-//   * half a line a weight row and block (e2m1: 64 bytes) named every line twice: tiles of up to 64 positions, whose weights are
-//     most of their bytes, take two blocks a turn and whole lines (the larger shapes: 2% at 192 rows an expert, and LDS holds
-//     three stages of one block only).
-// Together 895 -> 693 us; the whole call at T = 3000 (Zipf) 1777 -> 1546, at T = 300 1115 -> 878. Four to eight stages instead of
-// three return nothing, two cost 15%.
-template <int POS, int WF>
+// A tile's shape by its positions (32, 64 or 160; the shared expert's 64 or 128), its weights' format and the blocks of a turn.
+// What bounds these launches is what L2 does not hold, at 5.5 TB/s (hidden 5120, intermediate 2304, 256 experts, top-6, T = 3000:
+// gate/up 5.7 GB of missed lines in 1.02 ms, 3.2 of them weights and their scales once), and tiles of few rows:
+//   * two workgroups of four waves a CU (pf_gemm_fp8.cuh): whole call T = 60 / 300 / 3000 474 / 882 / 1537 -> 435 / 830 / 1470 us;
+//   * half a line a weight row and block (e2m1: 64 bytes) names every line twice: tiles of up to 64 positions take two blocks a
+//     turn, whole lines;
+//   * a line of scale words is a row's for 32 blocks and has left L2 when its next words are asked for: with four blocks' words a
+//     load scale words were 1.25 of the 5.7 GB; eight a load (the weight rows' in ONE buffer, which the wave frees by reading it) 5.3
+//     GB, gate/up 1022 -> 989 us;
+//   * an expert of many rows reads its weights once a tile: 160 positions instead of 128 (T = 2000 / 6000 1280 -> 1246, 2100 -> 2013).
+template <int POS, int WF, int TB_>
 struct Shape {
   static constexpr bool F4 = WF == DSGX_FMT_MXFP4_G32;
-  static constexpr int WP = POS == 256 ? 2 : 1;     // position groups of waves
-  static constexpr int kPos = POS, kSub = POS / 16, WR = 8 / WP, RA = 2 * WP;
-  static constexpr int TB = F4 && POS <= 64 ? 2 : 1;  // 128-k blocks a turn
+  static constexpr int kPos = POS, kSub = POS / 16, RA = 4, TB = TB_;
   static constexpr int kRowB = F4 ? 64 * TB : 128;  // bytes of a weight row in a turn
-  static constexpr int kStageW = kWgRows * kRowB;
-  static constexpr int kStageX = kPos * 128;        // one block's activations
-  static constexpr int kStageBytes = kStageW + TB * kStageX;
-  static constexpr int kWords = F4 ? 4 : 1;         // blocks whose scale words come together
-  static constexpr int kGroupW = kWgRows * 4 * kWords, kGroupX = kPos * 4 * kWords;  // their scale words: the weight rows', the positions'
-  static constexpr int kGroup = kGroupW + kGroupX, kGroups = F4 ? 2 : 3;  // (e4m3: a buffer a stage)
-  static constexpr int kStages = 3 * kStageBytes + kGroups * kGroup <= 160 * 1024 ? 3 : 2;
-  static constexpr int kLoadsW = kRowB == 64 ? 2 : 4;       // a wave's loads a turn: its two weight tiles ...
-  static constexpr int kHalfX = kPos / 64;                  // ... and its half tiles of eight positions, a load a block
-  static constexpr int kLoads = kLoadsW + TB * kHalfX + (F4 ? 0 : 2);  // (e4m3: and its two loads of scale words)
-  static constexpr int kLds = kStages * kStageBytes + kGroups * kGroup;  // (the epilogues reuse it: UP kPos x 256 B, DOWN 8 x 2 WP KiB)
+  static constexpr int kTileB = 16 * kRowB, LT = kRowB / 64;  // a 16-row weight tile, its loads
+  static constexpr int kRing = F4 ? (TB == 1 ? 5 : POS == 32 ? 6 : 4) : POS == 128 ? 4 : 6;  // the wave's own ring of weight tiles
+  static constexpr int kStageX = POS * 128;         // one block's activations; two stages of TB blocks
+  static constexpr int kHX = POS / 8 / kWaves;      // the 8-position half tiles that a wave brings
+  static constexpr int kOffX = kWaves * kRing * kTileB, kOffS = kOffX + 2 * TB * kStageX;
+  static constexpr int kScaleW = kWgRows * 32, kScaleX = POS * 32;  // eight blocks' scale words of the weight rows, and of the positions (two such buffers)
+  static constexpr int kOffSX = kOffS + kScaleW, kLds = kOffSX + 2 * kScaleX;   // (the epilogues reuse it: UP kPos x 256 B, DOWN 4 x 2 KiB)
+  static_assert(F4 || TB == 1, "pairs of blocks are for 64-byte rows");
 };
 
 // The shared expert's side of a launch that holds its tiles too (k_gemm_mixed): the first `grid` workgroups are theirs
@@ -72,7 +69,8 @@ struct Args {
   const uint8_t* aq;   // activations, e4m3 [rows][K]
   const uint8_t* as;   // their ue8m0 scales [rows][K / 32]
   const int* gather;   // position -> activation row (null: the position itself)
-  const int* tile_e;   // the tile list (null: the shared expert on rows [0, nrows))
+  const int* tile_e;   // the list of tiles of kMaxPos positions (null: the shared expert on rows [0, nrows))
+  pf8::Map map;
   const int* tile_m0;
   const int* ntiles;
   const int* off;
@@ -101,11 +99,10 @@ __device__ __forceinline__ v4f_t mfma_mx(v8i_t a, v8i_t b, v4f_t c, int sa, int 
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, CBSZ, 0, 0, sa, 0, sb);
 }
 
-template <bool UP, int POS, int WF>
+template <bool UP, int POS, int WF, int TB>
 __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, int m0, int mend, int ns) {
-  using S = Shape<POS, WF>;
+  using S = Shape<POS, WF, TB>;
   constexpr bool F4 = S::F4;
-  constexpr int WP = S::WP, kPosWave = S::kPos / 8;
   constexpr int CBSZ = F4 ? 4 : 0;
   const int K = UP ? g.H : g.I, KB = K / 128, G = K / 32;
   if (mend > m0 + S::kPos) mend = m0 + S::kPos;
@@ -113,106 +110,115 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   const uint8_t *wa = g.wa + eo * g.wstride, *sa = g.sa + eo * g.sstride;
   const uint8_t *wb = UP ? g.wb + eo * g.wstride : wa, *sb = UP ? g.sb + eo * g.sstride : sa;
   const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6), r16 = lane & 15, part = lane >> 4;
-  const int rg = wave % S::WR, pg = wave / S::WR;
   const int c0 = ns * (kWgRows / 2), r0 = ns * kWgRows;
-  auto tile_row = [&](int i, const uint8_t*& wbase, const uint8_t*& sbase) {  // first weight row of 16-row tile i, its tensors
-    if (UP) {
-      wbase = (i & 1) ? wb : wa, sbase = (i & 1) ? sb : sa;
-      return c0 + 16 * (i >> 1);
-    }
-    wbase = wa, sbase = sa;
-    return r0 + 16 * i;
-  };
+  // The workgroup's sixteen 16-row tiles, four a wave: first weight row of tile i. UP: tile 2 c is the gate rows, tile 2 c + 1 the
+  // up rows of channels c0 + 16 c ...
+  auto tile_row = [&](int i) { return UP ? c0 + 16 * (i >> 1) : r0 + 16 * i; };
+  const int RB = F4 ? K / 2 : K;  // bytes of a weight row
+  const uint8_t* wt[S::RA];
+#pragma unroll
+  for (int t = 0; t < S::RA; ++t) wt[t] = (UP && (t & 1) ? wb : wa) + (size_t)tile_row(S::RA * wave + t) * RB;
   const int nmt = uni(min(S::kSub, (mend - m0 + 15) / 16));
-  const int nj = uni(nmt > pg ? (nmt - pg + WP - 1) / WP : 0);
   // ---- what this lane fetches ----
-  // weights: the wave brings tiles 2 wave, 2 wave + 1. 64-byte rows: one instruction a tile, lane -> row lane / 4, piece
-  // (lane % 4) ^ sw4(row); 128-byte rows: two instructions a tile (rows 0-7, 8-15), lane -> row lane / 8, piece (lane % 8) ^
+  // weights: 64-byte rows: one instruction a tile, lane -> row lane / 4, piece (lane % 4) ^ sw4(row); 128-byte rows: two
+  // instructions a tile (rows 0-7, 8-15), lane -> row lane / 8, piece (lane % 8) ^
   // swz(row) (e4m3) or (lane % 8) ^ (row % 8) (two blocks of e2m1, whose lanes read pieces part and 4 + part)
-  const uint8_t* pw[2][2];
-  const uint8_t* pws;  // lanes 0-31: the scale words of row lane % 16 of tile 2 wave + lane / 16
+  uint32_t ow[2];
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const uint8_t *wbase, *sbase;
-    const int row = tile_row(2 * wave + t, wbase, sbase);
-    if (S::kRowB == 64) {
-      const int r = lane >> 2;
-      pw[t][0] = wbase + (size_t)(row + r) * (K / 2) + 16 * ((lane & 3) ^ sw4(r));
-      pw[t][1] = pw[t][0];
-    } else {
-#pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        const int r = 8 * hh + (lane >> 3);
-        pw[t][hh] = F4 ? wbase + (size_t)(row + r) * (K / 2) + 16 * ((lane & 7) ^ (r & 7)) : wbase + (size_t)(row + r) * K + 16 * pc8((lane & 7) ^ swz(r));
-      }
-    }
-    if (((lane >> 4) & 1) == t) pws = sbase + (size_t)(F4 ? row + r16 : (row + r16) / 32) * G;
+  for (int hh = 0; hh < 2; ++hh) {
+    const int r = S::kRowB == 64 ? lane >> 2 : 8 * hh + (lane >> 3);
+    const int piece = S::kRowB == 64 ? (lane & 3) ^ sw4(r) : F4 ? (lane & 7) ^ (r & 7) : pc8((lane & 7) ^ swz(r));
+    ow[hh] = (uint32_t)r * RB + 16 * piece;
   }
-  // activations: half tile kHalfX wave + i is positions 8 (kHalfX wave + i) ...; a wave whose half tiles hold no rows brings none
-  const bool brings_x = POS > 64 || m0 + 8 * wave < mend;
+  // the scale words of eight blocks of the wave's 64 rows: two loads, lane -> row 32 i + lane / 2 of them, half sc_half(row, lane)
+  const uint8_t* pws[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = 32 * i + (lane >> 1), row = tile_row(S::RA * wave + (r >> 4)) + (r & 15);
+    pws[i] = (UP && ((r >> 4) & 1) ? sb : sa) + (size_t)(F4 ? row : row / 32) * G + (KB >= 8 ? 16 * sc_half(r & 15, lane) : 0);
+  }
+  // activations: half tile kHX wave + i is positions 8 (kHX wave + i) ...; those past the tile's rows are not fetched
+  const int nhx = uni(min(S::kHX, max(0, (mend - m0 + 7) / 8 - S::kHX * wave)));
   auto row_of = [&](int p) {  // the activation row of the tile's position p (a ragged tile re-reads its last row: never stored)
     const int pos = min(m0 + p, mend - 1);
-    return (size_t)(g.gather ? g.gather[pos] : pos);
+    return (uint32_t)(g.gather ? g.gather[pos] : pos);
   };
-  const uint8_t* px[S::kHalfX];
+  uint32_t ox[S::kHX];
 #pragma unroll
-  for (int i = 0; i < S::kHalfX; ++i) {
-    const int p = 8 * (S::kHalfX * wave + i) + (lane >> 3);
-    px[i] = g.aq + row_of(p) * K + 16 * pc8((lane & 7) ^ swz(p & 15));
+  for (int i = 0; i < S::kHX; ++i) {
+    const int p = 8 * (S::kHX * wave + i) + (lane >> 3);
+    ox[i] = row_of(p) * (uint32_t)K + 16 * pc8((lane & 7) ^ swz(p & 15));
   }
-  const uint8_t* pxs = g.as + row_of(kPosWave * wave + (lane & (kPosWave - 1))) * G;  // lanes 0 .. kPosWave - 1: the scale words of the wave's positions
+  constexpr int kPosWave = POS / kWaves, kSI = (2 * kPosWave + 63) / 64;  // the wave's positions; the loads of eight blocks of their scale words: half a position's a lane
+  uint32_t oxs[kSI];
+#pragma unroll
+  for (int i = 0; i < kSI; ++i) {
+    const int p = kPosWave * wave + min((64 * i + lane) >> 1, kPosWave - 1);
+    oxs[i] = row_of(p) * (uint32_t)G + (KB >= 8 ? 16 * sc_half(p & 15, lane) : 0);
+  }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
-  constexpr int kGroups0 = S::kStages * S::kStageBytes;  // the groups' scale words behind the stages
-  // load number i (0 .. kLoads - 1) of turn t: the activations (L2 hits mostly), the weights last: a wave's loads return in
-  // issue order, so a load that waits for HBM holds back every later one of its wave and the cache's miss slots with them
-  // (weights first: 7% slower, measured). A turn issues them one at a time between its MFMAs (issue_some), so that the
-  // texture unit works through a block's 50 KB while the matrix unit runs instead of in front of it: issued together after
-  // the barrier they cost every wave the time the unit takes to accept them all (measured: a third of a turn).
-  const int TN = KB / S::TB;
-  constexpr int kFirst = F4 ? 0 : 2;  // (e4m3: the turn's scale words in front; 32 weight rows share a word, so they name few lines)
-  auto issue_one = [&](int t, int i) {
-    const int tc = t < TN ? t : TN - 1;  // (past the end: the last turn again, into a stage nobody reads)
-    const uint32_t st = lds0 + (uint32_t)(t % S::kStages) * S::kStageBytes;
-    const uint32_t wbase = st + (uint32_t)wave * (2 * 16 * S::kRowB), xbase = st + S::kStageW + (uint32_t)wave * (S::kHalfX * 1024);
-    if (i < kFirst) {
-      const uint32_t at = lds0 + kGroups0 + (uint32_t)(t % S::kStages) * S::kGroup;
-      if (i == 0) {
-        if (brings_x && lane < kPosWave) dma4(reinterpret_cast<const float*>(pxs + 4 * tc), uni(at + S::kGroupW + (uint32_t)wave * (4 * kPosWave)));
-      } else {
-        if (lane < 32) dma4(reinterpret_cast<const float*>(pws + 4 * tc), uni(at + (uint32_t)wave * 128));
-      }
-    } else if (i < kFirst + S::TB * S::kHalfX) {
-      const int b = (i - kFirst) / S::kHalfX, q = (i - kFirst) % S::kHalfX;
-      if (brings_x) dma16(px[q] + (size_t)tc * (128 * S::TB) + 128 * b, uni(xbase + b * S::kStageX + q * 1024));
-    } else {
-      const int q = i - kFirst - S::TB * S::kHalfX;
-      if (S::kRowB == 64) dma16(pw[q][0] + (size_t)tc * 64, uni(wbase + q * 1024));
-      else dma16(pw[q >> 1][q & 1] + (size_t)tc * 128, uni(wbase + (q >> 1) * 2048 + (q & 1) * 1024));
-    }
+  const uint32_t ring0 = lds0 + (uint32_t)wave * (S::kRing * S::kTileB);
+  // Weight tile i of the wave's sequence (tile i % 4 of turn i / 4, clamped: past the end the last turn again, into a slot nobody
+  // reads) goes to slot i % kRing of the wave's own ring, whose rows no other wave reads: a slot is free as soon as the wave has read
+  // its fragments. Activations: a stage a turn.
+  const int TN = KB / TB;
+  auto issue_w = [&](int t, int i, int slot, int hh) {
+    dma16(wt[i] + (size_t)min(t, TN - 1) * S::kRowB, ow[hh], uni(ring0 + (uint32_t)slot * S::kTileB + hh * 1024));
   };
-  // e2m1: the scale words of the group that turn t opens (blocks 4 q ... 4 q + 3; the last ones of a row from its end): two loads
-  // a wave. Rows of fewer than four blocks have no 16 bytes: their words are put in place by hand.
-  constexpr int kGroupTurns = 4 / S::TB;
-  auto first_block = [&](int q) { return min(4 * q, KB - 4); };
+  auto issue_x = [&](int t) {
+    const uint32_t xbase = lds0 + S::kOffX + (uint32_t)(t & 1) * (TB * S::kStageX) + (uint32_t)wave * (S::kHX * 1024);
+#pragma unroll
+    for (int b = 0; b < TB; ++b)
+#pragma unroll
+      for (int i = 0; i < S::kHX; ++i) {
+        if (i >= nhx) break;
+        dma16(g.aq + (size_t)min(t, TN - 1) * (128 * TB) + 128 * b, ox[i], uni(xbase + b * S::kStageX + i * 1024));
+      }
+  };
+  // The scale words of the group that turn t opens (blocks 8 q ... 8 q + 7; the last ones of a row from its end): the weight rows'
+  // into the wave's one buffer, which is free when the group's last words are read; the positions' into two. A line of L2 holds a
+  // row's words of 32 blocks and has left L2 when the next group comes, so what counts is how often it is named. Rows of fewer than
+  // eight blocks: their words are put in place by hand.
+  constexpr int kGroupTurns = 8 / TB;
+  auto first_block = [&](int q) { return min(8 * q, KB - 8); };
   auto issue_scales = [&](int t) {
     const int q = t / kGroupTurns, kb = first_block(q);
-    const uint32_t at = lds0 + kGroups0 + (uint32_t)(q & 1) * S::kGroup;
-    if (lane < 32) dma16(pws + 4 * kb, uni(at + (uint32_t)wave * 512));
-    if (brings_x && lane < kPosWave) dma16(pxs + 4 * kb, uni(at + S::kGroupW + (uint32_t)wave * (16 * kPosWave)));
+#pragma unroll
+    for (int i = 0; i < 2; ++i) dma16(pws[i] + 4 * kb, uni(lds0 + S::kOffS + (uint32_t)wave * 2048 + i * 1024));
+#pragma unroll
+    for (int i = 0; i < kSI; ++i)
+      if (nhx > 0 && 64 * i + lane < 2 * kPosWave) dma16(g.as + 4 * kb, oxs[i], uni(lds0 + S::kOffSX + (uint32_t)(q & 1) * S::kScaleX + (uint32_t)wave * (32 * kPosWave) + i * 1024));
   };
-  if (F4 && KB >= 4) {
+  if (KB >= 8) {
     issue_scales(0);
-  } else if (F4) {
-    for (int kb = 0; kb < KB; ++kb) {
-      uint32_t* at = reinterpret_cast<uint32_t*>(smem + kGroups0) + kb;
-      if (lane < 32) at[(32 * wave + lane) * 4] = ldg_u32(pws + 4 * kb);
-      if (lane < kPosWave) at[S::kGroupW / 4 + (kPosWave * wave + lane) * 4] = ldg_u32(pxs + 4 * kb);
+  } else {
+    uint32_t w[2][7], x[kSI][7];
+#pragma unroll
+    for (int i = 0; i < 7; ++i) {
+      const int o = 4 * min(i, KB - 1);
+      w[0][i] = ldg_u32(pws[0] + o), w[1][i] = ldg_u32(pws[1] + o);
+#pragma unroll
+      for (int k = 0; k < kSI; ++k) x[k][i] = ldg_u32(g.as + oxs[k] + o);
+    }
+    if (!(lane & 1)) {
+      const int r = lane >> 1;
+#pragma unroll
+      for (int i = 0; i < 7; ++i) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) reinterpret_cast<uint32_t*>(smem + S::kOffS)[(64 * wave + 32 * k + r) * 8 + 4 * sc_half(r & 15, i >> 2) + (i & 3)] = w[k][i];
+#pragma unroll
+        for (int k = 0; k < kSI; ++k) {
+          const int p = kPosWave * wave + 32 * k + r;
+          if (32 * k + r < kPosWave) reinterpret_cast<uint32_t*>(smem + S::kOffSX)[p * 8 + 4 * sc_half(p & 15, i >> 2) + (i & 3)] = x[k][i];
+        }
+      }
     }
   }
+  issue_x(0);
 #pragma unroll
-  for (int s = 0; s + 1 < S::kStages; ++s)
+  for (int i = 0; i < S::kRing; ++i)
 #pragma unroll
-    for (int i = 0; i < S::kLoads; ++i) issue_one(s, i);
+    for (int hh = 0; hh < S::LT; ++hh) issue_w(i / 4, i % 4, i, hh);
 
   // fragment reads. The instruction numbers an 8-bit operand's k as 64 h + 16 part + i (h: the lane's first or second four
   // registers, i: the byte) and a 4-bit operand's as 32 part + i, and takes the scale of k block g = k / 32 from the lanes
@@ -228,79 +234,76 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
     return v8i_t{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
   };
   auto frag4 = [&](const uint8_t* t, int b) {
-    const u32x4_t lo = *reinterpret_cast<const u32x4_t*>(t + (S::TB == 2 ? rd4b[b] : rd4));
+    const u32x4_t lo = *reinterpret_cast<const u32x4_t*>(t + (TB == 2 ? rd4b[b] : rd4));
     return v8i_t{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, 0, 0, 0, 0};
   };
-  constexpr int kScaleT = 64 * S::kWords;   // bytes of a 16-row (16-position) tile's scale words
-  const int rds = r16 * (4 * S::kWords);    // the lane's row's among them; its byte: `part`
   const int rsh = 8 * part;
 
-  v4f_t acc[S::RA][8];
+  v4f_t acc[S::RA][S::kSub];
 #pragma unroll
   for (int t = 0; t < S::RA; ++t)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[t][j] = v4f_t{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < S::kSub; ++j) acc[t][j] = v4f_t{0.f, 0.f, 0.f, 0.f};
 
   auto run = [&](auto nj_c) {
     constexpr int NJ = decltype(nj_c)::value;
+    int slot = 0;  // of the turn's first weight tile: 4 t % kRing
     for (int t = 0; t < TN; ++t) {
-      // turn t's loads have landed; with three stages turn t + 1's may be in flight (the scale words of the group that it opens,
-      // which come first, are waited for: a count of its own for those turns is a branch in every turn and 1% slower)
-      if (S::kStages == 2) wait_loads<0>();
-      else if (brings_x) wait_loads<S::kLoads>();
-      else wait_loads<S::kLoadsW + kFirst / 2>();
+      // this wave's loads of turn t have landed (weight tiles of later turns may be in flight); after the barrier everyone's have,
+      // and everyone is done reading the stage of turn t - 1, which the activations of turn t + 1 now overwrite
+      wait_loads<S::LT * (S::kRing - 4)>();
       __syncthreads();
-      const int tn = t + S::kStages - 1;
-      // loads i with i * NJ / kLoads == j go out after the fragment reads of 16-position tile j, a group's scale words after the
-      // first tile's (in front of the turn's first reads they cost the 256-position tiles 2%, at its end every shape 4%)
-      auto issue_some = [&](int j) {
-        if (F4 && j == 0 && tn % kGroupTurns == 0 && tn < TN) issue_scales(tn);
+      const int q = t / kGroupTurns, word = TB * t - (KB >= 8 ? first_block(q) : 0);  // the turn's first word of its group's
+      // (a turn of two blocks begins at an even word: both lie in one half)
+      const int at = r16 * 32 + 16 * sc_half(r16, word >> 2) + 4 * (word & 3);  // the lane's row's words of the turn in a 16-row (16-position) tile's 512 bytes; its byte: `part`
+      const uint8_t* WS = smem + S::kOffS + wave * 2048 + at;
+      const uint8_t* XS = smem + S::kOffSX + (size_t)(q & 1) * S::kScaleX + at;
+      const uint8_t* X = smem + S::kOffX + (size_t)(t & 1) * (TB * S::kStageX);
+      int sl[4];
 #pragma unroll
-        for (int i = 0; i < S::kLoads; ++i)
-          if (i * (NJ > 0 ? NJ : 1) / S::kLoads == j) issue_one(tn, i);
-      };
-      if (NJ == 0) issue_some(0);
-      if (NJ == 0) continue;
-      const uint8_t* st = smem + (size_t)(t % S::kStages) * S::kStageBytes;
-      const uint8_t* W = st + S::RA * rg * (16 * S::kRowB);
-      const uint8_t* X = st + S::kStageW + pg * 2048;
-      const int q = t / kGroupTurns, word = S::TB * t - (KB >= 4 ? first_block(q) : 0);  // e2m1: the turn's first word of its group's
-      const uint8_t* GS = smem + kGroups0 + (F4 ? (size_t)(q & 1) * S::kGroup + 4 * word : (size_t)(t % S::kStages) * S::kGroup);
-      const uint8_t* WS = GS + S::RA * rg * kScaleT + rds;
-      const uint8_t* XS = GS + S::kGroupW + pg * kScaleT + rds;
-      v8i_t fa[S::TB][S::RA];
-      int fs[S::TB][S::RA];
+      for (int i = 0; i < 4; ++i) sl[i] = slot + i >= S::kRing ? slot + i - S::kRing : slot + i;
+      v8i_t fa[TB][S::RA];
+      int fs[TB][S::RA];
 #pragma unroll
-      for (int b = 0; b < S::TB; ++b)
+      for (int b = 0; b < TB; ++b)
 #pragma unroll
         for (int i = 0; i < S::RA; ++i) {
-          fa[b][i] = F4 ? frag4(W + i * (16 * S::kRowB), b) : frag8(W + i * 2048);
-          fs[b][i] = (*reinterpret_cast<const uint32_t*>(WS + i * kScaleT + 4 * b) >> rsh) & 0xFFu;
+          const uint8_t* W = smem + wave * (S::kRing * S::kTileB) + sl[i] * S::kTileB;
+          fa[b][i] = F4 ? frag4(W, b) : frag8(W);
+          fs[b][i] = (*reinterpret_cast<const uint32_t*>(WS + i * 512 + 4 * b) >> rsh) & 0xFFu;
         }
+      issue_x(t + 1);
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        v8i_t fb[S::TB];
-        int xsb[S::TB];
+      for (int b = 0; b < TB; ++b)  // (read: what holds them may be written from here on)
+        asm volatile("" : "+v"(fa[b][0]), "+v"(fa[b][1]), "+v"(fa[b][2]), "+v"(fa[b][3]), "+v"(fs[b][0]), "+v"(fs[b][1]), "+v"(fs[b][2]), "+v"(fs[b][3]));
+      if ((t + 1) % kGroupTurns == 0 && t + 1 < TN) issue_scales(t + 1);
+      static_for<NJ>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        v8i_t fb[TB];
+        int xsb[TB];
 #pragma unroll
-        for (int b = 0; b < S::TB; ++b) {
-          fb[b] = frag8(X + b * S::kStageX + j * (2048 * WP));
-          xsb[b] = (*reinterpret_cast<const uint32_t*>(XS + j * (kScaleT * WP) + 4 * b) >> rsh) & 0xFFu;
+        for (int b = 0; b < TB; ++b) {
+          fb[b] = frag8(X + b * S::kStageX + j * 2048);
+          xsb[b] = (*reinterpret_cast<const uint32_t*>(XS + j * 512 + 4 * b) >> rsh) & 0xFFu;
         }
-        issue_some(j);
+        // (the weights' loads one by one between the MFMAs)
 #pragma unroll
-        for (int b = 0; b < S::TB; ++b)
+        for (int i = 0; i < 4 * S::LT; ++i)
+          if (i * NJ / (4 * S::LT) == j) issue_w(t + (S::kRing + i / S::LT) / 4, (S::kRing + i / S::LT) % 4, sl[i / S::LT], i % S::LT);
+#pragma unroll
+        for (int b = 0; b < TB; ++b)
 #pragma unroll
           for (int i = 0; i < S::RA; ++i) acc[i][j] = mfma_mx<CBSZ>(fa[b][i], fb[b], acc[i][j], fs[b][i], xsb[b]);
-      }
+      });
+      slot = slot + 4 >= S::kRing ? slot + 4 - S::kRing : slot + 4;
     }
   };
-  constexpr int kMaxNJ = S::kSub / WP, kMinNJ = WP == 2 ? 0 : 1;
   auto run_nj = [&](auto self, auto n) {
     constexpr int N = decltype(n)::value;
-    if (N == kMaxNJ || nj == N) run(n);
-    else if constexpr (N < kMaxNJ) self(self, std::integral_constant<int, N + 1>{});
+    if (N == S::kSub || nmt == N) run(n);
+    else if constexpr (N < S::kSub) self(self, std::integral_constant<int, N + 1>{});
   };
-  run_nj(run_nj, std::integral_constant<int, kMinNJ>{});
+  run_nj(run_nj, std::integral_constant<int, F4 && POS == 64 ? 3 : !F4 && POS == 128 ? 5 : 1>{});
   wait_loads<0>();
   __syncthreads();
 
@@ -308,10 +311,10 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   if (UP) {
     const int I = g.I;
     const float lim = g.limit;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (j >= nj) break;
-      const int p = 16 * (pg + WP * j) + r16;
+    static_for<S::kSub>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      if (j >= nmt) return;
+      const int p = 16 * j + r16;
       const float wv = (g.posw && m0 + p < mend) ? g.posw[m0 + p] : 1.f;
 #pragma unroll
       for (int b = 0; b < S::RA / 2; ++b) {
@@ -325,16 +328,16 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
           hv[q] = __fmul_rn(hv[q], up[q]);
           if (g.posw) hv[q] = __fmul_rn(wv, hv[q]);
         }
-        const int ch = 16 * (S::RA / 2 * rg + b) + 4 * part;
+        const int ch = 16 * (S::RA / 2 * wave + b) + 4 * part;
         const int piece = (ch >> 3) ^ (p & 15);
         *reinterpret_cast<uint2*>(smem + p * 256 + piece * 16 + (ch & 4) * 2) = make_uint2(pack_bf16(hv[0], hv[1]), pack_bf16(hv[2], hv[3]));
       }
-    }
+    });
     __syncthreads();
     // 16 lanes a position, 8 channels a lane: a scale group (32 channels) is 4 lanes. The scale byte is the exponent of
     // max(amax, 1e-4) / 448 rounded up to a power of two (ds41f engine/kernels/common.cuh:53-66); codes e4m3(h * 2^(127 - e)).
     const int l16 = tid & 15;
-    for (int p = tid >> 4; p < 16 * nmt; p += kThreads / 16) {
+    for (int p = tid >> 4; p < 16 * nmt; p += kThreads4 / 16) {
       const int pos = m0 + p;
       const u32x4_t hv = *reinterpret_cast<const u32x4_t*>(smem + p * 256 + (l16 ^ (p & 15)) * 16);
       float v[8];
@@ -361,74 +364,76 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
     }
   } else {
     // a 16-position tile of the wave at a time through its own piece of LDS: written as held (4 consecutive rows of one
-    // position = 8 bytes of bf16), read back as whole rows (32 WP rows = 64 WP bytes a position), 4 WP lanes a position
+    // position = 8 bytes of bf16), read back as whole rows (64 rows = 128 bytes a position), 8 lanes a position
     const int H = g.H;
-    constexpr int RB = 64 * WP, PC = RB / 16;  // bytes and 16-byte pieces of a position's rows of this wave
-    uint8_t* my = smem + wave * (1024 * WP);
-    const int row0 = r0 + 16 * S::RA * rg;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (j >= nj) break;
+    uint8_t* my = smem + wave * 2048;
+    const int row0 = r0 + 16 * S::RA * wave;
+    static_for<S::kSub>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      if (j >= nmt) return;
 #pragma unroll
       for (int t = 0; t < S::RA; ++t) {
         const uint32_t lo = pack_bf16(acc[t][j][0], acc[t][j][1]), hi = pack_bf16(acc[t][j][2], acc[t][j][3]);
         const int c = 2 * t + (part >> 1);  // the 16-byte piece: rows 16 t + 4 part ... are bytes 32 t + 8 part ...
-        *reinterpret_cast<uint2*>(my + r16 * RB + ((c ^ r16) & (PC - 1)) * 16 + (part & 1) * 8) = make_uint2(lo, hi);
+        *reinterpret_cast<uint2*>(my + r16 * 128 + ((c ^ r16) & 7) * 16 + (part & 1) * 8) = make_uint2(lo, hi);
       }
 #pragma unroll
-      for (int i = 0; i < (16 * PC + 63) / 64; ++i) {
-        const int idx = i * 64 + lane, p = idx / PC, c = idx % PC;
-        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(my + p * RB + ((c ^ p) & (PC - 1)) * 16);
-        const int pos = m0 + 16 * (pg + WP * j) + p;
+      for (int i = 0; i < 2; ++i) {
+        const int p = 8 * i + (lane >> 3), c = lane & 7;
+        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(my + p * 128 + ((c ^ p) & 7) * 16);
+        const int pos = m0 + 16 * j + p;
         if (pos < mend) *reinterpret_cast<u32x4_t*>(g.d + (size_t)pos * H + row0 + 8 * c) = v;
       }
-    }
+    });
   }
 }
+
+constexpr int kLds = std::max({Shape<kMaxPos, DSGX_FMT_MXFP4_G32, 1>::kLds, Shape<64, DSGX_FMT_MXFP4_G32, 2>::kLds, Shape<32, DSGX_FMT_MXFP4_G32, 2>::kLds,
+                               Shape<128, DSGX_FMT_FP8_B32E, 1>::kLds, Shape<64, DSGX_FMT_FP8_B32E, 1>::kLds});
+static_assert(2 * kLds <= 160 * 1024, "two workgroups a CU");
 
 // The tile of the shared expert's rows from m0 on (e4m3 weights), in the smallest shape that holds them
 template <bool UP>
 __device__ __forceinline__ void shared_tile(const Args& g, uint8_t* smem, int m0, int mend, int ns) {
   constexpr int F8 = DSGX_FMT_FP8_B32E;
-  if (mend - m0 > 128) gemm_tile<UP, 256, F8>(g, smem, -1, m0, mend, ns);
-  else if (mend - m0 > 64) gemm_tile<UP, 128, F8>(g, smem, -1, m0, mend, ns);
-  else gemm_tile<UP, 64, F8>(g, smem, -1, m0, mend, ns);
+  if (mend - m0 > 64) gemm_tile<UP, 128, F8, 1>(g, smem, -1, m0, mend, ns);
+  else gemm_tile<UP, 64, F8, 1>(g, smem, -1, m0, mend, ns);
 }
-// The shared expert (tile_e null: tiles of 256 rows over [0, nrows)).
+// The shared expert (tile_e null: tiles of 128 rows over [0, nrows)).
 template <bool UP>
-__global__ void __launch_bounds__(kThreads) k_gemm(Args g) {
+__global__ void __launch_bounds__(kThreads4, 2) k_gemm(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int NS = UP ? g.I / (kWgRows / 2) : g.H / kWgRows;
   int tile, ns;
   pf8::task_of<true>(NS, tile, ns);
-  if (ns >= NS || tile * 256 >= g.nrows) return;
-  shared_tile<UP>(g, smem, tile * 256, g.nrows, ns);
+  if (ns >= NS || tile * 128 >= g.nrows) return;
+  shared_tile<UP>(g, smem, tile * 128, g.nrows, ns);
 }
-// The routed experts' list of both tile shapes (bit 30 of tile_e: a 256-position tile), an expert's tiles next to each other.
-// A remainder of up to 64 rows runs two blocks a turn where K is pairs of blocks.
+// The routed experts' list of tiles, an expert's tiles next to each other.
+// A tile of up to 64 rows runs two blocks a turn where K is pairs of blocks.
 template <bool UP>
-__global__ void __launch_bounds__(kThreads) k_gemm_mixed(Args g) {
+__global__ void __launch_bounds__(kThreads4, 2) k_gemm_mixed(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   constexpr int F4 = DSGX_FMT_MXFP4_G32;
   const int NS = UP ? g.I / (kWgRows / 2) : g.H / kWgRows;
   int tile, ns;
   if (blockIdx.x < g.sh.grid) {  // (the same for the whole workgroup)
-    pf8::task_of<true>(NS, tile, ns);
-    if (ns >= NS || tile * 256 >= g.nrows) return;
+    pf8::task_of<true>(NS, tile, ns, blockIdx.x, g.map);
+    if (ns >= NS || tile * 128 >= g.nrows) return;
     Args q = g;
     q.aq = g.sh.aq, q.as = g.sh.as, q.gather = nullptr, q.posw = nullptr, q.wstride = q.sstride = 0;
     q.wa = g.sh.wa, q.sa = g.sh.sa, q.wb = g.sh.wb, q.sb = g.sh.sb, q.h = g.sh.h, q.hq = g.sh.hq, q.hs = g.sh.hs, q.d = g.sh.d;
-    shared_tile<UP>(q, smem, tile * 256, g.nrows, ns);
+    shared_tile<UP>(q, smem, tile * 128, g.nrows, ns);
     return;
   }
-  pf8::task_of<false>(NS, tile, ns, blockIdx.x - g.sh.grid);
+  pf8::task_of<false>(NS, tile, ns, blockIdx.x - g.sh.grid, g.map);
   if (ns >= NS || tile >= *g.ntiles) return;
-  const int te = g.tile_e[tile], e = te & 0xFFFF;
+  const int e = g.tile_e[tile];
   const int m0 = g.off[e] + g.tile_m0[tile], mend = g.off[e + 1];
   const bool pairs = (UP ? g.H : g.I) % 256 == 0;
-  if (te >> 30) gemm_tile<UP, 256, F4>(g, smem, e, m0, mend, ns);
-  else if (mend - m0 <= 64 && pairs) gemm_tile<UP, 64, F4>(g, smem, e, m0, mend, ns);
-  else gemm_tile<UP, 128, F4>(g, smem, e, m0, mend, ns);
+  if (mend - m0 > 64 || !pairs) gemm_tile<UP, kMaxPos, F4, 1>(g, smem, e, m0, mend, ns);
+  else if (mend - m0 > 32) gemm_tile<UP, 64, F4, 2>(g, smem, e, m0, mend, ns);
+  else gemm_tile<UP, 32, F4, 2>(g, smem, e, m0, mend, ns);
 }
 
 }  // namespace pfmx

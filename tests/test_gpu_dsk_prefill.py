@@ -208,10 +208,28 @@ def test_dsk_prefill_against_oracle(H, I, E, T, shared):
         assert np.array_equal(gpu.host(y2, np.uint32, (T, H)), got["y"].view(np.uint32))
 
 
+@pytest.mark.parametrize("H,I", [(256, 128), (512, 1152), (1280, 256)])
+def test_dsk_prefill_tile_shapes_give_the_same_bits(H, I):
+    """experts whose rows end at the edges of the tiles of 32, 64 and 160 positions (and one row beyond), K in whole pairs of blocks and
+    not: every row has the bits that it has alone in a chunk, in the smallest tile"""
+    counts, topk = [1, 8, 9, 32, 33, 64, 65, 160, 161, 321], 1
+    L = Stacked(43, H, I, len(counts), topk, 5, True)
+    idx = np.repeat(np.arange(len(counts), dtype=np.int32), counts)[:, None].copy()
+    T = len(idx)
+    x = orc.normal_bf16(43, 1, (T, H), 1.5)
+    w = (0.5 + np.abs(orc.normal_f32(43, 2, (T, topk), 1.0))).astype(np.float32)
+    xq, xs = orc.act_quant_ue8m0(x)
+    got = run_prefill(L, xq, xs, idx, w)
+    ends = np.cumsum(counts)
+    for t in sorted(set(int(v) for e, n in zip(ends, counts) for v in (e - n, e - 1 - n // 2, e - 1 - n % 16 * (n > 16), e - 1))):
+        one = run_prefill(L, xq[t:t + 1].copy(), xs[t:t + 1].copy(), idx[t:t + 1], w[t:t + 1])
+        assert np.array_equal(got["y"][t].view(np.uint32), one["y"][0].view(np.uint32)), t
+
+
 @pytest.mark.parametrize("H,I,T", [(256, 128, 17), (256, 384, 10), (512, 640, 64), (768, 1152, 90), (1024, 1280, 33)])
 def test_dsk_prefill_scale_groups_and_block_pairs(H, I, T):
-    """The scale words come for four 128-k blocks at a time and small tiles take blocks by pairs: rows of K with fewer than four
-    blocks (1, 2, 3), with a last group that is not whole (5, 6, 9, 10), odd numbers of blocks; 8 to 64 positions and over"""
+    """The scale words come for eight 128-k blocks at a time and small tiles take blocks by pairs: rows of K with fewer than eight
+    blocks (1, 2, 3, 5, 6), with a last group that is not whole (9, 10), odd numbers of blocks; 8 to 64 positions and over"""
     E, topk = 8, 6
     L = Stacked(43, H, I, E, topk, 5, True)
     x = orc.normal_bf16(43, 1, (T, H), 1.5)

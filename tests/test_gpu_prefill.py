@@ -182,8 +182,8 @@ def test_prefill_fp8_against_oracle(H, I, E, topk, T, shared, unit_rule):
 
 @pytest.mark.parametrize("H,I,T", [(512, 640, 20), (1280, 1152, 300)])
 def test_prefill_fp8_scale_groups(H, I, T, unit_rule):
-    """the rows' scales come for four 128-k blocks at a time: last groups that are not whole (5, 9 and 10 blocks; 4 are one group,
-    1, 2 and 3 are among the shapes above), tiles of a few rows and of 256"""
+    """the rows' scales come for eight 128-k blocks at a time, in the widest tile for four: last groups that are not whole (5, 9 and 10
+    blocks; 4 and 8 are one group, fewer are among the shapes above), tiles of a few rows and of 160"""
     test_prefill_fp8_against_oracle(H, I, 4, 2, T, "fp8", unit_rule)
 
 
@@ -197,9 +197,26 @@ def test_prefill_rows_do_not_depend_on_the_chunk():
     assert np.array_equal(yr[50:60], yr2) and np.array_equal(ys[50:60], ys2)
 
 
+@pytest.mark.parametrize("H,I", [(256, 128), (1280, 1152)])
+def test_prefill_fp8_tile_shapes_give_the_same_bits(H, I):
+    """experts whose rows end at the edges of the tiles of 32, 64 and 160 positions (and one row beyond): every row has the bits that it
+    has alone in a chunk, in the smallest tile"""
+    counts, topk = [1, 8, 9, 32, 33, 64, 65, 160, 161, 321], 1
+    hl = helpers.make_layer(abi.FMT_FP8, H, I, len(counts), topk, 5, seed=14, shared="fp8")
+    idx = np.repeat(np.arange(len(counts), dtype=np.int32), counts)[:, None].copy()
+    T = len(idx)
+    x, _, _, w = helpers.rows_and_routing(15, T, H, len(counts), topk, 1.0)
+    yr, ys, _, dl = _prefill(hl, x, idx, w, T)
+    ends = np.cumsum(counts)
+    for t in sorted(set(int(v) for e, n in zip(ends, counts) for v in (e - n, e - 1 - n // 2, e - 1 - n % 16 * (n > 16), e - 1))):
+        y1, s1, _, _ = _prefill(hl, x[t:t + 1], idx[t:t + 1], w[t:t + 1], 1)
+        assert np.array_equal(yr[t].view(np.uint32), y1[0].view(np.uint32)), t
+        assert np.array_equal(ys[t].view(np.uint32), s1[0].view(np.uint32)), t
+
+
 def test_prefill_tile_order_does_not_change_a_bit():
     """dsgx_prefill_cfg::tile_order (the reference's prefill_tuning tord, ds41f engine/kernels/dsk.h:252) only changes which
-    workgroup takes which tile: experts of 0, a few, 128, 129, 256 and several hundred rows (remainders, 256-position
+    workgroup takes which tile: experts of 0, a few, 128, 129, 256 and several hundred rows (remainders, full
     tiles and both), every order, the same yr, ys and workspace views as the order by expert id"""
     H, I, E, topk, T = 256, 256, 12, 2, 900
     hl = helpers.make_layer(abi.FMT_FP8, H, I, E, topk, 5, seed=9, shared="fp8")
