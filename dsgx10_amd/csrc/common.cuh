@@ -557,4 +557,36 @@ __device__ __forceinline__ float div_by(float v, float d, float r) {
   return fmaf(fmaf(-q, d, v), r, q);
 }
 
+// act_quant(x, 128): sixteen lanes a (row, 128-k block), eight values (one 16-byte load) a lane; the block's largest
+// magnitude by four DPP steps within the row of 16 lanes
+// (ds41f-4xgx10-switchless/ref/torchref/kernel.py:56-77 of the reference, scale_fmt None)
+__device__ __forceinline__ void act_quant_block(const uint16_t* __restrict__ x, int T, int K, size_t blk, uint8_t* __restrict__ q, float* __restrict__ s) {
+  const int KB = K / 128, l16 = threadIdx.x & 15;
+  if (blk >= (size_t)T * KB) return;  // (whole rows of 16 lanes leave together)
+  const size_t t = blk / KB, b = blk % KB, at = t * K + 128 * b + 8 * l16;
+  const u32x4_t xv = *reinterpret_cast<const DSGX_GLOBAL u32x4_t*>((uintptr_t)(x + at));
+  float v[8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[2 * i] = bf16_bits_to_f32(xv[i] & 0xFFFFu), v[2 * i + 1] = bf16_bits_to_f32(xv[i] >> 16);
+  float amax = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
+  amax = dpp_max<0xB1>(amax);
+  amax = dpp_max<0x4E>(amax);
+  amax = dpp_max<0x141>(amax);
+  amax = dpp_max<0x140>(amax);
+  amax = fmaxf(amax, 1e-4f);
+  const float sc = __fmul_rn(amax, 1.0f / 448.0f);
+  if (l16 == 0) s[t * KB + b] = sc;
+  float qv[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) qv[i] = fminf(448.f, fmaxf(-448.f, __fdiv_rn(v[i], sc)));
+  uint32_t o[2];
+  o[0] = __builtin_amdgcn_cvt_pk_fp8_f32(qv[0], qv[1], 0, false);
+  o[0] = __builtin_amdgcn_cvt_pk_fp8_f32(qv[2], qv[3], o[0], true);
+  o[1] = __builtin_amdgcn_cvt_pk_fp8_f32(qv[4], qv[5], 0, false);
+  o[1] = __builtin_amdgcn_cvt_pk_fp8_f32(qv[6], qv[7], o[1], true);
+  *reinterpret_cast<uint2*>(q + at) = make_uint2(o[0], o[1]);
+}
+
 }  // namespace dsgx

@@ -254,6 +254,141 @@ __global__ void __launch_bounds__(256) k_pf_place(const int* __restrict__ idx, c
   }
 }
 
+// The three launches as one, of one workgroup, for chunks of up to kBucketPicks picks whose masks fit its LDS: every launch is a few
+// microseconds of little but round trips, and that workgroup's own chain is shorter than theirs. The masks of all rows lie in LDS at
+// once; further workgroups quantise the chunk's rows for the FP8 layers (act_quant), which waits for nothing here. At T = 200, top-8
+// of 256: 6.5 us instead of 3.3 + 4.2 + 9.3 + 4.8 and three gaps (whole call 987 -> 974; 1024 x 512, 32 experts, top-4, T = 40: 38.2 -> 31.2).
+// One workgroup's scattered stores are what grows: 8888 picks take 20 us, as the three launches do, 16,000 are 1 us slower than those.
+struct BucketArgs {
+  const int* idx;
+  const float* w;
+  int T, topk, E;
+  const dsgx_mat_desc* desc;  // the combine's factor s2 * w (null: w)
+  int *cnt, *off, *perm, *pickpos, *rpos, *re;
+  float *rk, *posw;           // (posw null: not asked for)
+  TileLists tl;
+  const uint16_t* x;          // rows to quantise (workgroups 1 ...)
+  int H;
+  uint8_t* xq;
+  float* xs;
+};
+constexpr int kBucketThreads = 1024;
+constexpr int kBucketPicks = 4096;
+constexpr size_t kBucketLds = 112 * 1024;
+inline size_t bucket_lds(int T, int topk, int E) {
+  const size_t NW = ((size_t)T + 31) / 32;
+  return (NW * E * 6 + 15) / 16 * 16 + (size_t)T * topk * 2;
+}
+__global__ void __launch_bounds__(kBucketThreads) k_pf_bucket(BucketArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  __shared__ int s_cnt[DSGX_MAX_EXPERTS], s_off[DSGX_MAX_EXPERTS], s_wave[2][DSGX_MAX_EXPERTS / 64];
+  __shared__ float s_s2[DSGX_MAX_EXPERTS];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (blockIdx.x > 0) {
+    act_quant_block(a.x, a.T, a.H, (size_t)(blockIdx.x - 1) * (kBucketThreads / 16) + (tid >> 4), a.xq, a.xs);
+    return;
+  }
+  const int T = a.T, topk = a.topk, E = a.E, P = T * topk, NW = (T + 31) / 32;
+  uint32_t* mask = reinterpret_cast<uint32_t*>(smem);                    // [E][NW]: the rows that picked the expert
+  uint16_t* pre = reinterpret_cast<uint16_t*>(smem + (size_t)E * NW * 4);  // [E][NW]: how many of them lie in the words before
+  uint16_t* ids = reinterpret_cast<uint16_t*>(smem + ((size_t)E * NW * 6 + 15) / 16 * 16);  // [T][topk]
+  for (int i = tid; i < E * NW; i += kBucketThreads) mask[i] = 0;
+  float s2 = 1.f;
+  if (a.desc && tid < E) s2 = a.desc[(size_t)tid * 3 + 2].s2;
+  __syncthreads();
+  for (int i0 = tid; i0 < P; i0 += 4 * kBucketThreads) {  // (four picks' loads in flight together)
+    int e[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) e[u] = a.idx[min(i0 + u * kBucketThreads, P - 1)];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = i0 + u * kBucketThreads, t = i / topk;
+      if (i < P) ids[i] = (uint16_t)e[u], atomicOr(&mask[e[u] * NW + (t >> 5)], 1u << (t & 31));
+    }
+  }
+  __syncthreads();
+  // the words' counts summed along the rows: a wave takes as many experts at a time as NW words go into its lanes
+  {
+    const int wl = NW <= 8 ? 3 : NW <= 16 ? 4 : NW <= 32 ? 5 : 6, W = 1 << wl, per = 64 >> wl, l = lane & (W - 1);
+    for (int e = wave * per + (lane >> wl); e < E; e += (kBucketThreads / 64) * per) {
+      int carry = 0;
+      for (int b = 0; b < NW; b += W) {
+        const int c = b + l < NW ? __popc(mask[e * NW + b + l]) : 0;
+        int v = c;
+        for (int d = 1; d < W; d <<= 1) {
+          const int u = __shfl_up(v, d, W);
+          if (l >= d) v += u;
+        }
+        if (b + l < NW) pre[e * NW + b + l] = (uint16_t)(carry + v - c);
+        carry += __shfl(v, W - 1, W);
+      }
+      if (l == 0) s_cnt[e] = carry;
+    }
+  }
+  __syncthreads();
+  // the buckets' offsets and the lists: scans over the experts, a thread an expert (tiles of both lists in one word)
+  constexpr int kWide = pf8::kMaxPos;
+  int c = 0, n = 0, vc = 0, vn = 0;
+  if (tid < DSGX_MAX_EXPERTS) {
+    c = tid < E ? s_cnt[tid] : 0, n = (c + kTile - 1) / kTile | ((c + kWide - 1) / kWide) << 16;
+    vc = c, vn = n;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int uc = __shfl_up(vc, d), un = __shfl_up(vn, d);
+      if (lane >= d) vc += uc, vn += un;
+    }
+    if (lane == 63) s_wave[0][wave] = vc, s_wave[1][wave] = vn;
+  }
+  __syncthreads();
+  if (tid < E) {
+    for (int q = 0; q < wave; ++q) vc += s_wave[0][q], vn += s_wave[1][q];
+    const int off = vc - c, nt = n & 0xFFFF, nw = n >> 16, t0 = (vn - n) & 0xFFFF, w0 = (vn - n) >> 16;
+    s_off[tid] = off, s_s2[tid] = s2;
+    a.cnt[tid] = c, a.off[tid] = off;
+    if (tid == E - 1) a.off[E] = vc, *a.tl.ntiles = vn & 0xFFFF, *a.tl.nwide = vn >> 16;
+    for (int i = 0; i < nt; ++i) a.tl.tile_e[t0 + i] = tid, a.tl.tile_m0[t0 + i] = i * kTile;
+    for (int i = 0; i < nw; ++i) {
+      a.tl.wide_e[w0 + i] = a.tl.ord_e[w0 + i] = tid;
+      a.tl.wide_m0[w0 + i] = a.tl.ord_m0[w0 + i] = i * kWide;
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < P; i += kBucketThreads) {
+    const float wv = a.w[i];
+    const int e = ids[i], t = i / topk, m = e * NW + (t >> 5);
+    const int pos = s_off[e] + pre[m] + __popc(mask[m] & ((1u << (t & 31)) - 1));
+    int rank = 0;
+    for (int j = 0; j < topk; ++j) rank += ids[t * topk + j] < e;
+    const int o = t * topk + rank;
+    a.perm[pos] = t, a.pickpos[i] = pos;
+    a.re[o] = e, a.rpos[o] = pos, a.rk[o] = a.desc ? __fmul_rn(s_s2[e], wv) : wv;
+    if (a.posw) a.posw[pos] = wv;  // (DeepSeek's layers apply the routing weight to h, position by position)
+  }
+}
+// The bucketing of a chunk, and with `quant` (FP8 layers) the quantised rows
+static int bucket(const PfLayout& o, uint8_t* W, const int* idx, const float* w, int T, int topk, int E, const dsgx_mat_desc* desc, float* posw, int order,
+                  const uint16_t* x, int H, bool quant, hipStream_t st) {
+  auto I32 = [&](size_t off) { return reinterpret_cast<int*>(W + off); };
+  auto F32 = [&](size_t off) { return reinterpret_cast<float*>(W + off); };
+  const TileLists tl{I32(o.ntiles), I32(o.tile_e), I32(o.tile_m0), I32(o.nwide), I32(o.wide_e), I32(o.wide_m0), I32(o.ord_e), I32(o.ord_m0)};
+  if (T * topk <= kBucketPicks && bucket_lds(T, topk, E) <= kBucketLds && !order) {
+    if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(k_pf_bucket), kBucketLds)) return rc;
+    const BucketArgs a{idx, w, T, topk, E, desc, I32(o.cnt), I32(o.off), I32(o.perm), I32(o.pickpos), I32(o.rpos), I32(o.re), F32(o.rk), posw, tl, x, H, W + o.xq, F32(o.xs)};
+    const size_t nq = quant ? (size_t)T * (H / 128) : 0;
+    hipLaunchKernelGGL(k_pf_bucket, dim3((unsigned)(1 + (nq + kBucketThreads / 16 - 1) / (kBucketThreads / 16))), dim3(kBucketThreads), bucket_lds(T, topk, E), st, a);
+    DSGX_HIP(hipGetLastError());
+    return DSGX_OK;
+  }
+  const int NB = (T + kRowBlock - 1) / kRowBlock;
+  uint32_t* bmask = reinterpret_cast<uint32_t*>(W + o.bmask);
+  hipLaunchKernelGGL(k_pf_mask, dim3(NB), dim3(256), 0, st, idx, T, topk, E, I32(o.bcnt), bmask);
+  hipLaunchKernelGGL(k_pf_scan, dim3(1), dim3(DSGX_MAX_EXPERTS), 0, st, I32(o.bcnt), NB, E, I32(o.boff), I32(o.cnt), I32(o.off), tl, order);
+  hipLaunchKernelGGL(k_pf_place, dim3(NB), dim3(256), 0, st, idx, w, T, topk, E, I32(o.off), I32(o.boff), bmask, desc, I32(o.perm), I32(o.pickpos), I32(o.rpos),
+                     I32(o.re), F32(o.rk), posw);
+  DSGX_HIP(hipGetLastError());
+  return quant ? dsgx_act_quant(x, T, H, W + o.xq, F32(o.xs), st) : DSGX_OK;
+}
+
 // ---- the grouped GEMMs ---------------------------------------------------------------------------------------------------
 // FP8 activations (e4m3 MFMA): pf_gemm_fp8.cuh. bf16 activations (bf16 MFMA): k_pf_gemm16 below.
 constexpr int kWgRows = 256;                     // weight rows a workgroup (UP: 128 channels)
@@ -742,15 +877,10 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
   if (order > 2) return fail(DSGX_EINVAL, "moe_prefill: tile_order %d (-1, 0, 1, 2)", cfg.tile_order);
   if (i4 || !cfg.act_fp8) order = 0;  // (the bf16-activation kernels walk the 128-position list)
 
+  const bool fp8_rows = !i4 && cfg.act_fp8 && (cfg.phases & (2 | 16));  // the GEMMs read x quantised
+  if (fp8_rows && (H > 8192 || I > 8192)) return fail(DSGX_EUNSUPPORTED, "moe_prefill: FP8 activations: hidden %d, intermediate %d (up to 8192)", H, I);
   if (cfg.phases & 1) {
-    const int NB = (T + kRowBlock - 1) / kRowBlock;
-    uint32_t* bmask = reinterpret_cast<uint32_t*>(W + o.bmask);
-    hipLaunchKernelGGL(k_pf_mask, dim3(NB), dim3(256), 0, st, idx, T, topk, E, I32(o.bcnt), bmask);
-    const TileLists tl{I32(o.ntiles), I32(o.tile_e), I32(o.tile_m0), I32(o.nwide), I32(o.wide_e), I32(o.wide_m0), I32(o.ord_e), I32(o.ord_m0)};
-    hipLaunchKernelGGL(k_pf_scan, dim3(1), dim3(DSGX_MAX_EXPERTS), 0, st, I32(o.bcnt), NB, E, I32(o.boff), I32(o.cnt), I32(o.off), tl, order);
-    hipLaunchKernelGGL(k_pf_place, dim3(NB), dim3(256), 0, st, idx, w, T, topk, E, I32(o.off), I32(o.boff), bmask, L->desc, I32(o.perm),
-                       I32(o.pickpos), I32(o.rpos), I32(o.re), F32(o.rk), (float*)nullptr);
-    DSGX_HIP(hipGetLastError());
+    if (int rc = bucket(o, W, idx, w, T, topk, E, L->desc, nullptr, order, x, H, fp8_rows, st)) return rc;
   }
   if (i4 || !cfg.act_fp8) {
     // bf16 activations throughout: x -> h (bf16) -> d (f32 a pick) -> combine; the shared expert likewise -> ys.
@@ -845,7 +975,7 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
   // 2048, 256 experts: T = 17 387 -> 341 us, T = 200 1061 -> 973, T = 2000 1565 -> 1544, T = 8192 within the noise; same bits).
   const int sh_tiles = (T + pf8::kMaxPos - 1) / pf8::kMaxPos;
   const bool fused_sh = shared && (cfg.phases & (2 | 4 | 16)) == (2 | 4 | 16);
-  if (cfg.phases & (2 | 16)) {
+  if (fp8_rows && !(cfg.phases & 1)) {
     if (int rc = dsgx_act_quant(x, T, H, W + o.xq, F32(o.xs), stream)) return rc;
   }
   if (cfg.phases & 2) {
@@ -982,14 +1112,7 @@ int dsgx_dsk_moe_prefill(const dsgx_dsk_weights* Wt, const uint8_t* xq, const ui
   uint16_t* dsh = U16(o.d + align256((size_t)P * H * 2));  // the shared expert's outputs behind the picks', both bf16
   // phases (dsk::MoePCfg, dsk.h:278-282): 1 bucketing, 2 shared expert, 4 routed up, 8 routed down, 16 combine
   if (cfg.phases & 1) {
-    const int NB = (T + kRowBlock - 1) / kRowBlock;
-    uint32_t* bmask = reinterpret_cast<uint32_t*>(W + o.bmask);
-    hipLaunchKernelGGL(k_pf_mask, dim3(NB), dim3(256), 0, st, idx, T, topk, E, I32(o.bcnt), bmask);
-    const TileLists tl{I32(o.ntiles), I32(o.tile_e), I32(o.tile_m0), I32(o.nwide), I32(o.wide_e), I32(o.wide_m0), I32(o.ord_e), I32(o.ord_m0)};
-    hipLaunchKernelGGL(k_pf_scan, dim3(1), dim3(DSGX_MAX_EXPERTS), 0, st, I32(o.bcnt), NB, E, I32(o.boff), I32(o.cnt), I32(o.off), tl, 0);
-    hipLaunchKernelGGL(k_pf_place, dim3(NB), dim3(256), 0, st, idx, w, T, topk, E, I32(o.off), I32(o.boff), bmask, (const dsgx_mat_desc*)nullptr, I32(o.perm),
-                       I32(o.pickpos), I32(o.rpos), I32(o.re), F32(o.rk), F32(o.posw));
-    DSGX_HIP(hipGetLastError());
+    if (int rc = bucket(o, W, idx, w, T, topk, E, nullptr, F32(o.posw), 0, nullptr, 0, false, st)) return rc;
   }
   pfmx::Args g{};
   g.H = H, g.I = I, g.nrows = T, g.limit = cfg.swiglu_limit;

@@ -187,6 +187,26 @@ def test_prefill_fp8_scale_groups(H, I, T, unit_rule):
     test_prefill_fp8_against_oracle(H, I, 4, 2, T, "fp8", unit_rule)
 
 
+@pytest.mark.parametrize("E,topk,T", [(3, 1, 1), (40, 8, 31), (40, 8, 33), (256, 8, 512), (256, 8, 513), (512, 2, 2048), (5, 1, 4096), (5, 1, 4097)])
+def test_prefill_buckets_at_the_edges_of_one_workgroup(E, topk, T):
+    """the bucketing as one launch (up to 4096 picks whose masks fit LDS) and as three: offsets, rows in token order, each row's picks in
+    expert-id order and its factors, words of 32 rows that are full, one row more, and more words than lanes"""
+    H, I = 256, 128
+    hl = helpers.make_layer(abi.FMT_FP8, H, I, E, topk, 3, seed=8, shared=None)
+    x, _, idx, w = helpers.rows_and_routing(19, T, H, E, topk, 1.0)
+    _, _, ws, dl = _prefill(hl, x, idx, w, T)
+    v, P = lib.prefill_view(dl.w, ws, T), T * topk
+    off = gpu.host(gpu.view(ws, v.off, (E + 1) * 4), np.int32, (E + 1,))
+    assert np.array_equal(off, np.concatenate([[0], np.cumsum(np.bincount(idx.reshape(-1), minlength=E))]))
+    order = np.argsort(idx.reshape(-1), kind="stable")
+    assert np.array_equal(gpu.host(gpu.view(ws, v.perm, P * 4), np.int32, (P,)), order // topk)
+    pos = np.empty(P, np.int32)
+    pos[order] = np.arange(P)
+    by_e = np.argsort(idx, axis=1)
+    assert np.array_equal(gpu.host(gpu.view(ws, v.re, P * 4), np.int32, (T, topk)), np.take_along_axis(idx, by_e, 1))
+    assert np.array_equal(gpu.host(gpu.view(ws, v.rpos, P * 4), np.int32, (T, topk)), np.take_along_axis(pos.reshape(T, topk), by_e, 1))
+
+
 def test_prefill_rows_do_not_depend_on_the_chunk():
     """a row's result is the same bits whatever else is in the chunk (bucket positions differ)"""
     H, I, E, topk = 256, 256, 8, 2
