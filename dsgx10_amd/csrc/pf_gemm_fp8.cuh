@@ -2,7 +2,7 @@
 // (ds41f-4xgx10-switchless/ref/torchref/kernel.py:105-125, ref/inference/kernel.py:207-274 of the reference): per 128-k
 // block the e4m3 x e4m3 products summed in f32 from zero, then acc = fma(x_scale * w_scale, partial, acc).
 //
-// A workgroup (4 waves, two workgroups a CU) computes one tile of up to 32, 64 or 160 positions against 256 weight rows (UP: 128
+// A workgroup (4 waves, two workgroups a CU) computes one tile of up to 32 or 160 positions against 256 weight rows (UP: 128
 // channels, gate and up): a wave owns 64 weight rows and every position. Two workgroups a CU, because their barriers, first loads
 // and epilogues are not each other's: as one workgroup of eight waves and 256 positions, a tile's first stage and epilogue (4 and
 // 12 of 84 us) and every wait for its slowest load left the CU idle (hidden 4096, intermediate 2048, 256 experts, whole call,
@@ -51,15 +51,17 @@ constexpr int kWgRows = 256;      // weight rows a workgroup (UP: 128 channels)
 constexpr int kThreads = 512;     // (the other formats' kernels)
 constexpr int kWaves = 4, kThreads4 = 64 * kWaves;
 
-// LDS of one of two workgroups on a CU: the waves' own rings of weight tiles (as deep as fits beside the rest: a slot is free when its
-// fragments are read, so kRing - 4 tiles come two turns ahead and four one turn), two stages of activations, two buffers of scales.
+// LDS of one of two workgroups on a CU: the waves' own rings of weight tiles (a slot is free when its fragments are read, so RING - 4
+// tiles come two turns ahead and four one turn), two stages of activations, two buffers of scales. Deeper rings are no gain where many
+// tiles are in flight: a shape of 64 positions and 7 tiles was slower than the widest with 4 (T = 1200 1361 -> 1308 us), and
+// dsgx_moe_prefill says where 32 positions take 8.
 constexpr int kMaxPos = 160;
-template <int POS>
+template <int POS, int RING = 4>
 struct Shape {
   static constexpr int kPos = POS;                 // positions of a tile
   static constexpr int kSub = POS / 16;            // its 16-position tiles
   static constexpr int RA = 4;                     // 16-row tiles a wave
-  static constexpr int kRing = POS == kMaxPos ? 4 : POS == 64 ? 7 : 8; // the wave's own ring of weight tiles, 2 KiB each
+  static constexpr int kRing = RING;               // the wave's own ring of weight tiles, 2 KiB each
   static constexpr int kHX = POS / 32;             // 8-position half tiles that a wave brings
   static constexpr int kStageX = POS * 128;        // a block's activations; two stages
   static constexpr int kOffX = kWaves * kRing * 2048, kOffS = kOffX + 2 * kStageX;
@@ -67,7 +69,7 @@ struct Shape {
   static constexpr int kGroup = POS * 4 * kSB;
   static constexpr int kLds = kOffS + 2 * kGroup;  // (the epilogues reuse it: UP kPos x 256 B, DOWN 4 x 4 KiB)
 };
-constexpr int kLds = std::max({Shape<kMaxPos>::kLds, Shape<64>::kLds, Shape<32>::kLds});
+constexpr int kLds = std::max({Shape<kMaxPos>::kLds, Shape<32, 5>::kLds, Shape<32, 8>::kLds});
 static_assert(2 * kLds <= 160 * 1024, "two workgroups a CU");
 
 // Workgroup -> (position tile, group of weight rows): blocks of 2^tl consecutive tiles x 2^nl row groups get consecutive workgroup
@@ -122,6 +124,7 @@ struct Args {
   const int* off;
   int nrows;           // the shared expert's rows: T
   int fast_act;        // UP: SwiGLU by the plain formula (swiglu4)
+  int deep;            // small tiles take deep rings
   dsgx_layer_w L;
   uint16_t* h;         // UP: h bf16 [position][I]
   uint8_t* hq;         // UP: h quantised, e4m3 [position][I]
@@ -171,9 +174,9 @@ __device__ __forceinline__ int sc_half(int r, int h) { return (h ^ (r >> 3)) & 1
 __device__ __forceinline__ int sw4(int r) { return (((r >> 2) ^ (r >> 3)) & 1) << 1 | ((r >> 3) & 1); }
 
 // one tile: expert e (-1: the shared expert), rows [m0, mend) of the activations' positions, row group ns
-template <bool UP, int POS>
+template <bool UP, int POS, int RING>
 __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, int m0, int mend, int ns) {
-  using S = Shape<POS>;
+  using S = Shape<POS, RING>;
   const int K = UP ? g.L.H : g.L.I, KB = K / 128;
   if (mend > m0 + S::kPos) mend = m0 + S::kPos;  // (the tile's own rows)
   const uint8_t *wa, *wb;  // UP: gate, up; DOWN: down twice
@@ -338,7 +341,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
     if (N == S::kSub || nmt == N) run(n);
     else if constexpr (N < S::kSub) self(self, std::integral_constant<int, N + 1>{});
   };
-  run_nj(run_nj, std::integral_constant<int, POS == kMaxPos ? 5 : POS == 64 ? 3 : 1>{});
+  run_nj(run_nj, std::integral_constant<int, POS == kMaxPos ? 3 : 1>{});
   wait_loads<0>();   // the trailing loads into unused slots: nothing may still be landing in LDS from here on
   __syncthreads();   // ... in any wave's part of it: the epilogues reuse the stages
   PF_STAMP(g, 5);
@@ -421,9 +424,9 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
 // a tile in the shape that its rows take
 template <bool UP>
 __device__ __forceinline__ void any_tile(const Args& g, uint8_t* smem, int e, int m0, int mend, int ns) {
-  if (mend - m0 > 64) gemm_tile<UP, kMaxPos>(g, smem, e, m0, mend, ns);
-  else if (mend - m0 > 32) gemm_tile<UP, 64>(g, smem, e, m0, mend, ns);
-  else gemm_tile<UP, 32>(g, smem, e, m0, mend, ns);
+  if (mend - m0 > 32) gemm_tile<UP, kMaxPos, 4>(g, smem, e, m0, mend, ns);
+  else if (g.deep) gemm_tile<UP, 32, 8>(g, smem, e, m0, mend, ns);
+  else gemm_tile<UP, 32, 5>(g, smem, e, m0, mend, ns);
 }
 // The shared expert: tiles of 128 rows over [0, nrows).
 template <bool UP>

@@ -48,7 +48,7 @@ struct Shape {
   static constexpr int kPos = POS, kSub = POS / 16, RA = 4, TB = TB_;
   static constexpr int kRowB = F4 ? 64 * TB : 128;  // bytes of a weight row in a turn
   static constexpr int kTileB = 16 * kRowB, LT = kRowB / 64;  // a 16-row weight tile, its loads
-  static constexpr int kRing = F4 ? (TB == 1 ? 5 : POS == 32 ? 6 : 4) : POS == 128 ? 4 : 6;  // the wave's own ring of weight tiles
+  static constexpr int kRing = F4 ? (POS == 32 ? 6 : 4) : POS == 128 ? 4 : 6;  // the wave's own ring of weight tiles
   static constexpr int kStageX = POS * 128;         // one block's activations; two stages of TB blocks
   static constexpr int kHX = POS / 8 / kWaves;      // the 8-position half tiles that a wave brings
   static constexpr int kOffX = kWaves * kRing * kTileB, kOffS = kOffX + 2 * TB * kStageX;

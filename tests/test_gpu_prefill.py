@@ -219,8 +219,8 @@ def test_prefill_rows_do_not_depend_on_the_chunk():
 
 @pytest.mark.parametrize("H,I", [(256, 128), (1280, 1152)])
 def test_prefill_fp8_tile_shapes_give_the_same_bits(H, I):
-    """experts whose rows end at the edges of the tiles of 32, 64 and 160 positions (and one row beyond): every row has the bits that it
-    has alone in a chunk, in the smallest tile"""
+    """experts whose rows end at the edges of the tiles of 32 and 160 positions and of their 16-position tiles (and one row beyond): every
+    row has the bits that it has alone in a chunk, in the smallest tile (with deep rings there)"""
     counts, topk = [1, 8, 9, 32, 33, 64, 65, 160, 161, 321], 1
     hl = helpers.make_layer(abi.FMT_FP8, H, I, len(counts), topk, 5, seed=14, shared="fp8")
     idx = np.repeat(np.arange(len(counts), dtype=np.int32), counts)[:, None].copy()
