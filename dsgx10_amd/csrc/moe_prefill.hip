@@ -895,7 +895,8 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
     q.tile_e = I32(o.tile_e), q.tile_m0 = I32(o.tile_m0), q.ntiles = I32(o.ntiles), q.off = I32(o.off), q.nrows = P;
     // INT4 experts: the LDS-staged kernels of pf_gemm_i4.cuh (DSGX_PF_I4_OLD=1: the register-ring kernel they replaced, same bits)
     const char* old4 = std::getenv("DSGX_PF_I4_OLD");
-    const bool new4 = i4 && !(old4 && old4[0] == '1');
+    const bool small4 = std::max((size_t)T * H, (size_t)kTile * I) * 2 < ((size_t)1 << 32);  // (its offsets of activation rows are 32 bits)
+    const bool new4 = i4 && small4 && !(old4 && old4[0] == '1');
     const auto k_dn4 = I % 256 ? pfi4::k_gemm<false, false> : pfi4::k_gemm<false, true>;
     pfi4::Args q4{};
     if (new4) {
@@ -914,14 +915,14 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
       q.x = x, q.gather = I32(o.perm), q.h = reinterpret_cast<uint16_t*>(W + o.h), q.d = nullptr;
       if (fused_sh) q4.sh_grid = sh_gu, q4.sh = sh_up;
       q4.x = q.x, q4.gather = q.gather, q4.h = q.h, q4.d = nullptr;
-      if (new4) hipLaunchKernelGGL((pfi4::k_gemm<true, true>), dim3(q4.sh_grid + pf8::grid_of(o.max_tiles, I / (kWgRows / 2))), dim3(pf8::kThreads), pfi4::kLdsRun, st, q4);
+      if (new4) hipLaunchKernelGGL((pfi4::k_gemm<true, true>), dim3(q4.sh_grid + pf8::grid_of(o.max_tiles, I / (kWgRows / 2), pfi4::map_of(I / (kWgRows / 2)))), dim3(pf8::kThreads4), pfi4::kLdsRun, st, q4);
       else hipLaunchKernelGGL(k_up, dim3(pf_grid(o.max_tiles, I / (kWgRows / 2))), dim3(kGemmThreads), lds16, st, q);
     }
     if (cfg.phases & 4) {
       q.x = reinterpret_cast<const uint16_t*>(W + o.h), q.gather = nullptr, q.h = nullptr, q.d = F32(o.d);
       q4.x = q.x, q4.gather = nullptr, q4.h = nullptr, q4.d = q.d;
       if (fused_sh) q4.sh_grid = sh_gd, q4.sh = sh_dn;
-      if (new4) hipLaunchKernelGGL(k_dn4, dim3(q4.sh_grid + pf8::grid_of(o.max_tiles, H / kWgRows)), dim3(pf8::kThreads), pfi4::kLdsRun, st, q4);
+      if (new4) hipLaunchKernelGGL(k_dn4, dim3(q4.sh_grid + pf8::grid_of(o.max_tiles, H / kWgRows, pfi4::map_of(H / kWgRows))), dim3(pf8::kThreads4), pfi4::kLdsRun, st, q4);
       else hipLaunchKernelGGL(k_dn, dim3(pf_grid(o.max_tiles, H / kWgRows)), dim3(kGemmThreads), lds16, st, q);
     }
     if (cfg.phases & 8) {
@@ -931,8 +932,8 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
       if (i4) {
         for (const void* k : {(const void*)pfb16::k_gemm<true>, (const void*)pfb16::k_gemm<false>})
           if (int rc = allow_dynamic_lds(k, pfb16::kLds)) return rc;
-        hipLaunchKernelGGL(pfb16::k_gemm<true>, dim3(sh_gu), dim3(pf8::kThreads), pfb16::kLds, st, sh_up);
-        hipLaunchKernelGGL(pfb16::k_gemm<false>, dim3(sh_gd), dim3(pf8::kThreads), pfb16::kLds, st, sh_dn);
+        hipLaunchKernelGGL(pfb16::k_gemm<true>, dim3(sh_gu), dim3(pf8::kThreads4), pfb16::kLds, st, sh_up);
+        hipLaunchKernelGGL(pfb16::k_gemm<false>, dim3(sh_gd), dim3(pf8::kThreads4), pfb16::kLds, st, sh_dn);
       } else {
         const int tiles = (T + kTile - 1) / kTile;
         q.tile_e = q.tile_m0 = q.ntiles = q.off = nullptr, q.nrows = T;

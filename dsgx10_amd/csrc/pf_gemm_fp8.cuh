@@ -81,7 +81,7 @@ struct Map {
 constexpr Map kMap{3, 2};
 // ... with as many row groups as divide NS: a block of fewer groups than the others always falls to the same XCDs where the blocks of a tile
 // are 2, 4 or 8 (ten row groups as 8 + 2: four XCDs with four times the others' work)
-inline Map map_of(int tl, int nl, int NS) {
+__host__ __device__ inline Map map_of(int tl, int nl, int NS) {
   while (nl > 0 && NS % (1 << nl)) --nl;
   return Map{tl, nl};
 }
@@ -148,6 +148,10 @@ __device__ __forceinline__ void dma16(const uint8_t* src, uint32_t lds_base) {
 // ... from a wave-uniform address and the lane's offset
 __device__ __forceinline__ void dma16(const uint8_t* base, uint32_t off, uint32_t lds_base) {
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(off), "s"(base) : "memory");
+}
+// ... as a streaming load, for what one workgroup of an XCD reads once
+__device__ __forceinline__ void dma16_nt(const uint8_t* base, uint32_t off, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_base), "v"(off), "s"(base) : "memory");
 }
 // f(0), f(1), ... f(N - 1) as constants (a loop over 40 accumulators with a way out in it is past the size that the compiler unrolls)
 template <int... I, class F>

@@ -381,6 +381,32 @@ def test_prefill_int4_rings_at_the_edges_of_k_and_of_the_tiles(H, I, T):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("I", [256, 384])
+@pytest.mark.parametrize("T", [1, 16, 17, 33, 48, 49, 65, 96, 97, 128, 129, 161])
+def test_prefill_int4_tiles_of_every_height(I, T):
+    """pf_gemm_i4.cuh's tiles: 16-row MFMAs for up to 64 positions (by sixteens, odd numbers of them too), 32-row ones for more (96, 128), K in
+    pairs of 128-k blocks and an odd number of them, and each redone for large scales - the register-ring kernel's bits"""
+    import os
+    H, E, topk = 512, 3, 3
+    for large in (False, True):
+        if large:
+            hl, x, idx, w = helpers.int4_layer_with_large_scales(H, I, E, topk, 61, T)
+        else:
+            hl = helpers.make_layer(abi.FMT_INT4, H, I, E, topk, 3, seed=67, shared=None)
+            x, _, idx, w = helpers.rows_and_routing(71, T, H, E, topk, 2.5)
+        outs = []
+        for old in ("0", "1"):
+            os.environ["DSGX_PF_I4_OLD"] = old
+            try:
+                yr, _, ws, dl = _prefill(hl, x, idx, w, T)
+                v = lib.prefill_view(dl.w, ws, T)
+                outs.append((yr.view(np.uint32), gpu.host(gpu.view(ws, v.h, T * topk * I * 2), np.uint16, (-1,))))
+            finally:
+                os.environ.pop("DSGX_PF_I4_OLD", None)
+        for a, b in zip(*outs):
+            assert np.array_equal(a, b), large
+
+
 def test_prefill_int4_scales_above_the_fast_decodes_range():
     """scales of 2^116 and more make a workgroup do its tile once more by the routine for every scale: the bits of the
     register-ring kernel, which has that routine only, in tiles of 128 positions and in ragged ones"""
