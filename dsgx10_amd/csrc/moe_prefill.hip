@@ -1122,6 +1122,9 @@ int dsgx_dsk_moe_prefill(const dsgx_dsk_weights* Wt, const uint8_t* xq, const ui
   g.H = H, g.I = I, g.nrows = T, g.limit = cfg.swiglu_limit;
   // (as for the FP8 layers; 1 tile x 2 / 4 x 2, T = 20
   // 237 / 246 us, T = 60 411 / 419, T = 300 803 / 812, T = 1000 1076 / 1078, T = 2000 1267 / 1245, T = 6000 2103 / 2015)
+  // (streaming loads of small tiles' weights, as the FP8 layers', while tiles are small: T = 20 / 60 / 300 / 500 249 / 409 / 781 / 948 -> 226 / 366 /
+  // 771 / 947 us, T = 700 / 1000 / 3000 1021 / 1084 / 1460 -> 1034 / 1100 / 1472)
+  g.stream = P < 12 * E;
   auto map_for = [&](int NS) { return (long long)P >= 24LL * E ? pf8::map_of(2, 1, NS) : pf8::map_of(0, 1, NS); };
   // a whole step runs the shared expert's tiles in the routed experts' launches, in front of them (as the FP8 layers do;
   // hidden 5120, intermediate 2304, T = 17: 417 -> 362 us, T = 600: 1405 -> 1334, T = 3000: 1870 -> 1821)

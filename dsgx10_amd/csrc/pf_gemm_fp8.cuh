@@ -153,6 +153,11 @@ __device__ __forceinline__ void dma16(const uint8_t* base, uint32_t off, uint32_
 __device__ __forceinline__ void dma16_nt(const uint8_t* base, uint32_t off, uint32_t lds_base) {
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_base), "v"(off), "s"(base) : "memory");
 }
+template <bool STREAM>
+__device__ __forceinline__ void dma16_w(const uint8_t* base, uint32_t off, uint32_t lds_base) {
+  if constexpr (STREAM) dma16_nt(base, off, lds_base);
+  else dma16(base, off, lds_base);
+}
 // f(0), f(1), ... f(N - 1) as constants (a loop over 40 accumulators with a way out in it is past the size that the compiler unrolls)
 template <int... I, class F>
 __device__ __forceinline__ void static_for(std::integer_sequence<int, I...>, F f) {
@@ -178,7 +183,7 @@ __device__ __forceinline__ int sc_half(int r, int h) { return (h ^ (r >> 3)) & 1
 __device__ __forceinline__ int sw4(int r) { return (((r >> 2) ^ (r >> 3)) & 1) << 1 | ((r >> 3) & 1); }
 
 // one tile: expert e (-1: the shared expert), rows [m0, mend) of the activations' positions, row group ns
-template <bool UP, int POS, int RING>
+template <bool UP, int POS, int RING, bool STREAM>
 __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, int m0, int mend, int ns) {
   using S = Shape<POS, RING>;
   const int K = UP ? g.L.H : g.L.I, KB = K / 128;
@@ -236,7 +241,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   // its fragments. Activations: a stage a block.
   const uint32_t ring0 = lds0 + (uint32_t)wave * (S::kRing * 2048);
   auto issue_w = [&](int kb, int t, int slot, int hh) {
-    dma16(wt[t] + (size_t)min(kb, KB - 1) * 128, ow[hh], uni(ring0 + (uint32_t)slot * 2048 + hh * 1024));
+    dma16_w<STREAM>(wt[t] + (size_t)min(kb, KB - 1) * 128, ow[hh], uni(ring0 + (uint32_t)slot * 2048 + hh * 1024));
   };
   auto issue_x = [&](int kb) {
     const uint32_t xbase = lds0 + S::kOffX + (uint32_t)(kb & 1) * S::kStageX + (uint32_t)wave * (1024 * S::kHX);
@@ -425,12 +430,15 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   PF_STAMP(g, 6);
 }
 
-// a tile in the shape that its rows take
+// A tile in the shape that its rows take. `only`: it is its expert's only one. Nobody else reads its weights then, and as streaming loads they
+// leave what others share (activations, scales) in L2: T = 20 / 60 / 200 / 700 / 1500 345 / 590 / 964 / 1241 / 1380 -> 316 / 552 / 900 / 1199 /
+// 1373 us; a remainder's weights as well, T = 8192 2825 -> 2880, and the widest tiles' too, T = 200 929, T = 8192 3400.
 template <bool UP>
-__device__ __forceinline__ void any_tile(const Args& g, uint8_t* smem, int e, int m0, int mend, int ns) {
-  if (mend - m0 > 32) gemm_tile<UP, kMaxPos, 4>(g, smem, e, m0, mend, ns);
-  else if (g.deep) gemm_tile<UP, 32, 8>(g, smem, e, m0, mend, ns);
-  else gemm_tile<UP, 32, 5>(g, smem, e, m0, mend, ns);
+__device__ __forceinline__ void any_tile(const Args& g, uint8_t* smem, int e, int m0, int mend, int ns, bool only) {
+  if (mend - m0 > 32) gemm_tile<UP, kMaxPos, 4, false>(g, smem, e, m0, mend, ns);
+  else if (g.deep) gemm_tile<UP, 32, 8, true>(g, smem, e, m0, mend, ns);
+  else if (only) gemm_tile<UP, 32, 5, true>(g, smem, e, m0, mend, ns);
+  else gemm_tile<UP, 32, 5, false>(g, smem, e, m0, mend, ns);
 }
 // The shared expert: tiles of 128 rows over [0, nrows).
 template <bool UP>
@@ -440,7 +448,7 @@ __global__ void __launch_bounds__(kThreads4, 2) k_gemm(Args g) {
   int tile, ns;
   task_of<true>(NS, tile, ns);
   if (ns >= NS || tile * kMaxPos >= g.nrows) return;
-  any_tile<UP>(g, smem, -1, tile * kMaxPos, g.nrows, ns);
+  any_tile<UP>(g, smem, -1, tile * kMaxPos, g.nrows, ns, tile == 0);
 }
 // The routed experts' list, an expert's tiles next to each other, behind the shared expert's tiles.
 template <bool UP>
@@ -457,7 +465,7 @@ __global__ void __launch_bounds__(kThreads4, 2) k_gemm_mixed(Args g) {
     q.trace = nullptr;
 #endif
     q.aq = g.sh.aq, q.as = g.sh.as, q.gather = nullptr, q.h = g.sh.h, q.hq = g.sh.hq, q.hs = g.sh.hs, q.d = g.sh.d;
-    any_tile<UP>(q, smem, -1, m0, mend, ns);
+    any_tile<UP>(q, smem, -1, m0, mend, ns, tile == 0);
     return;
   }
   PF_STAMP(g, 0);
@@ -469,7 +477,7 @@ __global__ void __launch_bounds__(kThreads4, 2) k_gemm_mixed(Args g) {
 #ifdef DSGX_PF_TRACE
   if (g.trace && threadIdx.x == 0) g.trace[(size_t)(blockIdx.x - g.sh.grid) * 8 + 7] = min(mend - m0, kMaxPos);
 #endif
-  any_tile<UP>(g, smem, e, m0, mend, ns);
+  any_tile<UP>(g, smem, e, m0, mend, ns, g.tile_m0[tile] == 0);
 }
 
 }  // namespace pf8

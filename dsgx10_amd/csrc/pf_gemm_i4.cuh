@@ -32,7 +32,7 @@ namespace pfi4 {
 
 
 using pf8::dma16;
-using pf8::dma16_nt;
+using pf8::dma16_w;
 using pf8::kThreads4;
 using pf8::kWaves;
 using pf8::kWgRows;
@@ -164,11 +164,12 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
     for (int i = 0; i < loads_x(MT * NJ); ++i)
       dma16(x0 + (size_t)kb * 256 + (turn & 1) * 32, ox[i], uni(lds0 + (uint32_t)(stage * (NJ * MT * 128) + x_group(NJ, i) * 1024)));
   };
-  // (weights as streaming loads: gate/up with 8 / 64 rows an expert 539 / 753 -> 506 / 726 us)
+  // (small tiles' weights as streaming loads, mostly their expert's only tile: gate/up with 8 / 64 rows an expert 539 / 753 -> 506 / 726 us; tall
+  // tiles' not, their expert has others that find them in L2: hidden 3840, intermediate 768, 20 experts, T = 1500 406 -> 381)
   auto load_w = [&](int q, int i) {  // PAIR: pair q, rows 8 i ... of the wave's; else block q, rows 16 i ...
     constexpr int kRows = PAIR ? 8 : 16;
     const int t = kRows * i / MT;
-    dma16_nt(wt[t] + (size_t)min(q, PAIR ? KB / 2 - 1 : KB - 1) * (PAIR ? 128 : 64) + (size_t)(kRows * i % MT) * (K / 2), ow[PAIR ? i & 1 : 0],
+    dma16_w<MT == 16>(wt[t] + (size_t)min(q, PAIR ? KB / 2 - 1 : KB - 1) * (PAIR ? 128 : 64) + (size_t)(kRows * i % MT) * (K / 2), ow[PAIR ? i & 1 : 0],
              uni(lds0 + kOffW + (uint32_t)wave * kW + (PAIR ? 0 : (q & 1) * 4096) + i * 1024));
   };
   auto load_b = [&](int kb, bool odd, int i) {  // load i of loads()
@@ -359,8 +360,8 @@ __global__ void __launch_bounds__(kThreads4, 2) k_gemm(Args g) {
   if (ns >= NS || tile >= *g.ntiles) return;
   const int e = g.tile_e[tile];
   const int m0 = g.off[e] + g.tile_m0[tile], mend = g.off[e + 1];
-  if (mend - m0 > 64) gemm_tile<UP, PAIR, 32>(g, smem, e, m0, mend, ns);
-  else gemm_tile<UP, PAIR, 16>(g, smem, e, m0, mend, ns);
+  if (mend - m0 <= 64) gemm_tile<UP, PAIR, 16>(g, smem, e, m0, mend, ns);
+  else gemm_tile<UP, PAIR, 32>(g, smem, e, m0, mend, ns);
 }
 
 }  // namespace pfi4

@@ -75,6 +75,7 @@ struct Args {
   const int* ntiles;
   const int* off;
   int nrows;
+  int stream;          // weights of experts of one small tile as streaming loads
   int H, I;
   const uint8_t *wa, *sa, *wb, *sb;  // UP: gate (w1), up (w3); DOWN: w2 in wa / sa. Expert e at + e * wstride / sstride.
   size_t wstride, sstride;
@@ -99,7 +100,7 @@ __device__ __forceinline__ v4f_t mfma_mx(v8i_t a, v8i_t b, v4f_t c, int sa, int 
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, CBSZ, 0, 0, sa, 0, sb);
 }
 
-template <bool UP, int POS, int WF, int TB>
+template <bool UP, int POS, int WF, int TB, bool STREAM = false>
 __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, int m0, int mend, int ns) {
   using S = Shape<POS, WF, TB>;
   constexpr bool F4 = S::F4;
@@ -163,7 +164,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   // its fragments. Activations: a stage a turn.
   const int TN = KB / TB;
   auto issue_w = [&](int t, int i, int slot, int hh) {
-    dma16(wt[i] + (size_t)min(t, TN - 1) * S::kRowB, ow[hh], uni(ring0 + (uint32_t)slot * S::kTileB + hh * 1024));
+    pf8::dma16_w<STREAM>(wt[i] + (size_t)min(t, TN - 1) * S::kRowB, ow[hh], uni(ring0 + (uint32_t)slot * S::kTileB + hh * 1024));
   };
   auto issue_x = [&](int t) {
     const uint32_t xbase = lds0 + S::kOffX + (uint32_t)(t & 1) * (TB * S::kStageX) + (uint32_t)wave * (S::kHX * 1024);
@@ -433,6 +434,7 @@ __global__ void __launch_bounds__(kThreads4, 2) k_gemm_mixed(Args g) {
   const bool pairs = (UP ? g.H : g.I) % 256 == 0;
   if (mend - m0 > 64 || !pairs) gemm_tile<UP, kMaxPos, F4, 1>(g, smem, e, m0, mend, ns);
   else if (mend - m0 > 32) gemm_tile<UP, 64, F4, 2>(g, smem, e, m0, mend, ns);
+  else if (g.stream && g.tile_m0[tile] == 0) gemm_tile<UP, 32, F4, 2, true>(g, smem, e, m0, mend, ns);
   else gemm_tile<UP, 32, F4, 2>(g, smem, e, m0, mend, ns);
 }
 
