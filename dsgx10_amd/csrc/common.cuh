@@ -45,11 +45,11 @@ __device__ __forceinline__ void fp8x8_to_bf16(uint32_t w0, uint32_t w1, uint32_t
 // factor and gives (1024 + u) s - (1024 + u_z) s, or (1024 + 16 u) (s / 16) - (64 + u_z) s, and the packed conversion rounds
 // once to nearest even: 17 instructions for 8 values where byte conversions and fmas took 23 (the 1024-offset form of a nibble is
 // a widely used one). Every product and constant has at most 11 + 8 significant bits, so it is exact in f32, and so is the difference;
-// the constants stay finite for |s| < 2^116, which no checkpoint comes near: a decode step or a prefill tile that meets a larger
-// scale takes i4x8_to_bf16_any, whose terms are finite up to 2^124 (dequant_int4's own kernel uses the subtract-first form, for all).
+// the constants stay finite for |s| < 2^116, which no checkpoint comes near: a decode unit, a GEMV's rows or a prefill tile that meets a larger
+// scale is done once more by i4x8_to_bf16_any, whose terms are finite up to 2^124 (dequant_int4's own kernel uses the subtract-first form, for all).
 // Hidden 6144, intermediate 2048, 168 experts: gate/up's vector instructions at T = 1111 3.16e8 -> 2.69e8, the decode kernel's at 6
 // rows 8.6e7 -> 7.2e7; with the LDS slots that came with it the prefill call takes 1869 -> 1784 us, four decode layers 923 -> 909.
-// The vector-unit GEMV (rowdot.cuh) keeps i4x8_to_bf16_any: its two bodies cost it more (35.3 -> 36.7 us) than they save.
+// The split-K GEMV and the vector-unit decode kernels keep i4x8_to_bf16_any.
 struct I4Group {
   float s, c0;   // the scale, -(1024 + u_z) s
   float s1, c1;  // s / 16, -(64 + u_z) s

@@ -44,6 +44,35 @@ __device__ __forceinline__ void stage_rows(uint4* xs, const GemvArgs& a, float* 
 template <int FMT>
 __device__ __forceinline__ int last_seg_lanes(int K, int nsegk) { return (K - (nsegk - 1) * FmtT<FMT>::SEGK + FmtT<FMT>::KL - 1) / FmtT<FMT>::KL; }
 
+// A slice of a batch's rows (segments seg0, seg0 + sk, ...) by the INT4 routine for every scale, for the waves of k_gemv whose faster one
+// has met a scale of 2^116 or more (none in a checkpoint). The loop only keeps the largest (and these lines stand once, behind it: as part of
+// every step's code they made a call's first pass 10 us longer): 6144 x 16384 at 1 / 2 / 4 rows 17.9 / 19.7 / 24.1 ->
+// 17.2 / 19.1 / 23.3 us a call, 16384 x 2048 at one 9.2 -> 8.6 (a vote and both routines in every step were 4% slower than the long one alone).
+// k_gemv_sk's calls are over before it pays (768 x 6144 over 4 at one row 6.2 -> 6.45).
+template <int M, int RB>
+__device__ __forceinline__ void dot_any_scale(const GemvArgs& a, int row_, int seg0, int sk, const uint4* xs, int lane, float (&acc)[RB][M]) {
+  constexpr int FMT = DSGX_FMT_INT4_G32;
+  const int row = uni(row_);
+  int si = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxSegs; ++i)
+    if (i < a.nsegs && row >= a.sg[i].row0) si = i;
+  RowSrc src[RB];
+#pragma unroll
+  for (int i = 0; i < RB; ++i) {
+    src[i] = row_src<FMT>(a.sg[si].m, row - a.sg[si].row0 + i, a.K);
+#pragma unroll
+    for (int m = 0; m < M; ++m) acc[i][m] = 0.f;
+  }
+  for (int seg = seg0; seg < a.nsegk; seg += sk) {
+    const uint32_t le = lane < (seg == a.nsegk - 1 ? last_seg_lanes<FMT>(a.K, a.nsegk) : kWave) ? lane : 0;
+    Raw r[RB];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) load_row<FMT>(r[i], src[i], seg, le, 0, acc[i][0]);
+    step_dot<FMT, M, RB, true>(r, xs, a.nq, seg, lane, acc, a.K);
+  }
+}
+
 // NW: wavefronts a workgroup, in groups of four: the first batches of the walk go to every workgroup's first group, so that
 // fewer batches than wavefronts still spread over all CUs. SPLIT: the split-K order of adds (k_gemv_sk's slices, in their
 // order, the same bits) by one wavefront that walks the slices one after the other.
@@ -124,10 +153,10 @@ __global__ void __launch_bounds__(NW * 64) k_gemv(GemvArgs a) {
   };
   int cj = 0, csl = 0, cseg = 0;
   float mine = 0.f, mine2 = 0.f;  // lane r * M + m: output (row r, activation row m) of the batch, and the pair's other row (SwiGLU)
-  auto compute = [&](const Raw (&raw)[RB]) {
-    step_dot<FMT, M, RB, true>(raw, xs, a.nq, cseg, lane, acc, a.K);
-    if ((cseg += sk) < a.nsegk) return;
-    // the slice is complete: add the lanes' partials, then the slices' sums in their order
+  constexpr bool kI4 = FMT == DSGX_FMT_INT4_G32;
+  float smax = 0.f;  // INT4: the largest scale that the wave has met
+  // a slice is complete: add the lanes' partials, then the slices' sums in their order
+  auto slice_done = [&]() {
     float v1 = 0.f, v2 = 0.f;
 #pragma unroll
     for (int i = 0; i < RB; ++i)
@@ -158,6 +187,10 @@ __global__ void __launch_bounds__(NW * 64) k_gemv(GemvArgs a) {
       static_cast<uint16_t*>(sg.y)[(size_t)m * sg.ldy + n / 2] = (uint16_t)swiglu_bits(bf16_round(mine), bf16_round(mine2));
     }
   };
+  auto compute = [&](const Raw (&raw)[RB]) {
+    step_dot<FMT, M, RB, true, kI4>(raw, xs, a.nq, cseg, lane, acc, a.K, &smax);
+    if ((cseg += sk) >= a.nsegk) slice_done();
+  };
   // the first weight loads are issued before the activations are staged: one memory round trip, not two, before the
   // first product (these calls are a few microseconds long: latency is most of them)
 #pragma unroll
@@ -169,6 +202,15 @@ __global__ void __launch_bounds__(NW * 64) k_gemv(GemvArgs a) {
     for (int d = 0; d < D; ++d) {
       if (t + d < nsteps) compute(w[d]);
       load(w[d]);
+    }
+  }
+  if constexpr (kI4) {
+    if (__builtin_expect(i4_any_large(smax), 0)) {  // all of the wave's rows once more, each lane over its own results
+      cj = csl = 0;
+      while (cj < nmine) {
+        dot_any_scale<M, RB>(a, (gw + cj * GW) * RB, csl, sk, xs, lane, acc);
+        slice_done();
+      }
     }
   }
 }

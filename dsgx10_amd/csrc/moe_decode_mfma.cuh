@@ -268,6 +268,44 @@ __device__ __forceinline__ void mf_stream(const int M, uint8_t* smem, size_t row
     const u32x4_t bv = *reinterpret_cast<const u32x4_t*>(smem + xp + 2 * koff);
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf_t, av), __builtin_bit_cast(v8bf_t, bv), c, 0, 0, 0);
   };
+  // INT4: a step whose weights lie in W; any: by the routine for every scale. A stream that met a scale which i4x8_to_bf16 is not for
+  // (2^116 or more, none in a checkpoint) does the unit once more: the steps only keep the maximum. (With a vote and both routines
+  // in every step, and the longer one alone at one row, four layers of hidden 6144, intermediate 2048, 168 experts took 249 / 362 / 619 / 1056 us
+  // at 1 / 2 / 4 / 8 rows, 242 / 350 / 598 / 1027 like this.)
+  float smax = 0.f;
+  auto int4_step = [&](const Entry& e, auto any) {
+    const float s0 = bf16_bits_to_f32(e.s & 0xFFFFu), s1 = bf16_bits_to_f32(e.s >> 16);
+    const uint32_t z0 = (e.z.x >> zsh) & 15u, z1 = (e.z.y >> zsh) & 15u;
+    const I4Group g0 = i4_group(s0, z0), g1 = i4_group(s1, z1);
+    const float n0 = -((float)z0 * s0), n1 = -((float)z1 * s1);
+    smax = fmaxf(smax, fmaxf(fabsf(s0), fabsf(s1)));
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj) {
+      const u32x4_t pc = *reinterpret_cast<const u32x4_t*>(W + rd_off[jj]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        uint32_t o[4];
+        if constexpr (decltype(any)::value) i4x8_to_bf16_any(pc[j], jj ? s1 : s0, jj ? n1 : n0, o);
+        else i4x8_to_bf16(pc[j], jj ? g1 : g0, o);
+        acc = mfma(o, 32 * jj + 8 * j, acc);
+      }
+    }
+  };
+  auto int4_redo = [&](int u) {
+    const MfUnit m = open(u);
+    acc = v4f_t{0.f, 0.f, 0.f, 0.f};
+    xp = live ? xl + xoff_of(u) : zoff;
+    for (int st = 0; st < steps; ++st) {
+      Entry e;
+      const uint8_t* p = m.wp + (size_t)st * 128;
+      e.s = ldg_u32(m.sp + (size_t)st * 16);
+      e.z = *(const DSGX_GLOBAL u32x2_t*)(uintptr_t)(m.zp + (size_t)st * 32);
+      *reinterpret_cast<u32x4_t*>(W + wr_off[0]) = ldg_stream(p);
+      *reinterpret_cast<u32x4_t*>(W + wr_off[1]) = ldg_stream(p + m.half);
+      int4_step(e, std::true_type{});
+      xp += xstep;
+    }
+  };
   auto compute = [&](const Entry& e) {
     *reinterpret_cast<u32x4_t*>(W + wr_off[0]) = keep_whole(e.a);
     *reinterpret_cast<u32x4_t*>(W + wr_off[1]) = keep_whole(e.b);
@@ -312,31 +350,7 @@ __device__ __forceinline__ void mf_stream(const int M, uint8_t* smem, size_t row
         }
       }
     } else if constexpr (FMT == DSGX_FMT_INT4_G32) {
-      const float s0 = bf16_bits_to_f32(e.s & 0xFFFFu), s1 = bf16_bits_to_f32(e.s >> 16);
-      auto sums = [&](auto&& decode) {
-#pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
-          const u32x4_t pc = *reinterpret_cast<const u32x4_t*>(W + rd_off[jj]);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            uint32_t o[4];
-            decode(jj, pc[j], o);
-            acc = mfma(o, 32 * jj + 8 * j, acc);
-          }
-        }
-      };
-      const uint32_t z0 = (e.z.x >> zsh) & 15u, z1 = (e.z.y >> zsh) & 15u;
-      // (one row: the stream waits for its loads, not for the vector unit, and the vote costs more than the shorter decode saves:
-      // layers of 6144 x 2048, 168 experts, four of them 215.3 -> 209.4 us with one decode. With 96 experts, 28 shapes: 5120 x 2048
-      // 197.6 -> 189.6, 1024 x 2048 98.6 -> 94.8, the others 0-4%, except 1% the other way round at hidden 4096, 200.7 -> 203.0. At two
-      // rows the two are within 2%, at six the shorter decode gains 1%.)
-      if (M == 1 || __builtin_expect(i4_any_large(fmaxf(fabsf(s0), fabsf(s1))), 0)) {
-        const float n0 = -((float)z0 * s0), n1 = -((float)z1 * s1);
-        sums([&](int jj, uint32_t w, uint32_t (&o)[4]) { i4x8_to_bf16_any(w, jj ? s1 : s0, jj ? n1 : n0, o); });
-      } else {
-        const I4Group g0 = i4_group(s0, z0), g1 = i4_group(s1, z1);
-        sums([&](int jj, uint32_t w, uint32_t (&o)[4]) { i4x8_to_bf16(w, jj ? g1 : g0, o); });
-      }
+      int4_step(e, std::false_type{});
     } else {
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) {
@@ -349,6 +363,10 @@ __device__ __forceinline__ void mf_stream(const int M, uint8_t* smem, size_t row
     if (++cstep < steps) return;
     cstep = 0;
     // the unit is complete in this wave's slice
+    if constexpr (FMT == DSGX_FMT_INT4_G32) {
+      if (__builtin_expect(i4_any_large(smax), 0)) int4_redo(cu * ng + grp);
+      smax = 0.f;
+    }
     if (ns == 1) {
       done(cu * ng + grp, acc);
     } else {

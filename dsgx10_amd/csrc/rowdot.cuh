@@ -81,10 +81,11 @@ __device__ __forceinline__ void load_row(Raw& r, const RowSrc& s, int seg, uint3
 }
 
 // RB rows of one segment against M activation rows. xs: the workgroup's staged activations, row m at xs + m * nq
-// (nq chunks a row); acc[r][m] are the lanes' running sums.
-template <int FMT, int M, int RB, bool TAIL = false>
+// (nq chunks a row); acc[r][m] are the lanes' running sums. FAST (INT4): by i4x8_to_bf16, smax keeps the largest scale's magnitude: the
+// caller does the rows again without FAST if it is one that the routine is not for (i4_any_large).
+template <int FMT, int M, int RB, bool TAIL = false, bool FAST = false>
 __device__ __forceinline__ void step_dot(const Raw (&raw_in)[RB], const uint4* __restrict__ xs, int nq, int seg, int lane,
-                                         float (&acc)[RB][M], int K = 0) {
+                                         float (&acc)[RB][M], int K = 0, float* smax = nullptr) {
   using F = FmtT<FMT>;
   const uint4* xl = xs + (size_t)seg * F::XC * 64 + lane;
   Raw raw[RB];
@@ -129,10 +130,13 @@ __device__ __forceinline__ void step_dot(const Raw (&raw_in)[RB], const uint4* _
     }
   } else if constexpr (FMT == DSGX_FMT_INT4_G32) {
     float s[RB], nzs[RB];
+    I4Group grp[RB];
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
       s[r] = bf16_bits_to_f32(raw[r].aux & 0xFFFFu);
       nzs[r] = -((float)(raw[r].aux >> 16) * s[r]);
+      grp[r] = i4_group(s[r], raw[r].aux >> 16);
+      if constexpr (FAST) *smax = fmaxf(*smax, fabsf(s[r]));
     }
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
@@ -143,7 +147,8 @@ __device__ __forceinline__ void step_dot(const Raw (&raw_in)[RB], const uint4* _
       for (int r = 0; r < RB; ++r) {
         const uint32_t w = c == 0 ? raw[r].v.x : c == 1 ? raw[r].v.y : c == 2 ? raw[r].v.z : raw[r].v.w;
         uint32_t o[4];
-        i4x8_to_bf16_any(w, s[r], nzs[r], o);
+        if constexpr (FAST) i4x8_to_bf16(w, grp[r], o);
+        else i4x8_to_bf16_any(w, s[r], nzs[r], o);
 #pragma unroll
         for (int m = 0; m < M; ++m) {
           float t = acc[r][m];

@@ -201,6 +201,27 @@ def test_gemv_every_bit_against_the_oracle(case, sk):
     assert np.array_equal(got.view(np.uint32 if kind == abi.OUT_F32 else np.uint16), want.view(np.uint32 if kind == abi.OUT_F32 else np.uint16)), int((got != want).sum())
 
 
+@pytest.mark.parametrize("sk", [1, 2, 4])
+@pytest.mark.parametrize("N,K,M", [(4200, 2048 + 256, 1), (72, 4096, 3), (3080, 4096 + 256, 8)])
+def test_gemv_int4_scales_above_the_fast_decodes_range(N, K, M, sk):
+    """rows with scales of 2^116 and more, in first, inner and last groups of K, are done once more by the routine for every scale (several
+    batches a wave, a K over slices, a partial last segment): every bit against the oracle in the kernel's order of adds"""
+    x = orc.normal_bf16(31, 1, (M, K), 1.0)
+    packed, scale, zp = quant_int4(31, 2, N, K)
+    rng = np.random.default_rng(31)
+    G = K // 32
+    for rows, g in ((rng.permutation(N)[:N // 9], 0), (rng.permutation(N)[:N // 9], G // 2 + 1), (np.arange(N - 3, N), G - 1)):
+        scale[rows, g] = ((127 + rng.integers(116, 120, len(rows))) << 7 | rng.integers(0, 128, len(rows))).astype(np.uint16)
+    got = _run(x, abi.FMT_INT4, (packed, scale, zp), N, K, abi.OUT_F32, splitk=sk)
+    orc.set_dot_rule(4, sk)
+    try:
+        o = _oracle(x, abi.FMT_INT4, (packed, scale, zp), N, K, abi.OUT_F32)
+    finally:
+        orc.set_dot_rule(0)
+    assert np.isfinite(got).all() and (np.abs(got) > 2.0 ** 100).mean() > 0.1
+    assert np.array_equal(got.view(np.uint32), o["yf"].view(np.uint32)), int((got != o["yf"]).sum())
+
+
 @pytest.mark.parametrize("H", [2048, 4096, 6144])
 @pytest.mark.parametrize("mode", ["contract", "round2", "two_partials"])
 def test_add_norm(H, mode):
