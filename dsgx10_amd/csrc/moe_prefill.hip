@@ -728,8 +728,8 @@ __global__ void __launch_bounds__(256) k_pf_combine(const float* __restrict__ d,
 static void launch_pf_combine(const float* d, const int* rpos, const float* rk, int T, int H, int topk, float* yr, hipStream_t st) {
   const size_t n = (size_t)T * (H / 4);
   const dim3 grid((unsigned)((n + 255) / 256)), block(256);
-  if (topk == 8) hipLaunchKernelGGL(k_pf_combine<8>, grid, block, 0, st, d, rpos, rk, T, H, topk, yr);
-  else hipLaunchKernelGGL(k_pf_combine<0>, grid, block, 0, st, d, rpos, rk, T, H, topk, yr);
+  const auto k = topk == 8 ? k_pf_combine<8> : topk == 6 ? k_pf_combine<6> : topk == 4 ? k_pf_combine<4> : k_pf_combine<0>;
+  hipLaunchKernelGGL(k, grid, block, 0, st, d, rpos, rk, T, H, topk, yr);
 }
 
 // DeepSeek's combine (ds41f engine/kernels/moe.cu:974-981): y[t] = the f32 sum, in expert-id order, of the picks' outputs
@@ -1167,9 +1167,8 @@ int dsgx_dsk_moe_prefill(const dsgx_dsk_weights* Wt, const uint8_t* xq, const ui
     const size_t n = (size_t)T * (H / 8);
     const dim3 grid((unsigned)((n + 255) / 256)), block(256);
     const uint16_t* sh = shared ? dsh : (const uint16_t*)nullptr;
-    if (topk == 6) hipLaunchKernelGGL(k_pfmx_combine<6>, grid, block, 0, st, U16(o.d), sh, I32(o.rpos), T, H, topk, y);
-    else if (topk == 8) hipLaunchKernelGGL(k_pfmx_combine<8>, grid, block, 0, st, U16(o.d), sh, I32(o.rpos), T, H, topk, y);
-    else hipLaunchKernelGGL(k_pfmx_combine<0>, grid, block, 0, st, U16(o.d), sh, I32(o.rpos), T, H, topk, y);
+    const auto k = topk == 8 ? k_pfmx_combine<8> : topk == 6 ? k_pfmx_combine<6> : topk == 4 ? k_pfmx_combine<4> : k_pfmx_combine<0>;
+    hipLaunchKernelGGL(k, grid, block, 0, st, U16(o.d), sh, I32(o.rpos), T, H, topk, y);
     DSGX_HIP(hipGetLastError());
   }
   return DSGX_OK;

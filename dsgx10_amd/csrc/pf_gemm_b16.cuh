@@ -100,7 +100,7 @@ __device__ __forceinline__ void store_d(uint8_t* smem, const acc_t<MT> (&acc)[64
       const int p = 4 * i + (lane >> 4), c = lane & 15;
       const v4f_t v = *reinterpret_cast<const v4f_t*>(my + p * 256 + (c ^ (p & 15)) * 16);
       const int pos = m0 + MT * pt + p;
-      if (pos < mend) *reinterpret_cast<v4f_t*>(d + (size_t)pos * H + row0 + 4 * c) = v;
+      if (pos < mend) __builtin_nontemporal_store(v, reinterpret_cast<v4f_t*>(d + (size_t)pos * H + row0 + 4 * c));
     }
   });
 }

@@ -399,14 +399,16 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
       uint32_t o0 = __builtin_amdgcn_cvt_pk_fp8_f32(qv[0], qv[1], 0, false), o1 = __builtin_amdgcn_cvt_pk_fp8_f32(qv[4], qv[5], 0, false);
       o0 = __builtin_amdgcn_cvt_pk_fp8_f32(qv[2], qv[3], o0, true), o1 = __builtin_amdgcn_cvt_pk_fp8_f32(qv[6], qv[7], o1, true);
       if (pos < mend) {
-        *reinterpret_cast<u32x4_t*>(g.h + (size_t)pos * I + c0 + 8 * l16) = hv;
+        __builtin_nontemporal_store(hv, reinterpret_cast<u32x4_t*>(g.h + (size_t)pos * I + c0 + 8 * l16));
         *reinterpret_cast<uint2*>(g.hq + (size_t)pos * I + c0 + 8 * l16) = make_uint2(o0, o1);
         if (l16 == 0) g.hs[(size_t)pos * (I / 128) + ns] = sc;
       }
     }
   } else {
     // the wave's 16 positions x 64 rows of one 16-position tile at a time through its own piece of LDS (4 KiB):
-    // written as held, read back as whole rows, 16 lanes a position
+    // written as held, read back as whole rows, 16 lanes a position. Streaming stores, here and of h above, which only a caller's view reads: a
+    // chunk's d is 26 MB to 1 GB that would push the weights out of L2 (T = 700 / 1500 / 3000 / 8192 1202 / 1374 / 1682 / 2833 -> 1178 / 1332 / 1652 /
+    // 2810 us; MXFP4 T = 3000 1467 -> 1452, its h as well: no change).
     const int H = g.L.H;
     uint8_t* my = smem + wave * 4096;
     const int row0 = r0 + 16 * S::RA * wave;
@@ -423,7 +425,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
         const int p = 4 * i + part, c = r16;
         const v4f_t v = *reinterpret_cast<const v4f_t*>(my + p * 256 + ((c & ~7) | ((c ^ p) & 7)) * 16);
         const int pos = m0 + 16 * j + p;
-        if (pos < mend) *reinterpret_cast<v4f_t*>(g.d + (size_t)pos * H + row0 + 4 * c) = v;
+        if (pos < mend) __builtin_nontemporal_store(v, reinterpret_cast<v4f_t*>(g.d + (size_t)pos * H + row0 + 4 * c));
       }
     });
   }

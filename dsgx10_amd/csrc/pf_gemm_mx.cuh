@@ -383,7 +383,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
         const int p = 8 * i + (lane >> 3), c = lane & 7;
         const u32x4_t v = *reinterpret_cast<const u32x4_t*>(my + p * 128 + ((c ^ p) & 7) * 16);
         const int pos = m0 + 16 * j + p;
-        if (pos < mend) *reinterpret_cast<u32x4_t*>(g.d + (size_t)pos * H + row0 + 8 * c) = v;
+        if (pos < mend) __builtin_nontemporal_store(v, reinterpret_cast<u32x4_t*>(g.d + (size_t)pos * H + row0 + 8 * c));
       }
     });
   }
