@@ -208,6 +208,22 @@ def test_dsk_prefill_against_oracle(H, I, E, T, shared):
         assert np.array_equal(gpu.host(y2, np.uint32, (T, H)), got["y"].view(np.uint32))
 
 
+@pytest.mark.parametrize("topk", [4, 5, 8])
+def test_dsk_prefill_picks_a_row(topk):
+    """the combine with a row's loads batched (4, 6 and 8 picks) and one after the other: the ordered fold of the GPU's own outputs"""
+    H, I, E, T = 512, 256, 12, 40
+    L = Stacked(47, H, I, E, topk, 5, True)
+    x = orc.normal_bf16(47, 1, (T, H), 1.5)
+    idx, w = orc.route(orc.normal_f32(47, 2, (T, E), 1.0), orc.normal_f32(47, 3, (E,), 0.2), topk, 1.5, score_fn=1)
+    xq, xs = orc.act_quant_ue8m0(x)
+    got = run_prefill(L, xq, xs, idx, w)
+    for t in range(T):
+        fold = np.zeros(H, np.float32)
+        for v in [got["d"][p] for p in got["rpos"][t]] + [got["dsh"][t]]:
+            fold = fold + orc.bf16_to_f32(v)
+        assert np.array_equal(got["y"][t].view(np.uint32), fold.view(np.uint32)), t
+
+
 @pytest.mark.parametrize("H,I", [(256, 128), (512, 1152), (1280, 256)])
 def test_dsk_prefill_tile_shapes_give_the_same_bits(H, I):
     """experts whose rows end at the edges of the tiles of 32, 64 and 160 positions (and one row beyond), K in whole pairs of blocks and

@@ -180,6 +180,12 @@ def test_prefill_fp8_against_oracle(H, I, E, topk, T, shared, unit_rule):
         assert helpers.rel_l2(ys[:24], seq_s[:24]) <= 6e-3
 
 
+@pytest.mark.parametrize("topk", [5, 6])
+def test_prefill_fp8_picks_a_row(topk, unit_rule):
+    """the combine with a row's loads batched (4, 6 and 8 picks; the other tests have 4 and 8) and one after the other"""
+    test_prefill_fp8_against_oracle(256, 256, 12, topk, 40, "fp8", unit_rule)
+
+
 @pytest.mark.parametrize("H,I,T", [(512, 640, 20), (1280, 1152, 300)])
 def test_prefill_fp8_scale_groups(H, I, T, unit_rule):
     """the rows' scales come for eight 128-k blocks at a time, in the widest tile for four: last groups that are not whole (5, 9 and 10
