@@ -48,7 +48,6 @@ typedef int v8i_t __attribute__((ext_vector_type(8)));
 typedef float v4f_t __attribute__((ext_vector_type(4)));
 
 constexpr int kWgRows = 256;      // weight rows a workgroup (UP: 128 channels)
-constexpr int kThreads = 512;     // (the other formats' kernels)
 constexpr int kWaves = 4, kThreads4 = 64 * kWaves;
 
 // LDS of one of two workgroups on a CU: the waves' own rings of weight tiles (a slot is free when its fragments are read, so RING - 4
