@@ -48,7 +48,10 @@ __device__ __forceinline__ int last_seg_lanes(int K, int nsegk) { return (K - (n
 // has met a scale of 2^116 or more (none in a checkpoint). The loop only keeps the largest (and these lines stand once, behind it: as part of
 // every step's code they made a call's first pass 10 us longer): 6144 x 16384 at 1 / 2 / 4 rows 17.9 / 19.7 / 24.1 ->
 // 17.2 / 19.1 / 23.3 us a call, 16384 x 2048 at one 9.2 -> 8.6 (a vote and both routines in every step were 4% slower than the long one alone).
-// k_gemv_sk's calls are over before it pays (768 x 6144 over 4 at one row 6.2 -> 6.45).
+// k_gemv_sk's calls are over before it pays (768 x 6144 over 4 at one row 6.2 -> 6.45). Nor where one wave walks the slices of eight rows
+// (SPLIT, M = 8): there the largest scale and the code of the second pass are registers past 128 (136; 120 with the long routine) and more instructions between
+// the slices: 5120 x 1024 over 2 8.8 -> 9.6, 4096 x 4096 11.85 -> 12.35, 8064 x 2048 11.3 -> 11.6 us; at five to seven rows the two are within 2% (mean
+// +0.7 to +2.3%), unsplit at eight +1.3%.
 template <int M, int RB>
 __device__ __forceinline__ void dot_any_scale(const GemvArgs& a, int row_, int seg0, int sk, const uint4* xs, int lane, float (&acc)[RB][M]) {
   constexpr int FMT = DSGX_FMT_INT4_G32;
@@ -153,8 +156,8 @@ __global__ void __launch_bounds__(NW * 64) k_gemv(GemvArgs a) {
   };
   int cj = 0, csl = 0, cseg = 0;
   float mine = 0.f, mine2 = 0.f;  // lane r * M + m: output (row r, activation row m) of the batch, and the pair's other row (SwiGLU)
-  constexpr bool kI4 = FMT == DSGX_FMT_INT4_G32;
-  float smax = 0.f;  // INT4: the largest scale that the wave has met
+  constexpr bool kFast = FMT == DSGX_FMT_INT4_G32 && !(SPLIT && M == 8);  // (dot_any_scale)
+  float smax = 0.f;  // the largest scale that the wave has met
   // a slice is complete: add the lanes' partials, then the slices' sums in their order
   auto slice_done = [&]() {
     float v1 = 0.f, v2 = 0.f;
@@ -188,7 +191,7 @@ __global__ void __launch_bounds__(NW * 64) k_gemv(GemvArgs a) {
     }
   };
   auto compute = [&](const Raw (&raw)[RB]) {
-    step_dot<FMT, M, RB, true, kI4>(raw, xs, a.nq, cseg, lane, acc, a.K, &smax);
+    step_dot<FMT, M, RB, true, kFast>(raw, xs, a.nq, cseg, lane, acc, a.K, &smax);
     if ((cseg += sk) >= a.nsegk) slice_done();
   };
   // the first weight loads are issued before the activations are staged: one memory round trip, not two, before the
@@ -204,7 +207,7 @@ __global__ void __launch_bounds__(NW * 64) k_gemv(GemvArgs a) {
       load(w[d]);
     }
   }
-  if constexpr (kI4) {
+  if constexpr (kFast) {
     if (__builtin_expect(i4_any_large(smax), 0)) {  // all of the wave's rows once more, each lane over its own results
       cj = csl = 0;
       while (cj < nmine) {
