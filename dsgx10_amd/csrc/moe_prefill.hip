@@ -808,6 +808,39 @@ __global__ void __launch_bounds__(64) k_probe_mfma_bf16(const uint16_t* __restri
   for (int q = 0; q < 4; ++q) out[(4 * part + q) * 16 + row] = c[q];
 }
 
+// A launch of a shared expert's tiles alone. While tiles of 32 or 64 rows are one a CU at most, those, with a CU's LDS for the loads in flight
+// (k_few): four waves a CU hide less latency than the eight of the kernels before. Beyond, two workgroups a CU; FP8: tiles as tall as
+// makes the rounds over the chip even. Kernels of eight waves / two workgroups of four everywhere / this, whole phase, us:
+//   FP8 4096 x 2048, T = 17 40.0 / 54.0 / 34.0, T = 200 79.8 / 84.6 / 36.7, T = 1000 95.9 / 89.1 / 48.8, T = 4000 118 / 135 / 110, T = 8192 231 / 240 / 219
+// (FP8 tiles of up to 160 rows one a CU: 2304 x 1792 T = 2000 81 us, 47 like this; 2048 x 768, T = 6000 79 and 53.)
+template <class... A>
+int launch_alone(void (*k)(A...), unsigned grid, size_t lds, hipStream_t st, const A&... a) {
+  if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(k), lds)) return rc;
+  hipLaunchKernelGGL(k, dim3(grid), dim3(pf8::kThreads4), lds, st, a...);
+  DSGX_HIP(hipGetLastError());
+  return DSGX_OK;
+}
+inline long tiles_of(int T, int pos) { return ((long)T + pos - 1) / pos; }
+template <bool UP, int POS, int R>
+int launch_few_fp8(pf8::Args& g, int NS, hipStream_t st) {
+  const int tiles = tiles_of(g.nrows, POS);
+  g.map = pf8::map_of_few(tiles);
+  return launch_alone(pf8::k_few<UP, POS, R>, pf8::grid_of(tiles, NS, g.map), pf8::Shape<POS, 4 * R, R>::kLds, st, g);
+}
+template <bool UP>
+int launch_shared_fp8(pf8::Args& g, int NS, hipStream_t st) {
+  const int T = g.nrows, cus = num_cus_cached();
+  auto wgs = [&](int pos) { return tiles_of(T, pos) * NS; };
+  if (wgs(32) <= cus) return launch_few_fp8<UP, 32, 4>(g, NS, st);
+  if (wgs(64) <= cus) return launch_few_fp8<UP, 64, 3>(g, NS, st);
+  auto rounds = [&](int pos) { return (wgs(pos) + 2 * cus - 1) / (2 * cus) * pos; };  // two workgroups a CU: what the rounds take, in positions
+  g.height = pf8::kMaxPos;
+  for (int h = g.height - 16; h >= 48; h -= 16)
+    if (rounds(h) < rounds(g.height)) g.height = h;
+  g.map = pf8::map_of(3, 2, NS);
+  return launch_alone(pf8::k_gemm<UP>, pf8::grid_of(tiles_of(T, g.height), NS, g.map), pf8::kLds, st, g);
+}
+
 bool layer_has_fp8_shared(const dsgx_layer_w* L) { return L->sh.g && L->sh.u && L->sh.d && L->sh.gs && L->sh.us && L->sh.ds; }
 
 }  // namespace
@@ -951,11 +984,7 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
   if (H > 8192 || I > 8192) return fail(DSGX_EUNSUPPORTED, "moe_prefill: FP8 activations: hidden %d, intermediate %d (up to 8192)", H, I);
   void (*k_up)(pf8::Args) = pf8::k_gemm_mixed<true>;  // the routed experts (and the shared one's tiles)
   void (*k_dn)(pf8::Args) = pf8::k_gemm_mixed<false>;
-  void (*k_up2)(pf8::Args) = pf8::k_gemm<true>;        // the shared expert alone
-  void (*k_dn2)(pf8::Args) = pf8::k_gemm<false>;
   for (const void* k : {(const void*)k_up, (const void*)k_dn})
-    if (int rc = allow_dynamic_lds(k, pf8::kLds)) return rc;
-  for (const void* k : {(const void*)k_up2, (const void*)k_dn2})
     if (int rc = allow_dynamic_lds(k, pf8::kLds)) return rc;
   pf8::Args g{};
   g.L = *L;
@@ -977,7 +1006,7 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
   // A whole step runs the shared expert's tiles in the routed experts' launches, in front of them: alone they are a launch
   // of few workgroups at small T, and two more tails (as kernels of eight waves, whole call, hidden 4096, intermediate
   // 2048, 256 experts: T = 17 387 -> 341 us, T = 200 1061 -> 973, T = 2000 1565 -> 1544, T = 8192 within the noise; same bits).
-  const int sh_tiles = (T + pf8::kMaxPos - 1) / pf8::kMaxPos;
+  const int sh_tiles = tiles_of(T, pf8::kMaxPos);
   const bool fused_sh = shared && (cfg.phases & (2 | 4 | 16)) == (2 | 4 | 16);
   if (fp8_rows && !(cfg.phases & 1)) {
     if (int rc = dsgx_act_quant(x, T, H, W + o.xq, F32(o.xs), stream)) return rc;
@@ -1002,13 +1031,12 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
     DSGX_HIP(hipGetLastError());
   }
   if ((cfg.phases & 16) && shared && !fused_sh) {
-    const int tiles = sh_tiles;
     g.tile_e = g.tile_m0 = g.ntiles = g.off = nullptr;
     g.aq = W + o.xq, g.as = F32(o.xs), g.gather = nullptr;
     g.h = reinterpret_cast<uint16_t*>(W + o.hsh), g.hq = W + o.hshq, g.hs = F32(o.hshs), g.d = nullptr;
-    hipLaunchKernelGGL(k_up2, dim3(pf8::grid_of(tiles, NSU)), dim3(pf8::kThreads4), pf8::kLds, st, g);
+    if (int rc = launch_shared_fp8<true>(g, NSU, st)) return rc;
     g.aq = W + o.hshq, g.as = F32(o.hshs), g.h = nullptr, g.hq = nullptr, g.hs = nullptr, g.d = ys;
-    hipLaunchKernelGGL(k_dn2, dim3(pf8::grid_of(tiles, NSD)), dim3(pf8::kThreads4), pf8::kLds, st, g);
+    if (int rc = launch_shared_fp8<false>(g, NSD, st)) return rc;
     DSGX_HIP(hipGetLastError());
   }
   return DSGX_OK;

@@ -55,15 +55,18 @@ constexpr int kWaves = 4, kThreads4 = 64 * kWaves;
 // tiles are in flight: a shape of 64 positions and 7 tiles was slower than the widest with 4 (T = 1200 1361 -> 1308 us), and
 // dsgx_moe_prefill says where 32 positions take 8.
 constexpr int kMaxPos = 160;
-template <int POS, int RING = 4>
+// R > 0: a shape for one workgroup a CU (k_few): weights and activations R blocks ahead.
+template <int POS, int RING = 4, int R = 0>
 struct Shape {
+  static_assert(R == 0 || RING == 4 * R, "R blocks of weights");
   static constexpr int kPos = POS;                 // positions of a tile
   static constexpr int kSub = POS / 16;            // its 16-position tiles
   static constexpr int RA = 4;                     // 16-row tiles a wave
   static constexpr int kRing = RING;               // the wave's own ring of weight tiles, 2 KiB each
   static constexpr int kHX = POS / 32;             // 8-position half tiles that a wave brings
-  static constexpr int kStageX = POS * 128;        // a block's activations; two stages
-  static constexpr int kOffX = kWaves * kRing * 2048, kOffS = kOffX + 2 * kStageX;
+  static constexpr int kStageX = POS * 128;        // a block's activations
+  static constexpr int kAhead = R ? R : 1, kStages = kAhead + 1;
+  static constexpr int kOffX = kWaves * kRing * 2048, kOffS = kOffX + kStages * kStageX;
   static constexpr int kSB = POS == kMaxPos ? 4 : 8;  // blocks whose scales of the positions come together; two such buffers behind the stages
   static constexpr int kGroup = POS * 4 * kSB;
   static constexpr int kLds = kOffS + 2 * kGroup;  // (the epilogues reuse it: UP kPos x 256 B, DOWN 4 x 4 KiB)
@@ -83,6 +86,12 @@ constexpr Map kMap{3, 2};
 __host__ __device__ inline Map map_of(int tl, int nl, int NS) {
   while (nl > 0 && NS % (1 << nl)) --nl;
   return Map{tl, nl};
+}
+// ... of a launch with fewer workgroups than CUs: a row group's tiles (up to eight) on one XCD, the row groups over all of them
+inline Map map_of_few(int tiles) {
+  int tl = 0;
+  while (tl < 3 && (1 << tl) < tiles) ++tl;
+  return Map{tl, 0};
 }
 constexpr int kXcds = 8;
 __host__ __device__ inline unsigned grid_of(int tiles, int NS, Map m = kMap) {
@@ -124,6 +133,7 @@ struct Args {
   int nrows;           // the shared expert's rows: T
   int fast_act;        // UP: SwiGLU by the plain formula (swiglu4)
   int deep;            // small tiles take deep rings
+  int height;          // k_gemm: rows of a tile
   dsgx_layer_w L;
   uint16_t* h;         // UP: h bf16 [position][I]
   uint8_t* hq;         // UP: h quantised, e4m3 [position][I]
@@ -166,10 +176,6 @@ template <int N, class F>
 __device__ __forceinline__ void static_for(F f) {
   static_for(std::make_integer_sequence<int, N>{}, f);
 }
-// the active lanes' 4 bytes to lds_base + 4 l
-__device__ __forceinline__ void dma4(const float* src, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_base), "v"(src) : "memory");
-}
 template <int N>
 __device__ __forceinline__ void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
@@ -182,9 +188,9 @@ __device__ __forceinline__ int sc_half(int r, int h) { return (h ^ (r >> 3)) & 1
 __device__ __forceinline__ int sw4(int r) { return (((r >> 2) ^ (r >> 3)) & 1) << 1 | ((r >> 3) & 1); }
 
 // one tile: expert e (-1: the shared expert), rows [m0, mend) of the activations' positions, row group ns
-template <bool UP, int POS, int RING, bool STREAM>
+template <bool UP, int POS, int RING, bool STREAM, int R = 0>
 __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, int m0, int mend, int ns) {
-  using S = Shape<POS, RING>;
+  using S = Shape<POS, RING, R>;
   const int K = UP ? g.L.H : g.L.I, KB = K / 128;
   if (mend > m0 + S::kPos) mend = m0 + S::kPos;  // (the tile's own rows)
   const uint8_t *wa, *wb;  // UP: gate, up; DOWN: down twice
@@ -233,8 +239,9 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   const uint32_t oxs = row_of(sp) * (uint32_t)KB * 4 + (kPc == 2 && KB >= 8 ? 16 * sc_half(sp & 15, lane) : 0);  // lanes 0 .. kPc kPosWave - 1: a piece of a position's scales
   // (the dynamic segment's address inside LDS: the pointer in the LDS address space is that 32-bit offset)
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
-  // the half tiles this wave brings that hold rows: a ragged tile's others are not fetched
-  const int nhx = uni(min(S::kHX, max(0, (mend - m0 + 7) / 8 - S::kHX * wave)));
+  // the half tiles this wave brings that hold rows: a ragged tile's others are not fetched (R: they are, so that every wave has as many
+  // loads in flight as its waits count)
+  const int nhx = R ? S::kHX : uni(min(S::kHX, max(0, (mend - m0 + 7) / 8 - S::kHX * wave)));
   // Weight tile i of the wave's sequence (tile i % 4 of block i / 4, clamped: past the end the last block again, into a slot nobody
   // reads) goes to slot i % kRing of the wave's own ring, whose rows no other wave reads: a slot is free as soon as the wave has read
   // its fragments. Activations: a stage a block.
@@ -243,7 +250,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
     dma16_w<STREAM>(wt[t] + (size_t)min(kb, KB - 1) * 128, ow[hh], uni(ring0 + (uint32_t)slot * 2048 + hh * 1024));
   };
   auto issue_x = [&](int kb) {
-    const uint32_t xbase = lds0 + S::kOffX + (uint32_t)(kb & 1) * S::kStageX + (uint32_t)wave * (1024 * S::kHX);
+    const uint32_t xbase = lds0 + S::kOffX + (uint32_t)(kb % S::kStages) * S::kStageX + (uint32_t)wave * (1024 * S::kHX);
 #pragma unroll
     for (int i = 0; i < S::kHX; ++i) {
       if (i >= nhx) break;
@@ -283,7 +290,10 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   issue_x(0);
   if (KB >= S::kSB) issue_scales(0);
 #pragma unroll
-  for (int i = 0; i < S::kRing; ++i) issue_w(i / 4, i % 4, i, 0), issue_w(i / 4, i % 4, i, 1);
+  for (int i = 0; i < S::kRing; ++i) {
+    if (R && i > 0 && i % 4 == 0) issue_x(i / 4);
+    issue_w(i / 4, i % 4, i, 0), issue_w(i / 4, i % 4, i, 1);
+  }
 
   // fragment reads: lane (row r16, part) takes pieces 2 part and 2 part + 1 of its row (32 consecutive k)
   const int rd0 = (r16 >> 3) * 1024 + (r16 & 7) * 128 + ((2 * part) ^ swz(r16)) * 16;
@@ -303,22 +313,23 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
     constexpr int NJ = decltype(nj_c)::value;
     int slot = 0;  // of the block's first weight tile: 4 kb % kRing
     for (int kb = 0; kb < KB; ++kb) {
-      // this wave's loads of block kb have landed (weight tiles of later blocks may be in flight); after the barrier everyone's have,
-      // and everyone is done reading the stage of block kb - 1, which the activations of block kb + 1 now overwrite
-      wait_loads<2 * (S::kRing - 4)>();
+      // this wave's loads of block kb have landed (weight tiles of later blocks may be in flight; R: all of R - 1 later blocks, a load of
+      // scales among them only makes the wait longer); after the barrier everyone's have, and everyone is done reading the stage of
+      // block kb - 1, which the activations of block kb + kAhead now overwrite
+      wait_loads<R ? (R - 1) * (8 + S::kHX) : 2 * (S::kRing - 4)>();
       __syncthreads();
       if (kb == 0) PF_STAMP(g, 4);
-      if ((kb + 1) % S::kSB == 0 && kb + 1 < KB) issue_scales((kb + 1) / S::kSB);
+      if ((kb + S::kAhead) % S::kSB == 0 && kb + S::kAhead < KB) issue_scales((kb + S::kAhead) / S::kSB);
       int sl[4];
 #pragma unroll
       for (int t = 0; t < 4; ++t) sl[t] = slot + t >= S::kRing ? slot + t - S::kRing : slot + t;
       v8i_t fa[S::RA];
 #pragma unroll
       for (int t = 0; t < S::RA; ++t) fa[t] = frag(smem + wave * (S::kRing * 2048) + sl[t] * 2048);
-      issue_x(kb + 1);
+      issue_x(kb + S::kAhead);
       const float wsa = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wsa_l), kb & 63));
       const float wsb = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wsb_l), kb & 63));
-      const uint8_t* X = smem + S::kOffX + (kb & 1) * S::kStageX;
+      const uint8_t* X = smem + S::kOffX + (kb % S::kStages) * S::kStageX;
       const int sw = kb - (KB >= S::kSB ? first_block(kb / S::kSB) : 0);
       const uint8_t* XS = smem + S::kOffS + ((kb / S::kSB) & 1) * S::kGroup + r16 * (4 * S::kSB) + 16 * (kPc == 2 ? sc_half(r16, sw >> 2) : 0) + 4 * (sw & 3);
       v8i_t fn = frag(X);
@@ -441,15 +452,27 @@ __device__ __forceinline__ void any_tile(const Args& g, uint8_t* smem, int e, in
   else if (only) gemm_tile<UP, 32, 5, true>(g, smem, e, m0, mend, ns);
   else gemm_tile<UP, 32, 5, false>(g, smem, e, m0, mend, ns);
 }
-// The shared expert: tiles of 128 rows over [0, nrows).
+// The shared expert alone: tiles of g.height rows (up to kMaxPos) over [0, nrows).
 template <bool UP>
 __global__ void __launch_bounds__(kThreads4, 2) k_gemm(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int NS = UP ? g.L.I / (kWgRows / 2) : g.L.H / kWgRows;
   int tile, ns;
-  task_of<true>(NS, tile, ns);
-  if (ns >= NS || tile * kMaxPos >= g.nrows) return;
-  any_tile<UP>(g, smem, -1, tile * kMaxPos, g.nrows, ns, tile == 0);
+  task_of<true>(NS, tile, ns, blockIdx.x, g.map);
+  const int m0 = tile * g.height;
+  if (ns >= NS || m0 >= g.nrows) return;
+  any_tile<UP>(g, smem, -1, m0, min(g.nrows, m0 + g.height), ns, false);
+}
+// ... in no more tiles than the chip has CUs: one workgroup a CU, which has the CU's LDS for loads in flight (Shape's R). A launch of few
+// workgroups waits for its loads' latency, turn after turn (0.47 us a block with four blocks ahead).
+template <bool UP, int POS, int R>
+__global__ void __launch_bounds__(kThreads4, 2) k_few(Args g) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  const int NS = UP ? g.L.I / (kWgRows / 2) : g.L.H / kWgRows;
+  int tile, ns;
+  task_of<true>(NS, tile, ns, blockIdx.x, g.map);
+  if (ns >= NS || tile * POS >= g.nrows) return;
+  gemm_tile<UP, POS, 4 * R, false, R>(g, smem, -1, tile * POS, g.nrows, ns);
 }
 // The routed experts' list, an expert's tiles next to each other, behind the shared expert's tiles.
 template <bool UP>

@@ -287,6 +287,23 @@ def test_prefill_shared_expert_in_the_routed_launches(fmt, shared, T):
     assert np.array_equal(gpu.host(s2, np.uint32, (T, H)), ys.view(np.uint32))
 
 
+@pytest.mark.parametrize("fmt,shared", [(abi.FMT_FP8, "fp8"), (abi.FMT_INT4, "bf16")], ids=["fp8", "int4-bf16"])
+@pytest.mark.parametrize("H,I,T", [(256, 128, 1), (256, 384, 33), (1280, 4096, 250), (1280, 4096, 257), (1280, 4096, 520), (1280, 4096, 1400),
+                                   (4096, 1152, 512), (4096, 1152, 700), (4096, 1152, 1030)])
+def test_prefill_shared_expert_alone_in_every_shape(fmt, shared, H, I, T):
+    """the shared expert as a phase of its own takes tiles of 32, 64 and 160 (FP8) or 128 (BF16) rows while they are one a CU, then two workgroups a
+    CU in tiles whose height evens out their rounds: both GEMMs at each, ragged last tiles, K of 1 to 64 blocks, deeper stages than blocks
+    of K: the bits that the rows have in the routed experts' launches"""
+    E, topk = 3, 1
+    hl = helpers.make_layer(fmt, H, I, E, topk, 1, seed=37, shared=shared)
+    x, _, idx, w = helpers.rows_and_routing(39, T, H, E, topk, 2.5)
+    yr, ys, _, dl = _prefill(hl, x, idx, w, T)
+    ws, s2 = gpu.empty(lib.prefill_ws_bytes(dl.w, T), 0x5A), gpu.empty(T * H * 4, 0xFF)
+    lib.moe_prefill(dl.w, gpu.dev(x), gpu.dev(idx), gpu.dev(w), T, ws, gpu.empty(T * H * 4), s2, phases=16)
+    assert np.isfinite(ys).all() and (np.abs(ys).max(axis=1) > 0).all()
+    assert np.array_equal(gpu.host(s2, np.uint32, (T, H)), ys.view(np.uint32))
+
+
 def test_prefill_argument_errors():
     hl = helpers.make_layer(abi.FMT_BF16, 512, 256, 8, 2, 4, seed=1)
     dl = hl.upload()
