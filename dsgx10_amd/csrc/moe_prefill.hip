@@ -812,6 +812,7 @@ __global__ void __launch_bounds__(64) k_probe_mfma_bf16(const uint16_t* __restri
 // (k_few): four waves a CU hide less latency than the eight of the kernels before. Beyond, two workgroups a CU; FP8: tiles as tall as
 // makes the rounds over the chip even. Kernels of eight waves / two workgroups of four everywhere / this, whole phase, us:
 //   FP8 4096 x 2048, T = 17 40.0 / 54.0 / 34.0, T = 200 79.8 / 84.6 / 36.7, T = 1000 95.9 / 89.1 / 48.8, T = 4000 118 / 135 / 110, T = 8192 231 / 240 / 219
+//   BF16 6144 x 2048, T = 17 57.4 / 86.5 / 56.2, T = 168 96 / 106 / 58, T = 672 102 / 110 / 81, T = 1111 138 / 139 / 132, T = 2500 235 / 227 / 233
 // (FP8 tiles of up to 160 rows one a CU: 2304 x 1792 T = 2000 81 us, 47 like this; 2048 x 768, T = 6000 79 and 53.)
 template <class... A>
 int launch_alone(void (*k)(A...), unsigned grid, size_t lds, hipStream_t st, const A&... a) {
@@ -839,6 +840,20 @@ int launch_shared_fp8(pf8::Args& g, int NS, hipStream_t st) {
     if (rounds(h) < rounds(g.height)) g.height = h;
   g.map = pf8::map_of(3, 2, NS);
   return launch_alone(pf8::k_gemm<UP>, pf8::grid_of(tiles_of(T, g.height), NS, g.map), pf8::kLds, st, g);
+}
+template <bool UP, int POS, int R>
+int launch_few_b16(const pfb16::Args& g, int NS, int height, hipStream_t st) {
+  const int tiles = tiles_of(g.rows, height);
+  const pf8::Map map = pf8::map_of_few(tiles);
+  return launch_alone(pfb16::k_few<UP, POS, R>, pf8::grid_of(tiles, NS, map), pfb16::Shape<POS, R>::kLds, st, g, map, height);
+}
+template <bool UP>
+int launch_shared_b16(const pfb16::Args& g, int NS, hipStream_t st) {
+  const int T = g.rows, cus = num_cus_cached();
+  for (int h = 32; h <= pfb16::kPos; h += 32)
+    if (tiles_of(T, h) * NS <= cus)
+      return h == 32 ? launch_few_b16<UP, 32, 4>(g, NS, h, st) : h == 64 ? launch_few_b16<UP, 64, 3>(g, NS, h, st) : launch_few_b16<UP, pfb16::kPos, 2>(g, NS, h, st);
+  return launch_alone(pfb16::k_gemm<UP>, pf8::grid_of(tiles_of(T, pfb16::kPos), NS), pfb16::kLds, st, g);
 }
 
 bool layer_has_fp8_shared(const dsgx_layer_w* L) { return L->sh.g && L->sh.u && L->sh.d && L->sh.gs && L->sh.us && L->sh.ds; }
@@ -963,10 +978,8 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
     }
     if ((cfg.phases & 16) && shared && !fused_sh) {
       if (i4) {
-        for (const void* k : {(const void*)pfb16::k_gemm<true>, (const void*)pfb16::k_gemm<false>})
-          if (int rc = allow_dynamic_lds(k, pfb16::kLds)) return rc;
-        hipLaunchKernelGGL(pfb16::k_gemm<true>, dim3(sh_gu), dim3(pf8::kThreads4), pfb16::kLds, st, sh_up);
-        hipLaunchKernelGGL(pfb16::k_gemm<false>, dim3(sh_gd), dim3(pf8::kThreads4), pfb16::kLds, st, sh_dn);
+        if (int rc = launch_shared_b16<true>(sh_up, I / (kWgRows / 2), st)) return rc;
+        if (int rc = launch_shared_b16<false>(sh_dn, H / kWgRows, st)) return rc;
       } else {
         const int tiles = (T + kTile - 1) / kTile;
         q.tile_e = q.tile_m0 = q.ntiles = q.off = nullptr, q.nrows = T;

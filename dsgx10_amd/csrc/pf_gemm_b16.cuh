@@ -30,9 +30,15 @@ using pf8::wait_loads;
 typedef __bf16 v8bf_t __attribute__((ext_vector_type(8)));
 typedef float v16f_t __attribute__((ext_vector_type(16)));
 
-constexpr int kPos = 128, kRing = 5;
-constexpr int kStageX = kPos * 128, kOffX = kWaves * kRing * 2048;  // the waves' rings of weight tiles, 2 KiB each; two stages of activations
-constexpr int kLds = kOffX + 2 * kStageX;                           // 73,728
+constexpr int kPos = 128;
+// The waves' rings of weight tiles, 2 KiB each, and the stages of activations. R > 0: for one workgroup a CU (k_few), both R turns ahead.
+template <int POS = kPos, int R = 0>
+struct Shape {
+  static constexpr int kRing = R ? 4 * R : 5, kAhead = R ? R : 1, kStages = kAhead + 1;
+  static constexpr int kStageX = POS * 128, kOffX = kWaves * kRing * 2048;
+  static constexpr int kLds = kOffX + kStages * kStageX;
+};
+constexpr int kLds = Shape<>::kLds;  // 73,728
 static_assert(2 * kLds <= 160 * 1024, "two workgroups a CU");
 
 struct Args {
@@ -106,10 +112,12 @@ __device__ __forceinline__ void store_d(uint8_t* smem, const acc_t<MT> (&acc)[64
 }
 
 // rows [m0, mend) against row group ns
-template <bool UP>
+template <bool UP, int POS = kPos, int R = 0>
 __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int m0, int mend, int ns) {
+  using S = Shape<POS, R>;
+  constexpr int kRing = S::kRing, kStageX = S::kStageX, kOffX = S::kOffX, kXL = POS / 32;  // kXL: a wave's loads of a stage of activations
   const int K = UP ? g.H : g.I, TN = K / 64;
-  if (mend > m0 + kPos) mend = m0 + kPos;
+  if (mend > m0 + POS) mend = m0 + POS;
   const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6), r32 = lane & 31, half = lane >> 5;
   const int npt = uni((mend - m0 + 31) / 32);
   // what this lane fetches: row lane / 8 of eight, slot lane % 8. The wave's four 16-row tiles: UP the gate rows (t < 2) and
@@ -121,19 +129,20 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int m0, 
   for (int t = 0; t < 4; ++t) wt[t] = g.w + (size_t)(kWgRows * ns + 64 * wave + (UP ? 32 * (t & 1) + (t >> 1) : 16 * t)) * K * 2;
 #pragma unroll
   for (int hh = 0; hh < 2; ++hh) ow[hh] = (uint32_t)(8 * hh + lr) * (UP ? 4 : 2) * K + 16 * ((lane & 7) ^ (4 * hh + (lane >> 4)));
-  const uint8_t* px[4];  // positions 8 (wave + 4 i) ...
+  const uint8_t* px[kXL];  // positions 8 (wave + 4 i) ...
 #pragma unroll
-  for (int i = 0; i < 4; ++i)  // (a ragged tile re-reads its last row: never stored)
+  for (int i = 0; i < kXL; ++i)  // (a ragged tile re-reads its last row: never stored)
     px[i] = reinterpret_cast<const uint8_t*>(g.x) + (size_t)min(m0 + 8 * (wave + 4 * i) + lr, mend - 1) * K * 2 + 16 * ((lane & 7) ^ (4 * (wave & 1) + (lane >> 4)));
-  const int nhx = uni(min(4, max(0, ((mend - m0 + 7) / 8 - wave + 3) / 4)));  // ... and its empty eights are not fetched
+  // ... and its empty eights are not fetched (R: they are, so that every wave has as many loads in flight as its waits count)
+  const int nhx = R ? kXL : uni(min(kXL, max(0, ((mend - m0 + 7) / 8 - wave + 3) / 4)));
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
   // (past the end: the last turn's again, into slots nobody reads)
   auto issue_x = [&](int t) {
     const size_t off = (size_t)min(t, TN - 1) * 128;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < kXL; ++i) {
       if (i >= nhx) break;
-      dma16(px[i] + off, uni(lds0 + kOffX + (uint32_t)(t & 1) * kStageX + (uint32_t)(wave + 4 * i) * 1024));
+      dma16(px[i] + off, uni(lds0 + kOffX + (uint32_t)(t % S::kStages) * kStageX + (uint32_t)(wave + 4 * i) * 1024));
     }
   };
   auto issue_w = [&](int t, int tile, int slot, int hh) {  // half hh of the tile
@@ -141,13 +150,16 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int m0, 
   };
   issue_x(0);
 #pragma unroll
-  for (int i = 0; i < kRing; ++i) issue_w(i / 4, i % 4, i, 0), issue_w(i / 4, i % 4, i, 1);
+  for (int i = 0; i < kRing; ++i) {
+    if (R && i > 0 && i % 4 == 0) issue_x(i / 4);
+    issue_w(i / 4, i % 4, i, 0), issue_w(i / 4, i % 4, i, 1);
+  }
   const int rd = (half ^ ((r32 >> 1) & 7)) * 16;  // (step s: ^ 32 s)
-  v16f_t acc[2][kPos / 32];
+  v16f_t acc[2][POS / 32];
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int j = 0; j < kPos / 32; ++j)
+    for (int j = 0; j < POS / 32; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[t][j][r] = 0.f;
 
@@ -155,12 +167,12 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int m0, 
     constexpr int NJ = decltype(nj_c)::value;
     int slot = 0;  // of the turn's first weight tile: 4 t % kRing
     for (int t = 0; t < TN; ++t) {
-      wait_loads<2 * (kRing - 4)>();  // (the next turn's first tiles may be in flight)
+      wait_loads<R ? (R - 1) * (8 + kXL) : 2 * (kRing - 4)>();  // (the next turn's first tiles may be in flight, or all of R - 1 turns)
       __syncthreads();
       int sl[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) sl[i] = slot + i >= kRing ? slot + i - kRing : slot + i;
-      const uint8_t* X = smem + kOffX + (t & 1) * kStageX + r32 * 128;
+      const uint8_t* X = smem + kOffX + (t % S::kStages) * kStageX + r32 * 128;
       u32x4_t fa[2][4], fn;
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
@@ -168,7 +180,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int m0, 
 #pragma unroll
         for (int s = 0; s < 4; ++s) fa[i][s] = *reinterpret_cast<const u32x4_t*>(W + (rd ^ (32 * s)));
       }
-      issue_x(t + 1);
+      issue_x(t + S::kAhead);
       fn = *reinterpret_cast<const u32x4_t*>(X + rd);
 #pragma unroll
       for (int i = 0; i < 2; ++i) asm volatile("" : "+v"(fa[i][0]), "+v"(fa[i][1]), "+v"(fa[i][2]), "+v"(fa[i][3]));  // (read: their slots may be written from here on)
@@ -186,9 +198,10 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int m0, 
       slot = slot + 4 >= kRing ? slot + 4 - kRing : slot + 4;
     }
   };
-  if (npt <= 1) run(std::integral_constant<int, 1>{});
-  else if (npt <= 2) run(std::integral_constant<int, 2>{});
-  else run(std::integral_constant<int, 4>{});
+  if (POS == 32 || npt <= 1) run(std::integral_constant<int, 1>{});
+  else if (POS == 64 || npt <= 2) run(std::integral_constant<int, std::min(2, POS / 32)>{});
+  else if (R && npt <= 3) run(std::integral_constant<int, std::min(3, POS / 32)>{});
+  else run(std::integral_constant<int, POS / 32>{});
   wait_loads<0>();
   __syncthreads();
   if (UP) store_h<32>(smem, acc, 1.f, 1.f, m0, mend, ns * (kWgRows / 2), g.I, g.h);
@@ -208,6 +221,17 @@ template <bool UP>
 __global__ void __launch_bounds__(kThreads4, 2) k_gemm(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   tiles<UP>(g, smem, blockIdx.x);
+}
+// The rows in fewer tiles than the chip has CUs: one workgroup a CU, which has the CU's LDS for loads in flight.
+template <bool UP, int POS, int R>
+__global__ void __launch_bounds__(kThreads4, 2) k_few(Args g, pf8::Map map, int height) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  const int NS = UP ? g.I / (kWgRows / 2) : g.H / kWgRows;
+  int tile, ns;
+  pf8::task_of<true>(NS, tile, ns, blockIdx.x, map);
+  const int m0 = tile * height;
+  if (ns >= NS || m0 >= g.rows) return;
+  gemm_tile<UP, POS, R>(g, smem, m0, min(g.rows, m0 + height), ns);
 }
 
 }  // namespace pfb16
