@@ -813,6 +813,7 @@ __global__ void __launch_bounds__(64) k_probe_mfma_bf16(const uint16_t* __restri
 // makes the rounds over the chip even. Kernels of eight waves / two workgroups of four everywhere / this, whole phase, us:
 //   FP8 4096 x 2048, T = 17 40.0 / 54.0 / 34.0, T = 200 79.8 / 84.6 / 36.7, T = 1000 95.9 / 89.1 / 48.8, T = 4000 118 / 135 / 110, T = 8192 231 / 240 / 219
 //   BF16 6144 x 2048, T = 17 57.4 / 86.5 / 56.2, T = 168 96 / 106 / 58, T = 672 102 / 110 / 81, T = 1111 138 / 139 / 132, T = 2500 235 / 227 / 233
+//   MXFP4's FP8 5120 x 2304, T = 17 33.9 / 46.0 / 39.5, T = 40 38.9 / 54 / 38.4, T = 200 90.7 / 64.9 / 39.0, T = 1000 104 / 74.5 / 75.7
 // (FP8 tiles of up to 160 rows one a CU: 2304 x 1792 T = 2000 81 us, 47 like this; 2048 x 768, T = 6000 79 and 53.)
 template <class... A>
 int launch_alone(void (*k)(A...), unsigned grid, size_t lds, hipStream_t st, const A&... a) {
@@ -840,6 +841,18 @@ int launch_shared_fp8(pf8::Args& g, int NS, hipStream_t st) {
     if (rounds(h) < rounds(g.height)) g.height = h;
   g.map = pf8::map_of(3, 2, NS);
   return launch_alone(pf8::k_gemm<UP>, pf8::grid_of(tiles_of(T, g.height), NS, g.map), pf8::kLds, st, g);
+}
+template <bool UP>
+int launch_shared_mx(pfmx::Args& g, int NS, hipStream_t st) {
+  const int T = g.nrows, pos = tiles_of(T, 32) * NS <= num_cus_cached() ? 32 : 64;
+  if (tiles_of(T, pos) * NS > num_cus_cached()) {
+    g.map = pf8::map_of(3, 2, NS);
+    return launch_alone(pfmx::k_gemm<UP>, pf8::grid_of(tiles_of(T, 128), NS, g.map), pfmx::kLds, st, g);
+  }
+  g.map = pf8::map_of_few(tiles_of(T, pos));
+  const unsigned grid = pf8::grid_of(tiles_of(T, pos), NS, g.map);
+  if (pos == 32) return launch_alone(pfmx::k_few<UP, 32, 3>, grid, pfmx::Shape<32, DSGX_FMT_FP8_B32E, 1, 3>::kLds, st, g);
+  return launch_alone(pfmx::k_few<UP, 64, 3>, grid, pfmx::Shape<64, DSGX_FMT_FP8_B32E, 1, 3>::kLds, st, g);
 }
 template <bool UP, int POS, int R>
 int launch_few_b16(const pfb16::Args& g, int NS, int height, hipStream_t st) {
@@ -1147,11 +1160,7 @@ int dsgx_dsk_moe_prefill(const dsgx_dsk_weights* Wt, const uint8_t* xq, const ui
   const int H = Wt->H, I = Wt->I, E = Wt->E, topk = Wt->topk, P = o.P;
   void (*k_up)(pfmx::Args) = pfmx::k_gemm_mixed<true>;
   void (*k_dn)(pfmx::Args) = pfmx::k_gemm_mixed<false>;
-  void (*k_sup)(pfmx::Args) = pfmx::k_gemm<true>;
-  void (*k_sdn)(pfmx::Args) = pfmx::k_gemm<false>;
   for (const void* k : {(const void*)k_up, (const void*)k_dn})
-    if (int rc = allow_dynamic_lds(k, pfmx::kLds)) return rc;
-  for (const void* k : {(const void*)k_sup, (const void*)k_sdn})
     if (int rc = allow_dynamic_lds(k, pfmx::kLds)) return rc;
   const int NSU = I / (pf8::kWgRows / 2), NSD = H / pf8::kWgRows;
   uint16_t* dsh = U16(o.d + align256((size_t)P * H * 2));  // the shared expert's outputs behind the picks', both bf16
@@ -1169,18 +1178,16 @@ int dsgx_dsk_moe_prefill(const dsgx_dsk_weights* Wt, const uint8_t* xq, const ui
   auto map_for = [&](int NS) { return (long long)P >= 24LL * E ? pf8::map_of(2, 1, NS) : pf8::map_of(0, 1, NS); };
   // a whole step runs the shared expert's tiles in the routed experts' launches, in front of them (as the FP8 layers do;
   // hidden 5120, intermediate 2304, T = 17: 417 -> 362 us, T = 600: 1405 -> 1334, T = 3000: 1870 -> 1821)
-  const int sh_tiles = (T + 127) / 128;
+  const int sh_tiles = tiles_of(T, 128);
   const bool fused_sh = shared && (cfg.phases & (2 | 4 | 8)) == (2 | 4 | 8);
   if ((cfg.phases & 2) && shared && !fused_sh) {
-    const int tiles = sh_tiles;
     g.tile_e = g.tile_m0 = g.ntiles = g.off = nullptr, g.gather = nullptr, g.posw = nullptr, g.wstride = g.sstride = 0;
     g.aq = xq, g.as = xs, g.wa = Wt->sh_w1, g.sa = Wt->sh_s1, g.wb = Wt->sh_w3, g.sb = Wt->sh_s3;
     g.h = U16(o.hsh), g.hq = W + o.hshq, g.hs = W + o.hshs, g.d = nullptr;
-    hipLaunchKernelGGL(k_sup, dim3(pf8::grid_of(tiles, NSU)), dim3(pf8::kThreads4), pfmx::kLds, st, g);
+    if (int rc = launch_shared_mx<true>(g, NSU, st)) return rc;
     g.aq = W + o.hshq, g.as = W + o.hshs, g.wa = Wt->sh_w2, g.sa = Wt->sh_s2, g.wb = g.sb = nullptr;
     g.h = nullptr, g.hq = g.hs = nullptr, g.d = dsh;
-    hipLaunchKernelGGL(k_sdn, dim3(pf8::grid_of(tiles, NSD)), dim3(pf8::kThreads4), pfmx::kLds, st, g);
-    DSGX_HIP(hipGetLastError());
+    if (int rc = launch_shared_mx<false>(g, NSD, st)) return rc;
   }
   g.tile_e = I32(o.wide_e), g.tile_m0 = I32(o.wide_m0), g.ntiles = I32(o.nwide), g.off = I32(o.off);
   auto launch = [&](bool up) {

@@ -42,19 +42,23 @@ using pf8::wait_loads;
 //     load scale words were 1.25 of the 5.7 GB; eight a load (the weight rows' in ONE buffer, which the wave frees by reading it) 5.3
 //     GB, gate/up 1022 -> 989 us;
 //   * an expert of many rows reads its weights once a tile: 160 positions instead of 128 (T = 2000 / 6000 1280 -> 1246, 2100 -> 2013).
-template <int POS, int WF, int TB_>
+// R > 0: the shared expert's shape for one workgroup a CU (k_few): weights and activations R turns ahead, and two buffers of the weight
+// rows' scale words.
+template <int POS, int WF, int TB_, int R = 0>
 struct Shape {
   static constexpr bool F4 = WF == DSGX_FMT_MXFP4_G32;
   static constexpr int kPos = POS, kSub = POS / 16, RA = 4, TB = TB_;
   static constexpr int kRowB = F4 ? 64 * TB : 128;  // bytes of a weight row in a turn
   static constexpr int kTileB = 16 * kRowB, LT = kRowB / 64;  // a 16-row weight tile, its loads
-  static constexpr int kRing = F4 ? (POS == 32 ? 6 : 4) : POS == 128 ? 4 : 6;  // the wave's own ring of weight tiles
-  static constexpr int kStageX = POS * 128;         // one block's activations; two stages of TB blocks
+  static constexpr int kRing = R ? 4 * R : F4 ? (POS == 32 ? 6 : 4) : POS == 128 ? 4 : 6;  // the wave's own ring of weight tiles
+  static constexpr int kAhead = R ? R : 1, kStages = kAhead + 1;
+  static constexpr int kStageX = POS * 128;         // one block's activations; a stage is TB blocks
   static constexpr int kHX = POS / 8 / kWaves;      // the 8-position half tiles that a wave brings
-  static constexpr int kOffX = kWaves * kRing * kTileB, kOffS = kOffX + 2 * TB * kStageX;
+  static constexpr int kOffX = kWaves * kRing * kTileB, kOffS = kOffX + kStages * TB * kStageX;
   static constexpr int kScaleW = kWgRows * 32, kScaleX = POS * 32;  // eight blocks' scale words of the weight rows, and of the positions (two such buffers)
-  static constexpr int kOffSX = kOffS + kScaleW, kLds = kOffSX + 2 * kScaleX;   // (the epilogues reuse it: UP kPos x 256 B, DOWN 4 x 2 KiB)
+  static constexpr int kOffSX = kOffS + (R ? 2 : 1) * kScaleW, kLds = kOffSX + 2 * kScaleX;   // (the epilogues reuse it: UP kPos x 256 B, DOWN 4 x 2 KiB)
   static_assert(F4 || TB == 1, "pairs of blocks are for 64-byte rows");
+  static_assert(R == 0 || TB == 1, "R blocks of weights");
 };
 
 // The shared expert's side of a launch that holds its tiles too (k_gemm_mixed): the first `grid` workgroups are theirs
@@ -100,9 +104,9 @@ __device__ __forceinline__ v4f_t mfma_mx(v8i_t a, v8i_t b, v4f_t c, int sa, int 
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, CBSZ, 0, 0, sa, 0, sb);
 }
 
-template <bool UP, int POS, int WF, int TB, bool STREAM = false>
+template <bool UP, int POS, int WF, int TB, bool STREAM = false, int R = 0>
 __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, int m0, int mend, int ns) {
-  using S = Shape<POS, WF, TB>;
+  using S = Shape<POS, WF, TB, R>;
   constexpr bool F4 = S::F4;
   constexpr int CBSZ = F4 ? 4 : 0;
   const int K = UP ? g.H : g.I, KB = K / 128, G = K / 32;
@@ -138,8 +142,9 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
     const int r = 32 * i + (lane >> 1), row = tile_row(S::RA * wave + (r >> 4)) + (r & 15);
     pws[i] = (UP && ((r >> 4) & 1) ? sb : sa) + (size_t)(F4 ? row : row / 32) * G + (KB >= 8 ? 16 * sc_half(r & 15, lane) : 0);
   }
-  // activations: half tile kHX wave + i is positions 8 (kHX wave + i) ...; those past the tile's rows are not fetched
-  const int nhx = uni(min(S::kHX, max(0, (mend - m0 + 7) / 8 - S::kHX * wave)));
+  // activations: half tile kHX wave + i is positions 8 (kHX wave + i) ...; those past the tile's rows are not fetched (R: they are, so that
+  // every wave has as many loads in flight as its waits count)
+  const int nhx = R ? S::kHX : uni(min(S::kHX, max(0, (mend - m0 + 7) / 8 - S::kHX * wave)));
   auto row_of = [&](int p) {  // the activation row of the tile's position p (a ragged tile re-reads its last row: never stored)
     const int pos = min(m0 + p, mend - 1);
     return (uint32_t)(g.gather ? g.gather[pos] : pos);
@@ -167,7 +172,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
     pf8::dma16_w<STREAM>(wt[i] + (size_t)min(t, TN - 1) * S::kRowB, ow[hh], uni(ring0 + (uint32_t)slot * S::kTileB + hh * 1024));
   };
   auto issue_x = [&](int t) {
-    const uint32_t xbase = lds0 + S::kOffX + (uint32_t)(t & 1) * (TB * S::kStageX) + (uint32_t)wave * (S::kHX * 1024);
+    const uint32_t xbase = lds0 + S::kOffX + (uint32_t)(t % S::kStages) * (TB * S::kStageX) + (uint32_t)wave * (S::kHX * 1024);
 #pragma unroll
     for (int b = 0; b < TB; ++b)
 #pragma unroll
@@ -177,7 +182,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
       }
   };
   // The scale words of the group that turn t opens (blocks 8 q ... 8 q + 7; the last ones of a row from its end): the weight rows'
-  // into the wave's one buffer, which is free when the group's last words are read; the positions' into two. A line of L2 holds a
+  // into the wave's one buffer, which is free when the group's last words are read (R: into two); the positions' into two. A line of L2 holds a
   // row's words of 32 blocks and has left L2 when the next group comes, so what counts is how often it is named. Rows of fewer than
   // eight blocks: their words are put in place by hand.
   constexpr int kGroupTurns = 8 / TB;
@@ -185,7 +190,7 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   auto issue_scales = [&](int t) {
     const int q = t / kGroupTurns, kb = first_block(q);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) dma16(pws[i] + 4 * kb, uni(lds0 + S::kOffS + (uint32_t)wave * 2048 + i * 1024));
+    for (int i = 0; i < 2; ++i) dma16(pws[i] + 4 * kb, uni(lds0 + S::kOffS + (R ? (uint32_t)(q & 1) * S::kScaleW : 0) + (uint32_t)wave * 2048 + i * 1024));
 #pragma unroll
     for (int i = 0; i < kSI; ++i)
       if (nhx > 0 && 64 * i + lane < 2 * kPosWave) dma16(g.as + 4 * kb, oxs[i], uni(lds0 + S::kOffSX + (uint32_t)(q & 1) * S::kScaleX + (uint32_t)wave * (32 * kPosWave) + i * 1024));
@@ -217,9 +222,11 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
   }
   issue_x(0);
 #pragma unroll
-  for (int i = 0; i < S::kRing; ++i)
+  for (int i = 0; i < S::kRing; ++i) {
+    if (R && i > 0 && i % 4 == 0) issue_x(i / 4);
 #pragma unroll
     for (int hh = 0; hh < S::LT; ++hh) issue_w(i / 4, i % 4, i, hh);
+  }
 
   // fragment reads. The instruction numbers an 8-bit operand's k as 64 h + 16 part + i (h: the lane's first or second four
   // registers, i: the byte) and a 4-bit operand's as 32 part + i, and takes the scale of k block g = k / 32 from the lanes
@@ -250,16 +257,17 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
     constexpr int NJ = decltype(nj_c)::value;
     int slot = 0;  // of the turn's first weight tile: 4 t % kRing
     for (int t = 0; t < TN; ++t) {
-      // this wave's loads of turn t have landed (weight tiles of later turns may be in flight); after the barrier everyone's have,
-      // and everyone is done reading the stage of turn t - 1, which the activations of turn t + 1 now overwrite
-      wait_loads<S::LT * (S::kRing - 4)>();
+      // this wave's loads of turn t have landed (weight tiles of later turns may be in flight; R: all of R - 1 later turns, loads of scales
+      // among them only make the wait longer); after the barrier everyone's have, and everyone is done reading the stage of turn
+      // t - 1, which the activations of turn t + kAhead now overwrite
+      wait_loads<R ? (R - 1) * (4 * S::LT + S::kHX) : S::LT * (S::kRing - 4)>();
       __syncthreads();
       const int q = t / kGroupTurns, word = TB * t - (KB >= 8 ? first_block(q) : 0);  // the turn's first word of its group's
       // (a turn of two blocks begins at an even word: both lie in one half)
       const int at = r16 * 32 + 16 * sc_half(r16, word >> 2) + 4 * (word & 3);  // the lane's row's words of the turn in a 16-row (16-position) tile's 512 bytes; its byte: `part`
-      const uint8_t* WS = smem + S::kOffS + wave * 2048 + at;
+      const uint8_t* WS = smem + S::kOffS + (R ? (q & 1) * S::kScaleW : 0) + wave * 2048 + at;
       const uint8_t* XS = smem + S::kOffSX + (size_t)(q & 1) * S::kScaleX + at;
-      const uint8_t* X = smem + S::kOffX + (size_t)(t & 1) * (TB * S::kStageX);
+      const uint8_t* X = smem + S::kOffX + (size_t)(t % S::kStages) * (TB * S::kStageX);
       int sl[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) sl[i] = slot + i >= S::kRing ? slot + i - S::kRing : slot + i;
@@ -273,19 +281,30 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
           fa[b][i] = F4 ? frag4(W, b) : frag8(W);
           fs[b][i] = (*reinterpret_cast<const uint32_t*>(WS + i * 512 + 4 * b) >> rsh) & 0xFFu;
         }
-      issue_x(t + 1);
+      if (R && (t + S::kAhead) % kGroupTurns == 0 && t + S::kAhead < TN) issue_scales(t + S::kAhead);
+      issue_x(t + S::kAhead);
 #pragma unroll
       for (int b = 0; b < TB; ++b)  // (read: what holds them may be written from here on)
         asm volatile("" : "+v"(fa[b][0]), "+v"(fa[b][1]), "+v"(fa[b][2]), "+v"(fa[b][3]), "+v"(fs[b][0]), "+v"(fs[b][1]), "+v"(fs[b][2]), "+v"(fs[b][3]));
-      if ((t + 1) % kGroupTurns == 0 && t + 1 < TN) issue_scales(t + 1);
+      if (!R && (t + 1) % kGroupTurns == 0 && t + 1 < TN) issue_scales(t + 1);
+      // (R: a wave has its SIMD for itself, so the next step's fragment is read before this one's MFMAs)
+      v8i_t fn;
+      int xn;
+      auto next = [&](int j) { fn = frag8(X + j * 2048), xn = (*reinterpret_cast<const uint32_t*>(XS + j * 512) >> rsh) & 0xFFu; };
+      if constexpr (R) next(0);
       static_for<NJ>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
         v8i_t fb[TB];
         int xsb[TB];
+        if constexpr (R) {
+          fb[0] = fn, xsb[0] = xn;
+          if (j + 1 < NJ) next(j + 1);
+        } else {
 #pragma unroll
-        for (int b = 0; b < TB; ++b) {
-          fb[b] = frag8(X + b * S::kStageX + j * 2048);
-          xsb[b] = (*reinterpret_cast<const uint32_t*>(XS + j * 512 + 4 * b) >> rsh) & 0xFFu;
+          for (int b = 0; b < TB; ++b) {
+            fb[b] = frag8(X + b * S::kStageX + j * 2048);
+            xsb[b] = (*reinterpret_cast<const uint32_t*>(XS + j * 512 + 4 * b) >> rsh) & 0xFFu;
+          }
         }
         // (the weights' loads one by one between the MFMAs)
 #pragma unroll
@@ -406,9 +425,19 @@ __global__ void __launch_bounds__(kThreads4, 2) k_gemm(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int NS = UP ? g.I / (kWgRows / 2) : g.H / kWgRows;
   int tile, ns;
-  pf8::task_of<true>(NS, tile, ns);
+  pf8::task_of<true>(NS, tile, ns, blockIdx.x, g.map);
   if (ns >= NS || tile * 128 >= g.nrows) return;
   shared_tile<UP>(g, smem, tile * 128, g.nrows, ns);
+}
+// ... in fewer tiles than the chip has CUs: one workgroup a CU, which has the CU's LDS for loads in flight.
+template <bool UP, int POS, int R>
+__global__ void __launch_bounds__(kThreads4, 2) k_few(Args g) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  const int NS = UP ? g.I / (kWgRows / 2) : g.H / kWgRows;
+  int tile, ns;
+  pf8::task_of<true>(NS, tile, ns, blockIdx.x, g.map);
+  if (ns >= NS || tile * POS >= g.nrows) return;
+  gemm_tile<UP, POS, DSGX_FMT_FP8_B32E, 1, false, R>(g, smem, -1, tile * POS, g.nrows, ns);
 }
 // The routed experts' list of tiles, an expert's tiles next to each other.
 // A tile of up to 64 rows runs two blocks a turn where K is pairs of blocks.

@@ -256,6 +256,22 @@ def test_dsk_prefill_scale_groups_and_block_pairs(H, I, T):
 
 
 
+@pytest.mark.parametrize("H,I,T", [(256, 128, 1), (1280, 2048, 130), (1280, 2048, 1024), (1280, 2048, 1030), (4096, 1152, 200)])
+def test_dsk_prefill_shared_expert_alone(H, I, T):
+    """the shared expert as a phase of its own: tiles of 64 rows while they are one a CU (K of 1 to 32 blocks, last groups of scale words that
+    are not whole, a ragged last tile), of 128 and 64 beyond: the bits of a whole step"""
+    E, topk = 3, 1
+    L = Stacked(43, H, I, E, topk, 3, True)
+    x = orc.normal_bf16(43, 1, (T, H), 1.5)
+    idx, w = orc.route(orc.normal_f32(43, 2, (T, E), 1.0), orc.normal_f32(43, 3, (E,), 0.2), topk, 1.5, score_fn=1)
+    xq, xs = orc.act_quant_ue8m0(x)
+    got = run_prefill(L, xq, xs, idx, w)
+    ws, y2 = gpu.empty(lib.dsk_prefill_ws_bytes(H, I, E, topk, T), 0x11), gpu.empty(T * H * 4, 0)
+    for ph in (2, 1, 4, 8, 16):
+        lib.dsk_moe_prefill(L.w, gpu.dev(xq), gpu.dev(xs), gpu.dev(idx), gpu.dev(w), T, ws, y2, phases=ph)
+    assert np.isfinite(got["y"]).all() and np.array_equal(gpu.host(y2, np.uint32, (T, H)), got["y"].view(np.uint32))
+
+
 def test_dsk_prefill_refuses_what_it_cannot_run():
     L = Stacked(42, 1024, 512, 16, 6, 2, False)
     xq = gpu.empty(4 * 1024, 0)
