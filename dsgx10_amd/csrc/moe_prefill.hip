@@ -1014,11 +1014,21 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
     if (int rc = allow_dynamic_lds(k, pf8::kLds)) return rc;
   pf8::Args g{};
   g.L = *L;
+  const bool mixed = order >= 1;
   // Which workgroups share an XCD. Few rows an expert: eight row groups of one tile, an expert is a tile and the chip is even in small
-  // blocks; many rows: eight tiles x four row groups, so that an expert's tiles find its weights in L2. 4096 x 2048, 256 experts, top-8,
-  // 1 x 8 / 8 x 4: T = 20 340 / 358 us, T = 200 991 / 1019, T = 700 1271 / 1313, T = 1500 1432 / 1440, T = 3000 1715 / 1716, T = 5000
-  // 2115 / 2106, T = 8192 2844 / 2814 (other shapes of 1 to 8 tiles x 1 to 32 groups lie between or above).
-  auto map_for = [&](int NS) { return (long long)P >= 94LL * E ? pf8::map_of(3, 2, NS) : pf8::map_of(0, 3, NS); };
+  // blocks; many rows: blocks of several tiles, so that an expert's tiles find its weights in L2 - eight tiles x four row groups where the launch
+  // is many rounds of workgroups over the chip, four x two where blocks of 32 would be too few to be even over the XCDs; tiles
+  // that are not an expert's next to each other share nothing. 1 x 8 / 4 x 2 / 8 x 4, us:
+  //   4096 x 2048, 256 experts, top-8: T = 200 872 / 877 / 903, 700 1164 / 1163 / 1174, 1500 1325 / 1310 / 1322, 3100 1585 / 1584 / 1598,
+  //   5000 1981 / 1976 / 1949, 8192 2695 / 2674 / 2651 (2048 x 1024: 8192 850 / 835 / 829)
+  //   64 experts, top-8: T = 400 367 / 356 / 367, 700 443 / 429 / 435, 1000 492 / 480 / 515, 1500 583 / 577 / 587, 4000 1204 / 1175 / 1176
+  //   32 experts, top-4: T = 400 206 / 197 / 226, 800 252 / 246 / 278, 1500 353 / 334 / 384, 2500 469 / 462 / 468; 16 experts: T = 250 140 / 131 / 132
+  //   3072 x 1536, 128 experts, top-6: T = 1000 445 / 448 / 465, 1500 483 / 497 / 530, 2200 552 / 552 / 566, 5000 849 / 831 / 818
+  auto map_for = [&](int NS) {
+    const long long rounds = (long long)o.max_wide * NS / (2 * num_cus_cached());
+    if (mixed || (long long)P < (rounds < 4 ? 48LL : 94LL) * E) return pf8::map_of(0, 3, NS);
+    return rounds >= 6 ? pf8::map_of(3, 2, NS) : pf8::map_of(2, 1, NS);
+  };
   g.fast_act = cfg.fast_act;
   // Small tiles' rings: deep where few are in flight (T = 17 / 30 / 50 320 / 437 / 538 -> 301 / 418 / 530 us), else the chip's loads stand
   // in each other's way (at T = 200 and beyond rings of 4 to 6 tiles and of 8 are within 2%, on most chunks the shorter ahead).
@@ -1027,7 +1037,6 @@ int dsgx_moe_prefill(const dsgx_layer_w* L, const uint16_t* x, const int* idx, c
   if (const char* tp = std::getenv("DSGX_PF_TRACE_PTR")) g.trace = reinterpret_cast<unsigned long long*>(std::strtoull(tp, nullptr, 0));
 #endif
   const int NSU = I / (pf8::kWgRows / 2), NSD = H / pf8::kWgRows;
-  const bool mixed = order >= 1;
   g.tile_e = I32(mixed ? o.ord_e : o.wide_e), g.tile_m0 = I32(mixed ? o.ord_m0 : o.wide_m0), g.ntiles = I32(o.nwide), g.off = I32(o.off), g.nrows = T;
   // A whole step runs the shared expert's tiles in the routed experts' launches, in front of them: alone they are a launch
   // of few workgroups at small T, and two more tails (as kernels of eight waves, whole call, hidden 4096, intermediate
