@@ -1199,11 +1199,18 @@ int dsgx_dsk_moe_prefill(const dsgx_dsk_weights* Wt, const uint8_t* xq, const ui
     if (int rc = launch_shared_mx<false>(g, NSD, st)) return rc;
   }
   g.tile_e = I32(o.wide_e), g.tile_m0 = I32(o.wide_m0), g.ntiles = I32(o.nwide), g.off = I32(o.off);
+  g.tile_e_low = I32(o.tile_e), g.tile_m0_low = I32(o.tile_m0), g.ntiles_low = I32(o.ntiles);
+  int max_tiles = o.max_wide;
+  auto few_rounds = [&](int NS) {  // whether the launch may be of two rounds or less (lower_tiles): by full tiles alone
+    const bool few = (long long)(P / pf8::kMaxPos) * NS <= 4LL * num_cus_cached();
+    g.slots = few ? 2 * num_cus_cached() : 0, max_tiles = few ? o.max_tiles : o.max_wide;
+  };
   auto launch = [&](bool up) {
-    hipLaunchKernelGGL(up ? k_up : k_dn, dim3(g.sh.grid + pf8::grid_of(o.max_wide, up ? NSU : NSD, g.map)), dim3(pf8::kThreads4), pfmx::kLds, st, g);
+    hipLaunchKernelGGL(up ? k_up : k_dn, dim3(g.sh.grid + pf8::grid_of(max_tiles, up ? NSU : NSD, g.map)), dim3(pf8::kThreads4), pfmx::kLds, st, g);
   };
   if (cfg.phases & 4) {
     g.aq = xq, g.as = xs, g.gather = I32(o.perm), g.posw = F32(o.posw), g.map = map_for(NSU);
+    few_rounds(NSU);
     g.wa = Wt->w1, g.sa = Wt->s1, g.wb = Wt->w3, g.sb = Wt->s3, g.wstride = (size_t)I * H / 2, g.sstride = (size_t)I * H / 32;
     g.h = U16(o.h), g.hq = W + o.hq, g.hs = W + o.hs, g.d = nullptr;
     if (fused_sh)
@@ -1213,6 +1220,7 @@ int dsgx_dsk_moe_prefill(const dsgx_dsk_weights* Wt, const uint8_t* xq, const ui
   }
   if (cfg.phases & 8) {
     g.aq = W + o.hq, g.as = W + o.hs, g.gather = nullptr, g.posw = nullptr, g.map = map_for(NSD);
+    few_rounds(NSD);
     g.wa = Wt->w2, g.sa = Wt->s2, g.wb = g.sb = nullptr, g.wstride = (size_t)I * H / 2, g.sstride = (size_t)I * H / 32;
     g.h = nullptr, g.hq = g.hs = nullptr, g.d = U16(o.d);
     if (fused_sh)

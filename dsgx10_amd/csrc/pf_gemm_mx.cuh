@@ -79,6 +79,8 @@ struct Args {
   const int* ntiles;
   const int* off;
   int nrows;
+  const int *tile_e_low, *tile_m0_low, *ntiles_low;  // the same rows as a list of tiles of kLowPos positions
+  int slots;           // workgroups that the chip holds at once (lower_tiles)
   int stream;          // weights of experts of one small tile as streaming loads
   int H, I;
   const uint8_t *wa, *sa, *wb, *sb;  // UP: gate (w1), up (w3); DOWN: w2 in wa / sa. Expert e at + e * wstride / sstride.
@@ -439,6 +441,19 @@ __global__ void __launch_bounds__(kThreads4, 2) k_few(Args g) {
   if (ns >= NS || tile * POS >= g.nrows) return;
   gemm_tile<UP, POS, DSGX_FMT_FP8_B32E, 1, false, R>(g, smem, -1, tile * POS, g.nrows, ns);
 }
+// Whether the routed experts' rows go in tiles of 128 positions instead of 160. Many rounds of workgroups over the chip: 160, an expert's
+// weights are read less often. Up to two: what the rounds take by the tallest tile of each, from the very counts of tiles (a fortieth of a
+// round does not count: its workgroups find the slots of small tiles). Top-4 of 32, 160 / 128: hidden 1024, intermediate 512, T = 1000 / 2000 / 3000 /
+// 4500 / 6000 50.8 / 45.3, 55.6 / 57.4, 68.1 / 61.5, 77.7 / 91, 111.5 / 102.4 us, hidden 2048 62.9 / 56.4, 70.8 / 78.3, 98.2 / 89.3, 112 / 129, 155.5 /
+// 149.5. As kernels of eight waves and 256 positions 58, 60.4, 62.7, 102, 105 and 70.6, 83.3, 88.1, 138, 154.
+constexpr int kLowPos = 128;
+__device__ __forceinline__ bool lower_tiles(const Args& g, int NS) {
+  if (!g.slots) return false;
+  const int shared = g.sh.grid ? (g.nrows + 127) / 128 : 0;
+  auto rounds = [&](int n) { return (40 * (n + shared) * NS + 39 * g.slots - 1) / (40 * g.slots); };
+  const int r = rounds(*g.ntiles);
+  return r <= 2 && rounds(*g.ntiles_low) * kLowPos < r * kMaxPos;
+}
 // The routed experts' list of tiles, an expert's tiles next to each other.
 // A tile of up to 64 rows runs two blocks a turn where K is pairs of blocks.
 template <bool UP>
@@ -457,13 +472,15 @@ __global__ void __launch_bounds__(kThreads4, 2) k_gemm_mixed(Args g) {
     return;
   }
   pf8::task_of<false>(NS, tile, ns, blockIdx.x - g.sh.grid, g.map);
-  if (ns >= NS || tile >= *g.ntiles) return;
-  const int e = g.tile_e[tile];
-  const int m0 = g.off[e] + g.tile_m0[tile], mend = g.off[e + 1];
+  const bool low = lower_tiles(g, NS);
+  const int *tile_e = low ? g.tile_e_low : g.tile_e, *tile_m0 = low ? g.tile_m0_low : g.tile_m0;
+  if (ns >= NS || tile >= *(low ? g.ntiles_low : g.ntiles)) return;
+  const int e = tile_e[tile];
+  const int m0 = g.off[e] + tile_m0[tile], mend = min(g.off[e + 1], m0 + (low ? kLowPos : kMaxPos));
   const bool pairs = (UP ? g.H : g.I) % 256 == 0;
   if (mend - m0 > 64 || !pairs) gemm_tile<UP, kMaxPos, F4, 1>(g, smem, e, m0, mend, ns);
   else if (mend - m0 > 32) gemm_tile<UP, 64, F4, 2>(g, smem, e, m0, mend, ns);
-  else if (g.stream && g.tile_m0[tile] == 0) gemm_tile<UP, 32, F4, 2, true>(g, smem, e, m0, mend, ns);
+  else if (g.stream && tile_m0[tile] == 0) gemm_tile<UP, 32, F4, 2, true>(g, smem, e, m0, mend, ns);
   else gemm_tile<UP, 32, F4, 2>(g, smem, e, m0, mend, ns);
 }
 

@@ -224,12 +224,11 @@ def test_dsk_prefill_picks_a_row(topk):
         assert np.array_equal(got["y"][t].view(np.uint32), fold.view(np.uint32)), t
 
 
-@pytest.mark.parametrize("H,I", [(256, 128), (512, 1152), (1280, 256)])
-def test_dsk_prefill_tile_shapes_give_the_same_bits(H, I):
-    """experts whose rows end at the edges of the tiles of 32, 64 and 160 positions (and one row beyond), K in whole pairs of blocks and
-    not: every row has the bits that it has alone in a chunk, in the smallest tile"""
-    counts, topk = [1, 8, 9, 32, 33, 64, 65, 160, 161, 321], 1
-    L = Stacked(43, H, I, len(counts), topk, 5, True)
+def _rows_have_their_bits_alone(H, I, counts, shared):
+    """a chunk of counts[e] rows of each expert: rows at the ends and inside of each have the bits that they have alone in a chunk, in
+    the smallest tile"""
+    topk = 1
+    L = Stacked(43, H, I, len(counts), topk, 5, shared)
     idx = np.repeat(np.arange(len(counts), dtype=np.int32), counts)[:, None].copy()
     T = len(idx)
     x = orc.normal_bf16(43, 1, (T, H), 1.5)
@@ -237,9 +236,25 @@ def test_dsk_prefill_tile_shapes_give_the_same_bits(H, I):
     xq, xs = orc.act_quant_ue8m0(x)
     got = run_prefill(L, xq, xs, idx, w)
     ends = np.cumsum(counts)
-    for t in sorted(set(int(v) for e, n in zip(ends, counts) for v in (e - n, e - 1 - n // 2, e - 1 - n % 16 * (n > 16), e - 1))):
+    rows = set(int(v) for e, n in zip(ends, counts) if n > 1 for v in (e - n, e - 1 - n // 2, e - 1 - n % 16 * (n > 16), e - 1))
+    for t in sorted(rows | {0, T - 1}):
         one = run_prefill(L, xq[t:t + 1].copy(), xs[t:t + 1].copy(), idx[t:t + 1], w[t:t + 1])
         assert np.array_equal(got["y"][t].view(np.uint32), one["y"][0].view(np.uint32)), t
+
+
+@pytest.mark.parametrize("H,I", [(256, 128), (512, 1152), (1280, 256)])
+def test_dsk_prefill_tile_shapes_give_the_same_bits(H, I):
+    """experts whose rows end at the edges of the tiles of 32, 64, 128 and 160 positions (and one row beyond), K in whole pairs of blocks and
+    not; so small a launch takes the list of 128-position tiles"""
+    _rows_have_their_bits_alone(H, I, [1, 8, 9, 32, 33, 64, 65, 128, 129, 160, 161, 257, 321], True)
+
+
+@pytest.mark.parametrize("H,I,counts", [(256, 6144, [160, 159, 130, 321, 161, 33, 64]), (256, 6144, [160, 159, 130, 321, 161, 33, 64, 96]),
+                                        (4096, 256, [1] * 60 + [159, 160, 161, 320, 321, 33]), (4096, 384, [1] * 60 + [160, 321, 65])])
+def test_dsk_prefill_tiles_of_160_positions(H, I, counts):
+    """launches that take the list of 160-position tiles: a round of workgroups where tiles of 128 are two (gate/up of the first; of the second
+    both are two), and more than two rounds (down of the last two)"""
+    _rows_have_their_bits_alone(H, I, counts, False)
 
 
 @pytest.mark.parametrize("H,I,T", [(256, 128, 17), (256, 384, 10), (512, 640, 64), (768, 1152, 90), (1024, 1280, 33)])
