@@ -1179,12 +1179,13 @@ int dsgx_dsk_moe_prefill(const dsgx_dsk_weights* Wt, const uint8_t* xq, const ui
   }
   pfmx::Args g{};
   g.H = H, g.I = I, g.nrows = T, g.limit = cfg.swiglu_limit;
-  // (as for the FP8 layers; 1 tile x 2 / 4 x 2, T = 20
-  // 237 / 246 us, T = 60 411 / 419, T = 300 803 / 812, T = 1000 1076 / 1078, T = 2000 1267 / 1245, T = 6000 2103 / 2015)
+  // (as for the FP8 layers; 1 tile x 2 / 4 x 2 / 4 x 4, us: 5120 x 2304, 256 experts, top-6: T = 60 358 / 369 / 371, T = 250 712 / 723 / 724, T = 1000 1059 / 1060 /
+  // 1061, T = 2000 1241 / 1231 / 1237, T = 3000 1428 / 1396 / 1393, T = 6000 2066 / 1965 / 1952; 6144 x 1536, 96 experts: T = 600 371 / 369 / 368, T = 800 411 /
+  // 411 / 401, T = 3000 699 / 678 / 657; 3072 x 1536, 128 experts: T = 600 261 / 264 / 265, T = 2000 367 / 361 / 355, T = 6000 743 / 726 / 712)
   // (streaming loads of small tiles' weights, as the FP8 layers', while tiles are small: T = 20 / 60 / 300 / 500 249 / 409 / 781 / 948 -> 226 / 366 /
   // 771 / 947 us, T = 700 / 1000 / 3000 1021 / 1084 / 1460 -> 1034 / 1100 / 1472)
   g.stream = P < 12 * E;
-  auto map_for = [&](int NS) { return (long long)P >= 24LL * E ? pf8::map_of(2, 1, NS) : pf8::map_of(0, 1, NS); };
+  auto map_for = [&](int NS) { return (long long)P >= 24LL * E ? pf8::map_of(2, 2, NS) : pf8::map_of(0, 1, NS); };
   // a whole step runs the shared expert's tiles in the routed experts' launches, in front of them (as the FP8 layers do;
   // hidden 5120, intermediate 2304, T = 17: 417 -> 362 us, T = 600: 1405 -> 1334, T = 3000: 1870 -> 1821)
   const int sh_tiles = tiles_of(T, 128);
