@@ -256,8 +256,8 @@ def test_decode_mfma_variant_every_bit_against_the_matrix_unit_oracle(fmt, H, I,
 
 @pytest.mark.parametrize("up", [0, 1])
 def test_decode_int4_scales_above_the_fast_decodes_range(up):
-    """a wave of variant 1 that meets a scale of 2^116 or more decodes the step by the routine for every scale, which variant 0 has
-    only: every bit against the oracle in the kernels' order of adds"""
+    """a wave of variant 1 that met a scale of 2^116 or more in a unit does the unit once more by the routine for every scale, the only one
+    that variant 0 has: every bit against the oracle in the kernels' order of adds"""
     H, I, E, topk = 2048, 2048, 8, 4
     hl, x, idx, w = int4_layer_with_large_scales(H, I, E, topk, 62, 8)
     dl = hl.upload()
@@ -273,6 +273,36 @@ def test_decode_int4_scales_above_the_fast_decodes_range(up):
             assert np.array_equal(yr.view(np.uint32), dn["yr32"].view(np.uint32)), (M, int((yr != dn["yr32"]).sum()))
     finally:
         orc.set_dot_rule(0)
+
+
+@pytest.mark.parametrize("shared", [None, "bf16", "fp8"])
+def test_decode_int4_large_scales_beside_a_shared_expert_and_over_eight_rows(shared):
+    """the units done once more in a stream that also holds the shared expert's units (BF16, FP8), and in the pass of 9 to 16 rows, whose
+    dots are kept by pick: one row against the oracle in the kernels' order of adds, every row of more against the row alone"""
+    H, I, E, topk, rows = 2048, 1024, 8, 4, 16
+    hl, x, idx, w = int4_layer_with_large_scales(H, I, E, topk, 62, rows)
+    if shared:
+        sh = make_layer(abi.FMT_INT4, H, I, E, topk, 1, seed=63, shared=shared)
+        hl = HostLayer(abi.FMT_INT4, H, I, E, topk, hl.experts, shared_fp8=sh.shared_fp8, shared_bf16=sh.shared_bf16)
+    dl = hl.upload()
+    alone = [gpu.decode_layer(dl, x[m:m + 1], idx[m:m + 1], w[m:m + 1], 1, up=1)[:2] for m in range(rows)]
+    orc.set_dot_rule(2)
+    try:
+        for m in (0, 7):
+            uni = orc.union(idx[m:m + 1], E)
+            dn = orc.moe_down(hl, orc.moe_up(hl, x[m:m + 1], uni)["h32"], idx[m:m + 1], w[m:m + 1], uni)
+            assert np.isfinite(alone[m][0]).all() and (alone[m][0] != 0).mean() > 0.9
+            assert np.array_equal(alone[m][0].view(np.uint32), dn["yr32"].view(np.uint32)), m
+            if shared:
+                assert np.array_equal(alone[m][1].view(np.uint32), dn["ys32"].view(np.uint32)), m
+    finally:
+        orc.set_dot_rule(0)
+    for M in (2, 8, 9, 16):
+        yr, ys, _ = gpu.decode_layer(dl, x[:M], idx[:M], w[:M], M, up=1)
+        for m in range(M):
+            assert np.array_equal(yr[m].view(np.uint32), alone[m][0][0].view(np.uint32)), (M, m)
+            if shared:
+                assert np.array_equal(ys[m].view(np.uint32), alone[m][1][0].view(np.uint32)), (M, m)
 
 
 @pytest.mark.parametrize("fmt,H,I,E,topk,shared,scale", [(abi.FMT_FP8, 2048, 1024, 32, 8, "fp8", 1.0), (abi.FMT_FP8, 1024, 2048, 256, 8, None, 1.0),

@@ -179,7 +179,7 @@ def check_chunk(L, x, idx, w, rows, got, note="", e2e=3e-3):
 
 @pytest.mark.parametrize("H,I,E,T,shared", [(1024, 512, 16, 300, True), (2048, 768, 8, 700, True), (1024, 256, 32, 37, False), (1024, 512, 16, 1, True)])
 def test_dsk_prefill_against_oracle(H, I, E, T, shared):
-    """T = 700 over 8 experts: buckets of ~500 rows, i.e. 256-position tiles and ragged remainders; T = 37 over 32: experts
+    """T = 700 over 8 experts: buckets of ~500 rows, i.e. 160-position tiles and ragged remainders; T = 37 over 32: experts
     with no rows at all; T = 1"""
     topk = 6
     L = Stacked(41, H, I, E, topk, 5, shared)

@@ -222,6 +222,57 @@ def test_gemv_int4_scales_above_the_fast_decodes_range(N, K, M, sk):
     assert np.array_equal(got.view(np.uint32), o["yf"].view(np.uint32)), int((got != o["yf"]).sum())
 
 
+def _large_scales(tid, N, K, rows):
+    """an INT4 matrix whose `rows` have scales of 2^116 and more in their first, an inner and their last group of K"""
+    packed, scale, zp = quant_int4(31, tid, N, K)
+    rng = np.random.default_rng(tid)
+    for g in (0, K // 64 + 1, K // 32 - 1):
+        r = rows[rng.random(len(rows)) < 0.6]
+        scale[r, g] = ((127 + rng.integers(116, 120, len(r))) << 7 | rng.integers(0, 128, len(r))).astype(np.uint16)
+    return packed, scale, zp
+
+
+@pytest.mark.parametrize("sk", [1, 2])
+@pytest.mark.parametrize("out", [abi.OUT_BF16, abi.OUT_SWIGLU])
+@pytest.mark.parametrize("N,K,M", [(4200, 2048 + 256, 1), (3080, 4096 + 256, 8)])
+def test_gemv_int4_large_scales_in_every_output_kind(N, K, M, out, sk):
+    """the rows done once more are stored once more: bf16 outputs, and SwiGLU pairs of which gate, up or both are such rows, K whole and
+    over two slices of one wave. bf16: every bit of the oracle in the kernel's order of adds; SwiGLU: at most 0.2% one bf16 step off, where
+    the host's expf and the device's round silu to neighbours (the bar of the prefill's h)"""
+    x = orc.normal_bf16(31, 1, (M, K), 1.0)
+    rows = np.random.default_rng(5).permutation(N)[:N // 5]
+    parts = _large_scales(2, N, K, rows)
+    got = _run(x, abi.FMT_INT4, parts, N, K, out, splitk=sk)
+    orc.set_dot_rule(4, sk)
+    try:
+        want = _oracle(x, abi.FMT_INT4, parts, N, K, out)["y16"]
+    finally:
+        orc.set_dot_rule(0)
+    with np.errstate(over="ignore"):
+        assert (np.abs(orc.bf16_to_f32(want).astype(np.float64)) > 2.0 ** 100).mean() > 0.05
+    if out == abi.OUT_BF16:
+        assert np.array_equal(got, want), int((got != want).sum())
+    else:
+        assert (got != want).mean() <= 0.002 and np.abs(got.astype(np.int32) - want.astype(np.int32)).max() <= 1, int((got != want).sum())
+
+
+@pytest.mark.parametrize("sk", [1, 2, 4])
+@pytest.mark.parametrize("out", [abi.OUT_BF16, abi.OUT_F32])
+def test_gemv_int4_large_scales_in_later_segments(out, sk):
+    """three matrices in a call, large scales in rows of the second and the third only (a wave's rows done once more lie in another segment
+    than its first): each segment's outputs are those of a call of its own, which the test above and the one for f32 hold to the oracle"""
+    M, K, ns = 3, 2048 + 256, (1032, 4104, 1048)
+    x = orc.normal_bf16(33, 1, (M, K), 1.0)
+    mats = [_large_scales(50 + i, n, K, np.arange(0) if i == 0 else np.arange(i, n, 7)) for i, n in enumerate(ns)]
+    esz, dt = (4, np.uint32) if out == abi.OUT_F32 else (2, np.uint16)
+    keep = [[gpu.dev(p) for p in m] for m in mats]
+    ys = [gpu.empty(M * n * esz, 0xFF) for n in ns]
+    lib.gemv(gpu.dev(x), K, M, K, [dict(fmt=abi.FMT_INT4, w=k[0], s=k[1], zp=k[2], n=n, y=y, ldy=n) for k, n, y in zip(keep, ns, ys)], out, splitk=sk)
+    for i, (n, m, y) in enumerate(zip(ns, mats, ys)):
+        alone = _run(x, abi.FMT_INT4, m, n, K, out, splitk=sk).view(dt)
+        assert np.array_equal(gpu.host(y, dt, (M, n)), alone), i
+
+
 @pytest.mark.parametrize("H", [2048, 4096, 6144])
 @pytest.mark.parametrize("mode", ["contract", "round2", "two_partials"])
 def test_add_norm(H, mode):

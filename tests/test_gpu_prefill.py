@@ -196,11 +196,19 @@ def test_prefill_fp8_scale_groups(H, I, T, unit_rule):
 @pytest.mark.parametrize("E,topk,T", [(3, 1, 1), (40, 8, 31), (40, 8, 33), (256, 8, 512), (256, 8, 513), (512, 2, 2048), (5, 1, 4096), (5, 1, 4097)])
 def test_prefill_buckets_at_the_edges_of_one_workgroup(E, topk, T):
     """the bucketing as one launch (up to 4096 picks whose masks fit LDS) and as three: offsets, rows in token order, each row's picks in
-    expert-id order and its factors, words of 32 rows that are full, one row more, and more words than lanes"""
+    expert-id order, words of 32 rows that are full, one row more, and more words than lanes; the factors s2_down * w and the lists of
+    tiles by what comes out: the rows that a chunk of some rows more (at 512 and 4096 rows beyond the one launch's picks) or fewer holds
+    too have its bits, and some rows the oracle's, from the h that the GPU made"""
     H, I = 256, 128
     hl = helpers.make_layer(abi.FMT_FP8, H, I, E, topk, 3, seed=8, shared=None)
-    x, _, idx, w = helpers.rows_and_routing(19, T, H, E, topk, 1.0)
-    _, _, ws, dl = _prefill(hl, x, idx, w, T)
+    hl.desc["s2"] = (0.5 + np.arange(3 * E, dtype=np.float32) % 7 / 5)  # (factors that tell the experts apart)
+    x, _, idx, w = helpers.rows_and_routing(19, T + 1, H, E, topk, 1.0)
+    more, _, _, _ = _prefill(hl, x, idx, w, T + 1)
+    few = (T + 1) // 2
+    fewer, _, _, _ = _prefill(hl, x[:few], idx[:few], w[:few], few)
+    x, idx, w = x[:T], idx[:T], w[:T]
+    yr, _, ws, dl = _prefill(hl, x, idx, w, T)
+    assert np.array_equal(yr.view(np.uint32), more[:T].view(np.uint32)) and np.array_equal(yr[:few].view(np.uint32), fewer.view(np.uint32))
     v, P = lib.prefill_view(dl.w, ws, T), T * topk
     off = gpu.host(gpu.view(ws, v.off, (E + 1) * 4), np.int32, (E + 1,))
     assert np.array_equal(off, np.concatenate([[0], np.cumsum(np.bincount(idx.reshape(-1), minlength=E))]))
@@ -210,7 +218,16 @@ def test_prefill_buckets_at_the_edges_of_one_workgroup(E, topk, T):
     pos[order] = np.arange(P)
     by_e = np.argsort(idx, axis=1)
     assert np.array_equal(gpu.host(gpu.view(ws, v.re, P * 4), np.int32, (T, topk)), np.take_along_axis(idx, by_e, 1))
-    assert np.array_equal(gpu.host(gpu.view(ws, v.rpos, P * 4), np.int32, (T, topk)), np.take_along_axis(pos.reshape(T, topk), by_e, 1))
+    rpos = np.take_along_axis(pos.reshape(T, topk), by_e, 1)
+    assert np.array_equal(gpu.host(gpu.view(ws, v.rpos, P * 4), np.int32, (T, topk)), rpos)
+    hg = gpu.host(gpu.view(ws, v.h, P * I * 2), np.uint16, (P, I))
+    orc.set_fp8_block_rule(1)
+    try:
+        for t in sorted({0, T // 2, T - 1}):
+            o = orc.moe_prefill_fp8_row(hl, x[t], idx[t], w[t], h_in=np.concatenate([hg[rpos[t]], np.zeros((1, I), np.uint16)]))
+            assert np.array_equal(yr[t].view(np.uint32), o["yr"].view(np.uint32)), t
+    finally:
+        orc.set_fp8_block_rule(0)
 
 
 def test_prefill_rows_do_not_depend_on_the_chunk():
@@ -240,17 +257,23 @@ def test_prefill_fp8_tile_shapes_give_the_same_bits(H, I):
         assert np.array_equal(ys[t].view(np.uint32), s1[0].view(np.uint32)), t
 
 
-def test_prefill_tile_order_does_not_change_a_bit():
+@pytest.mark.parametrize("T,want", [
+    (900, [0, 1, 17, 128, 129, 256, 257, 300, 421, 291]),       # (the rest of the picks over two more experts)
+    (580, [159, 160, 161, 320, 321, 0, 1, 33, 5]),              # at the edges of the 160-position tiles
+    (640, [160, 320, 0, 160, 480, 160]),                        # full tiles only: no remainders
+    (274, [159, 1, 32, 33, 100, 0, 64, 159]),                   # remainders only
+], ids=["any", "edges", "full", "remainders"])
+def test_prefill_tile_order_does_not_change_a_bit(T, want):
     """dsgx_prefill_cfg::tile_order (the reference's prefill_tuning tord, ds41f engine/kernels/dsk.h:252) only changes which
-    workgroup takes which tile: experts of 0, a few, 128, 129, 256 and several hundred rows (remainders, full
-    tiles and both), every order, the same yr, ys and workspace views as the order by expert id"""
-    H, I, E, topk, T = 256, 256, 12, 2, 900
+    workgroup takes which tile: experts of no rows, of a few, of full tiles, of remainders and of both, every order, the same h, yr and
+    ys as the order by expert id"""
+    H, I, topk = 256, 256, 2
+    # rows an expert as given (pairs (a, b), a < b, dealt so that the counts come out)
+    if sum(want) < 2 * T:
+        want = want + [(2 * T - sum(want)) // 2, (2 * T - sum(want) + 1) // 2]
+    E = len(want)
     hl = helpers.make_layer(abi.FMT_FP8, H, I, E, topk, 5, seed=9, shared="fp8")
     x, _, _, w = helpers.rows_and_routing(21, T, H, E, topk, 1.0)
-    # rows an expert: 0, 1, 17, 128, 129, 256, 257, 300, 421, ... (pairs (a, b), a < b, dealt so that the counts come out)
-    want = [0, 1, 17, 128, 129, 256, 257, 300, 421, 291, 0, 0]
-    want[10] = (2 * T - sum(want)) // 2
-    want[11] = 2 * T - sum(want)
     left = list(want)
     idx = np.zeros((T, topk), np.int32)
     for t in range(T):
@@ -263,11 +286,12 @@ def test_prefill_tile_order_does_not_change_a_bit():
     ref = None
     for order in (0, 1, 2, -1):
         yr, ys, ws, dl = _prefill(hl, x, idx, w, T, tile_order=order)
-        got = (yr.view(np.uint32), ys.view(np.uint32))
+        h = gpu.host(gpu.view(ws, lib.prefill_view(dl.w, ws, T).h, T * topk * I * 2), np.uint16, (-1,))
+        got = (yr.view(np.uint32), ys.view(np.uint32), h)
         if ref is None:
             ref = got
-            assert np.isfinite(yr).all() and np.isfinite(ys).all() and np.abs(yr).max() > 0
-        assert np.array_equal(ref[0], got[0]) and np.array_equal(ref[1], got[1]), order
+            assert np.isfinite(yr).all() and np.isfinite(ys).all() and (np.abs(yr).max(axis=1) > 0).all()
+        assert all(np.array_equal(a, b) for a, b in zip(ref, got)), order
     with pytest.raises(lib.DsgxError):
         _prefill(hl, x, idx, w, T, tile_order=3)
 
