@@ -49,7 +49,7 @@ __device__ __forceinline__ void fp8x8_to_bf16(uint32_t w0, uint32_t w1, uint32_t
 // scale is done once more by i4x8_to_bf16_any, whose terms are finite up to 2^124 (dequant_int4's own kernel uses the subtract-first form, for all).
 // Hidden 6144, intermediate 2048, 168 experts: gate/up's vector instructions at T = 1111 3.16e8 -> 2.69e8, the decode kernel's at 6
 // rows 8.6e7 -> 7.2e7; with the LDS slots that came with it the prefill call takes 1869 -> 1784 us, four decode layers 923 -> 909.
-// The split-K GEMV and the vector-unit decode kernels keep i4x8_to_bf16_any.
+// k_gemv_sk, k_gemv over K slices at eight rows and the vector-unit decode kernels keep i4x8_to_bf16_any.
 struct I4Group {
   float s, c0;   // the scale, -(1024 + u_z) s
   float s1, c1;  // s / 16, -(64 + u_z) s
@@ -516,7 +516,7 @@ __device__ __forceinline__ void silu4(const float (&g)[4], float (&s)[4]) {
 // are a quarter of theirs, which keeps the reciprocal normal up to the largest finite divisor, and the quarter of the divisor's 1 is one
 // step above 1/4: of the 65536 bf16 values, NaN, infinities and zeros included, every one rounds to the bits that the exact sequence
 // (expf, IEEE division) rounds to (all compared; with 1/4 itself 5.9375 alone does not). The prefill GEMMs' epilogues are bound by the
-// vector unit (the FP8 256-position gate/up tile spends an eighth of
+// vector unit (as kernels of eight waves the FP8 gate/up tile of 256 positions spent an eighth of
 // its time there): FP8 gate/up at 256 rows an expert 1366 -> 1326 us, Zipf T = 8192 2919 -> 2876; INT4 at 64 rows an expert 1490 -> 1461.
 __device__ __forceinline__ float silu_for_bf16(float g) {
   const float e = __builtin_amdgcn_exp2f(fmaf(g, -1.44269504088896341f, -2.f));

@@ -12,8 +12,8 @@
 // to the accumulator one after the other, the 16 x 16 x 32 one its four parts' in the same way, so two of the former (k = 16 s + 8 half)
 // are one of the latter (k = 8 part), bit for bit; and the former leaves the vector unit more of its issue slots (a loop with three
 // vector instructions a 16 x 16 x 32's worth: 17.6 against 23.1 clocks, without any 16.4 against 17.9).
-// A whole step runs these tiles in the routed experts' launches (pfi4::k_gemm), in front of them: as launches of their own they are
-// 16 and 24 workgroups a 128 rows, most of the chip idle. (Hidden 6144, intermediate 2048, 168 experts, kernels of eight waves, T = 1111:
+// A whole step runs these tiles in the routed experts' launches (pfi4::k_gemm), in front of them: as launches of their own (k_few, k_gemm) they
+// are 16 and 24 workgroups a 128 rows, most of the chip idle. (Hidden 6144, intermediate 2048, 168 experts, kernels of eight waves, T = 1111:
 // 1660 -> 1590 us; hidden 3840, intermediate 768, 16 experts, T = 200: 244 -> 134.)
 #pragma once
 #include "pf_gemm_fp8.cuh"
@@ -222,7 +222,7 @@ __global__ void __launch_bounds__(kThreads4, 2) k_gemm(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   tiles<UP>(g, smem, blockIdx.x);
 }
-// The rows in fewer tiles than the chip has CUs: one workgroup a CU, which has the CU's LDS for loads in flight.
+// The rows in no more tiles than the chip has CUs: one workgroup a CU, which has the CU's LDS for loads in flight.
 template <bool UP, int POS, int R>
 __global__ void __launch_bounds__(kThreads4, 2) k_few(Args g, pf8::Map map, int height) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];

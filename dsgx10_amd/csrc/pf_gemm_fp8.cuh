@@ -6,9 +6,9 @@
 // channels, gate and up): a wave owns 64 weight rows and every position. Two workgroups a CU, because their barriers, first loads
 // and epilogues are not each other's: as one workgroup of eight waves and 256 positions, a tile's first stage and epilogue (4 and
 // 12 of 84 us) and every wait for its slowest load left the CU idle (hidden 4096, intermediate 2048, 256 experts, whole call,
-// T = 8192: 2975 -> 2813 us; 3.45M -> 2.88M clocks of gate/up). What bounds it now is what L2 does not hold: 9.1 GB of lines missed
-// in gate/up at T = 8192 (4.3 of them the weights once), which come at 5.5 to 6 TB/s whatever their kind; the chip also lowers its
-// clock in this launch (1.75 GHz). Hence 160 positions and not 128 (an expert's weights are read again for each of its tiles: T = 3000
+// T = 8192: 2975 -> 2813 us; 3.45M -> 2.88M clocks of gate/up). What bounds it now is what L2 does not hold: 8.6 GB of lines missed
+// in gate/up at T = 8192 (4.3 of them the weights once), which come at 5.3 to 6 TB/s whatever their kind; the chip also lowers its
+// clock in this launch (1.8 GHz). Hence 160 positions and not 128 (an expert's weights are read again for each of its tiles: T = 3000
 // 1744 -> 1718, T = 8192 2858 -> 2836; 160 is what 256 registers a lane hold), and the scales' loads below.
 // Weights are the MFMA's A operand, so a lane's four accumulators of a 16 x 16 tile belong to ONE position and the
 // block's combined scale is one value a lane.
@@ -82,7 +82,8 @@ struct Map {
 };
 constexpr Map kMap{3, 2};
 // ... with as many row groups as divide NS: a block of fewer groups than the others always falls to the same XCDs where the blocks of a tile
-// are 2, 4 or 8 (ten row groups as 8 + 2: four XCDs with four times the others' work)
+// are 2, 4 or 8 (ten row groups as 8 + 2: four XCDs with four times the others' work; hidden 2560, intermediate 1280, 256 experts, as many groups as nl
+// says / this: FP8 T = 200 467 / 386 us, T = 1000 691 / 568, T = 8192 1237 / 1141, MXFP4 T = 4000 501 / 459, INT4 T = 200 337 / 313, T = 4000 989 / 921)
 __host__ __device__ inline Map map_of(int tl, int nl, int NS) {
   while (nl > 0 && NS % (1 << nl)) --nl;
   return Map{tl, nl};
@@ -98,9 +99,9 @@ __host__ __device__ inline unsigned grid_of(int tiles, int NS, Map m = kMap) {
   const int blocks = ((tiles + (1 << m.tl) - 1) >> m.tl) * ((NS + (1 << m.nl) - 1) >> m.nl);
   return ((unsigned)((blocks + kXcds - 1) / kXcds) * kXcds) << (m.tl + m.nl);
 }
-// TILE_MINOR: neighbouring workgroup numbers are neighbouring tiles of one row group (the dense GEMM of the shared expert,
-// where every tile streams the same weights: 0.241 against 0.250 ms at 8192 rows); else the row groups of one tile (the
-// routed experts' list: 1.63 against 1.75 ms for gate/up).
+// TILE_MINOR: neighbouring workgroup numbers are neighbouring tiles of one row group (the shared expert, whose tiles all stream the same
+// weights: in a whole call of 4096 x 2048, 64 experts, T = 2500 827 against 847 us, 256 experts, T = 8192 2762 / 2784; alone no difference); else the row
+// groups of one tile (the routed experts' list: 256 experts, T = 5000 / 8192 1977 / 2770 against 2067 / 2852).
 template <bool TILE_MINOR>
 __device__ __forceinline__ void task_of(int NS, int& tile, int& ns, unsigned wg = blockIdx.x, Map m = kMap) {
   const int x = wg % kXcds, j = wg / kXcds;

@@ -66,7 +66,9 @@ constexpr int loads_x(int pos) { return (pos + 31) / 32; }    // a wave's instru
 constexpr int young(bool pair, int pos, int i) { return stages(pos) == 2 ? loads(pair, i - 1) : loads(pair, i - 2) + loads_x(pos) + loads(pair, i - 1); }
 
 // Which workgroups share an XCD: four tiles x four row groups (gate/up with 8 / 64 / 224 rows an expert, eight tiles x four groups 622 / 756 /
-// 1846 us, one x eight 511 / 737 / 1924, this 512 / 748 / 1828).
+// 1846 us, one x eight 511 / 737 / 1924, this 512 / 748 / 1828; whole calls, this / 1 x 8 / 8 x 4 / 4 x 2: 6144 x 2048, 168 experts, T = 250 / 1200 / 2500 887 / 888 /
+// 897 / 893, 1413 / 1439 / 1421 / 1426, 2184 / 2219 / 2231 / 2233; 3072 x 1536, 48 experts, T = 250 / 1200 139 / 141 / 159 / 142, 295 / 305 / 304 / 306; 2048 x 768, 64
+// experts, T = 2500 175 / 179 / 186 / 175; 16 experts of 6144 x 2048, T = 250 219 / 220 / 214 / 201).
 __host__ __device__ inline pf8::Map map_of(int NS) { return pf8::map_of(2, 2, NS); }
 
 struct Args {
@@ -342,11 +344,8 @@ __device__ __forceinline__ void gemm_tile(const Args& g, uint8_t* smem, int e, i
 }
 
 // The routed experts' tiles, and in front of them (workgroups 0 .. sh_grid - 1) the BF16 shared expert's, if the launch holds those.
-// PAIR: K is an even number of 128-k blocks; only down has an odd number (up to 64 rows of one: in the 128-position shape every wave
-// fetches activations that nobody reads; whole call of hidden 2048, intermediate 384, 64 experts, T = 17 / 60: 69.5 / 75.7 us there, 68.1 /
-// 74.8 like this). A kernel of its own: as a third shape of one kernel it cost the others up to 1.3% (hidden 6144, intermediate 2048, 168
-// experts, T = 17 / 40 / 60: 396.5 / 551 / 685 us, 391.5 / 544 / 677.5 like this). The check of K under PAIR is always true; it is
-// there for the code that the compiler makes of it: without it 394 / 547.5 / 681.
+// PAIR: K is an even number of 128-k blocks; only down has an odd number. A kernel of its own: its shapes in the other's code cost
+// that up to 1.3% when a workgroup was eight waves.
 template <bool UP, bool PAIR>
 __global__ void __launch_bounds__(kThreads4, 2) k_gemm(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];

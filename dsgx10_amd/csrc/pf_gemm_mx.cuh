@@ -40,7 +40,7 @@ using pf8::wait_loads;
 //     turn, whole lines;
 //   * a line of scale words is a row's for 32 blocks and has left L2 when its next words are asked for: with four blocks' words a
 //     load scale words were 1.25 of the 5.7 GB; eight a load (the weight rows' in ONE buffer, which the wave frees by reading it) 5.3
-//     GB, gate/up 1022 -> 989 us;
+//     GB, gate/up 1022 -> 989 us (5.9 GB with the shared expert's tiles and the stores);
 //   * an expert of many rows reads its weights once a tile: 160 positions instead of 128 (T = 2000 / 6000 1280 -> 1246, 2100 -> 2013).
 // R > 0: the shared expert's shape for one workgroup a CU (k_few): weights and activations R turns ahead, and two buffers of the weight
 // rows' scale words.
@@ -431,7 +431,7 @@ __global__ void __launch_bounds__(kThreads4, 2) k_gemm(Args g) {
   if (ns >= NS || tile * 128 >= g.nrows) return;
   shared_tile<UP>(g, smem, tile * 128, g.nrows, ns);
 }
-// ... in fewer tiles than the chip has CUs: one workgroup a CU, which has the CU's LDS for loads in flight.
+// ... in no more tiles than the chip has CUs: one workgroup a CU, which has the CU's LDS for loads in flight.
 template <bool UP, int POS, int R>
 __global__ void __launch_bounds__(kThreads4, 2) k_few(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
@@ -455,7 +455,9 @@ __device__ __forceinline__ bool lower_tiles(const Args& g, int NS) {
   return r <= 2 && rounds(*g.ntiles_low) * kLowPos < r * kMaxPos;
 }
 // The routed experts' list of tiles, an expert's tiles next to each other.
-// A tile of up to 64 rows runs two blocks a turn where K is pairs of blocks.
+// A tile of up to 64 rows runs two blocks a turn where K is pairs of blocks; where K is an odd number (only down) every tile takes the
+// one shape without pairs (down of hidden 2048, intermediate 384, top-6 of 64, T = 17 / 100 / 600, whole call, kernels of eight waves with 128 positions for
+// those tiles / this: 41.7 / 50.2 / 80.3 and 30.3 / 43.1 / 62.9 us; 5120 x 1152, top-6 of 256, T = 40 / 250 / 1500 242 / 485 / 730 and 177 / 393 / 625).
 template <bool UP>
 __global__ void __launch_bounds__(kThreads4, 2) k_gemm_mixed(Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];

@@ -259,8 +259,8 @@ typedef struct dsgx_prefill_cfg {
   int32_t tile_order; /* FP8 activations only: the order in which the grouped GEMMs walk the tiles (the reference's
                        prefill_tuning tord, ds41f-4xgx10-switchless/engine/kernels/dsk.h:252, prefill.cu:658-668). 0: by
                        expert id, an expert's tiles next to each other; 1: the experts by falling count, their
-                       256-position tiles and the remainders merged evenly (tiles bound by the matrix unit beside tiles
-                       bound by the weight stream); 2: every 256-position tile first, then the remainders by falling
+                       full tiles (of 160 positions) and the remainders merged evenly (tiles bound by the matrix unit beside
+                       tiles bound by the weight stream); 2: every full tile first, then the remainders by falling
                        size; -1 (the default): the library's choice (0: on MI355X 1 and 2 measured no faster). The
                        results do not depend on it; a call that runs later phases alone names the same order as the
                        call that ran the bucketing (any order finds a valid list). */
@@ -320,9 +320,10 @@ DSGX_API int dsgx_add_norm_gemv(const dsgx_norm_in* n, int rows, int K, const ds
 DSGX_API int dsgx_dequant_int4(const void* packed, const void* scale, const void* zp, int N, int K, uint16_t* out,
                                size_t ld, void* stream);
 /* The same through the streaming kernels' own in-register decodes: the probes that pin the hot loops' INT4 arithmetic to
-   the contract bit for bit, as the reference's k_deq does (engine/experts/tests/test_experts.cu:217-235): the first the decode of
-   the matrix-unit kernels (prefill, decode variant 1), which takes the other's from 2^116 on; _any the decode of the
-   vector-unit kernels (dsgx_gemv, decode variant 0), at every scale. Bit-exact for
+   the contract bit for bit, as the reference's k_deq does (engine/experts/tests/test_experts.cu:217-235): the first the short decode,
+   of scales below 2^116: the matrix-unit kernels' (prefill, decode variant 1) and dsgx_gemv's, which do what met a larger scale once
+   more by the other (the probe takes the other from 2^116 on); _any the decode for every scale: decode variant 0, and
+   dsgx_gemv where waves of their own take a matrix's K slices or one wave walks them with eight rows. Bit-exact for
    positive scales below 2^124 (the checkpoint's are 2^-15 .. 2^-4; a negative scale, which the format forbids, gives
    +0 instead of -0 where u = u_z); dsgx_dequant_int4 is exact for every finite scale. */
 DSGX_API int dsgx_probe_dequant_int4(const void* packed, const void* scale, const void* zp, int N, int K, uint16_t* out,
