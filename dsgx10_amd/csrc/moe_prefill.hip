@@ -814,6 +814,7 @@ __global__ void __launch_bounds__(64) k_probe_mfma_bf16(const uint16_t* __restri
 //   FP8 4096 x 2048, T = 17 40.0 / 54.0 / 34.0, T = 200 79.8 / 84.6 / 36.7, T = 1000 95.9 / 89.1 / 48.8, T = 4000 118 / 135 / 110, T = 8192 231 / 240 / 219
 //   BF16 6144 x 2048, T = 17 57.4 / 86.5 / 56.2, T = 168 96 / 106 / 58, T = 672 102 / 110 / 81, T = 1111 138 / 139 / 132, T = 2500 235 / 227 / 233
 //   MXFP4's FP8 5120 x 2304, T = 17 33.9 / 46.0 / 39.5, T = 40 38.9 / 54 / 38.4, T = 200 90.7 / 64.9 / 39.0, T = 1000 104 / 74.5 / 75.7
+// (MXFP4's at up to 32 rows: 18 workgroups wait for a CU's share of the stream; four turns ahead are 38.3 us, and 20.5 instead of 19.1 at 2048 x 768.)
 // (FP8 tiles of up to 160 rows one a CU: 2304 x 1792 T = 2000 81 us, 47 like this; 2048 x 768, T = 6000 79 and 53.)
 template <class... A>
 int launch_alone(void (*k)(A...), unsigned grid, size_t lds, hipStream_t st, const A&... a) {
